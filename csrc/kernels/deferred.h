@@ -6,7 +6,8 @@
 // executor's backward runs, the finishing kernels can go to its side stream (the one running the
 // weight-gradient GEMMs) instead of sitting on the critical path: the side stream waits for the
 // producer with an event, and the partial buffers are recorded on it for the caching allocator.
-// set_deferred_reduce_stream(0) (the default) keeps everything on the current stream.
+// set_deferred_reduce_stream(0) (the default) keeps everything on the current stream. The choice is the calling
+// thread's: an executor on another thread has streams of its own to join.
 #pragma once
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -20,7 +21,7 @@ struct DeferredReduce {
   hipStream_t stream = nullptr;
   int device = 0;
 };
-DeferredReduce& deferred_reduce();  // defined in elementwise.hip
+DeferredReduce& deferred_reduce();  // this thread's; defined in elementwise.hip
 
 // out[a][c] += Σ_g part[a][g][c] for a < A (part fp32 [A][G][C]); on the deferred stream if set
 inline void reduce_partials_auto(const torch::Tensor& part, int A, int G, int C, float* const* outs, hipStream_t cur) {

@@ -732,7 +732,7 @@ std::vector<torch::Tensor> tensor_stats(torch::Tensor x, int64_t bins) {
 
 namespace penroz {
 DeferredReduce& deferred_reduce() {
-  static DeferredReduce d;
+  static thread_local DeferredReduce d;
   return d;
 }
 }  // namespace penroz
@@ -742,3 +742,5 @@ void set_deferred_reduce_stream(int64_t stream, int64_t device) {
   penroz::deferred_reduce().stream = reinterpret_cast<hipStream_t>(stream);
   penroz::deferred_reduce().device = (int)device;
 }
+
+int64_t get_deferred_reduce_stream() { return reinterpret_cast<int64_t>(penroz::deferred_reduce().stream); }

@@ -844,9 +844,11 @@ class GPTExecutor:
             stale.clear()
 
     def _defer_reductions(self, on: bool):
-        """LayerNorm / bias column-reduction finishing kernels go to the side stream (on) or not."""
-        if getattr(self, "_side", None) is not None:
-            _ext.kernels().set_deferred_reduce_stream(self._side.cuda_stream if on else 0, self.device.index or 0)
+        """LayerNorm / bias column-reduction finishing kernels go to the side stream (on) or not. A step without a side
+        stream says so too: whatever ran before on this thread, its reductions stay on the main stream."""
+        if self.device.type == "cuda":
+            side = self._side if on else None
+            _ext.kernels().set_deferred_reduce_stream(0 if side is None else side.cuda_stream, self.device.index or 0)
 
     def _reuse(self, buf: Tensor) -> Tensor:
         """Main stream: wait until the side stream no longer reads ``buf`` (before overwriting)."""
@@ -886,6 +888,12 @@ class GPTExecutor:
                 self._opt_mode = "per-bucket-in-backward" if self._opt_bucketed else None
         try:
             loss = self._train_micro_step(idx, targets, scale, sync, capture)
+        except BaseException:
+            # the next step may be of one stream: nothing stays deferred, and the main stream (its allocations too)
+            # comes behind what the side stream still has to do
+            self._defer_reductions(False)
+            self._join_side()
+            raise
         finally:
             self._opt_done = self._opt_apply is not None
             self._opt_apply = None

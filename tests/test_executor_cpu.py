@@ -195,3 +195,66 @@ def test_zero_gap_minus_skip_range():
     assert _minus([(0, 10)], (0, 10)) == []
     assert _minus([(0, 100)], (40, 60)) == [(0, 40), (60, 100)]
     assert _minus([(10, 20)], (30, 40)) == [(10, 20)]
+
+
+class _Stream:
+    """A stream that notes what waits for what."""
+
+    def __init__(self, cuda_stream, log):
+        self.cuda_stream, self.log = cuda_stream, log
+
+    def wait_stream(self, other):
+        self.log.append((self.cuda_stream, other.cuda_stream))
+
+
+def test_a_failed_step_defers_nothing_to_the_next(monkeypatch):
+    """A step on two streams that raises in its backward, then one on a single stream: the second step's reductions stay
+    on the main stream, which has waited for the side stream."""
+    from types import SimpleNamespace
+
+    import torch
+    from penroz.models import executor
+    waits, deferred = [], []
+    main = _Stream(1, waits)
+    monkeypatch.setattr(executor._ext, "kernels", lambda: SimpleNamespace(
+        set_deferred_reduce_stream=lambda stream, device: deferred.append(stream)))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: main)
+    ex = GPTExecutor.__new__(GPTExecutor)
+    ex.device, ex.flat, ex._opt_flat, ex.reducer = torch.device("cuda", 0), torch.empty(10), False, None
+    ex._side_stream, ex._buf_free, seen = _Stream(7, waits), {1: "event"}, []
+
+    def micro(idx, targets, scale, sync, capture):
+        ex._plan_step(idx.numel())
+        ex._defer_reductions(True)
+        seen.append(deferred[-1] if deferred else 0)
+        if ex._side is not None:
+            raise MemoryError("in the backward")
+        ex._defer_reductions(False)
+        ex._join_side()
+
+    ex._train_micro_step = micro
+    ex.SIDE_MIN_FLOPS = 6 * 100 * 10
+    with pytest.raises(MemoryError):
+        ex.train_micro_step(torch.empty(4, 64), None, 1.0)
+    assert deferred[-1] == 0 and waits == [(1, 7)] and not ex._buf_free
+    deferred.append(7)  # whatever was left of it
+    ex.train_micro_step(torch.empty(1, 64), None, 1.0)
+    assert seen == [7, 0] and deferred[-1] == 0
+
+
+def test_deferred_reductions_are_a_threads_own():
+    """One thread's executor defers its reductions, another's does not."""
+    import threading
+
+    from penroz.ops import _ext
+    if not _ext.available("penroz_kernels"):
+        pytest.skip("extension not built")
+    k, seen = _ext.kernels(), []
+    k.set_deferred_reduce_stream(64, 0)
+    try:
+        t = threading.Thread(target=lambda: seen.append(k.get_deferred_reduce_stream()))
+        t.start()
+        t.join()
+        assert seen == [0] and k.get_deferred_reduce_stream() == 64
+    finally:
+        k.set_deferred_reduce_stream(0, 0)
