@@ -328,6 +328,33 @@ def test_experts(target, N, E, top, C, F, spread):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("dt,N", [(torch.float32, 300), (torch.bfloat16, 300), (torch.bfloat16, 1300)])
+def test_gated_activations_over_the_whole_range(kind, dt, N):
+    """Gates down to where exp(-g) is the largest finite value: every result within what fp32 exp, add and divide round
+    (a reciprocal there is subnormal, which the hardware's approximate one returns as zero)."""
+    z = torch.linspace(-88.5, 30, N).to(dt).float() / (1.702 if kind else 1.0)
+    h = torch.zeros(N, 32)
+    h[:, 0], h[:, 1] = z, 1.0
+    h = h.to(dt)
+    z = h[:, 0].double()
+    g, u, d = torch.zeros(1, 32, 32), torch.zeros(1, 32, 32), torch.eye(32)[None]
+    g[:, :, 0], u[:, :, 1] = 1.0, 1.0  # every product one term: exact
+    limit = 40.0
+    s = 1.702 * z if kind else z
+    want = (z * torch.sigmoid(s) * (2 if kind else 1))[:, None]
+    bound = (2 * s.abs() + 8)[:, None] * 2.0 ** -24 + (0 if dt == torch.float32 else 2.0 ** -8)
+    w = {k: v.cuda() for k, v in P.pack_experts(g.to(dt), u.to(dt), d.to(dt)).items()}
+    got = [P.experts(h.cuda(), torch.zeros(N, 1, dtype=torch.int32, device="cuda"), w, kind, limit)]
+    if kind == 1:
+        got.append(P.gated_linear(h.cuda(), torch.cat([g[0], u[0]]).to(dt).cuda(), kind, limit))
+    for y in got:
+        e = (y.double().cpu() - want).abs() / want.abs().clamp_min(1e-300)
+        e[z == 0] = 0
+        assert bool((e <= bound).all()), (e / bound).max()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("kind", [0, 1, P.UNGATED])
 @pytest.mark.parametrize("C,F", [(544, 288), (576, 512)])
 def test_experts_in_large_tiles(kind, C, F):
