@@ -416,80 +416,39 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
   // a lane or behind an earlier load's use: with the residual, delta and bias of each chunk added as they came, and
   // γ, β and the bias loaded where they were needed, a LayerNorm kernel spent five memory round trips one after the
   // other (GPT-2 B = 1: 6.8 us against 3.6 for the same bytes without it).
+  // Where all of that is more than 256 registers, one wave per SIMD (the estimate is the compiler's count within 15), the
+  // weights come first and the LayerNorm's operands a row of x at a time (all at once / so, us: 4 rows of x, K 768,
+  // N 50257 52.6 / 42.9; 3 rows, K 1024 64.1 / 44.4; but 3 rows, K 768, 245 registers, 29.7 / 36.6).
+  constexpr bool EARLY = CPL * (28 + 12 * M + 5 * RP) <= 260;
   int cc[CPL];  // chunks past the row are read from its last one and count as zero
 #pragma unroll
   for (int i = 0; i < CPL; ++i) cc[i] = min(cl + CS * i, nc - 1);
-  float v[LN ? M : 1][LN ? CPL : 1][8];
-  float4_t gm[LN ? CPL : 1][2], bt4[LN ? CPL : 1][2], r4[LN ? M : 1][LN ? CPL : 1][2], db4[LN ? CPL : 1][2];
-  uint4 d8[LN ? M : 1][LN ? CPL : 1], e8[LN ? M : 1][LN ? CPL : 1];
-  if constexpr (LN) {
-    if (ewte) {  // embedding mode: the residual row is wte[token] + wpe[position] (the first block of a decode
-                 // step, embed_fwd_kernel's arithmetic: clamped token, position min(*epos, P - 1))
-      const int epos_v = min((int)*epos, eP - 1);
+  uint4 wv[RP][CPL], xb[M][CPL];
+  auto weights = [&]() {
 #pragma unroll
-      for (int m = 0; m < M; ++m) {
-        int64_t tok = eidx[m];
-        tok = tok < 0 ? 0 : (tok >= eV ? eV - 1 : tok);
+    for (int rp = 0; rp < RP; ++rp) {
+      const bf16* wr = w + (size_t)row_of(rp) * K;
 #pragma unroll
-        for (int i = 0; i < CPL; ++i) {
-          d8[m][i] = *reinterpret_cast<const uint4*>(ewte + (size_t)tok * K + 8 * cc[i]);
-          e8[m][i] = *reinterpret_cast<const uint4*>(ewpe + (size_t)epos_v * K + 8 * cc[i]);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int m = 0; m < M; ++m)
-#pragma unroll
-        for (int i = 0; i < CPL; ++i) {
-          const float4_t* rp = reinterpret_cast<const float4_t*>(rin + (size_t)m * K + 8 * cc[i]);
-          r4[m][i][0] = rp[0];
-          r4[m][i][1] = rp[1];
-        }
-      if (delta) {
-#pragma unroll
-        for (int m = 0; m < M; ++m)
-#pragma unroll
-          for (int i = 0; i < CPL; ++i) d8[m][i] = *reinterpret_cast<const uint4*>(delta + (size_t)m * K + 8 * cc[i]);
-      }
-      if (dbias) {
-#pragma unroll
-        for (int i = 0; i < CPL; ++i) {
-          const float4_t* e = reinterpret_cast<const float4_t*>(dbias + 8 * cc[i]);
-          db4[i][0] = e[0];
-          db4[i][1] = e[1];
-        }
+      for (int i = 0; i < CPL; ++i) {
+        const int c = cl + CS * i;
+        wv[rp][i] = c < nc ? *reinterpret_cast<const uint4*>(wr + 8 * c) : uint4{0u, 0u, 0u, 0u};
       }
     }
-#pragma unroll
-    for (int i = 0; i < CPL; ++i) {
-      const float4_t* gp = reinterpret_cast<const float4_t*>(gamma + 8 * cc[i]);
-      const float4_t* bp = reinterpret_cast<const float4_t*>(beta + 8 * cc[i]);
-      gm[i][0] = gp[0];
-      gm[i][1] = gp[1];
-      bt4[i][0] = bp[0];
-      bt4[i][1] = bp[1];
-    }
-  }
+  };
   float bias_v[RP];  // (paired rows have none)
 #pragma unroll
   for (int rp = 0; rp < RP; ++rp) bias_v[rp] = 0.f;
-  if constexpr (EPI == 0 || WR) {
-    if (bias) {
+  auto biases = [&]() {
+    if constexpr (EPI == 0 || WR) {
+      if (bias) {
 #pragma unroll
-      for (int rp = 0; rp < RP; ++rp) bias_v[rp] = bf2f(bias[row_of(rp)]);
+        for (int rp = 0; rp < RP; ++rp) bias_v[rp] = bf2f(bias[row_of(rp)]);
+      }
     }
-  }
-  uint4 wv[RP][CPL], xb[M][CPL];
-#pragma unroll
-  for (int rp = 0; rp < RP; ++rp) {
-    const bf16* wr = w + (size_t)row_of(rp) * K;
-#pragma unroll
-    for (int i = 0; i < CPL; ++i) {
-      const int c = cl + CS * i;
-      wv[rp][i] = c < nc ? *reinterpret_cast<const uint4*>(wr + 8 * c) : uint4{0u, 0u, 0u, 0u};
-    }
-  }
+  };
   if constexpr (!LN) {
+    biases();
+    weights();
 #pragma unroll
     for (int m = 0; m < M; ++m)
 #pragma unroll
@@ -498,28 +457,96 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
         xb[m][i] = c < nc ? *reinterpret_cast<const uint4*>(x + (size_t)m * x_rs + 8 * c) : uint4{0u, 0u, 0u, 0u};
       }
   } else {
+    // a chunk's values before they are added: the fp32 residual (or in embedding mode the position row's 16 bytes in
+    // its first piece), then delta (the token's row)
+    typedef uint32_t raw4 __attribute__((ext_vector_type(4)));
+    constexpr int ME = EARLY ? M : 1;
+    raw4 r4[ME][CPL][2], d4[ME][CPL];
+    float4_t db4[CPL][2], gm[CPL][2], bt4[CPL][2];
+    float v[M][CPL][8];
+    const int epos_v = ewte ? min((int)*epos, eP - 1) : 0;
+    auto load_row = [&](int m) {
+      const int q = EARLY ? m : 0;
+      if (ewte) {  // embedding mode: the residual row is wte[token] + wpe[position] (the first block of a decode
+                   // step, embed_fwd_kernel's arithmetic: clamped token, position min(*epos, P - 1))
+        int64_t tok = eidx[m];
+        tok = tok < 0 ? 0 : (tok >= eV ? eV - 1 : tok);
 #pragma unroll
-    for (int m = 0; m < M; ++m)
+        for (int i = 0; i < CPL; ++i) {
+          d4[q][i] = *reinterpret_cast<const raw4*>(ewte + (size_t)tok * K + 8 * cc[i]);
+          r4[q][i][0] = *reinterpret_cast<const raw4*>(ewpe + (size_t)epos_v * K + 8 * cc[i]);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) {
+          const raw4* rp = reinterpret_cast<const raw4*>(rin + (size_t)m * K + 8 * cc[i]);
+          r4[q][i][0] = rp[0];
+          r4[q][i][1] = rp[1];
+        }
+        if (delta) {
+#pragma unroll
+          for (int i = 0; i < CPL; ++i) d4[q][i] = *reinterpret_cast<const raw4*>(delta + (size_t)m * K + 8 * cc[i]);
+        }
+      }
+    };
+    auto add_row = [&](int m) {
+      const int q = EARLY ? m : 0;
 #pragma unroll
       for (int i = 0; i < CPL; ++i) {
         const bool ok = l32 + 32 * i < nc;
-        const uint32_t dw[4] = {d8[m][i].x, d8[m][i].y, d8[m][i].z, d8[m][i].w};
-        const uint32_t ew[4] = {e8[m][i].x, e8[m][i].y, e8[m][i].z, e8[m][i].w};
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-          const auto half16 = [&](const uint32_t* u) {
+          const auto half16 = [&](const raw4& u) {
             return __uint_as_float(k & 1 ? u[k >> 1] & 0xffff0000u : u[k >> 1] << 16);
           };
           float r;
           if (ewte) {
-            r = half16(dw) + half16(ew);
+            r = half16(d4[q][i]) + half16(r4[q][i][0]);
           } else {
-            r = r4[m][i][k >> 2][k & 3];
-            if (delta) r += dbias ? half16(dw) + db4[i][k >> 2][k & 3] : half16(dw);
+            r = __uint_as_float(r4[q][i][k >> 2][k & 3]);
+            if (delta) r += dbias ? half16(d4[q][i]) + db4[i][k >> 2][k & 3] : half16(d4[q][i]);
           }
           v[m][i][k] = ok ? r : 0.f;
         }
       }
+    };
+    auto load_dbias = [&]() {
+      if (dbias) {
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) {
+          const float4_t* e = reinterpret_cast<const float4_t*>(dbias + 8 * cc[i]);
+          db4[i][0] = e[0];
+          db4[i][1] = e[1];
+        }
+      }
+    };
+    auto scales = [&](int i) {
+      const float4_t* gp = reinterpret_cast<const float4_t*>(gamma + 8 * cc[i]);
+      const float4_t* bp = reinterpret_cast<const float4_t*>(beta + 8 * cc[i]);
+      gm[i][0] = gp[0];
+      gm[i][1] = gp[1];
+      bt4[i][0] = bp[0];
+      bt4[i][1] = bp[1];
+    };
+    if constexpr (EARLY) {
+#pragma unroll
+      for (int m = 0; m < M; ++m) load_row(m);
+      load_dbias();
+#pragma unroll
+      for (int i = 0; i < CPL; ++i) scales(i);
+      biases();
+      weights();
+#pragma unroll
+      for (int m = 0; m < M; ++m) add_row(m);
+    } else {
+      weights();
+      load_dbias();
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        load_row(m);
+        add_row(m);
+      }
+    }
     if ((delta || ewte) && rout && blockIdx.x == 0 && h == 0) {
 #pragma unroll
       for (int m = 0; m < M; ++m)
@@ -561,6 +588,7 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
 #pragma unroll
     for (int i = 0; i < CPL; ++i) {
       const bool ok = l32 + 32 * i < nc;
+      if constexpr (!EARLY) scales(i);
 #pragma unroll
       for (int m = 0; m < M; ++m) {
         float y[8];
@@ -572,6 +600,7 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
       }
     }
   }
+  if constexpr (LN && !EARLY) biases();
   // 2. products and the half-wave reductions
   float acc[RP][M];
 #pragma unroll
@@ -585,7 +614,7 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
       if constexpr (WR) a += other_half(a, h);
       acc[rp][m] = a;
     }
-  // 3. epilogue: lane 0 of each half stores its rows
+  // 3. epilogue
   if constexpr (WR) {
     if (lane != 0) return;
 #pragma unroll
@@ -629,18 +658,17 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
     }
     return;
   }
-  if (l32 != 0) return;
+  // a lane per output: one after the other on one lane the activations of 8 rows, 4 of x, take as long as the loads
+  static_assert(RP * M <= 32, "");
+  float mine = 0.f;
 #pragma unroll
-  for (int rp = 0; rp < RP; ++rp) {
-    const int n = n0 + 2 * rp + h;
-    if (n >= N) continue;
+  for (int rp = 0; rp < RP; ++rp)
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
-      float y = acc[rp][m] + bias_v[rp];
-      if (act) y = gelu_f(bf2f(from_f<bf16>(y)), act - 1);
-      out[(size_t)m * o_rs + n] = from_f<bf16>(y);
-    }
-  }
+    for (int m = 0; m < M; ++m) mine = l32 == rp * M + m ? acc[rp][m] + bias_v[rp] : mine;
+  const int n = n0 + 2 * (l32 / M) + h;
+  if (l32 >= RP * M || n >= N) return;
+  if (act) mine = gelu_f(bf2f(from_f<bf16>(mine)), act - 1);
+  out[(size_t)(l32 % M) * o_rs + n] = from_f<bf16>(mine);
 }
 
 }  // namespace penroz
@@ -842,8 +870,8 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
   int rpw = (int)rows_per_wave;
   // by shape: the vocabulary projection wants fewer, longer-lived waves (8 rows); behind a LayerNorm 4 rows, since every
   // wave reads and normalises the whole operand again (2 / 4 / 8 rows, us: K 768, N 2304, one row of x 4.8 / 4.2 / 4.3,
-  // four 10.4 / 8.8 / 9.7; K 1024, N 4096 7.0 / 5.3 / 5.1 and 24.2 / 13.8 / 13.2); else 2 rows per wave — the most
-  // workgroups in flight. PENROZ_DECODE_GEMV_RPW forces 2 / 4 / 8 below 16k rows (A/B).
+  // four 10.5 / 9.0 / 8.8; K 1024, N 4096 6.7 / 5.3 / 4.9 and 13.8 / 12.1 / 12.0; K 512, N 512 3.1 / 3.2 / 3.3); else 2
+  // rows per wave — the most workgroups in flight. PENROZ_DECODE_GEMV_RPW forces 2 / 4 / 8 below 16k rows (A/B).
   static const int rpw_env = [] {
     const char* e = std::getenv("PENROZ_DECODE_GEMV_RPW");
     return e ? std::atoi(e) : 0;
@@ -909,17 +937,15 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
     }
     if (ln) {
       TORCH_CHECK(cpl <= 4, "decode_gemv: LN mode needs K <= 1024");
-      // LN mode instantiates only the small chunk counts (K <= 1024)
-      if (RPv == 1) {
-        if (cpl <= 3) launch(mt, std::true_type{}, std::integral_constant<int, 1>{}, std::integral_constant<int, 3>{});
-        else launch(mt, std::true_type{}, std::integral_constant<int, 1>{}, std::integral_constant<int, 4>{});
-      } else if (RPv == 2) {
-        if (cpl <= 3) launch(mt, std::true_type{}, std::integral_constant<int, 2>{}, std::integral_constant<int, 3>{});
-        else launch(mt, std::true_type{}, std::integral_constant<int, 2>{}, std::integral_constant<int, 4>{});
-      } else {
-        if (cpl <= 3) launch(mt, std::true_type{}, std::integral_constant<int, 4>{}, std::integral_constant<int, 3>{});
-        else launch(mt, std::true_type{}, std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
-      }
+      auto by_chunks = [&](auto rpt) {  // K <= 1024
+        if (cpl <= 1) launch(mt, std::true_type{}, rpt, std::integral_constant<int, 1>{});
+        else if (cpl <= 2) launch(mt, std::true_type{}, rpt, std::integral_constant<int, 2>{});
+        else if (cpl <= 3) launch(mt, std::true_type{}, rpt, std::integral_constant<int, 3>{});
+        else launch(mt, std::true_type{}, rpt, std::integral_constant<int, 4>{});
+      };
+      if (RPv == 1) by_chunks(std::integral_constant<int, 1>{});
+      else if (RPv == 2) by_chunks(std::integral_constant<int, 2>{});
+      else by_chunks(std::integral_constant<int, 4>{});
     } else {
       by_rp(mt, std::false_type{});
     }

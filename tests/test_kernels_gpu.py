@@ -1232,6 +1232,38 @@ def test_decode_gemv_ln(M, K, N, act, with_delta, rpw):
         _close(rout, s, 1e-6, 1e-6, "resid_out")
 
 
+@pytest.mark.parametrize("K", [8, 248, 264, 512, 768, 1016, 1024])
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("emb", [False, True])
+def test_decode_gemv_ln_forms(K, M, emb):
+    """LN mode with every chunk count, operands all held at once or a row of x at a time: the same bits at 2, 4 and 8
+    rows per wave (one order of every sum), within rounding of fp32 torch."""
+    torch.manual_seed(K + M)
+    k, N = _ext.kernels(), 45
+    gamma, beta = torch.randn(K, device=DEV), torch.randn(K, device=DEV)
+    w = (torch.randn(N, K, device=DEV) / K ** 0.5).to(torch.bfloat16)
+    b = torch.randn(N, device=DEV).to(torch.bfloat16)
+    if emb:
+        wte, wpe = (torch.randn(9, K, device=DEV).to(torch.bfloat16) for _ in range(2))
+        idx, pos = torch.tensor([8, 0, 3, 11][:M], device=DEV), torch.tensor([12], device=DEV)  # (past the ends: the last row)
+        s, rin, delta, dbias = wte[idx.clamp(max=8)].float() + wpe[8].float(), None, None, None
+        tail = (idx, wte, wpe, pos)
+    else:
+        rin, dbias = torch.randn(M, K, device=DEV) * 2 + 0.5, torch.randn(K, device=DEV)
+        delta = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+        s, tail = rin + (delta.float() + dbias), ()
+    got = []
+    for rpw in (2, 4, 8):
+        rout, out = torch.empty(M, K, device=DEV), torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+        k.decode_gemv(None, rin, delta, dbias, rout, gamma, beta, 1e-5, w, b, out, 2, rpw, *tail)
+        _close(rout, s, 1e-6, 1e-6, "resid_out")
+        got.append(out)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+    y = F.layer_norm(s, (K,), gamma, beta, 1e-5).to(torch.bfloat16).float()
+    ref = F.gelu((y @ w.float().t() + b.float()).to(torch.bfloat16).float(), approximate="tanh")
+    _close(got[0], ref, 2e-2, 2e-2, "out")
+
+
 @pytest.mark.parametrize("M,K,N", [(1, 768, 768), (1, 3072, 768), (4, 768, 50304), (2, 6912, 1152), (3, 40, 33),
                                    (1, 8192, 16)])
 @pytest.mark.parametrize("rpw", [0, 2, 4, 8])
