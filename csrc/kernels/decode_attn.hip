@@ -558,15 +558,16 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
     for (int s2 = 0; s2 < KS; ++s2)
       sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[s2]),
                                                      __builtin_bit_cast(bf16x8_t, qf[s2]), sacc, 0, 0, 0);
+    const int nk = min(16, k1 - kb);
     float vf[4][4];  // this block's V values (fp32), taken before the next block's loads land
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
+      if (4 * qd + j >= nk) vraw[j] = uint2{0u, 0u};  // (the last key's row again, whose infinities count once)
       vf[j][0] = __uint_as_float(vraw[j].x << 16);
       vf[j][1] = __uint_as_float(vraw[j].x & 0xffff0000u);
       vf[j][2] = __uint_as_float(vraw[j].y << 16);
       vf[j][3] = __uint_as_float(vraw[j].y & 0xffff0000u);
     }
-    const int nk = min(16, k1 - kb);
     if (kb + 16 < k1) load_block(kb + 16);
     // scores of keys kb + 4qd + r for head r16 (masked past the wave's range)
     float sc[4], bmax = -INFINITY;
@@ -577,12 +578,12 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
     }
     bmax = fmaxf(bmax, lane_xor16(bmax, qd & 1));
     bmax = fmaxf(bmax, lane_xor32(bmax, qd >> 1));
-    const float mn = fmaxf(m, bmax);
+    const float mn = fmaxf(m, bmax), base = mn == -INFINITY ? 0.f : mn;  // (no score above -inf yet: nothing counts)
     const float alpha = m == -INFINITY ? 0.f : exp2f(m - mn);
     float ps = 0.f;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const float pv = exp2f(sc[r] - mn);
+      const float pv = exp2f(sc[r] - base);
       ps += pv;
       pl[w][4 * qd + r][r16] = pv;
     }

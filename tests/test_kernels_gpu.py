@@ -913,6 +913,24 @@ def test_decode_attention_small_edges(B, H, Hkv, D, S):
     assert torch.equal(kc[:, :, :S], want[0]) and torch.equal(vc[:, :, :S], want[1])
 
 
+@pytest.mark.parametrize("H,Hkv,D", [(3, 3, 64), (4, 1, 256), (8, 4, 128)])
+@pytest.mark.parametrize("S", [33, 70, 300])
+def test_decode_attention_small_infinities(H, Hkv, D, S):
+    """Keys whose scores are -inf (a whole block of them first) weigh nothing beside finite ones, and an infinite value
+    of the last key reaches its own column only, wherever the last block ends."""
+    torch.manual_seed(S)
+    q, cap = torch.randn(1, 1, H, D, device=DEV).bfloat16(), 512
+    kc, vc = (torch.randn(1, Hkv, cap, D, device=DEV).bfloat16() for _ in range(2))
+    q[..., 0], kc[..., 0] = 1e20, 0.0
+    kc[:, :, :32, 0] = -1e38
+    vc[:, :, S - 1, 3] = float("inf")
+    out = A.decode_attention(q, kc, vc, S).view(1, H, D)
+    ref = A.reference_cache_attention(q.double(), kc[:, :, 32:S].double(), vc[:, :, 32:S].double(), S - 33).view(1, H, D)
+    assert torch.isinf(out[..., 3]).all() and torch.isinf(ref[..., 3]).all()
+    out[..., 3], ref[..., 3] = 0, 0
+    _close(out, ref, 0.02, 0.01)
+
+
 @pytest.mark.parametrize("B,H,Hkv,D,S", [(64, 4, 1, 256, 1), (64, 4, 1, 256, 700), (17, 4, 1, 256, 1024),
                                           (3, 8, 2, 128, 40), (2, 8, 2, 128, 300), (5, 8, 4, 64, 77)])
 def test_decode_attention_rope_in_kernel(B, H, Hkv, D, S):
