@@ -754,7 +754,7 @@ torch::Tensor decode_attn(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, c
   TORCH_CHECK(!quant || (k_scale.has_value() && v_scale.has_value()), "int8 cache needs scales");
   TORCH_CHECK(quant || kc.scalar_type() == q.scalar_type(), "cache dtype must match q");
   auto out = torch::empty({B, Tq, H * D}, q.options());
-  const int64_t q_rs = Tq == 1 ? q.stride(0) : q.stride(1);
+  int64_t q_rs = Tq == 1 ? q.stride(0) : q.stride(1);
   const int items = B * Hkv * Tq;
   // keys per split (each workgroup sweeps its keys in chunks of 256; a graph captures S = the cache
   // capacity and the kernel stops at the device-side length). With zeroed arrival counters
@@ -818,6 +818,11 @@ torch::Tensor decode_attn(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, c
   const float* rsp = rope ? rope_sin->data_ptr<float>() : nullptr;
   if (small) {
     const int G0 = H / Hkv;
+    // it reads the queries 16 bytes at a time (the general kernel one by one)
+    if (q_rs % 8 != 0 || reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 != 0) {
+      q = q.clone(at::MemoryFormat::Contiguous);
+      q_rs = q.stride(0);
+    }
     const bf16* qp = reinterpret_cast<const bf16*>(q.data_ptr());
     bf16* kp = reinterpret_cast<bf16*>(kc.data_ptr());
     bf16* vp = reinterpret_cast<bf16*>(vc.data_ptr());

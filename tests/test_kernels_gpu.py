@@ -931,6 +931,17 @@ def test_decode_attention_small_infinities(H, Hkv, D, S):
     _close(out, ref, 0.02, 0.01)
 
 
+@pytest.mark.parametrize("H,D", [(3, 64), (2, 256)])
+@pytest.mark.parametrize("pad,off", [(0, 4), (3, 0), (5, 1)])
+def test_decode_attention_of_unaligned_queries(H, D, pad, off):
+    """Query rows that lie anywhere in wider rows: the same bits as from rows of their own."""
+    torch.manual_seed(pad)
+    rows = torch.randn(3 * (H * D + pad) + off, device=DEV).bfloat16()
+    q = rows[off:].view(3, -1)[:, :H * D].unflatten(1, (H, D))[:, None]
+    kc, vc = (torch.randn(3, H, 256, D, device=DEV).bfloat16() for _ in range(2))
+    assert torch.equal(A.decode_attention(q, kc, vc, 201), A.decode_attention(q.clone(), kc, vc, 201))
+
+
 @pytest.mark.parametrize("B,H,Hkv,D,S", [(64, 4, 1, 256, 1), (64, 4, 1, 256, 700), (17, 4, 1, 256, 1024),
                                           (3, 8, 2, 128, 40), (2, 8, 2, 128, 300), (5, 8, 4, 64, 77)])
 def test_decode_attention_rope_in_kernel(B, H, Hkv, D, S):
