@@ -414,8 +414,8 @@ __global__ void __launch_bounds__(256) decode_kernel(const TQ* __restrict__ q, c
   }
 }
 
-// Small-batch decode attention (bf16 cache, one query row, query group G <= 16): D / 64 workgroups
-// per (batch, KV head), each for 64 of the output columns — no split-K launch, no hand-over between
+// Small-batch decode attention (bf16 cache, one query row, query group G <= 16): D / DC workgroups
+// per (batch, KV head), each for DC of the output columns — no split-K launch, no hand-over between
 // workgroups, no barrier inside the key loop. Each computes all the scores; its 8 waves own a
 // contiguous eighth of the keys. Per 16-key block a wave computes the scores of all G heads with
 // v_mfma_f32_16x16x32_bf16 (A = 16 K rows straight from global memory, B = the group's queries,
@@ -426,7 +426,9 @@ __global__ void __launch_bounds__(256) decode_kernel(const TQ* __restrict__ q, c
 // Bound by what one CU can read and by a wave's blocks one after the other, so the keys go over 8
 // waves and V over D / 64 workgroups, whose K rows meet in the L2 of one XCD (they are 8 apart in
 // the grid). 232 keys, D = 256, G = 4, 3 rows: 12.6 us with
-// one workgroup of 4 waves per item, 11.4 with 8 waves, 9.0 so. Made for the batch-1 GQA shapes where the
+// one workgroup of 4 waves per item, 11.4 with 8 waves, 9.0 so. 128 columns where 64 would make more workgroups than
+// CUs (D = 512, more than 32 items; G <= 4, for the registers): 64 items, 200 keys, G = 1 16.1 us with one workgroup of
+// 4 waves per item, 19.8 / 12.1 with 64 / 128 columns. Made for the batch-1 GQA shapes where the
 // general kernel's thread-per-key loop is serial (Gemma-3 1B: G = 4, D = 256 — 19 µs per layer).
 // Fused append as in decode_kernel: key S-1 comes from k_new / v_new and is written to the cache.
 // rc / rs (optional, fp32 [D/2]: this step's RoPE cos / sin): the query and the new key arrive
@@ -435,8 +437,9 @@ __global__ void __launch_bounds__(256) decode_kernel(const TQ* __restrict__ q, c
 // the same lane, so the rotation stays in registers.
 // ROPE is a template flag so the default instantiations compile exactly as without it (as a run-time
 // branch it cost the D = 512 kernels 320 B/lane of scratch).
-constexpr int kSmallWaves = 8, kSmallCols = 64;
-template <int D, int GMAX, bool ROPE = false>  // GMAX: the exact query-group size H / Hkv
+constexpr int kSmallWaves = 8;
+// GMAX: the exact query-group size H / Hkv; DC: output columns per workgroup
+template <int D, int GMAX, bool ROPE = false, int DC = 64>
 __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf16* __restrict__ q, bf16* __restrict__ kc,
                                                            bf16* __restrict__ vc, bf16* __restrict__ out, int items,
                                                            int H, int Hkv, int cap, int S, float scale,
@@ -446,11 +449,11 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
                                                            const float* __restrict__ rc,
                                                            const float* __restrict__ rs) {
   constexpr int KS = D / 32;   // MFMA k-steps per score block
-  constexpr int CG = D / kSmallCols;  // workgroups of an item
+  constexpr int CG = D / DC, CL = DC / 64;  // workgroups of an item, quads of output columns per lane
   static_assert(CG >= 1 && GMAX <= 16, "decode_small geometry");
   typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
   typedef float f32x4_t __attribute__((ext_vector_type(4)));
-  constexpr int G = GMAX, NW = kSmallWaves, DC = kSmallCols;
+  constexpr int G = GMAX, NW = kSmallWaves;
   const int item = blockIdx.x / (8 * CG) * 8 + blockIdx.x % 8, cg = blockIdx.x / 8 % CG;
   if (item >= items) return;
   const int g = item % Hkv, b = item / Hkv;
@@ -504,14 +507,14 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
   const int per = (S + 16 * NW - 1) / (16 * NW) * 16;  // 16-key blocks, an equal share each
   const int k0 = w * per, k1 = min(S, k0 + per);
   float m = -INFINITY, l = 0.f;  // for head r16 (replicated over qd)
-  float o[GMAX][4];  // columns 64 cg + 4 r16 + e, over the keys 4 qd .. + 3 of each block
+  float o[GMAX][4 * CL];  // columns DC cg + 64 (e / 4) + 4 r16 + e % 4, over the keys 4 qd .. + 3 of each block
 #pragma unroll
   for (int i = 0; i < GMAX; ++i)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[i][e] = 0.f;
+    for (int e = 0; e < 4 * CL; ++e) o[i][e] = 0.f;
 
   uint4 kf[KS];
-  uint2 vraw[4];  // this lane's 4 bf16 of its 4 V rows
+  uint2 vraw[4][CL];  // this lane's quads of bf16 of its 4 V rows
   auto load_block = [&](int kb) {
     const int key = min(kb + r16, S - 1);
     const bool fresh = k_new != nullptr && key == S - 1;
@@ -525,7 +528,9 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
     for (int j = 0; j < 4; ++j) {
       const int kj = min(kb + 4 * qd + j, S - 1);
       const bool fr = v_new != nullptr && kj == S - 1;
-      vraw[j] = *reinterpret_cast<const uint2*>((fr ? v_new + new_off : vc + (head_base + kj) * D) + DC * cg + 4 * r16);
+      const bf16* vr = (fr ? v_new + new_off : vc + (head_base + kj) * D) + DC * cg + 4 * r16;
+#pragma unroll
+      for (int c4 = 0; c4 < CL; ++c4) vraw[j][c4] = *reinterpret_cast<const uint2*>(vr + 64 * c4);
     }
   };
   // fused append: the wave holding key S-1 writes this step's K / V row into the cache (no workgroup reads it there)
@@ -559,15 +564,18 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
       sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[s2]),
                                                      __builtin_bit_cast(bf16x8_t, qf[s2]), sacc, 0, 0, 0);
     const int nk = min(16, k1 - kb);
-    float vf[4][4];  // this block's V values (fp32), taken before the next block's loads land
+    float vf[4][4 * CL];  // this block's V values (fp32), taken before the next block's loads land
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (4 * qd + j >= nk) vraw[j] = uint2{0u, 0u};  // (the last key's row again, whose infinities count once)
-      vf[j][0] = __uint_as_float(vraw[j].x << 16);
-      vf[j][1] = __uint_as_float(vraw[j].x & 0xffff0000u);
-      vf[j][2] = __uint_as_float(vraw[j].y << 16);
-      vf[j][3] = __uint_as_float(vraw[j].y & 0xffff0000u);
-    }
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int c4 = 0; c4 < CL; ++c4) {
+        uint2 u = vraw[j][c4];
+        if (4 * qd + j >= nk) u = uint2{0u, 0u};  // (the last key's row again, whose infinities count once)
+        vf[j][4 * c4] = __uint_as_float(u.x << 16);
+        vf[j][4 * c4 + 1] = __uint_as_float(u.x & 0xffff0000u);
+        vf[j][4 * c4 + 2] = __uint_as_float(u.y << 16);
+        vf[j][4 * c4 + 3] = __uint_as_float(u.y & 0xffff0000u);
+      }
     if (kb + 16 < k1) load_block(kb + 16);
     // scores of keys kb + 4qd + r for head r16 (masked past the wave's range)
     float sc[4], bmax = -INFINITY;
@@ -599,7 +607,7 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
 #pragma unroll
     for (int i = 0; i < G; ++i)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[i][e] *= al[i];
+      for (int e = 0; e < 4 * CL; ++e) o[i][e] *= al[i];
     // keys past the range have p = 0 (their scores are -inf): all 16 rows, no branch
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -607,7 +615,7 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
       for (int i = 0; i < G; ++i) {
         const float pw = pl[w][4 * qd + j][i];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[i][e] += pw * vf[j][e];
+        for (int e = 0; e < 4 * CL; ++e) o[i][e] += pw * vf[j][e];
       }
   }
   // merge the waves
@@ -615,14 +623,26 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
     wm[w][r16] = m;
     wl[w][r16] = l;
   }
+  // the quarters' sums, a lane of each left with one column of a quad: two exchanges per two columns, not four
+  if (k0 < k1) {
+    auto sum2 = [](float a, float b, auto rows32) {  // the lower rows' sum of a, the upper rows' sum of b
+      const uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+      if constexpr (decltype(rows32)::value) {
+        const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+      } else {
+        const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+      }
+    };
 #pragma unroll
-  for (int i = 0; i < GMAX; ++i) {
+    for (int i = 0; i < GMAX; ++i)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      o[i][e] += lane_xor16(o[i][e], qd & 1);
-      o[i][e] += lane_xor32(o[i][e], qd >> 1);
-    }
-    if (qd == 0) *reinterpret_cast<float4_t*>(&wo[w][i][4 * r16]) = float4_t{o[i][0], o[i][1], o[i][2], o[i][3]};
+      for (int c4 = 0; c4 < CL; ++c4) {
+        const float e0 = sum2(o[i][4 * c4], o[i][4 * c4 + 1], std::false_type{});
+        const float e1 = sum2(o[i][4 * c4 + 2], o[i][4 * c4 + 3], std::false_type{});
+        wo[w][i][64 * c4 + 4 * r16 + qd] = sum2(e0, e1, std::true_type{});
+      }
   }
   __syncthreads();
   for (int idx = t; idx < G * DC; idx += 64 * NW) {
@@ -633,6 +653,7 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
     float O = 0.f, L = 0.f;
 #pragma unroll
     for (int x = 0; x < NW; ++x) {
+      if (x * per >= S) break;  // a wave without keys
       const float e = wm[x][i] == -INFINITY ? 0.f : exp2f(wm[x][i] - M);
       O += e * wo[x][i][d];
       L += e * wl[x][i];
@@ -719,9 +740,11 @@ bool decode_small_applies(int64_t B, int64_t Tq, int64_t H, int64_t Hkv, int64_t
   if (Hkv <= 0 || H % Hkv) return false;
   const int64_t G0 = H / Hkv;
   // decode_small takes contexts up to 1024 keys (a workgroup goes over the whole cache, so longer ones keep the
-  // key-split grid). General / small kernel, us per launch at a 1024-slot cache, G = 1, D = 64: 12 heads, 1 row, 40
-  // keys 4.2 / 3.2, 200 5.4 / 4.2, 500 9.1 / 6.5, 1000 9.6 / 9.5; 5 rows 4.7 / 3.3, 5.7 / 4.9, 12.2 / 6.8, 14.1 / 11.8;
-  // 4 heads, 1 row 4.1 / 3.2, 4.9 / 4.2, 8.2 / 5.8, 8.7 / 9.3
+  // key-split grid) and up to 64 items. General / small kernel, us per launch at a 1024-slot cache, 40, 200, 500 and 1000
+  // keys: D = 64, G = 1, 12 items 4.9 / 4.0, 5.7 / 5.1, 9.2 / 6.5, 9.9 / 9.8, 64 items 4.9 / 4.0, 6.3 / 5.1, 13.1 / 7.5,
+  // 15.1 / 10.4; D = 256, G = 4, 64 items 11.1 / 5.1, 29.8 / 8.5, .., 47.5 / 23.7; D = 512, G = 1, 64 items 17.6 / 6.0,
+  // 56.8 / 12.1, .., 81.1 / 45.5. Of D 64 to 512, G 1 to 16, 1 to 64 items only D = 256, G = 1 with 1 to 4 items is
+  // slower at 1000 keys (19.0 / 20.2), and faster up to 500 (18.5 / 11.8).
   const int64_t small_keys = split_keys_env ? split_keys_env : 1024;
   return Tq == 1 && B * Hkv <= small_items && S <= small_keys &&
          (G0 == 1 || G0 == 2 || G0 == 4 || G0 == 8 || G0 == 16) && (D == 64 || D == 128 || D == 256 || D == 512) &&
@@ -831,7 +854,7 @@ torch::Tensor decode_attn(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, c
     const bf16* vnp = fuse ? reinterpret_cast<const bf16*>(v_new->data_ptr()) : nullptr;
 #define PENROZ_DSMALL(DD, GG)                                                                                   \
   do {                                                                                                          \
-    const dim3 grid((items + 7) / 8 * 8 * (DD / kSmallCols));                                                   \
+    const dim3 grid((items + 7) / 8 * 8 * (DD / 64));                                                           \
     if (rope && DD <= 256)                                                                                      \
       hipLaunchKernelGGL((decode_small_kernel<DD, GG, true>), grid, dim3(64 * kSmallWaves), 0, stream, qp, kp,  \
                          vp, op, items, H, Hkv, cap, (int)S, (float)scale, sdev, q_rs, knp, vnp, kv_rs, rcp, rsp); \
@@ -851,6 +874,16 @@ torch::Tensor decode_attn(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, c
     if (D == 64) PENROZ_DSMALL_G(64)
     else if (D == 128) PENROZ_DSMALL_G(128)
     else if (D == 256) PENROZ_DSMALL_G(256)
+    else if (items > 32 && G0 <= 4) {  // more workgroups of 64 columns than CUs: of 128
+      auto wide = [&](auto g0) {
+        hipLaunchKernelGGL((decode_small_kernel<512, decltype(g0)::value, false, 128>), dim3((items + 7) / 8 * 8 * 4),
+                           dim3(64 * kSmallWaves), 0, stream, qp, kp, vp, op, items, H, Hkv, cap, (int)S, (float)scale,
+                           sdev, q_rs, knp, vnp, kv_rs, nullptr, nullptr);
+      };
+      if (G0 == 1) wide(std::integral_constant<int, 1>{});
+      else if (G0 == 2) wide(std::integral_constant<int, 2>{});
+      else wide(std::integral_constant<int, 4>{});
+    }
     else if (G0 == 1) PENROZ_DSMALL(512, 1);
     else if (G0 == 2) PENROZ_DSMALL(512, 2);
     else if (G0 == 4) PENROZ_DSMALL(512, 4);
