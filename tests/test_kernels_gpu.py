@@ -896,7 +896,8 @@ def test_decode_attention_fused_append(dtype, int8, D, H, Hkv, S):
 
 
 @pytest.mark.parametrize("B,H,Hkv,D", [(3, 4, 1, 256), (3, 6, 3, 64), (1, 16, 1, 128), (9, 2, 2, 128), (1, 4, 2, 512),
-                                       (5, 12, 12, 64)])
+                                       (5, 12, 12, 64), (33, 1, 1, 512), (18, 4, 2, 512), (16, 16, 4, 512),
+                                       (34, 8, 1, 512)])
 @pytest.mark.parametrize("S", [1, 16, 17, 127, 129, 145, 1024])
 def test_decode_attention_small_edges(B, H, Hkv, D, S):
     """One-row attention of few heads at the edges of its key blocks (16) and waves (8 blocks), its rows taken as
@@ -1068,6 +1069,24 @@ def test_rms_residual(C, mode, with_y):
         _close(gy.float(), Nm.reference_rms_norm(gh, w2, 1e-5).float(), 0.02, 0.02)
     else:
         assert gy is None  # an undefined tensor crosses pybind as None
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+@pytest.mark.parametrize("C", [40, 1536, 2048, 2056, 4096, 6144])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_rms_residual_other_types(C, mode, dt):
+    """The same in the other types, on either side of the width from which fp32 loads the weights where they are used."""
+    from penroz.ops import norms as Nm
+    torch.manual_seed(C + mode)
+    x, a = (torch.randn(5, C, device=DEV).to(dt) * s for s in (3, 1))
+    w1, w2 = ((1 + torch.rand(C, device=DEV)).to(dt) for _ in range(2))
+    h = x + a if mode != 1 else x + Nm.reference_rms_norm(a, w1, 1e-6)
+    if mode == 0:
+        h = Nm.reference_rms_norm(h, w1, 1e-6)
+    gh, gy = _ext.kernels().rms_residual(x, a, w1 if mode != 2 else None, w2, mode, 1e-6, 1e-5)
+    tol = 1e-5 if dt == torch.float32 else 4e-3  # fp32 sums in another order; two to three roundings of 2^-11
+    _close(gh, h, tol, tol)
+    _close(gy, Nm.reference_rms_norm(gh, w2, 1e-5), tol, tol)
 
 
 @pytest.mark.parametrize("kind", ["gelu", "gelu_tanh", "silu"])
