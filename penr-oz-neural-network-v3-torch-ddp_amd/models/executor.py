@@ -752,16 +752,26 @@ class GPTExecutor:
         self._side_stream = self._side  # what _plan_step chooses for large enough steps
         self._buf_free = {}
 
-    # The side stream costs an event and a wait on either stream per weight gradient, ≈ 5 ms per GPT-2 step and hidden
-    # only behind enough work; a step of fewer operations (6 · tokens · parameters) runs on one stream. GPT-2 124M, ms
-    # per step with / without it: 256 tokens 9.8 / 5.3, 4096 9.9 / 8.7, 5120 10.0 / 9.4, 6026 10.8 / 11.3, 7860 12.8 /
-    # 13.3, 65536 62.0 / 63.7.
-    SIDE_MIN_FLOPS = 4e12
+    # The side stream costs the host an event and a wait on either stream per weight gradient: it takes 0.75 to 0.85 ms
+    # per layer to enqueue a step on two streams, whatever its size, and the card has nothing to do meanwhile unless the
+    # step is long enough. On one stream a step lasts about 0.45 ms per layer, 6 ms per 1e9 parameters (AdamW) and
+    # 1 ms per 1.1e12 operations, 6 · tokens · parameters; two streams from where that is more than the host's time. ms
+    # per step, two streams / one: GPT-2 124M (12 layers, 163e6 parameters with its own head) 256 tokens 9.0 / 5.2, 2048
+    # 9.3 / 7.2, 4096 9.7 / 9.4, 6144 11.1 / 11.7, 65536 62.0 / 63.7; 4 of its layers 1024 3.4 / 2.7, 3072 3.8 / 4.0;
+    # 24 layers, 406e6 2048 18.1 / 15.9, 5120 24.0 / 24.3; 48 layers, 1638e6 512 34.7 / 32.1, 1024 36.2 / 39.0; 6 layers,
+    # 17e6 8192 4.9 / 3.6; Gemma-3 1B (26 layers, 1302e6) 256 20.6 / 19.4, 512 20.9 / 22.2; 18 layers, 436e6 1024
+    # 14.5 / 12.4, 3072 15.8 / 17.3; 8 layers, 819e6 64 7.8 / 8.1.
+    SIDE_MIN_FLOPS = None  # operations of the smallest step on two streams; None: side_min_flops
+
+    @staticmethod
+    def side_min_flops(layers: int, parameters: int) -> float:
+        return 1.1e12 * (0.39 * layers - 6e-9 * parameters)
 
     def _plan_step(self, tokens: int):
         """The streams of a micro-step of this size (each micro-step ends with its streams joined)."""
-        large = 6 * tokens * self.flat.numel() >= self.SIDE_MIN_FLOPS
-        self._side = self._side_stream if large else None
+        params = self.flat.numel()
+        least = self.side_min_flops(self.L, params) if self.SIDE_MIN_FLOPS is None else self.SIDE_MIN_FLOPS
+        self._side = self._side_stream if 6 * tokens * params >= least else None
 
     def _side_call(self, operand: Tensor, fn):
         """Run ``fn`` (gradient-only work reading ``operand``) on the side stream, or inline."""

@@ -102,9 +102,6 @@ class GemmaExecutor(GPTExecutor):
     # 65.86 / 65.86 -> 65.14 / 65.32 and 65.82 / 65.72 -> 65.09 / 65.06 ms on two boxes, Gemma-4 e2b
     # neutral (profiles/notes_r6.md §16; PENROZ_SEGMENT_TRANSPOSE=1 / 0 overrides)
     SEGMENT_TRANSPOSE = False
-    # fewer events per operation than GPT-2 124M: Gemma-3 1B, ms per step with / without the side stream: 256 tokens
-    # 19.2 / 18.7, 512 19.8 / 20.9, 1024 23.0 / 26.1
-    SIDE_MIN_FLOPS = 2e12
 
     # ------------------------------------------------------------------ pattern match
     @staticmethod

@@ -258,3 +258,30 @@ def test_deferred_reductions_are_a_threads_own():
         assert seen == [0] and k.get_deferred_reduce_stream() == 64
     finally:
         k.set_deferred_reduce_stream(0, 0)
+
+
+# layers, parameters, tokens, ms per step on two streams / on one
+SIDE_STREAM_MS = [
+    (12, 163109376, 256, 9.0, 5.2), (12, 163109376, 2048, 9.3, 7.2), (12, 163109376, 4096, 9.7, 9.4),
+    (12, 163109376, 6144, 11.1, 11.7), (12, 163109376, 65536, 62.0, 63.7), (4, 106406400, 1024, 3.4, 2.7),
+    (4, 106406400, 3072, 3.8, 4.0), (24, 406382592, 2048, 18.1, 15.9), (24, 406382592, 5120, 24.0, 24.3),
+    (48, 1638172800, 512, 34.7, 32.1), (48, 1638172800, 1024, 36.2, 39.0), (6, 17332224, 8192, 4.9, 3.6),
+    (26, 1301862528, 256, 20.6, 19.4), (26, 1301862528, 512, 20.9, 22.2), (18, 435861120, 1024, 14.5, 12.4),
+    (18, 435861120, 3072, 15.8, 17.3), (8, 818713728, 64, 7.8, 8.1)]
+
+
+@pytest.mark.parametrize("layers,params,tokens,two,one", SIDE_STREAM_MS)
+def test_steps_take_the_streams_measured_faster(layers, params, tokens, two, one):
+    import torch
+    ex = GPTExecutor.__new__(GPTExecutor)
+    ex.L, ex._side_stream = layers, "side"
+    ex.flat = torch.empty(params, device="meta")
+    ex._plan_step(tokens)
+    assert (ex._side is not None) == (two < one)
+
+
+def test_the_stream_rule_counts_the_models_own_parameters():
+    import torch
+    with torch.device("meta"):
+        m = _model(bench.gpt2_layers())
+    assert sum(p.numel() for p in m.parameters()) == SIDE_STREAM_MS[0][1]
