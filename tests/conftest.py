@@ -27,6 +27,24 @@ def workdir(tmp_path, monkeypatch):
     return tmp_path
 
 
+@pytest.fixture(params=["two", "one"])
+def training_streams(request, monkeypatch):
+    """The training executors' steps on two streams, as every large step runs, and on one, as small ones do: by their
+    size the steps of a test all take one. (An executor given a limit of its own keeps to that.)"""
+    from penroz.models.executor import GPTExecutor
+    two, plan, taken = request.param == "two", GPTExecutor._plan_step, []
+
+    def checked(self, tokens):
+        plan(self, tokens)
+        if "SIDE_MIN_FLOPS" not in vars(self) and self._side_stream is not None:
+            taken.append(self._side is not None)
+
+    monkeypatch.setattr(GPTExecutor, "SIDE_MIN_FLOPS", 0 if two else float("inf"))
+    monkeypatch.setattr(GPTExecutor, "_plan_step", checked)
+    yield request.param
+    assert all(t == two for t in taken)
+
+
 def gpu_available() -> bool:
     try:
         import torch

@@ -77,6 +77,7 @@ def _worker(rank, world, port, out, bucket_mb, overlap, model_type):
             for p in model.parameters():
                 p.add_(0.01)
     ex = GemmaExecutor(model, dev)
+    ex.SIDE_MIN_FLOPS = 0  # the buckets start from the side stream, as in large steps (the single process: one stream)
     ex.setup_training(True)
     assert ex.reducer is not None and len(ex.reducer.buckets) > 1
     x, y = _batch(rank)
@@ -89,7 +90,7 @@ def _worker(rank, world, port, out, bucket_mb, overlap, model_type):
             xs, ys = _batch(rank + 10 * step)
             ex.zero_grad()
             ex.train_micro_step(xs.to(dev), ys.to(dev), 1.0, sync=True, fuse_optimizer=True)
-            assert ex.opt_overlap_mode() == "per-bucket-in-backward" and ex._opt_done
+            assert ex.opt_overlap_mode() == "per-bucket-in-backward" and ex._opt_done and ex._side is not None
             assert ex._opt_buckets_done == set(range(len(ex.reducer.buckets)))
             ex.optimizer_step()  # nothing left to do
         torch.cuda.synchronize()
@@ -99,7 +100,7 @@ def _worker(rank, world, port, out, bucket_mb, overlap, model_type):
         dist.destroy_process_group()
         return
     ex.train_micro_step(x.to(dev), y.to(dev), 1.0, sync=True)
-    assert ex._reduce_pending == bool(overlap)
+    assert ex._reduce_pending == bool(overlap) and ex._side is not None
     if rank == 0:
         ex.optimizer_step()
         ex.wait_gradients()

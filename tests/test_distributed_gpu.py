@@ -65,6 +65,7 @@ def _worker(rank, world, port, out, bucket_mb, overlap):
             for p in model.parameters():
                 p.add_(0.01)
     ex = GPTExecutor(model, dev)
+    ex.SIDE_MIN_FLOPS = 0  # the buckets start from the side stream, as in large steps (the single process: one stream)
     ex.setup_training(True)
     assert ex.reducer is not None and len(ex.reducer.buckets) > 1
     x, y = _batch(rank)
@@ -74,7 +75,7 @@ def _worker(rank, world, port, out, bucket_mb, overlap):
         # as the bucket's all-reduce has landed; the embedding bucket is cut into pieces
         assert len(ex.reducer.buckets) >= 4
         ex.train_micro_step(x.to(dev), y.to(dev), 1.0, sync=True, fuse_optimizer=True)
-        assert ex.opt_overlap_mode() == "per-bucket-in-backward" and ex._opt_done
+        assert ex.opt_overlap_mode() == "per-bucket-in-backward" and ex._opt_done and ex._side is not None
         assert ex._opt_buckets_done == set(range(len(ex.reducer.buckets)))
         ex.optimizer_step()  # nothing left to do
         torch.cuda.synchronize()
@@ -85,6 +86,7 @@ def _worker(rank, world, port, out, bucket_mb, overlap):
         return
     ex.train_micro_step(x.to(dev), y.to(dev), 1.0, sync=True)
     assert ex._reduce_pending == bool(overlap)  # overlap: the last buckets are still reducing
+    assert ex._side is not None
     if rank == 0:  # the optimizer consumes the in-flight buckets one by one
         ex.optimizer_step()
         ex.wait_gradients()

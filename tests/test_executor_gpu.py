@@ -5,7 +5,7 @@ import math
 import pytest
 import torch
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("training_streams")]
 if not torch.cuda.is_available():  # pragma: no cover
     pytest.skip("needs a GPU", allow_module_level=True)
 
@@ -271,3 +271,32 @@ def test_step_sizes_share_one_executor(family):
     torch.cuda.synchronize()
     # two such runs differ by AdamW updates whose gradient is within a rounding of zero: 2 lr on a few weights of 0.02
     assert ((got[0] - got[1]).norm() / got[1].norm()).item() < 2e-3
+
+
+def test_a_failed_step_leaves_the_next_one_alone(monkeypatch):
+    """A step on two streams that raises in its backward, then a small step on one: gradients as a fresh executor's."""
+    from penroz.models import executor
+    x = torch.randint(0, 512, (4, 129), generator=torch.Generator().manual_seed(1)).cuda()
+    grads = []
+    for fail in (True, False):
+        torch.manual_seed(0)
+        ex = GPTExecutor(tiny().cuda(), torch.device("cuda", 0))
+        ex.SIDE_MIN_FLOPS = 0
+        ex.setup_training(False)
+        if fail:
+            with monkeypatch.context() as mp:
+                def stop(*args, **kwargs):
+                    assert _ext.kernels().get_deferred_reduce_stream() == ex._side.cuda_stream
+                    raise MemoryError("in the backward")
+                mp.setattr(executor.attn_ops, "flash_bwd", stop)
+                ex.zero_grad()
+                with pytest.raises(MemoryError):
+                    ex.train_micro_step(x[:, :-1].contiguous(), x[:, 1:].contiguous(), 1.0)
+            assert _ext.kernels().get_deferred_reduce_stream() == 0
+        ex.SIDE_MIN_FLOPS = float("inf")
+        ex.flat_grad.zero_()
+        ex.train_micro_step(x[:2, :-1].contiguous(), x[:2, 1:].contiguous(), 1.0)
+        assert ex._side is None and _ext.kernels().get_deferred_reduce_stream() == 0
+        grads.append(ex.flat_grad.clone())
+    # (the embedding gradient's atomics may sum in another order)
+    assert ((grads[0] - grads[1]).norm() / grads[1].norm()).item() < 1e-5

@@ -15,7 +15,7 @@ from types import SimpleNamespace
 import pytest
 import torch
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("training_streams")]
 if not torch.cuda.is_available():  # pragma: no cover
     pytest.skip("needs a GPU", allow_module_level=True)
 
@@ -322,8 +322,8 @@ def test_row_split_embedding_adamw_matches_dense(monkeypatch, V, steps):
     and touched rows (after the embedding backward, gradient cleared) == the dense fused step; the
     gradient buffer's table range stays zero between steps (zero_grad skips it). Rows no token
     touches (the training tokens are < 512) are BITWISE equal — only the scatter order of touched
-    rows may differ; at V = 16384 the untouched-row update (side stream) runs while the forward
-    is still executing (ADVICE r5)."""
+    rows may differ; on two streams, at V = 16384, the untouched-row update runs while the forward
+    is still executing."""
     from penroz.models.model import _FusedRunner
     a, b = _gemma("gemma3_text", V=V, seed=4).to(DEV), _gemma("gemma3_text", V=V, seed=4).to(DEV)
     monkeypatch.setenv("PENROZ_EMB_ROW_ADAM", "0")
