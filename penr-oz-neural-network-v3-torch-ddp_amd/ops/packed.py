@@ -128,10 +128,11 @@ def _conv_torch(x: Tensor, cw: Tensor, state: Tensor, b: PackedBatch) -> Tensor:
     return out
 
 
-def _norm_conv_fits(x: Tensor, y: Tensor, w: Tensor, groups: int, cw: Tensor, state: Tensor) -> bool:
+def _norm_conv_fits(x: Tensor, y: Tensor, w: Tensor, groups: int, cw: Tensor, state: Tensor, dtype: torch.dtype) -> bool:
     """Whether the residual add, its norm and the convolution of a prompt run as one pass: a norm group is what one
-    wave holds, and its registers keep the rows of up to 4 taps (8192 rows of 2048: 56 us as two passes, 38 as one)."""
-    return (x.shape[1] in (256 * groups, 512 * groups) and cw.shape[0] <= 4
+    wave holds, its registers keep the rows of up to 4 taps (8192 rows of 2048: 56 us as two passes, 38 as one), and y
+    and the output are of one type."""
+    return (y.dtype == dtype and x.shape[1] in (256 * groups, 512 * groups) and cw.shape[0] <= 4
             and all(t.data_ptr() % 16 == 0 for t in (x, y, w, cw, state)))
 
 
@@ -155,7 +156,7 @@ def residual_conv(b: PackedBatch, dtype: torch.dtype, *, x: Tensor | None = None
         if conv is None or b.single:
             adv = b.advance and embed is not None
             K.row_norm_add(tok, table, x, xo, y, pair_w, w, g, eps, cw, st, b.slot, b.pos, adv, h)
-        elif embed is None and y is not None and pair_w is None and _norm_conv_fits(x, y, w, g, cw, st):
+        elif embed is None and y is not None and pair_w is None and _norm_conv_fits(x, y, w, g, cw, st, dtype):
             xo = torch.empty_like(x)
             K.norm_conv_rows(x, xo, y, w, g, eps, cw, st, b.slot, b.pos, b.first, b.cu, b.seq_slot, h)
         else:

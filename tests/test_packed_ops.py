@@ -87,28 +87,33 @@ def test_convolution_in_portions(target, C, taps):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("y_dt,dt", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32),
+                                     (torch.bfloat16, torch.float32)])
 @pytest.mark.parametrize("C,groups,taps,top,cuts", [
-    (512, 2, 4, 0, [[1, 5, 6, 2], [3, 1, 7, 12], [40, 2, 3, 1]]), (1536, 6, 3, 2, [[4, 9, 14], [1, 1, 30]]),
-    (512, 1, 1, 3, [[7, 6], [2, 2]]), (1024, 4, 4, 6, [[1, 6700, 3], [2, 3, 29]]), (2048, 4, 2, 0, [[1, 2, 19000]])])
-def test_norm_and_convolution_in_one_pass(C, groups, taps, top, cuts, dt):
-    """Residual add, norm and convolution of prompts at the edges of the wave's spans (5 rows, and one round
-    or two of longer ones), every sequence in portions, with fewer groups than waves and more; and with expert rows,
-    which take the kernels one by one: as the step-by-step form computes them."""
+    (512, 2, 4, 0, [[1, 5, 6, 2], [3, 1, 7, 12], [40, 2, 3, 1]]), (1536, 6, 3, 0, [[4, 9, 14], [1, 1, 30]]),
+    (512, 1, 1, 0, [[7, 6], [2, 2]]), (2048, 4, 4, 0, [[1, 6700, 3], [2, 3, 29]]), (2048, 4, 2, 0, [[1, 2, 19000]]),
+    (5120, 10, 4, 0, [[9, 1, 70], [5, 2, 3]]), (2048, 8, 1, 0, [[3, 30]]), (1536, 6, 3, 2, [[4, 9, 14], [1, 1, 30]]),
+    (512, 2, 5, 0, [[7, 6], [2, 2]]), (768, 6, 4, 0, [[7, 6], [2, 2]])])
+def test_norm_and_convolution_in_one_pass(C, groups, taps, top, cuts, y_dt, dt):
+    """Residual add, norm and convolution of prompts as the step-by-step form computes them. In one pass (x left as it
+    was): at the edges of the wave's spans (5 rows, and one round or two of longer ones), every sequence in portions, 1 to
+    4 taps, groups of 256 and 512, fewer of them than a workgroup has waves and more. One kernel after the other (x
+    updated in place): expert rows, 5 taps, other groups, and an output of another type than the sublayer's."""
+    one_pass = top == 0 and taps <= 4 and C // groups in (256, 512) and y_dt == dt
     g = torch.Generator().manual_seed(C + taps)
     w, cw = torch.rand(C, generator=g) + 0.5, torch.randn(taps, C, generator=g)
     state = {d: SequenceState([], [(C, taps)], [], dt, d, slots=len(cuts[0])) for d in ("cpu", "cuda")}
     slots = {d: [st.acquire() for _ in cuts[0]][::-1] for d, st in state.items()}
     for counts in cuts:
         N = sum(counts)
-        x, y = torch.randn(N, C, generator=g), torch.randn(N * max(top, 1), C, generator=g).to(dt)
+        x0, y = torch.randn(N, C, generator=g), torch.randn(N * max(top, 1), C, generator=g).to(y_dt)
         pw = torch.rand(N, top, generator=g) if top else None
         out = {}
         for d, st in state.items():
-            b = st.begin(list(zip(slots[d], counts)))
-            out[d] = P.residual_conv(b, dt, x=x.clone().to(d), y=y.to(d), pair_w=None if pw is None else pw.to(d),
+            b, x = st.begin(list(zip(slots[d], counts))), x0.clone().to(d)
+            out[d] = P.residual_conv(b, dt, x=x, y=y.to(d), pair_w=None if pw is None else pw.to(d),
                                      norm=(w.to(d), groups, 1e-5), conv=(cw.to(d), st.conv[0]))
-        assert P._norm_conv_fits(x, y, w, groups, cw, st.conv[0])
+        assert (out["cuda"][0].data_ptr() != x.data_ptr()) == one_pass
         near(out["cuda"][0], out["cpu"][0], torch.float32)
         near(out["cuda"][1], out["cpu"][1], dt)
         for a, c in zip(slots["cuda"], slots["cpu"]):
