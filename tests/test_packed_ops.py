@@ -400,10 +400,12 @@ def test_experts_in_large_tiles(kind, C, F):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", [1, P.UNGATED])
-@pytest.mark.parametrize("E,C,F", [(512, 1024, 64), (512, 992, 32), (40, 96, 160)])
+@pytest.mark.parametrize("E,C,F", [(512, 1024, 64), (512, 992, 32), (40, 96, 160), (20, 512, 544), (20, 544, 512),
+                                   (20, 1056, 1024), (70, 992, 512), (70, 992, 544)])
 def test_experts_of_few_pairs(kind, E, C, F):
-    """Few pairs at both widths of the second product's workgroups (64 weight rows from 16384 workgroups of 32), with an
-    odd number of them, and at widths that end in half of one."""
+    """Few pairs at both widths of the second product's workgroups (64 weight rows from 1024 workgroups of 32, F up to
+    512), with an odd number of them, and at widths that end in half of one; reductions of one round of loads (4 or 8 steps of 32 per
+    wave), of one step more and of less."""
     dev, N, top = "cuda", 130, 4
     h = rand(N, C, dtype=torch.bfloat16).to(dev)
     ids = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(i))[:top] for i in range(N)]).to(dev)
