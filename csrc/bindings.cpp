@@ -189,7 +189,7 @@ PYBIND11_MODULE(penroz_kernels, m) {
         pybind11::arg("seq_len_dev") = pybind11::none(), pybind11::arg("k_new") = pybind11::none(),
         pybind11::arg("v_new") = pybind11::none(), pybind11::arg("counters") = pybind11::none(),
         pybind11::arg("rope_cos") = pybind11::none(), pybind11::arg("rope_sin") = pybind11::none());
-  m.def("decode_small_applies", &decode_small_applies, "decode_attn takes the one-workgroup-per-item kernel");
+  m.def("decode_small_applies", &decode_small_applies, "decode_attn takes the kernel for few heads and short contexts");
   m.def("set_deferred_reduce_stream", &set_deferred_reduce_stream);
   m.def("get_deferred_reduce_stream", &get_deferred_reduce_stream);
   m.def("kv_append", &kv_append, pybind11::arg("k"), pybind11::arg("v"), pybind11::arg("kc"), pybind11::arg("vc"),

@@ -275,7 +275,8 @@ __global__ void __launch_bounds__(kPrThreads) conv_rows_kernel(const float* __re
 // whose rows the neighbour before still reads.
 // Bound by memory: x and y are read and x_out and h written once (the halo adds 3 / span to the reads). With the
 // state's launch, against norm and convolution one after the other: 8192 rows of 2048, 4 groups, 56 -> 38 us; 16384
-// 105 -> 91; 1024 16.3 -> 13.0. (With the weighted sum of 6 expert rows instead of y: 90 -> 91, so not here.)
+// 105 -> 91; 1024 16.3 -> 13.0 (called alone over and over; between the other kernels of a prompt, 8192 rows, it takes
+// 42 us, the state's launch 5). (With the weighted sum of 6 expert rows instead of y: 90 -> 91, so not here.)
 constexpr int kNcTaps = 4;
 template <typename T> struct Raw4 { using type = uint2; };
 template <> struct Raw4<float> { using type = float4_t; };
@@ -290,9 +291,10 @@ template <int Q> constexpr int norm_conv_blocks() { return Q == 1 ? 4 : 2; }  //
 
 template <typename T, int Q>
 __global__ void __launch_bounds__(kPrThreads, norm_conv_blocks<Q>()) norm_conv_kernel(
-    const float* __restrict__ x, float* __restrict__ x_out, const T* __restrict__ y, const float* __restrict__ nw, int groups, float eps, const float* __restrict__ cw, int taps,
-    const float* __restrict__ state, const int* __restrict__ slot, const int* __restrict__ pos,
-    const int* __restrict__ first, T* __restrict__ h, int N, int C, int span) {
+    const float* __restrict__ x, float* __restrict__ x_out, const T* __restrict__ y, const float* __restrict__ nw,
+    int groups, float eps, const float* __restrict__ cw, int taps, const float* __restrict__ state,
+    const int* __restrict__ slot, const int* __restrict__ pos, const int* __restrict__ first, T* __restrict__ h, int N,
+    int C, int span) {
   using R = typename Raw4<T>::type;
   const int lane = threadIdx.x & 63, g = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (g >= groups) return;
