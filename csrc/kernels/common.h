@@ -49,6 +49,15 @@ __device__ __forceinline__ float dpp_f32(float v) {
 __device__ __forceinline__ float lane_f32(float v, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
+// the value of lane ^ 16 (odd: lane bit 4) and of lane ^ 32 (odd: lane bit 5), without a trip through the LDS crossbar
+__device__ __forceinline__ float lane_xor16(float v, int odd) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(odd ? r[0] : r[1]);
+}
+__device__ __forceinline__ float lane_xor32(float v, int odd) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(odd ? r[0] : r[1]);
+}
 template <typename Op>
 __device__ __forceinline__ float wave_reduce(float v, Op op) {
   v = op(v, dpp_f32<0xB1>(v));   // quad_perm [1,0,3,2]

@@ -18,22 +18,13 @@
 // counters, a second kernel). Enough splits are used to put ≥ 512 workgroups in
 // flight (256 CUs) even at batch 1.
 #include "common.h"
+#include "prompt_attn.h"
 #include <cstdlib>
 #include <type_traits>
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
 namespace penroz {
-
-// the value of lane ^ 16 (odd: lane bit 4) and of lane ^ 32 (odd: lane bit 5), without a trip through the LDS crossbar
-__device__ __forceinline__ float lane_xor16(float v, int odd) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(odd ? r[0] : r[1]);
-}
-__device__ __forceinline__ float lane_xor32(float v, int odd) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(odd ? r[0] : r[1]);
-}
 
 constexpr int kMaxGroup = 16;
 constexpr int kMaxMergeSplits = 16;
@@ -662,7 +653,8 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
   }
 }
 
-template <typename TQ>
+// LOG2: the parts' maxima are in powers of two (prompt_attn_kernel's)
+template <typename TQ, bool LOG2 = false>
 __global__ void __launch_bounds__(256) decode_combine_kernel(const float* __restrict__ ws_o,
                                                              const float* __restrict__ ws_ml, TQ* __restrict__ out,
                                                              int rows, int D, int splits) {
@@ -676,7 +668,7 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(const float* __rest
     for (int s = 0; s < splits; ++s) {
       const int64_t rr = (int64_t)s * rows + r;
       const float ms = ws_ml[2 * rr];
-      const float f = ms == -INFINITY ? 0.f : __expf(ms - M);
+      const float f = ms == -INFINITY ? 0.f : LOG2 ? exp2f(ms - M) : __expf(ms - M);
       L += ws_ml[2 * rr + 1] * f;
       O += ws_o[rr * D + d] * f;
     }
@@ -892,6 +884,19 @@ torch::Tensor decode_attn(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, c
 #undef PENROZ_DSMALL
     return out;
   }
+  // several query rows per sequence (prompts): 64 of them share each key and value that is read. Wide heads from 1024
+  // tokens: below, the gain is small beside the rest of a prompt of the models that have them (one of 9 tokens 9.0 / 6.7
+  // us, 3 of 200 38.6 / 19.8 in a layer of 190), and their bf16 residual stream turns another rounding of one value into
+  // a difference of 3 % in the logits of a few rows: those keep the results they had.
+  const bool prompt = Tq > 1 && !quant && q.scalar_type() == torch::kBFloat16 && sdev == nullptr && D >= 64 &&
+                      (D <= 128 || (int64_t)B * Tq >= 1024);
+  if (prompt) {
+    splits = prompt_attn_splits((int64_t)B * Hkv, (int64_t)Tq * (H / Hkv), q_offset + Tq, D);
+    if (q_rs % 8 != 0 || reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 != 0) {  // it reads 16 bytes at a time
+      q = q.clone(at::MemoryFormat::Contiguous);
+      q_rs = (int64_t)H * D;
+    }
+  }
   torch::Tensor ws_o, ws_ml;
   float* wo = nullptr;
   float* wm = nullptr;
@@ -900,6 +905,17 @@ torch::Tensor decode_attn(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, c
     ws_ml = torch::empty({(int64_t)splits * B * Tq * H * 2}, q.options().dtype(torch::kFloat32));
     wo = ws_o.data_ptr<float>();
     wm = ws_ml.data_ptr<float>();
+  }
+  if (prompt) {
+    const int rows = B * Tq * H;
+    bf16* op = reinterpret_cast<bf16*>(out.data_ptr());
+    prompt_attn_launch(reinterpret_cast<const bf16*>(q.data_ptr()), reinterpret_cast<const bf16*>(kc.data_ptr()),
+                       reinterpret_cast<const bf16*>(vc.data_ptr()), op, wo, wm, B, Tq, H, Hkv, D, cap, (int)q_offset,
+                       splits, (float)scale, q_rs, stream);
+    if (splits > 1)
+      hipLaunchKernelGGL((decode_combine_kernel<bf16, true>), dim3(std::min(2048, (rows * D + 255) / 256)), dim3(256), 0,
+                         stream, wo, wm, op, rows, D, splits);
+    return out;
   }
   dim3 grid(items * splits);
   auto launch = [&](auto qtag, auto ktag) {
