@@ -548,6 +548,165 @@ __global__ void __launch_bounds__(512, 1) wgrad256_ring16o_kernel(const bf16* __
   else run(std::integral_constant<int, 8>{});
 }
 
+// ---- several weight gradients of one step in one launch ----------------------------------------
+// The four linears of a layer at K tokens: as launches of their own, GPT-2's gradients of 256 tokens are 9 to 36 workgroups of
+// the 256-tile kernel on 256 CUs, and those of 4096 need seven slabs each to fill them. Together the layer's tiles fill the card
+// unsplit, so there is no slab and every gradient is written once.
+struct WgradItem {
+  const bf16* a;  // dy [K, M]
+  const bf16* b;  // x [K, N]
+  float* g;       // [M, N]
+  int M, N, lda, ldb, tiles_n, tile0, acc_in;  // tile0: tiles of the items before
+};
+constexpr int kGroupItems = 8;
+struct WgradItems {
+  WgradItem item[kGroupItems];
+  int n, K;
+};
+
+// Tile 64·WM × 64·WN, a wave per 64×64, the ring and the swizzle of ring16o: 128×128 is two workgroups to a CU, 256×128 one that
+// reads a quarter less (plan_wgrad_group has the times of both). The product is taken transposed (rows of the MFMA result are
+// columns n of the gradient), so a lane holds four consecutive n and writes 16 bytes. Sums of 8 stages (256 tokens) are added to
+// a total of their own, which keeps the chains of fp32 additions as short as the split kernel's. Bound by the writes (28 MB for
+// GPT-2's layer: 5 us of 14) below about 512 tokens, by LDS reads and MFMAs (equal at 64×64 per wave) above: 0.75 PFLOP/s at
+// 3885 tokens with 216 of 256 CUs at work. A ring of three stages (three workgroups per CU) measured the same.
+template <int WM, int WN>
+__global__ void __launch_bounds__(64 * WM * WN, WM * WN == 4 ? 2 : 1) wgrad_group_kernel(const WgradItems items) {
+  extern __shared__ __attribute__((aligned(16))) char smem2[];  // [NBUF][A|B]
+  constexpr int NBUF = 4, TM = 64 * WM, TN = 64 * WN, NW = WM * WN;
+  constexpr int ABYTES = 32 * TM * 2, BBYTES = 32 * TN * 2, STAGE = ABYTES + BBYTES;
+  constexpr int PA = ABYTES / 1024 / NW, PB = BBYTES / 1024 / NW, G = PA + PB;
+  constexpr int CA = TM / 8, CB = TN / 8;  // 16-byte chunks of a row
+  static_assert(CA >= 16 && CB >= 16 && PA >= 1 && PB >= 1, "swz16 permutes at least 16 chunks");
+  const int nwg = gridDim.x, wg = blockIdx.x;
+  const int xcd = wg & 7, qd = nwg >> 3, rd = nwg & 7;
+  const int id = (xcd < rd ? xcd * (qd + 1) : rd * (qd + 1) + (xcd - rd) * qd) + (wg >> 3);
+  int which = 0;
+  for (int i = 1; i < items.n; ++i) which = id >= items.item[i].tile0 ? i : which;
+  const WgradItem& it = items.item[which];
+  const int M = it.M, N = it.N, lda = it.lda, ldb = it.ldb, K = items.K;
+  const bf16* const A = it.a;
+  const bf16* const B = it.b;
+  const int tile = id - it.tile0;
+  const int tm = tile / it.tiles_n, tn = tile - tm * it.tiles_n;
+  const int m0 = tm * TM, n0 = tn * TN;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = w / WN, wn = w % WN;
+
+  // piece i of a wave: 1024 consecutive bytes of the stage; columns past M / N are those of the last chunk
+  const int mlast = ((M + 7) & ~7) - 8, nlast = N - 8;
+  unsigned aoff[PA], boff[PB];
+  int arow[PA], brow[PB];
+#pragma unroll
+  for (int i = 0; i < PA; ++i) {
+    const int c = 64 * (PA * w + i) + lane;
+    arow[i] = c / CA;
+    aoff[i] = (unsigned)(arow[i] * lda + min(m0 + 8 * ((c % CA) ^ swz16(arow[i])), mlast)) * 2u;
+  }
+#pragma unroll
+  for (int i = 0; i < PB; ++i) {
+    const int c = 64 * (PB * w + i) + lane;
+    brow[i] = c / CB;
+    boff[i] = (unsigned)(brow[i] * ldb + min(n0 + 8 * ((c % CB) ^ swz16(brow[i])), nlast)) * 2u;
+  }
+  const unsigned lds_base = (unsigned)(size_t)(lds_void_t*)smem2;
+  const char* zero = reinterpret_cast<const char*>(g_zero16);
+  auto dma = [&](int st) {
+    const int kr = st * 32;
+    const unsigned la = __builtin_amdgcn_readfirstlane(lds_base + (st % NBUF) * STAGE + PA * w * 1024);
+    const unsigned lb = __builtin_amdgcn_readfirstlane(lds_base + (st % NBUF) * STAGE + ABYTES + PB * w * 1024);
+    const char* sa = reinterpret_cast<const char*>(A + (size_t)kr * lda);
+    const char* sb = reinterpret_cast<const char*>(B + (size_t)kr * ldb);
+    if (kr + 32 <= K) {
+#pragma unroll
+      for (int i = 0; i < PA; ++i) glds16_s(sa, aoff[i], la + i * 1024);
+#pragma unroll
+      for (int i = 0; i < PB; ++i) glds16_s(sb, boff[i], lb + i * 1024);
+    } else {  // rows >= K read the zero page
+#pragma unroll
+      for (int i = 0; i < PA; ++i) glds16(kr + arow[i] < K ? sa + aoff[i] : zero, la + i * 1024);
+#pragma unroll
+      for (int i = 0; i < PB; ++i) glds16(kr + brow[i] < K ? sb + boff[i] : zero, lb + i * 1024);
+    }
+  };
+
+  // fragment: k = 8·(lane>>4) + j of column c0 + (lane&15); rows r and r + 4
+  const int g = lane >> 4, q = (lane & 15) >> 2, p4 = 4 * (lane & 3);
+  unsigned fa[4], fb[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = 8 * g + q, ca = 64 * wm + 16 * i + p4, cb = 64 * wn + 16 * i + p4;
+    fa[i] = (unsigned)(row * TM * 2 + (((ca >> 3) ^ swz16(row)) << 4) + ((ca & 4) << 1));
+    fb[i] = (unsigned)(row * TN * 2 + (((cb >> 3) ^ swz16(row)) << 4) + ((cb & 4) << 1));
+  }
+  auto frag = [&](const char* t, unsigned off, int stride) -> uint4 {
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(t + off));
+    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(t + off + 4 * stride));
+    const uint2 ua = __builtin_bit_cast(uint2, a), ub = __builtin_bit_cast(uint2, b);
+    return uint4{ua.x, ua.y, ub.x, ub.y};
+  };
+
+  f32x4 acc[4][4], tot[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = tot[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int nsteps = (K + 31) / 32;
+#pragma unroll
+  for (int t = 0; t < NBUF - 1; ++t) dma(t);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NBUF - 2) * G) : "memory");
+  __syncthreads();
+  auto step = [&](int st, auto stage_tag) {
+    constexpr int ST = decltype(stage_tag)::value;
+    dma(st + NBUF - 1);  // into the stage consumed at step st-1 (freed by its barrier)
+    const char* At = smem2 + ST * STAGE;
+    const char* Bt = At + ABYTES;
+    uint4 af[4], bf[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) bf[j] = frag(Bt, fb[j], TN * 2);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) af[i] = frag(At, fa[i], TM * 2);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = mfma16(bf[j], af[i], acc[i][j]);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NBUF - 2) * G) : "memory");  // stage st+1 landed
+    __syncthreads();
+  };
+  int st = 0, held = 0;
+  for (; st + NBUF <= nsteps; st += NBUF) {
+    unroll_steps<0, NBUF>([&](auto ic) { step(st + decltype(ic)::value, ic); });
+    held += NBUF;
+    if (held >= 8) {
+      held = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) tot[i][j] += acc[i][j], acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  unroll_steps<0, NBUF - 1>([&](auto ic) {
+    if (st + decltype(ic)::value < nsteps) step(st + decltype(ic)::value, ic);
+  });
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // drain the zero-page prefetches
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int m = m0 + 64 * wm + 16 * i + (lane & 15);
+    float* row = it.g + (size_t)m * N + n0 + 64 * wn + 4 * g;
+    float4_t cur[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      cur[j] = it.acc_in && m < M && n0 + 64 * wn + 16 * j + 4 * g < N ? *reinterpret_cast<const float4_t*>(row + 16 * j)
+                                                                     : float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 v = tot[i][j] + acc[i][j];
+      if (m < M && n0 + 64 * wn + 16 * j + 4 * g < N)
+        *reinterpret_cast<float4_t*>(row + 16 * j) = float4_t{cur[j].x + v[0], cur[j].y + v[1], cur[j].z + v[2], cur[j].w + v[3]};
+    }
+  }
+}
+
 // G[e] += Σ_s slab[s][e]  (vectorised, fixed order)
 __global__ void __launch_bounds__(256) slab_reduce_kernel(const float* __restrict__ slab, float* __restrict__ g,
                                                           int64_t n4, int splits, int64_t stride4, int acc_in) {
@@ -584,9 +743,18 @@ __global__ void __launch_bounds__(256) tile_slab_reduce_kernel(const float* __re
 
 using namespace penroz;
 
-// grad[M][N] += dyᵀ·x with dy [K, M], x [K, N] (bf16, row-major, contiguous rows).
-// tile = 256 (default, 8 waves) or 128 (4 waves); variant selects the 256-tile pipeline (see below).
-void wgrad_gemm(torch::Tensor dy, torch::Tensor x, torch::Tensor grad, int64_t tile, int64_t variant, bool accumulate) {
+namespace {
+
+int cu_count(int device) {
+  static int n_cu = 0;
+  if (n_cu == 0) {
+    hipDeviceProp_t prop;
+    n_cu = hipGetDeviceProperties(&prop, device) == hipSuccess ? prop.multiProcessorCount : 256;
+  }
+  return n_cu;
+}
+
+void check_wgrad(const torch::Tensor& dy, const torch::Tensor& x, const torch::Tensor& grad) {
   TORCH_CHECK(dy.is_cuda() && x.is_cuda() && grad.is_cuda());
   TORCH_CHECK(dy.scalar_type() == torch::kBFloat16 && x.scalar_type() == torch::kBFloat16 &&
               grad.scalar_type() == torch::kFloat32, "wgrad: bf16 operands, fp32 gradient");
@@ -604,6 +772,15 @@ void wgrad_gemm(torch::Tensor dy, torch::Tensor x, torch::Tensor grad, int64_t t
   TORCH_CHECK(M % 8 == 0 || dy.storage().nbytes() >= (size_t)(dy.storage_offset() + (int64_t)(K - 1) * dy.stride(0) +
                                                              Mp) * 2,
               "wgrad: dy's last row padding must be allocated");
+}
+
+}  // namespace
+
+// grad[M][N] += dyᵀ·x with dy [K, M], x [K, N] (bf16, row-major, contiguous rows).
+// tile = 256 (default, 8 waves) or 128 (4 waves); variant selects the 256-tile pipeline (see below).
+void wgrad_gemm(torch::Tensor dy, torch::Tensor x, torch::Tensor grad, int64_t tile, int64_t variant, bool accumulate) {
+  check_wgrad(dy, x, grad);
+  const int K = dy.size(0), M = dy.size(1), N = x.size(1);
   TORCH_CHECK(tile == 128 || tile == 256, "wgrad: tile must be 128 or 256");
   if (K == 0) {
     if (!accumulate) grad.zero_();
@@ -612,11 +789,7 @@ void wgrad_gemm(torch::Tensor dy, torch::Tensor x, torch::Tensor grad, int64_t t
   const int T = (int)tile;
   const int tiles_m = (M + T - 1) / T, tiles_n = (N + T - 1) / T;
   const int ntiles = tiles_m * tiles_n;
-  static int n_cu = 0;
-  if (n_cu == 0) {
-    hipDeviceProp_t prop;
-    n_cu = hipGetDeviceProperties(&prop, grad.get_device()) == hipSuccess ? prop.multiProcessorCount : 256;
-  }
+  const int n_cu = cu_count(grad.get_device());
   // split-K from the wave-quantisation cost model (host_plan.h, sanitizer-tested on the host);
   // the ring16o variants (6, 8) may also take a split-tail plan (plan_wgrad)
   const SplitK uplan = plan_wgrad_splits(M, N, K, T, n_cu, T == 256 ? BK2 : BK);
@@ -692,4 +865,57 @@ void wgrad_gemm(torch::Tensor dy, torch::Tensor x, torch::Tensor grad, int64_t t
   const int64_t n4 = (int64_t)M * N / 4;
   hipLaunchKernelGGL(slab_reduce_kernel, dim3((int)std::min<int64_t>((n4 + 255) / 256, 2048)), dim3(256), 0, stream,
                      slab.data_ptr<float>(), grad.data_ptr<float>(), n4, splits, n4, acc_in);
+}
+
+// grads[i][M_i][N_i] (+)= dys[i]ᵀ·xs[i]: in one launch where plan_wgrad_group says that this is faster, else (and for more than 8
+// products, several K, or operands that are not 16-byte aligned) one after the other by wgrad_gemm's 256-tile kernel.
+void wgrad_group(std::vector<torch::Tensor> dys, std::vector<torch::Tensor> xs, std::vector<torch::Tensor> grads,
+                 std::vector<bool> accumulate, int64_t variant) {
+  const size_t n = dys.size();
+  TORCH_CHECK(xs.size() == n && grads.size() == n && accumulate.size() == n, "wgrad_group: one of each per product");
+  if (n == 0) return;
+  auto aligned = [](const torch::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+  bool together = n <= (size_t)kGroupItems;
+  int Ms[kGroupItems], Ns[kGroupItems];
+  for (size_t i = 0; i < n; ++i) {
+    check_wgrad(dys[i], xs[i], grads[i]);
+    together = together && dys[i].size(0) == dys[0].size(0) && dys[i].get_device() == dys[0].get_device() &&
+               dys[i].stride(0) >= dys[i].size(1) && xs[i].stride(0) >= xs[i].size(1) && aligned(dys[i]) && aligned(xs[i]) &&
+               aligned(grads[i]);
+    if (together) Ms[i] = dys[i].size(1), Ns[i] = xs[i].size(1);
+  }
+  const int K = dys[0].size(0);
+  const int TN = 128, TM = together ? plan_wgrad_group(Ms, Ns, (int)n, K, cu_count(dys[0].get_device())) : 0;
+  if (TM == 0) {
+    for (size_t i = 0; i < n; ++i) wgrad_gemm(dys[i], xs[i], grads[i], 256, variant, accumulate[i]);
+    return;
+  }
+  WgradItems items{};
+  items.n = (int)n;
+  items.K = K;
+  int64_t tiles = 0;
+  for (size_t i = 0; i < n; ++i) {
+    const int tn = (Ns[i] + TN - 1) / TN;
+    items.item[i] = WgradItem{reinterpret_cast<const bf16*>(dys[i].data_ptr()), reinterpret_cast<const bf16*>(xs[i].data_ptr()),
+                              grads[i].data_ptr<float>(), Ms[i], Ns[i], (int)dys[i].stride(0), (int)xs[i].stride(0), tn,
+                              (int)tiles, accumulate[i] ? 1 : 0};
+    tiles += (int64_t)((Ms[i] + TM - 1) / TM) * tn;
+    TORCH_CHECK(tiles < (int64_t)1 << 31, "wgrad_group: too many tiles");
+  }
+  auto stream = at::hip::getCurrentHIPStream();
+  auto launch = [&](auto wm) {
+    constexpr int WM = decltype(wm)::value, lds = 4 * 64 * (64 * WM + 128);
+    hipFuncSetAttribute(reinterpret_cast<const void*>(wgrad_group_kernel<WM, 2>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                        lds);
+    hipLaunchKernelGGL((wgrad_group_kernel<WM, 2>), dim3((unsigned)tiles), dim3(128 * WM), lds, stream, items);
+  };
+  if (TM == 256) launch(std::integral_constant<int, 4>{});
+  else launch(std::integral_constant<int, 2>{});
+}
+
+// the tile that plan_wgrad_group takes for products [Ms[i], Ns[i]] over K (0: each by itself)
+int64_t wgrad_group_tile(std::vector<int64_t> Ms, std::vector<int64_t> Ns, int64_t K, int64_t n_cu) {
+  std::vector<int> m(Ms.begin(), Ms.end()), k(Ns.begin(), Ns.end());
+  TORCH_CHECK(m.size() == k.size());
+  return plan_wgrad_group(m.data(), k.data(), (int)m.size(), (int)K, (int)n_cu);
 }

@@ -83,6 +83,39 @@ inline WgradPlan plan_wgrad(int M, int N, int K, int tile, int n_cu, int bk) {
   return r;
 }
 
+// Several weight gradients over the same K tokens: one launch of wgrad_group_kernel with tiles of tile_m × 128 (128 or 256), or
+// each by the split kernel on its own (0). All estimates are fits (µs) to GPT-2's and Gemma-3 1B's layers, their heads and a
+// layer of width 256 at 17 to 16384 tokens: a 32-token stage takes 0.43 with a card full of tiles (0.30 for one tile of 128 to a
+// CU), 0.6 to 0.75 in the split kernel, which costs 20 whatever its size; outputs are written at 5.5 TB/s. Measured, one by one /
+// together: GPT-2's layer 99 / 14 at 256 tokens, 134 / 62 at 3885, 275 / 243 at 16384; Gemma's 117 / 38, 302 / 239, 886 / 953; a
+// head of 50304 x 768 119 / 104 at 1024, 176 / 189 at 2048; a layer of width 256 104 / 81 at 8192, 120 / 154 at 16384.
+inline int plan_wgrad_group(const int* M, const int* N, int n, int K, int n_cu) {
+  if (n <= 0 || K <= 0) return 0;
+  const double steps = (double)(((int64_t)K + 31) / 32);
+  const int64_t cus = std::max(1, n_cu);
+  double single = 0, store = 0;
+  int64_t small = 0, large = 0;
+  for (int i = 0; i < n; ++i) {
+    if (M[i] <= 0 || N[i] <= 0) return 0;
+    const int64_t tm = ((int64_t)M[i] + 127) / 128, tn = ((int64_t)N[i] + 127) / 128;
+    small += tm * tn;
+    large += (tm + 1) / 2 * tn;
+    const double out = 4.0 * M[i] * N[i] / 5.5e6;
+    store += out;
+    const WgradPlan p = plan_wgrad(M[i], N[i], K, 256, n_cu, 32);
+    const int64_t main = (int64_t)p.main_tiles * p.main_splits;
+    single += 20 + (main > cus ? 0.75 : 0.6) * (double)((main + cus - 1) / cus) * p.main_klen / 32;
+    if (p.tail_splits > 0) single += 0.75 * p.tail_klen / 32;
+    single += p.main_splits > 1 ? 3 + 8.0 * p.main_splits * M[i] * N[i] / 20e6 : out;
+  }
+  const int64_t rest = small % (2 * cus);
+  const double t128 = steps * (0.43 * (double)(small / (2 * cus)) + (rest > cus ? 0.43 : rest > 0 ? 0.30 : 0.0)) *
+                      (1.0 + std::max(0, K - 4096) / 32768.0);  // operands from beyond the XCD's L2
+  const double t256 = steps * 0.43 * (double)((large + cus - 1) / cus);
+  if (std::min(t128, t256) + store + 6 >= single) return 0;
+  return t128 <= t256 ? 128 : 256;
+}
+
 // Slices of the two-stage deterministic column reduction (reduce.h): ~sqrt(G) balances stages.
 inline int reduce_slices(int G) {
   int s = 1;

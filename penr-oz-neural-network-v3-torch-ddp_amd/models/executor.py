@@ -491,7 +491,9 @@ class GPTExecutor:
         self.dresid = torch.empty(N, C, dtype=f32, device=dev)
         # gradient buffers read by the side-stream weight-gradient GEMMs rotate between two
         # copies, so the main stream can produce the next one while the side stream still reads
-        self.dresid_bf2 = [torch.empty(N, C, dtype=bf, device=dev) for _ in range(2)]
+        # (four of the residual's gradient where a layer's weight gradients run together and read two of them)
+        self.dresid_bf2 = [torch.empty(N, C, dtype=bf, device=dev)
+                           for _ in range(4 if N <= self.WGRAD_GROUP_TOKENS else 2)]
         self.d_f2 = [torch.empty(N, F, dtype=bf, device=dev) for _ in range(2)]
         self.dqkv2 = [torch.empty(N, 3 * C, dtype=bf, device=dev) for _ in range(2)]
         self.d_c = torch.empty(N, C, dtype=bf, device=dev)
@@ -773,8 +775,8 @@ class GPTExecutor:
         least = self.side_min_flops(self.L, params) if self.SIDE_MIN_FLOPS is None else self.SIDE_MIN_FLOPS
         self._side = self._side_stream if 6 * tokens * params >= least else None
 
-    def _side_call(self, operand: Tensor, fn):
-        """Run ``fn`` (gradient-only work reading ``operand``) on the side stream, or inline."""
+    def _side_call(self, operands, fn):
+        """Run ``fn`` (gradient-only work reading ``operands``, one tensor or several) on the side stream, or inline."""
         if getattr(self, "_side", None) is None:
             fn()
             return
@@ -786,7 +788,29 @@ class GPTExecutor:
             fn()
             done = torch.cuda.Event()
             done.record(self._side)
-        self._buf_free[operand.data_ptr()] = done
+        for t in (operands,) if isinstance(operands, Tensor) else operands:
+            self._buf_free[t.data_ptr()] = done
+
+    # a layer's weight gradients go in one launch up to this many tokens (GPT-2's four by themselves 275 us at 16384, together
+    # 243; longer ones fill the card each and start as soon as their operand is there)
+    WGRAD_GROUP_TOKENS = 16384
+
+    def _gather_wgrads(self, tokens: int):
+        """From here to :meth:`_flush_wgrads` weight gradients are gathered; their operands stay untouched until then."""
+        self._wgrad_queue = [] if tokens <= self.WGRAD_GROUP_TOKENS else None
+
+    def _flush_wgrads(self):
+        queue, self._wgrad_queue = getattr(self, "_wgrad_queue", None), None
+        if queue:
+            dys, xs, grads, accumulate = zip(*queue)
+            self._side_call(dys, lambda: gemm_ops.wgrad_group(dys, xs, grads, accumulate))
+
+    def _emit_wgrad(self, dy: Tensor, x: Tensor, g: Tensor, accumulate: bool):
+        queue = getattr(self, "_wgrad_queue", None)
+        if queue is None:
+            self._side_call(dy, lambda: gemm_ops.wgrad(dy, x, g, accumulate))
+        else:
+            queue.append((dy, x, g, accumulate))
 
     def _wgrad(self, dy: Tensor, x: Tensor, p: Tensor):
         self._wgrad_into(id(p), dy, x, self.grad(p))
@@ -817,7 +841,7 @@ class GPTExecutor:
         parts = stale.get(key)
         if parts and parts == [rng]:  # the whole learned range, untouched this step: overwrite
             del stale[key]
-            self._side_call(dy, lambda: gemm_ops.wgrad(dy, x, g, False))
+            self._emit_wgrad(dy, x, g, False)
             return
         if parts:
             keep = []
@@ -836,7 +860,7 @@ class GPTExecutor:
                 stale[key] = keep
             else:
                 del stale[key]
-        self._side_call(dy, lambda: gemm_ops.wgrad(dy, x, g, True))
+        self._emit_wgrad(dy, x, g, True)
 
     def _finish_wgrad_bookkeeping(self):
         """End of a backward: learn the ranges once; clear any part of a range zero_grad skipped
@@ -902,6 +926,7 @@ class GPTExecutor:
             # the next step may be of one stream: nothing stays deferred, and the main stream (its allocations too)
             # comes behind what the side stream still has to do
             self._defer_reductions(False)
+            self._wgrad_queue = None
             self._join_side()
             raise
         finally:
@@ -961,6 +986,7 @@ class GPTExecutor:
             layer_range = trace_range(f"backward.block{l}")
             layer_range.__enter__()
             b = s.blocks[l]
+            self._gather_wgrads(N)
             d_f, dqkv = self._reuse(self.d_f2[l & 1]), self._reuse(self.dqkv2[l & 1])
             dres_bf = self.dresid_bf2[rb]
             # ---- MLP branch
@@ -971,7 +997,7 @@ class GPTExecutor:
             torch.mm(d_f, self._dgrad_w(b.fc.weight), out=self.d_c)
             self._wgrad(d_f, self.ln2[l], b.fc.weight)
             _, _, mean, rstd = self.stats[l]
-            rb ^= 1
+            rb = (rb + 1) % len(self.dresid_bf2)
             dres_bf = self._reuse(self.dresid_bf2[rb])
             dp, ds = self._drop(True, seed, l, 0)
             norm_ops.ln_bwd(self.d_c, self.resid_mid[l], mean, rstd, self.f32(b.ln2.weight), self.dresid, True,
@@ -987,9 +1013,10 @@ class GPTExecutor:
                                dbias=self.grad(b.qkv.bias))
             torch.mm(dqkv, self._dgrad_w(b.qkv.weight), out=self.d_c)
             self._wgrad(dqkv, self.ln1[l], b.qkv.weight)
+            self._flush_wgrads()
             mean, rstd, _, _ = self.stats[l]
             prev_bias = self.grad(s.blocks[l - 1].fc2.bias) if l > 0 else None
-            rb ^= 1
+            rb = (rb + 1) % len(self.dresid_bf2)
             dp, ds = self._drop(True, seed, l - 1, 1) if l > 0 else (0.0, 0)
             norm_ops.ln_bwd(self.d_c, self.resid[l], mean, rstd, self.f32(b.ln1.weight), self.dresid, True,
                             self._reuse(self.dresid_bf2[rb]) if l > 0 else None, self.grad(b.ln1.weight),

@@ -521,6 +521,7 @@ class GemmaExecutor(GPTExecutor):
             layer_range = trace_range(f"backward.block{l}")
             layer_range.__enter__()
             b = s.blocks[l]
+            self._gather_wgrads(N)
             H, Hkv, D = b.H, b.Hkv, b.D
             QKV = (H + 2 * Hkv) * D
             db = self.d_branch2[rb]
@@ -552,6 +553,7 @@ class GemmaExecutor(GPTExecutor):
             k.rope_qkv(d_qkv.view(B, T, -1), cos, sin, H, Hkv, D, True, dqr)
             torch.mm(dqr, self._dgrad(b.qkv.weight, self.bf16(b.qkv.weight)), out=self.d_c)
             self._wgrad(dqr, self.y_in[l], b.qkv.weight)
+            self._flush_wgrads()
             # ---- the combine that produced y_in[l]: block l-1's MLP combine (or the embedding norm)
             if l > 0:
                 pb = s.blocks[l - 1]

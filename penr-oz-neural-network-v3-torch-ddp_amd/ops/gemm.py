@@ -47,17 +47,34 @@ def reference_wgrad(dy: Tensor, x: Tensor, grad: Tensor, accumulate: bool = True
         grad.copy_(dy.float().t() @ x.float())
 
 
+def _native_wgrad(dy: Tensor, x: Tensor) -> bool:
+    return (use_kernels(dy) and _native_ok(dy.shape[1], x.shape[1], dy.stride(0)) and dy.dtype == torch.bfloat16
+            and x.dtype == torch.bfloat16 and dy.stride(0) % 8 == 0 and x.stride(0) % 8 == 0)
+
+
 def wgrad(dy: Tensor, x: Tensor, grad: Tensor, accumulate: bool = True) -> None:
     """grad += dyᵀ·x, or grad = dyᵀ·x with accumulate=False (the first weight-gradient write of a
     step whose zero_grad skipped this range)."""
-    if (use_kernels(dy) and _native_ok(dy.shape[1], x.shape[1], dy.stride(0)) and dy.dtype == torch.bfloat16
-            and x.dtype == torch.bfloat16 and dy.stride(0) % 8 == 0 and x.stride(0) % 8 == 0):
-        kernels().wgrad_gemm(dy, x, grad, 256, _wgrad_variant(dy.shape[0]), accumulate)
+    if _native_wgrad(dy, x):
+        if WGRAD_VARIANT:
+            kernels().wgrad_gemm(dy, x, grad, 256, WGRAD_VARIANT, accumulate)
+        else:
+            kernels().wgrad_group([dy], [x], [grad], [accumulate], _wgrad_variant(dy.shape[0]))
     elif dy.is_cuda:
         prod = torch.mm(dy.t(), x, out_dtype=torch.float32)
         grad.add_(prod) if accumulate else grad.copy_(prod)
     else:
         reference_wgrad(dy, x, grad, accumulate)
+
+
+def wgrad_group(dys, xs, grads, accumulate) -> None:
+    """:func:`wgrad` for each of several products over the same tokens, in one launch where that is faster (the rule,
+    ``plan_wgrad_group`` in ``csrc/kernels/host_plan.h``, knows their sizes)."""
+    if not WGRAD_VARIANT and all(_native_wgrad(dy, x) for dy, x in zip(dys, xs)):
+        kernels().wgrad_group(list(dys), list(xs), list(grads), list(accumulate), _wgrad_variant(dys[0].shape[0]))
+        return
+    for args in zip(dys, xs, grads, accumulate):
+        wgrad(*args)
 
 
 # ---- library GEMM solution choice (hipBLASLt / rocBLAS through torch) -----------------------
