@@ -29,6 +29,10 @@ void decode_gemv_pair(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64
 void decode_gemm_acc(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias, torch::Tensor resid,
                      int64_t flags);
 void decode_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64_t kind);
+// rows_gemm.hip
+c10::optional<torch::Tensor> rows_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
+                                       c10::optional<torch::Tensor> out, bool fp32, bool in_order);
+int64_t rows_gemm_tile(int64_t M, int64_t N, int64_t K, bool in_order);
 // packed_rows.hip
 void row_norm_add(c10::optional<torch::Tensor> tok, c10::optional<torch::Tensor> table,
                   c10::optional<torch::Tensor> x_in, c10::optional<torch::Tensor> x_out,
@@ -145,6 +149,10 @@ PYBIND11_MODULE(penroz_serve, m) {
         pybind11::arg("cos") = pybind11::none(), pybind11::arg("sin") = pybind11::none(),
         pybind11::arg("pairs_per_wave") = 0,
         "paired-row decode GEMV for 1..4 rows: gated MLP (mode 1) or RoPE QKV (mode 2) epilogue");
+  m.def("rows_gemm", &rows_gemm, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("bias"), pybind11::arg("out"),
+        pybind11::arg("fp32") = false, pybind11::arg("in_order") = false);
+  m.def("rows_gemm_tile", &rows_gemm_tile, pybind11::arg("M"), pybind11::arg("N"), pybind11::arg("K"),
+        pybind11::arg("in_order") = false);
   m.def("decode_gemm_acc", &decode_gemm_acc, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("bias"),
         pybind11::arg("resid"), pybind11::arg("flags") = 0,
         "batched decode: resid += x·wᵀ + bias (fp32 residual, in place)");

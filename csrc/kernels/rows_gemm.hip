@@ -1,0 +1,224 @@
+// Linear layers of a few rows to a few thousand: out[M, N] = x[M, K] · W[N, K]ᵀ (+ bias), bf16 operands, fp32 sums, bf16 or fp32 out.
+//
+// Below products that fill the card with tiles of 256 lie the short steps: batches of up to 64 sequences, 256 training tokens,
+// prompts of a few hundred rows. Their products need 1 to 5 us of memory or matrix time; what bounds them is how many bytes the
+// card has on the way (about 1.1 us a trip, the ring's 96 KB per CU), so the tile is the largest that still gives nearly every CU
+// one (rows_gemm_plan, host_plan.h). A workgroup of 4 waves owns 32×32, 32×64, 64×64 or 64×128 outputs; stages of 64 to 256 columns
+// arrive by LDS-DMA in a ring (128-byte row pieces, whole cache lines, chunks permuted on the source side so that a fragment read
+// covers all banks); the waves split the tile (WM × WN) or the columns of a stage (WK, added through LDS at the end, in order).
+// Tiles that share weights run on one XCD. In order (WK = 1) a sum is one chain of MFMAs over k, as in the library's unsplit
+// kernels, and bit for bit theirs at K = 768: training steps take that form, where a rounding that falls otherwise changes every
+// later layer's. With the columns split, 64 x 2048 x 2048 takes 6.1 us instead of 7.0, 64 x 768 x 3072 7.4 instead of 9.0. us, library / here (weights from memory): 64 x 768 x 768 7.1 / 3.8, 64 x 2048 x 2048
+// 8.9 / 6.1, 64 x 2048 x 6144 19.0 / 16.3, 256 x 2304 x 768 7.7 / 6.5, 1024 x 1152 x 1024 9.7 / 9.2; at 16 rows, skinny_gemm / here:
+// 768 x 768 9.7 / 3.6, 2048 x 2048 7.1 / 5.7, 7232 x 2048 12.3 / 8.2. A call costs the host 4 us, the library's 19. Tiles of 128×128
+// in rings of two to four stages were no faster than the library anywhere.
+#include "common.h"
+#include "host_plan.h"
+#include <torch/extension.h>
+#include <ATen/hip/HIPContext.h>
+
+namespace penroz {
+namespace {
+
+typedef __bf16 rg_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float rg_f32x4 __attribute__((ext_vector_type(4)));
+
+template <int P, int LEFT>
+__device__ __forceinline__ void wait_stages(int left) {  // all but the newest `left` stages of P loads have landed
+  if constexpr (LEFT > 0) {
+    if (left >= LEFT) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEFT * P) : "memory");
+      return;
+    }
+    wait_stages<P, LEFT - 1>(left);
+  } else {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+}
+
+template <int FM, int FN, int WM, int WN, int WK, int KS, int NBUF, typename OUT>
+__global__ void __launch_bounds__(64 * WM * WN * WK) rows_gemm_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
+                                                                      const bf16* __restrict__ bias, OUT* __restrict__ out, int M,
+                                                                      int N, int K, int ldx, int ldw, int ldo, int tiles_m) {
+  constexpr int TM = 16 * FM * WM, TN = 16 * FN * WN, NW = WM * WN * WK;
+  constexpr int SUB = (TM + TN) * 128, STAGE = WK * KS * SUB;  // a sub-slice of 64 columns: x rows, then W rows
+  constexpr int COLS = 64 * WK * KS, PIECES = STAGE / 1024 / NW, PER_SUB = SUB / 1024;
+  static_assert(STAGE % (1024 * NW) == 0 && (NBUF - 2) * PIECES <= 63 && NBUF >= 2, "ring geometry");
+  static_assert(WK == 1 || WK * WM * WN * FM * FN * 1024 <= NBUF * STAGE, "the waves' sums fit the ring");
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int nwg = gridDim.x, wg = blockIdx.x;
+  const int xcd = wg & 7, qd = nwg >> 3, rd = nwg & 7;
+  const int id = (xcd < rd ? xcd * (qd + 1) : rd * (qd + 1) + (xcd - rd) * qd) + (wg >> 3);
+  const int tn = id / tiles_m, tm = id - tn * tiles_m;
+  const int m0 = tm * TM, n0 = tn * TN;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wk = wv / (WM * WN), wm = wv / WN % WM, wn = wv % WN;
+
+  // piece p of a stage: 8 rows of a sub-slice; lane -> row (lane >> 3), 16-byte chunk (lane & 7) ^ swizzle
+  const char* src[PIECES];
+  int kofs[PIECES];
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    const int p = wv * PIECES + i, sub = p / PER_SUB, row = (p % PER_SUB) * 8 + (lane >> 3);
+    const int ch = (lane & 7) ^ ((row >> 1) & 7);
+    kofs[i] = 64 * sub + 8 * ch;
+    const bf16* r = row < TM ? x + (size_t)min(m0 + row, M - 1) * ldx : w + (size_t)min(n0 + row - TM, N - 1) * ldw;
+    src[i] = reinterpret_cast<const char*>(r + kofs[i]);
+  }
+  const unsigned lds = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_void_t*)smem + wv * PIECES * 1024);
+  const char* zero = reinterpret_cast<const char*>(g_zero16);
+  auto dma = [&](int st, int buf) {
+    const int k0 = st * COLS;
+    if (k0 + COLS <= K) {
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i) glds16(src[i] + (size_t)k0 * 2, lds + buf * STAGE + i * 1024);
+    } else {
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i)
+        glds16(k0 + kofs[i] < K ? src[i] + (size_t)k0 * 2 : zero, lds + buf * STAGE + i * 1024);
+    }
+  };
+
+  const int r16 = lane & 15, kq = lane >> 4;
+  auto frag = [&](const char* t, int row, int ch) {
+    return *reinterpret_cast<const uint4*>(t + row * 128 + ((ch ^ ((row >> 1) & 7)) << 4));
+  };
+  rg_f32x4 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = rg_f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int nst = (K + COLS - 1) / COLS;
+#pragma unroll
+  for (int t = 0; t < NBUF - 1; ++t)
+    if (t < nst) dma(t, t);
+  wait_stages<PIECES, NBUF - 2>(nst - 1);
+  __syncthreads();
+  int buf = 0;
+  for (int st = 0; st < nst; ++st) {
+    if (st + NBUF - 1 < nst) dma(st + NBUF - 1, buf == 0 ? NBUF - 1 : buf - 1);  // freed by the barrier of the step before
+#pragma unroll
+    for (int s = 0; s < 2 * KS; ++s) {
+      const char* xt = smem + buf * STAGE + (wk * KS + (s >> 1)) * SUB;
+      const char* wt = xt + TM * 128;
+      uint4 a[FM], b[FN];
+#pragma unroll
+      for (int j = 0; j < FN; ++j) b[j] = frag(wt, 16 * (FN * wn + j) + r16, 4 * (s & 1) + kq);
+#pragma unroll
+      for (int i = 0; i < FM; ++i) a[i] = frag(xt, 16 * (FM * wm + i) + r16, 4 * (s & 1) + kq);
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(rg_bf16x8, b[j]),
+                                                              __builtin_bit_cast(rg_bf16x8, a[i]), acc[i][j], 0, 0, 0);
+    }
+    if (st + 1 < nst) wait_stages<PIECES, NBUF - 2>(nst - 2 - st);
+    __syncthreads();
+    buf = buf + 1 == NBUF ? 0 : buf + 1;
+  }
+  // a lane holds row m = r16 of a block, columns 4·kq .. + 3
+  auto store = [&](int i, int j, rg_f32x4 v) {
+    const int m = m0 + 16 * (FM * wm + i) + r16, n = n0 + 16 * (FN * wn + j) + 4 * kq;
+    if (m >= M || n >= N) return;
+    OUT* o = out + (size_t)m * ldo + n;
+    const int cnt = min(4, N - n);
+    if (bias != nullptr)
+      for (int r = 0; r < cnt; ++r) v[r] += to_f(bias[n + r]);
+    if (cnt == 4 && (ldo & 3) == 0) {
+      if constexpr (sizeof(OUT) == 2) {
+        bf16 h[4] = {from_f<bf16>(v[0]), from_f<bf16>(v[1]), from_f<bf16>(v[2]), from_f<bf16>(v[3])};
+        *reinterpret_cast<uint2*>(o) = *reinterpret_cast<const uint2*>(h);
+      } else {
+        *reinterpret_cast<float4*>(o) = float4{v[0], v[1], v[2], v[3]};
+      }
+    } else {
+      for (int r = 0; r < cnt; ++r) o[r] = from_f<OUT>(v[r]);
+    }
+  };
+  if constexpr (WK == 1) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) store(i, j, acc[i][j]);
+  } else {
+    // every wave leaves its sums, then adds FM·FN / WK blocks of all WK slices
+    static_assert(FM * FN % WK == 0, "blocks per wave");
+    rg_f32x4* red = reinterpret_cast<rg_f32x4*>(smem);
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) red[(wv * FM * FN + i * FN + j) * 64 + lane] = acc[i][j];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        if ((i * FN + j) % WK != wk) continue;
+        rg_f32x4 v = rg_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < WK; ++k) v += red[((k * WM * WN + wm * WN + wn) * FM * FN + i * FN + j) * 64 + lane];
+        store(i, j, v);
+      }
+  }
+}
+
+}  // namespace
+}  // namespace penroz
+
+using namespace penroz;
+
+// x · wᵀ (+ bias) into out, or (none given) into a new tensor, fp32 or of x's type; in_order: each sum in one chain over k. None where rows_gemm_plan leaves the product to
+// the library or a row is not of 16-byte pieces.
+c10::optional<torch::Tensor> rows_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
+                                       c10::optional<torch::Tensor> out_opt, bool fp32, bool in_order) {
+  const bool given = out_opt.has_value() && out_opt->defined(), has_bias = bias.has_value() && bias->defined();
+  if (!(x.is_cuda() && w.is_cuda() && x.get_device() == w.get_device() && x.scalar_type() == torch::kBFloat16 &&
+        w.scalar_type() == torch::kBFloat16 && x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1)))
+    return c10::nullopt;
+  const int64_t M = x.size(0), N = w.size(0), K = x.size(1);
+  auto rows_ok = [&](const torch::Tensor& t) {
+    return t.stride(1) == 1 && t.stride(0) >= K && t.stride(0) % 8 == 0 && t.stride(0) < (int64_t)1 << 30 &&
+           reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  const int tile = rows_gemm_plan(M, N, K, in_order);
+  if (tile == 0 || !rows_ok(x) || !rows_ok(w)) return c10::nullopt;
+  if (has_bias && !(bias->is_cuda() && bias->scalar_type() == torch::kBFloat16 && bias->is_contiguous() && bias->numel() == N))
+    return c10::nullopt;
+  if (given) {
+    const torch::Tensor& o = *out_opt;
+    if (!(o.is_cuda() && o.scalar_type() == (fp32 ? torch::kFloat32 : torch::kBFloat16) && o.dim() == 2 && o.size(0) == M &&
+          o.size(1) == N && o.stride(1) == 1 && o.stride(0) >= N && o.stride(0) < (int64_t)1 << 30 &&
+          (o.stride(0) % 4 != 0 || reinterpret_cast<uintptr_t>(o.data_ptr()) % (4 * o.element_size()) == 0)))
+      return c10::nullopt;
+  }
+  torch::Tensor out = given ? *out_opt : torch::empty({M, N}, x.options().dtype(fp32 ? torch::kFloat32 : torch::kBFloat16));
+  const bf16* bp = has_bias ? reinterpret_cast<const bf16*>(bias->data_ptr()) : nullptr;
+  auto stream = at::hip::getCurrentHIPStream();
+  auto launch = [&](auto kern, int threads, int lds, int TM, int TN, auto* o) {
+    const int64_t tiles_m = (M + TM - 1) / TM, tiles = tiles_m * ((N + TN - 1) / TN);
+    hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(threads), lds, stream, reinterpret_cast<const bf16*>(x.data_ptr()),
+                       reinterpret_cast<const bf16*>(w.data_ptr()), bp, o, (int)M, (int)N, (int)K, (int)x.stride(0),
+                       (int)w.stride(0), (int)out.stride(0), (int)tiles_m);
+  };
+#define PENROZ_RG(FM, FN, WM, WN, WK, KS, NB)                                                                    \
+  launch(rows_gemm_kernel<FM, FN, WM, WN, WK, KS, NB, OUT>, 64 * WM * WN * WK,                                   \
+         NB * WK * KS * 128 * 16 * (FM * WM + FN * WN), 16 * FM * WM, 16 * FN * WN, o)
+  auto typed = [&](auto* o) {
+    using OUT = std::remove_pointer_t<decltype(o)>;
+    if (tile == 1 && in_order) PENROZ_RG(1, 1, 2, 2, 1, 2, 4);
+    else if (tile == 1) PENROZ_RG(2, 2, 1, 1, 4, 1, 4);
+    else if (tile == 2) PENROZ_RG(2, 4, 1, 1, 4, 1, 3);
+    else if (tile == 3) PENROZ_RG(2, 2, 2, 2, 1, 2, 4);
+    else if (tile == 4) PENROZ_RG(2, 2, 2, 2, 1, 2, 2);
+    else PENROZ_RG(2, 4, 2, 2, 1, 1, 3);
+  };
+#undef PENROZ_RG
+  if (fp32) typed(out.data_ptr<float>());
+  else typed(reinterpret_cast<bf16*>(out.data_ptr()));
+  return out;
+}
+
+int64_t rows_gemm_tile(int64_t M, int64_t N, int64_t K, bool in_order) { return rows_gemm_plan(M, N, K, in_order); }

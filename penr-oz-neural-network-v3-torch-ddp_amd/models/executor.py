@@ -509,10 +509,7 @@ class GPTExecutor:
     # ------------------------------------------------------------------ forward
     def _linear(self, x: Tensor, lin: nn.Linear, out: Tensor | None = None) -> Tensor:
         w = self.bf16(lin.weight)
-        if lin.bias is not None:
-            return torch.addmm(self.bf16(lin.bias), x, w.t(), out=out) if out is not None else \
-                torch.addmm(self.bf16(lin.bias), x, w.t())
-        return torch.mm(x, w.t(), out=out) if out is not None else torch.mm(x, w.t())
+        return gemm_ops.train_linear(x, w, None if lin.bias is None else self.bf16(lin.bias), out)
 
     def _drop(self, training: bool, seed: int, l: int, branch: int) -> tuple[float, int]:
         """(p, mask seed) of residual-dropout site (layer l, branch 0 = attention / 1 = MLP)."""
@@ -571,7 +568,7 @@ class GPTExecutor:
         """lm_head GEMM of token rows [r0, r1) into ``buf`` ([rows, ld]); returns the [rows, Vp]
         view (columns V..Vp-1 are the pad rows' exact zeros; slice [:, :V] for the logits)."""
         lg = buf[: r1 - r0, : self.Vp]
-        torch.mm(self.lnf_out[r0:r1], self.head_w().t(), out=lg)
+        gemm_ops.train_linear(self.lnf_out[r0:r1], self.head_w(), None, lg)
         return lg
 
     def _full_logits(self, padded: bool = False) -> Tensor:
@@ -966,7 +963,7 @@ class GPTExecutor:
             # CE rewrites the V real columns with dlogits; the pad columns stay the exact zeros of
             # the pad rows, so the padded dgrad / wgrad equal the unpadded ones (pad rows get 0)
             loss += fused_ops.cross_entropy_fwd_bwd(lg[:, :V], tg[r0:r1], scale / N).sum()
-            torch.mm(lg[:, : w_dgrad.shape[0]], w_dgrad, out=self.d_c[r0:r1])
+            gemm_ops.train_linear(lg[:, : w_dgrad.shape[0]], w_dgrad.t(), None, self.d_c[r0:r1])
             self._wgrad_into(id(s.head.weight), lg, self.lnf_out[r0:r1], self.head_grad())
         loss *= scale / N
         mean, rstd = self.statsf
@@ -994,7 +991,7 @@ class GPTExecutor:
             gemm_ops.dgrad_gelu(dres_bf, self._dgrad_w(b.fc2.weight).t(), self.fcpre[l], d_f, self.grad(b.fc.bias),
                                 s.gelu_approx)
             self._wgrad(dres_bf, self.fcact[l], b.fc2.weight)
-            torch.mm(d_f, self._dgrad_w(b.fc.weight), out=self.d_c)
+            gemm_ops.train_linear(d_f, self._dgrad_w(b.fc.weight).t(), None, self.d_c)
             self._wgrad(d_f, self.ln2[l], b.fc.weight)
             _, _, mean, rstd = self.stats[l]
             rb = (rb + 1) % len(self.dresid_bf2)
@@ -1004,14 +1001,14 @@ class GPTExecutor:
                             dres_bf, self.grad(b.ln2.weight), self.grad(b.ln2.bias), self.grad(b.proj.bias),
                             dropout_p=dp, dropout_seed=ds)
             # ---- attention branch
-            torch.mm(dres_bf, self._dgrad_w(b.proj.weight), out=self.d_c)
+            gemm_ops.train_linear(dres_bf, self._dgrad_w(b.proj.weight).t(), None, self.d_c)
             self._wgrad(dres_bf, self.att[l], b.proj.weight)
             # the qkv bias gradient comes out of the attention-backward epilogues (partials finished
             # on the side stream by the deferred reduction)
             attn_ops.flash_bwd(self.d_c.view(B, T, C), self.qkv[l].view(B, T, 3 * C), self.att[l].view(B, T, C),
                                self.lse[l], s.H, s.H, s.D, b.attn.dropout, seed + l, dqkv=dqkv.view(B, T, 3 * C),
                                dbias=self.grad(b.qkv.bias))
-            torch.mm(dqkv, self._dgrad_w(b.qkv.weight), out=self.d_c)
+            gemm_ops.train_linear(dqkv, self._dgrad_w(b.qkv.weight).t(), None, self.d_c)
             self._wgrad(dqkv, self.ln1[l], b.qkv.weight)
             self._flush_wgrads()
             mean, rstd, _, _ = self.stats[l]

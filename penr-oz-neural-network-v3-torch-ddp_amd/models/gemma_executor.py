@@ -357,7 +357,7 @@ class GemmaExecutor(GPTExecutor):
         return tab
 
     def _mm(self, x: Tensor, w: Tensor, out: Tensor) -> Tensor:
-        return torch.mm(x, w.t(), out=out)
+        return gemm_ops.train_linear(x, w, None, out)
 
     # ---- row-split AdamW of the embedding table ------------------------------------------------
     # The table's gradient is zero on every row this step's tokens do not touch (8k of 262k rows
@@ -501,7 +501,7 @@ class GemmaExecutor(GPTExecutor):
             if lg is None:
                 lg = self._head_logits(r0, r1, self._reuse(self._head_bufs[i % len(self._head_bufs)]))
             loss += fused_ops.cross_entropy_fwd_bwd(lg, tg[r0:r1], scale / N).sum()
-            torch.mm(lg, w_head, out=self.d_c[r0:r1])
+            gemm_ops.train_linear(lg, w_head.t(), None, self.d_c[r0:r1])
             self._wgrad(lg, self.lnf_out[r0:r1], s.head.weight)
         loss *= scale / N
         if cap:
@@ -527,11 +527,11 @@ class GemmaExecutor(GPTExecutor):
             db = self.d_branch2[rb]
             # ---- MLP: down dgrad / wgrad, packed gated backward, gate|up dgrad / wgrad
             d_g = self._rows(self.d_g, N, b.F)
-            torch.mm(db, self._dgrad(b.mlp.down_proj.weight, self.bf16(b.mlp.down_proj.weight)), out=d_g)
+            gemm_ops.train_linear(db, self._dgrad(b.mlp.down_proj.weight, self.bf16(b.mlp.down_proj.weight)).t(), None, d_g)
             self._wgrad(db, self.g[l], b.mlp.down_proj.weight)
             dgu = self._rows(self._reuse(self.d_gu2[l & 1]), N, 2 * b.F)
             k.gated_act_bwd_packed(d_g, self.gu[l], dgu, s.act)
-            torch.mm(dgu, self._dgrad(b.mlp.gate_proj.weight, self.gu_bf16(b)), out=self.d_c)
+            gemm_ops.train_linear(dgu, self._dgrad(b.mlp.gate_proj.weight, self.gu_bf16(b)).t(), None, self.d_c)
             self._wgrad_into(id(b.mlp.gate_proj.weight), dgu, self.y_mlp[l], self.gu_grad(b))
             # ---- attention combine: dy = d(pre-MLP norm output), dh_in = dresid (grad of mid[l])
             pa = b.post_attn
@@ -543,7 +543,7 @@ class GemmaExecutor(GPTExecutor):
                               gr(pa.weight) if pa is not None else None, gr(b.pre_mlp.weight))
             # ---- attention: O dgrad / wgrad, flash backward, inverse RoPE, QKV dgrad / wgrad
             datt = self._rows(self._reuse(self.d_att2[l & 1]), N, H * D)
-            torch.mm(db, self._dgrad(b.o.weight, self.bf16(b.o.weight)), out=datt)
+            gemm_ops.train_linear(db, self._dgrad(b.o.weight, self.bf16(b.o.weight)).t(), None, datt)
             self._wgrad(db, self.att[l], b.o.weight)
             d_qkv = self._rows(self.d_qkv, N, QKV)
             attn_ops.flash_bwd(datt.view(B, T, H * D), self.qkv[l].view(B, T, -1), self.att[l].view(B, T, H * D),
@@ -551,7 +551,7 @@ class GemmaExecutor(GPTExecutor):
             cos, sin = self._rope(b, T)
             dqr = self._rows(self._reuse(self.d_qkv_raw2[l & 1]), N, QKV)
             k.rope_qkv(d_qkv.view(B, T, -1), cos, sin, H, Hkv, D, True, dqr)
-            torch.mm(dqr, self._dgrad(b.qkv.weight, self.bf16(b.qkv.weight)), out=self.d_c)
+            gemm_ops.train_linear(dqr, self._dgrad(b.qkv.weight, self.bf16(b.qkv.weight)).t(), None, self.d_c)
             self._wgrad(dqr, self.y_in[l], b.qkv.weight)
             self._flush_wgrads()
             # ---- the combine that produced y_in[l]: block l-1's MLP combine (or the embedding norm)

@@ -198,6 +198,9 @@ class GPTDecodeProgram:
 
     def _linear(self, x: Tensor, lin, bias: bool = True) -> Tensor:
         b = lin.bias if bias else None
+        y = gemm_ops.rows_linear(x, lin.weight, b)
+        if y is not None:
+            return y
         if x.shape[0] <= SKINNY_MAX_ROWS and gemm_ops.skinny_ok(x, lin.weight):
             return gemm_ops.skinny_linear(x, lin.weight, b)
         if b is not None:
@@ -582,7 +585,11 @@ def _gated(x: Tensor, gu: Tensor, kind: int) -> Tensor:
 
 
 def _linear(x: Tensor, w: Tensor) -> Tensor:
-    """x [M, K] · wᵀ without bias: the decode-shaped MFMA kernels up to 64 rows."""
+    """x [M, K] · wᵀ without bias: the kernel of short steps, what its rule leaves by the decode-shaped MFMA kernels up to
+    32 rows, else by the library."""
+    y = gemm_ops.rows_linear(x, w)
+    if y is not None:
+        return y
     if x.shape[0] <= SKINNY_MAX_ROWS and gemm_ops.skinny_ok(x, w):
         return gemm_ops.skinny_linear(x, w, None)
     if _decode_gemm_ok(x, w):

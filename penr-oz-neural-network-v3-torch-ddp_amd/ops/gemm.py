@@ -77,6 +77,50 @@ def wgrad_group(dys, xs, grads, accumulate) -> None:
         wgrad(*args)
 
 
+# ---- linear layers of short steps (csrc/kernels/rows_gemm.hip) ------------------------------
+ROWS_GEMM = os.environ.get("PENROZ_ROWS_GEMM", "1") != "0"  # "0": the library (A/B)
+
+
+def rows_linear(x: Tensor, w: Tensor, bias: Tensor | None = None, out: Tensor | None = None,
+                fp32: bool = False, in_order: bool = False) -> Tensor | None:
+    """x [M, K] · wᵀ (+ bias), bf16 (``fp32``: the sums themselves; ``in_order``: each sum in one chain over k), by the
+    kernel of short steps; None for what its rule (``rows_gemm_plan`` in ``csrc/kernels/host_plan.h``) leaves to the
+    library."""
+    if not (ROWS_GEMM and x.is_cuda and x.dtype == torch.bfloat16 and use_kernels(x)):
+        return None
+    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
+        return None
+    return kernels().rows_gemm(x, w, bias, out, fp32, in_order)
+
+
+def linear(x: Tensor, w: Tensor, bias: Tensor | None = None, out: Tensor | None = None) -> Tensor:
+    """x [M, K] · wᵀ (+ bias): :func:`rows_linear` or the library."""
+    y = rows_linear(x, w, bias, out)
+    if y is not None:
+        return y
+    return torch.mm(x, w.t(), out=out) if bias is None else torch.addmm(bias, x, w.t(), out=out)
+
+
+# Training steps take the kernel where its sums are the library's bit for bit: up to this many columns the library does not
+# split them (17 to 1100 rows measured; of 2304 and 3072 columns it splits the sums of some row counts and not of others). A
+# rounding that falls otherwise is as good, but AdamW's first steps carry it through every weight.
+TRAIN_ROWS_MAX_K = 1024
+
+
+def train_linear(x: Tensor, w: Tensor, bias: Tensor | None = None, out: Tensor | None = None) -> Tensor:
+    """x [M, K] · wᵀ (+ bias) of a training step's forward or data gradient."""
+    y = rows_linear(x, w, bias, out, in_order=True) if x.shape[1] <= TRAIN_ROWS_MAX_K else None
+    if y is not None:
+        return y
+    return torch.mm(x, w.t(), out=out) if bias is None else torch.addmm(bias, x, w.t(), out=out)
+
+
+def linear_fp32(x: Tensor, w: Tensor) -> Tensor:
+    """x [M, K] · wᵀ of bf16 operands in fp32."""
+    y = rows_linear(x, w, fp32=True)
+    return torch.mm(x, w.t(), out_dtype=torch.float32) if y is None else y
+
+
 # ---- library GEMM solution choice (hipBLASLt / rocBLAS through torch) -----------------------
 # The forward / dgrad GEMMs stay library calls; which hipBLASLt (or rocBLAS) solution runs each
 # shape is measured, not left to the heuristic: bench/tune_gemms.sh runs PyTorch TunableOp's
@@ -149,9 +193,9 @@ def guard_tuned_gemms(run_steps, steps: int = 3, rounds: int = 2, margin: float 
 # shape and on the headline step (profiles/gemm_epi_r4.log, profiles/native_gemm_r4.md), so the
 # forward / dgrad GEMMs are hipBLASLt and the GELU work stays in elementwise.hip.
 def linear_gelu(x: Tensor, w: Tensor, bias: Tensor, pre: Tensor, act: Tensor, approximate: str = "none"):
-    """pre = x·wᵀ + bias (library GEMM), act = GELU(pre) (bf16; ``approximate`` "none" = erf,
+    """pre = x·wᵀ + bias (:func:`train_linear`), act = GELU(pre) (bf16; ``approximate`` "none" = erf,
     "tanh" = gelu_new; the HIP GELU kernel)."""
-    torch.addmm(bias, x, w.t(), out=pre)
+    train_linear(x, w, bias, pre)
     if use_kernels(pre):
         from penroz.ops import activations as act_ops
         act_ops.gelu_fwd(pre, approximate, out=act)
@@ -161,11 +205,11 @@ def linear_gelu(x: Tensor, w: Tensor, bias: Tensor, pre: Tensor, act: Tensor, ap
 
 
 def dgrad_gelu(dy: Tensor, wt: Tensor, pre: Tensor, out: Tensor, dbias: Tensor | None, approximate: str = "none"):
-    """Data gradient into a GELU's input: out = bf16(dy·wtᵀ) (library GEMM; ``wt`` = the
+    """Data gradient into a GELU's input: out = bf16(dy·wtᵀ) (:func:`train_linear`; ``wt`` = the
     transposed weight copy, [in, out] row-major), then out *= GELU'(pre) and dbias (fp32) += the
     column sums of out in one HIP kernel. The GPT executor's fc2 data gradient + GELU backward +
     fc bias gradient."""
-    torch.mm(dy, wt.t(), out=out)
+    train_linear(dy, wt, None, out)
     from penroz.ops import activations as act_ops
     act_ops.gelu_bwd(out, pre, approximate, dbias, out=out)
     return out

@@ -13,7 +13,7 @@ from dataclasses import dataclass
 import torch
 from torch import Tensor
 
-from penroz.ops import packed as P
+from penroz.ops import gemm as gemm_ops, packed as P
 from penroz.ops._ext import kernels, use_kernels
 from penroz.ops.window import head_columns, head_rows
 
@@ -113,7 +113,7 @@ def linear_attention(s: LinearSizes, w: dict, z: Tensor, state: Tensor, b: P.Pac
             spans, cs = b.spans(length)
             zdec = ws = wdec = None
             if s.rank:  # bf16 operands: the products are exact, their sums fp32
-                zdec = torch.mm(z[:, s.width - s.r8:s.width], w["a2"].t(), out_dtype=torch.float32)
+                zdec = gemm_ops.linear_fp32(z[:, s.width - s.r8:s.width], w["a2"])
             if spans.shape[0] > len(b.counts):
                 ws = torch.empty(spans.shape[0], *s.state, dtype=torch.float32, device=z.device)
                 wdec = torch.empty(spans.shape[0], s.heads, s.d8, dtype=torch.float32, device=z.device)

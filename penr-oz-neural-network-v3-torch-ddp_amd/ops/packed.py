@@ -252,8 +252,9 @@ def logits(h: Tensor, table: Tensor) -> Tensor:
         if h.shape[0] <= 4 and _gemv_ok(h, table, 8192):
             return linear(h, table)
         if h.shape[0] <= 16 and gemm_ops.skinny_ok(h, table):
-            return gemm_ops.skinny_linear(h, table, None)
-        return torch.mm(h, table.t(), out_dtype=torch.float32)
+            y = gemm_ops.rows_linear(h, table)
+            return gemm_ops.skinny_linear(h, table, None) if y is None else y
+        return gemm_ops.linear_fp32(h, table)
     return torch.mm(h, table.t()).float()
 
 
@@ -429,7 +430,7 @@ def _latent_attention_gpu(s, w, z, cache, nw, tab, b):
                        c if fresh else None, kr if fresh else None, True)
         if not fresh:
             K.latent_gather(cache, kcu, b.seq_slot, s.R8, s.r8, c, kr)
-        K.latent_flash(z, torch.mm(c, w["ukv"].t()), kr, b.query_blocks(), b.cu, kcu, s.heads, s.d8, s.r8, s.v8,
+        K.latent_flash(z, gemm_ops.linear(c, w["ukv"]), kr, b.query_blocks(), b.cu, kcu, s.heads, s.d8, s.r8, s.v8,
                        s.scale, out)
         return out
     qa = torch.empty(N, s.heads, s.cache_width, dtype=z.dtype, device=dev)
@@ -476,7 +477,7 @@ def route(h: Tensor, wr: Tensor, top: int, renorm: bool = False, *, sigmoid: boo
         if N <= 64:
             kernels().router_topk(None, h, wr, *rule, ids, wts)
         else:
-            z = torch.mm(h, wr.t(), out_dtype=torch.float32) if h.dtype == torch.bfloat16 else torch.mm(h, wr.t())
+            z = gemm_ops.linear_fp32(h, wr) if h.dtype == torch.bfloat16 else torch.mm(h, wr.t())
             kernels().router_topk(z, None, None, *rule, ids, wts)
         return ids, wts
     z = h.float() @ wr.float().t()

@@ -103,7 +103,7 @@ def build_module(name: str, sources: list[str], extra_libs: list[str], jobs: int
 
 # module -> its kernel sources under csrc/kernels; every other .hip belongs to penroz_kernels
 SERVE_SOURCES = ("packed_rows", "latent_attn", "latent_mfma", "experts", "window_attn", "window_mfma", "linear_attn", "linear_mfma",
-                 "skinny_gemm", "decode_linear")
+                 "skinny_gemm", "decode_linear", "rows_gemm")
 
 
 def _module_sources(name: str) -> list[str]:

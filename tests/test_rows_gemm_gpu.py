@@ -1,0 +1,75 @@
+"""Linear layers of short steps (csrc/kernels/rows_gemm.hip) against float64."""
+import pytest
+import torch
+
+from penroz.ops import _ext, gemm
+
+
+@pytest.mark.skipif(not _ext.available("penroz_serve"), reason="HIP extension not built")
+@pytest.mark.parametrize("M,N,K,tile", [(1, 8, 8, 1), (64, 768, 768, 1), (256, 1024, 1024, 1), (257, 1024, 1024, 2),
+                                        (64, 8192, 2048, 2), (256, 3072, 768, 3), (64, 12288, 2048, 3), (65, 12288, 2048, 0),
+                                        (512, 3072, 768, 4), (1024, 3072, 768, 5), (64, 32768, 2048, 5), (4096, 3072, 768, 0),
+                                        (64, 768, 772, 0), (0, 768, 768, 0), (64, 1 << 21, 768, 0)])
+def test_rows_gemm_rule(M, N, K, tile):
+    assert _ext.kernels().rows_gemm_tile(M, N, K) == tile
+    in_order = _ext.kernels().rows_gemm_tile(M, N, K, True)
+    assert in_order == {(257, 1024, 1024): 1, (64, 8192, 2048): 1}.get((M, N, K), tile)
+
+
+# every tile: less than one, its edges, ragged rows and columns; K of less than a stage, whole stages, ragged ones
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,tile", [(1, 8, 1), (31, 33, 1), (33, 250, 1), (256, 1024, 1), (300, 1026, 2), (17, 9001, 2),
+                                      (200, 3001, 3), (64, 12288, 3), (500, 3001, 4), (700, 3100, 5), (64, 40000, 5)])
+@pytest.mark.parametrize("K", [8, 56, 64, 72, 256, 264, 760, 1024])
+def test_rows_gemm(M, N, tile, K):
+    assert _ext.kernels().rows_gemm_tile(M, N, K) == tile
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K + 8, generator=g, device="cuda").bfloat16()[:, :K]  # strided rows
+    w = torch.randn(N, K, generator=g, device="cuda").bfloat16()
+    bias = torch.randn(N, generator=g, device="cuda").bfloat16()
+    want = x.double() @ w.double().t()
+    full = gemm.rows_linear(x, w, fp32=True)
+    # fp32 sums of K products: in blocks of 32 in the MFMA, K / 32 of them
+    assert full.dtype == torch.float32
+    assert torch.linalg.norm(full.double() - want) <= 2.0 ** -24 * (K / 32 + 32) ** 0.5 * torch.linalg.norm(want)
+    for b, in_order in ((None, True), (None, False), (bias, True), (bias, False)):
+        ref = want if b is None else want + b.double()
+        got = gemm.rows_linear(x, w, b, in_order=in_order)
+        if got is None:
+            assert in_order and tile == 2
+            continue
+        assert got.dtype == torch.bfloat16
+        # half a step of bf16 at each value, and the sums' own error where they cancel
+        assert ((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -18 * K ** 0.5).all()
+    buf = torch.full((M, N + 8), 7.0, device="cuda", dtype=torch.bfloat16)  # rows of a wider buffer
+    assert gemm.rows_linear(x, w, bias, buf[:, :N]) is not None
+    assert torch.equal(buf[:, :N], got) and (buf[:, N:] == 7.0).all()
+
+
+@pytest.mark.gpu
+def test_rows_gemm_leaves_other_forms():
+    """What the kernel does not read goes to the library with the result it always had."""
+    x, w = (torch.randn(64, 256, device="cuda").bfloat16() for _ in range(2))
+    forms = [(x[:, 1:249], w[:, 1:249]), (x.t().contiguous().t(), w), (x, w.t().contiguous().t()), (x[:, :100], w[:, :100])]
+    for a, b in forms:
+        assert gemm.rows_linear(a, b) is None
+        assert torch.equal(gemm.linear(a, b), torch.mm(a, b.t()))
+    off = torch.randn(64 * 256 + 1, device="cuda").bfloat16()[1:].view(64, 256)
+    assert gemm.rows_linear(off, w) is None
+    assert gemm.rows_linear(x, w, torch.zeros(64, device="cuda")) is None  # an fp32 bias
+    assert gemm.rows_linear(x.float(), w.float()) is None
+    with pytest.raises(RuntimeError):
+        gemm.linear(x, w[:, :248])
+    wp = w.clone().requires_grad_()
+    gemm.linear(x, wp).sum().backward()
+    assert wp.grad is not None
+
+
+@pytest.mark.gpu
+def test_rows_gemm_propagates_what_is_not_finite():
+    x = torch.ones(40, 96, device="cuda").bfloat16()
+    w = torch.ones(72, 96, device="cuda").bfloat16()
+    x[3, 95], w[5, 0], x[7, 1] = float("inf"), float("nan"), -float("inf")
+    got, ref = gemm.rows_linear(x, w), torch.mm(x.float(), w.float().t())
+    assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(got[3, :5], ref[3, :5].bfloat16())
+    assert torch.equal(got[7, :5], ref[7, :5].bfloat16())
