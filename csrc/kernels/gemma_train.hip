@@ -18,7 +18,7 @@
 // gradient of h through the residual path, from the LATER combine; absent for the last one) and
 // produces dx (fp32 gradient of x, in place over dh_in allowed), da (bf16 gradient of the
 // branch output, the input of the branch's dgrad GEMM) and per-wave partial rows of dw1, dw2
-// (finished by the deterministic two-stage column reduction, on the deferred stream):
+// (finished by the deterministic column reduction, on the deferred stream):
 //   dh  = r2·w2·dy − h·r2³·mean(h·w2·dy) + dh_in            dw2 += dy·h·r2
 //   mode 0: ds = r1·w1·dh − s·r1³·mean(s·w1·dh)  -> dx = da = ds,   dw1 += dh·s·r1
 //   mode 1: dx = dh;  da = r1·w1·dh − a·r1³·mean(a·w1·dh),          dw1 += dh·a·r1
@@ -352,7 +352,7 @@ void gemma_combine_fwd(int64_t mode, torch::Tensor x, c10::optional<torch::Tenso
 
 // dy bf16 [N, C]; dh_in fp32 (optional; may alias dx); h fp32 (mode 3: x); s fp32 (mode 0);
 // a bf16 (mode 1); dx fp32 out; da bf16 out (modes 0-2); dw1 (modes 0, 1) / dw2 fp32 [C]
-// accumulated (+=) through the two-stage column reduction; dh_save (optional): dL/dh
+// accumulated (+=) through the column reduction; dh_save (optional): dL/dh
 void gemma_combine_bwd(int64_t mode, torch::Tensor dy, c10::optional<torch::Tensor> dh_in, torch::Tensor h,
                        c10::optional<torch::Tensor> s_save, c10::optional<torch::Tensor> a_save,
                        c10::optional<torch::Tensor> r1, torch::Tensor r2, c10::optional<torch::Tensor> w1,

@@ -134,7 +134,7 @@ inline int rows_gemm_plan(int64_t M, int64_t N, int64_t K, bool in_order) {
   return 0;
 }
 
-// Slices of the two-stage deterministic column reduction (reduce.h): ~sqrt(G) balances stages.
+// Slices of the deterministic column reduction (reduce.h): ~sqrt(G) balances its two steps.
 inline int reduce_slices(int G) {
   int s = 1;
   while ((int64_t)s * s < G) ++s;

@@ -272,13 +272,11 @@ std::vector<torch::Tensor> rmsnorm_bwd(torch::Tensor dy, torch::Tensor x, torch:
                          reinterpret_cast<const TW*>(wc.data_ptr()), rstd.data_ptr<float>(),
                          reinterpret_cast<TX*>(dx.data_ptr()), part.data_ptr<float>(), N, C))))
   }
-  // dγ = Σ of the G partial rows: the sliced two-stage column reduction (reduce.h), on the CURRENT
+  // dγ = Σ of the G partial rows: the sliced column reduction (reduce.h), on the CURRENT
   // stream — dw goes straight back to autograd, so it must not be finished on the executor's
   // deferred side stream (nothing would order the caller's reads after it)
-  const int S = reduce_slices(G);
-  auto mid = torch::empty({1, S, C}, part.options());
   float* outs[1] = {dw.data_ptr<float>()};
-  reduce_partials_add(part.data_ptr<float>(), 1, G, C, outs, mid.data_ptr<float>(), S, stream);
+  reduce_partials_add(part.data_ptr<float>(), 1, G, C, outs, stream);
   return {dx, dw};
 }
 
