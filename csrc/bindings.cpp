@@ -37,6 +37,7 @@ void gemma_combine_bwd(int64_t mode, torch::Tensor dy, c10::optional<torch::Tens
                        torch::Tensor w2, torch::Tensor dx, c10::optional<torch::Tensor> da,
                        c10::optional<torch::Tensor> dw1, torch::Tensor dw2, c10::optional<torch::Tensor> dh_save);
 void transpose_bf16(torch::Tensor in, torch::Tensor out);
+void transpose_bf16_group(std::vector<torch::Tensor> ins, std::vector<torch::Tensor> outs);
 void embedding_fwd(torch::Tensor idx, torch::Tensor wte, torch::Tensor wpe, int64_t off, torch::Tensor out,
                    c10::optional<torch::Tensor> off_dev, double dropout_p, int64_t dropout_seed);
 void embedding_bwd(torch::Tensor dout, torch::Tensor idx, torch::Tensor dwte, torch::Tensor dwpe, int64_t off,
@@ -163,6 +164,7 @@ PYBIND11_MODULE(penroz_kernels, m) {
         pybind11::arg("w1"), pybind11::arg("w2"), pybind11::arg("dx"), pybind11::arg("da"), pybind11::arg("dw1"),
         pybind11::arg("dw2"), pybind11::arg("dh_save") = pybind11::none(),
         "backward of gemma_combine_fwd (dw1 / dw2 accumulated; dh_save: dL/dh for diagnostics)");
+  m.def("transpose_bf16_group", &transpose_bf16_group, "transpose_bf16 of each, in one launch");
   m.def("transpose_bf16", &transpose_bf16, "out [C, R] = in [R, C]^T (bf16, dims % 64 == 0)");
   m.def("embedding_fwd", &embedding_fwd, pybind11::arg("idx"), pybind11::arg("wte"), pybind11::arg("wpe"),
         pybind11::arg("off"), pybind11::arg("out"), pybind11::arg("off_dev") = pybind11::none(),

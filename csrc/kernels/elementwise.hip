@@ -191,11 +191,32 @@ __global__ void __launch_bounds__(256) embed_fwd_kernel(const int64_t* __restric
 // for the weight copies of the data-gradient GEMMs (dx = dy·W runs ~12-22 % faster on
 // hipBLASLt with W stored transposed: both operands then reduction-contiguous, the forward's
 // layout — profiles/dgrad_layout_r1.log).
-__global__ void __launch_bounds__(256) transpose_bf16_kernel(const uint16_t* __restrict__ in,
-                                                             uint16_t* __restrict__ out, int R, int C) {
+struct Transpose {
+  const uint16_t* in;
+  uint16_t* out;
+  int R, C, tile0;  // tile0: tiles of the matrices before
+};
+constexpr int kTransposes = 64;
+struct Transposes {
+  Transpose m[kTransposes];
+  int n;
+};
+
+// All copies of a step in one launch: by themselves GPT-2's 49 take 3 to 4 us each, little above an empty launch, and 5 us of the
+// host's time. A workgroup finds its matrix by halving.
+__global__ void __launch_bounds__(256) transpose_bf16_kernel(const Transposes all) {
   __shared__ uint16_t tile[64][66];
+  int lo = 0, hi = all.n - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if ((int)blockIdx.x >= all.m[mid].tile0) lo = mid;
+    else hi = mid - 1;
+  }
+  const uint16_t* __restrict__ in = all.m[lo].in;
+  uint16_t* __restrict__ out = all.m[lo].out;
+  const int R = all.m[lo].R, C = all.m[lo].C, id = blockIdx.x - all.m[lo].tile0;
   const int tiles_c = C / 64;
-  const int r0 = (blockIdx.x / tiles_c) * 64, c0 = (blockIdx.x % tiles_c) * 64;
+  const int r0 = (id / tiles_c) * 64, c0 = (id % tiles_c) * 64;
   const int t = threadIdx.x;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -609,18 +630,36 @@ void embedding_fwd(torch::Tensor idx, torch::Tensor wte, torch::Tensor wpe, int6
                        (float)dropout_p))
 }
 
-void transpose_bf16(torch::Tensor in, torch::Tensor out) {
-  TORCH_CHECK(in.is_cuda() && in.scalar_type() == torch::kBFloat16 && out.scalar_type() == torch::kBFloat16 &&
-                  in.dim() == 2 && out.dim() == 2, "transpose_bf16: 2-D bf16");
-  const int R = in.size(0), C = in.size(1);
-  TORCH_CHECK(in.is_contiguous() && out.is_contiguous() && out.size(0) == C && out.size(1) == R,
-              "transpose_bf16: out must be the contiguous [C, R]");
-  TORCH_CHECK(R % 64 == 0 && C % 64 == 0, "transpose_bf16: dims must be multiples of 64");
-  if (R == 0 || C == 0) return;
+void transpose_bf16_group(std::vector<torch::Tensor> ins, std::vector<torch::Tensor> outs) {
+  TORCH_CHECK(ins.size() == outs.size(), "transpose_bf16: one output per input");
   auto stream = at::hip::getCurrentHIPStream();
-  hipLaunchKernelGGL(transpose_bf16_kernel, dim3((R / 64) * (C / 64)), dim3(256), 0, stream,
-                     reinterpret_cast<const uint16_t*>(in.data_ptr()), reinterpret_cast<uint16_t*>(out.data_ptr()), R, C);
+  Transposes all{};
+  int64_t tiles = 0;
+  auto launch = [&] {
+    if (all.n > 0)
+      hipLaunchKernelGGL(transpose_bf16_kernel, dim3((unsigned)tiles), dim3(256), 0, stream, all);
+    all.n = 0;
+    tiles = 0;
+  };
+  for (size_t i = 0; i < ins.size(); ++i) {
+    const torch::Tensor &in = ins[i], &out = outs[i];
+    TORCH_CHECK(in.is_cuda() && out.is_cuda() && in.scalar_type() == torch::kBFloat16 &&
+                    out.scalar_type() == torch::kBFloat16 && in.dim() == 2 && out.dim() == 2, "transpose_bf16: 2-D bf16");
+    const int64_t R = in.size(0), C = in.size(1);
+    TORCH_CHECK(in.is_contiguous() && out.is_contiguous() && out.size(0) == C && out.size(1) == R,
+                "transpose_bf16: out must be the contiguous [C, R]");
+    TORCH_CHECK(R % 64 == 0 && C % 64 == 0, "transpose_bf16: dims must be multiples of 64");
+    if (R == 0 || C == 0) continue;
+    const int64_t more = (R / 64) * (C / 64);
+    if (all.n == kTransposes || tiles + more >= (int64_t)1 << 31) launch();
+    all.m[all.n++] = Transpose{reinterpret_cast<const uint16_t*>(in.data_ptr()), reinterpret_cast<uint16_t*>(out.data_ptr()),
+                               (int)R, (int)C, (int)tiles};
+    tiles += more;
+  }
+  launch();
 }
+
+void transpose_bf16(torch::Tensor in, torch::Tensor out) { transpose_bf16_group({in}, {out}); }
 
 void embedding_bwd(torch::Tensor dout, torch::Tensor idx, torch::Tensor dwte, torch::Tensor dwpe, int64_t off,
                    double dropout_p, int64_t dropout_seed) {

@@ -398,8 +398,7 @@ class GPTExecutor:
         todo = [(key, e) for key, e in self._tw.items() if key not in self._t_fresh]
         self._t_fresh.clear()
         if side is None:
-            for _, e in todo:
-                k.transpose_bf16(self._tw_source(e), e[1])
+            k.transpose_bf16_group([self._tw_source(e) for _, e in todo], [e[1] for _, e in todo])
             return
         if not todo:  # all rebuilt after their segments' optimizer passes (the main stream joined)
             return
@@ -410,8 +409,7 @@ class GPTExecutor:
         main = torch.cuda.current_stream(self.device)
         with torch.cuda.stream(side):
             side.wait_stream(main)
-            for _, e in todo:
-                k.transpose_bf16(self._tw_source(e), e[1])
+            k.transpose_bf16_group([self._tw_source(e) for _, e in todo], [e[1] for _, e in todo])
             self._t_ready = torch.cuda.Event()
             self._t_ready.record(side)
 
@@ -430,12 +428,14 @@ class GPTExecutor:
         env = os.environ.get("PENROZ_SEGMENT_TRANSPOSE")  # (A/B: 1 / 0 overrides the class default)
         if not getattr(self, "_tw", None) or not (self.SEGMENT_TRANSPOSE if env is None else env == "1"):
             return
-        k = _ext.kernels()
+        ins, outs = [], []
         for key, ent in self._tw.items():
             off = self.offsets.get(key)
             if off is not None and s <= off and off + ent[1].numel() <= e:  # the whole weight is final
-                k.transpose_bf16(self._tw_source(ent), ent[1])
+                ins.append(self._tw_source(ent))
+                outs.append(ent[1])
                 self._t_fresh.add(key)
+        _ext.kernels().transpose_bf16_group(ins, outs)
 
     def _dgrad_w(self, w: Tensor) -> Tensor:
         """The weight operand of dx = dy·W: the transposed copy (viewed back as [out, in]) or the shadow

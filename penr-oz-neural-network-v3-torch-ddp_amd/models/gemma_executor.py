@@ -244,21 +244,17 @@ class GemmaExecutor(GPTExecutor):
             return
         k = _ext.kernels()
         side = getattr(self, "_side", None)
-        if side is None:
-            for key, (f, t) in self._tw.items():
-                if key not in self._t_fresh:
-                    k.transpose_bf16(f(), t)
-            self._t_fresh.clear()
-            return
         todo = [(f, t) for key, (f, t) in self._tw.items() if key not in self._t_fresh]
         self._t_fresh.clear()
+        if side is None:
+            k.transpose_bf16_group([f() for f, _ in todo], [t for _, t in todo])
+            return
         if not todo:  # all rebuilt after their segments' optimizer passes (the main stream joined)
             return
         main = torch.cuda.current_stream(self.device)
         with torch.cuda.stream(side):
             side.wait_stream(main)
-            for f, t in todo:
-                k.transpose_bf16(f(), t)
+            k.transpose_bf16_group([f() for f, _ in todo], [t for _, t in todo])
             self._t_ready = torch.cuda.Event()
             self._t_ready.record(side)
 
