@@ -73,9 +73,8 @@ def main():
         out = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
         y = torch.randn(M, K, device=dev, dtype=torch.bfloat16)
         row = {"kernel": "decode_ln_gemm", "shape": name, "M": M, "N": N, "K": K}
-        for flags in (0, 1, 2, 4, 3, 7, 15, 23, 31):
-            row[f"f{flags}_us"] = round(timeit([lambda w=w, b=b: k.decode_ln_gemm(resid, gamma, beta, 1e-5, w, b, out,
-                                                                                   0, flags) for w, b in zip(ws, bs)]), 2)
+        row["us"] = round(timeit([lambda w=w, b=b: k.decode_ln_gemm(resid, gamma, beta, 1e-5, w, b, out, 0)
+                                  for w, b in zip(ws, bs)]), 2)
         row["blas_mm_us"] = round(timeit([lambda w=w: torch.mm(y, w.t(), out=out) for w in ws]), 2)
         print(json.dumps(row), flush=True)
     for name, N, K in (("proj", C, C), ("fc2", C, 4 * C)):
@@ -84,8 +83,7 @@ def main():
         r = torch.zeros(M, N, device=dev)
         out = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
         row = {"kernel": "decode_gemm_acc", "shape": name, "M": M, "N": N, "K": K}
-        for flags in (0, 1, 2, 4, 3, 7):
-            row[f"f{flags}_us"] = round(timeit([lambda w=w: k.decode_gemm_acc(x, w, None, r, flags) for w in ws]), 2)
+        row["us"] = round(timeit([lambda w=w: k.decode_gemm_acc(x, w, None, r) for w in ws]), 2)
         row["blas_mm_us"] = round(timeit([lambda w=w: torch.mm(x, w.t(), out=out) for w in ws]), 2)
         print(json.dumps(row), flush=True)
     # an empty-ish kernel for the per-launch floor inside a graph

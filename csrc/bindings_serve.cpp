@@ -16,7 +16,7 @@ void decode_ln_linear(torch::Tensor rin, c10::optional<torch::Tensor> delta, c10
                       c10::optional<torch::Tensor> rout, torch::Tensor gamma, torch::Tensor beta, double eps,
                       torch::Tensor w, c10::optional<torch::Tensor> bias, torch::Tensor out, int64_t act);
 void decode_ln_gemm(torch::Tensor resid, torch::Tensor gamma, torch::Tensor beta, double eps, torch::Tensor w,
-                    c10::optional<torch::Tensor> bias, torch::Tensor out, int64_t act, int64_t flags);
+                    c10::optional<torch::Tensor> bias, torch::Tensor out, int64_t act);
 void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> rin, c10::optional<torch::Tensor> delta,
                  c10::optional<torch::Tensor> dbias, c10::optional<torch::Tensor> rout,
                  c10::optional<torch::Tensor> gamma, c10::optional<torch::Tensor> beta, double eps, torch::Tensor w,
@@ -26,12 +26,11 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
 void decode_gemv_pair(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64_t mode, int64_t kind, int64_t D,
                       int64_t nrot, c10::optional<torch::Tensor> cosv, c10::optional<torch::Tensor> sinv,
                       int64_t pairs_per_wave);
-void decode_gemm_acc(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias, torch::Tensor resid,
-                     int64_t flags);
+void decode_gemm_acc(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias, torch::Tensor resid);
 void decode_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64_t kind);
 // rows_gemm.hip
 c10::optional<torch::Tensor> rows_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
-                                       c10::optional<torch::Tensor> out, bool fp32, bool in_order);
+                                       c10::optional<torch::Tensor> out, bool fp32, bool in_order, bool gelu);
 int64_t rows_gemm_tile(int64_t M, int64_t N, int64_t K, bool in_order);
 // packed_rows.hip
 void row_norm_add(c10::optional<torch::Tensor> tok, c10::optional<torch::Tensor> table,
@@ -135,7 +134,7 @@ PYBIND11_MODULE(penroz_serve, m) {
         "resid_out receives the residual sum");
   m.def("decode_ln_gemm", &decode_ln_gemm, pybind11::arg("resid"), pybind11::arg("gamma"), pybind11::arg("beta"),
         pybind11::arg("eps"), pybind11::arg("w"), pybind11::arg("bias"), pybind11::arg("out"), pybind11::arg("act") = 0,
-        pybind11::arg("flags") = 0, "batched decode: out = act(LayerNorm(resid)·wᵀ + bias), fp32 resid [M, K <= 1024]");
+        "batched decode: out = act(LayerNorm(resid)·wᵀ + bias), fp32 resid [M, K <= 1024]");
   m.def("decode_gemv", &decode_gemv, pybind11::arg("x"), pybind11::arg("resid_in"), pybind11::arg("delta"),
         pybind11::arg("dbias"), pybind11::arg("resid_out"), pybind11::arg("gamma"), pybind11::arg("beta"),
         pybind11::arg("eps"), pybind11::arg("w"), pybind11::arg("bias"), pybind11::arg("out"), pybind11::arg("act") = 0,
@@ -150,11 +149,11 @@ PYBIND11_MODULE(penroz_serve, m) {
         pybind11::arg("pairs_per_wave") = 0,
         "paired-row decode GEMV for 1..4 rows: gated MLP (mode 1) or RoPE QKV (mode 2) epilogue");
   m.def("rows_gemm", &rows_gemm, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("bias"), pybind11::arg("out"),
-        pybind11::arg("fp32") = false, pybind11::arg("in_order") = false);
+        pybind11::arg("fp32") = false, pybind11::arg("in_order") = false, pybind11::arg("gelu") = false);
   m.def("rows_gemm_tile", &rows_gemm_tile, pybind11::arg("M"), pybind11::arg("N"), pybind11::arg("K"),
         pybind11::arg("in_order") = false);
   m.def("decode_gemm_acc", &decode_gemm_acc, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("bias"),
-        pybind11::arg("resid"), pybind11::arg("flags") = 0,
+        pybind11::arg("resid"),
         "batched decode: resid += x·wᵀ + bias (fp32 residual, in place)");
   m.def("decode_gemm", &decode_gemm, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("out"),
         pybind11::arg("kind") = -1,

@@ -1,28 +1,21 @@
-// Batched decode linears (M = decode rows, 16..64 typical): the two kernels of a GPT block's
-// decode step besides attention, shaped so that a block costs 5 launches instead of 8.
+// Decode linears. A GPT block's decode step of 5 to 64 rows costs 5 launches instead of 8:
 //
 //   decode_ln_gemm : out = act(LN(resid) · Wᵀ + bias)          (QKV; fc + GELU)
-//   decode_gemm_acc: resid += x · Wᵀ + bias                     (proj; fc2)
+//   decode_gemm_acc: resid += x · Wᵀ + bias                     (proj; fc2; rows_gemm.hip)
 //
 // The residual stream stays fp32 and is updated IN PLACE by decode_gemm_acc's epilogue, so
 // the separate "residual add + LayerNorm" kernel between the GEMMs disappears: the next
 // decode_ln_gemm normalises the rows it needs itself. Two choices keep that redundant
 // normalisation cheap (the round-2 fused kernel normalised all 64 rows in every 16-column
 // workgroup and lost at 64 rows, profiles/decode_fused_rows_r2.log):
-//   * a decode_ln_gemm workgroup owns 16 ROWS × 64 columns (4 waves × one 16x16x32 MFMA column
-//     block over the full K), so it normalises only its 16 rows (4 per wave) — 16× less
-//     prologue work per workgroup than 64 rows × 16 columns, for the same 144-192 workgroups;
-//   * the weight fragments of the whole K range (K ≤ 1024: ≤ 32 × 16 B per lane) are issued
-//     BEFORE the prologue, so their HBM latency hides under the normalisation.
-// decode_gemm_acc owns 16 rows × 16 columns (N = 768 → 48 column blocks × 4 row blocks = 192
-// workgroups without split-K), its 4 waves split K and reduce through LDS; the epilogue is a
-// deterministic float4 read-modify-write of the residual (one owner per element, no atomics).
+//   * a decode_ln_gemm workgroup owns 16 ROWS × 32 columns, so it normalises only its 16 rows;
+//   * four waves bring the weights while the other four normalise.
 // Row blocks of one column tile are placed on one XCD (blockIdx % 8 picks the XCD), so the
 // 4 row blocks' weight reads after the first hit that XCD's L2.
 //
 // MFMA: v_mfma_f32_16x16x32_bf16 with A = 16 weight rows (output columns n), B = 16 x rows
 // (decode rows m): lane holds D[n = 4(lane>>4) + r][m = lane & 15], r = 0..3 — four
-// consecutive outputs of one row, stored as 8 B (bf16) or RMW'd as 16 B (fp32).
+// consecutive outputs of one row, stored as 8 B.
 #include "common.h"
 #include <type_traits>
 #include <torch/extension.h>
@@ -34,8 +27,8 @@ typedef short dl_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float dl_f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t dl_u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kDlMaxSteps = 32;  // decode_ln_gemm: K <= 1024 (32 k-steps of 32)
-constexpr int kDlGroup = 32;     // decode_gemm_acc: k-steps per wave whose loads are issued together
+constexpr int kDlMaxSteps = 32;  // decode_ln_gemm: K <= 1024 (16 values of a row per lane)
+constexpr int kDlGroup = 32;     // decode_gemm: k-steps per wave whose loads are issued together
 
 // (row block, column tile) of a workgroup: the nrb row blocks of column tile ct share
 // blockIdx % 8 (one XCD) for the full groups of 8 tiles; the tail is row-block-major.
@@ -52,133 +45,122 @@ __device__ __forceinline__ void dl_tile(int id, int nrb, int nct, int& rb, int& 
   }
 }
 
-// grid = ceil(M/16) * ceil(N/(64/KS)), block 256. LDS: 16 normalised rows [16][K + 8] bf16.
-// KS = 2: 32-column tiles, the two waves of a column block split K in halves and meet in LDS —
-// twice the workgroups (qkv at 64 rows: 288 instead of 144 on 256 CUs), half the weight bytes per
-// workgroup.
-template <int KS>
-__global__ void __launch_bounds__(256) decode_ln_gemm_kernel(const float* __restrict__ resid,
+// grid = ceil(M/16) * ceil(N/32), block 512: waves 0-3 normalise 16 rows, 4 each, into LDS ([16][K + 8] bf16) while waves 4-7
+// bring the 32 weight rows by LDS-DMA (sub-slices of 64 columns, 16-byte chunks permuted on the source side: fragment reads cover
+// all banks); then the 8 waves take 2 column blocks × 4 shares of K, which meet in LDS. Bound by the chain launch, loads, two wave
+// sums per row, MFMAs, store: with the weights in the registers of the waves that normalise, their loads (memory) stood before
+// the residual's (L2) in the wave's queue: qkv / fc of GPT-2 at 64 rows 9.1 / 9.7 us so, 7.2 / 7.8 now; at 8 rows 7.0 / 7.5, 5.7 /
+// 6.2. (8 waves that each hold weights and normalise two rows: 12.7 at 64 rows.)
+__global__ void __launch_bounds__(512) decode_ln_gemm_kernel(const float* __restrict__ resid,
                                                              const float* __restrict__ gamma,
                                                              const float* __restrict__ beta, float eps,
                                                              const bf16* __restrict__ w, const bf16* __restrict__ bias,
                                                              bf16* __restrict__ out, int64_t o_rs, int M, int N, int K,
-                                                             int act, int flags) {
-  __shared__ __attribute__((aligned(16))) bf16 xs[16 * (1024 + 8)];
-  __shared__ __attribute__((aligned(16))) dl_f32x4 kred[KS > 1 ? (KS - 1) * (4 / KS) * 64 : 1];
-  constexpr int TW = 64 / KS, NCB = 4 / KS, MS = kDlMaxSteps / KS;
+                                                             int act) {
+  extern __shared__ __attribute__((aligned(16))) char dl_smem[];
+  __shared__ __attribute__((aligned(16))) dl_f32x4 kred[3 * 2 * 64];
+  const int subs = (K + 63) / 64, steps = K / 32;
+  char* const wt = dl_smem;                                        // [subs][32 rows][128 B]
+  bf16* const xs = reinterpret_cast<bf16*>(dl_smem + subs * 4096);  // [16][LDX]
   const int LDX = K + 8;  // +16 B per row: a fragment's 16 row reads spread over the banks
-  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
-  const int cb = wid % NCB, kh = wid / NCB;  // column block, K part (KS = 2: halves)
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int rb, ct;
-  dl_tile(blockIdx.x, (M + 15) / 16, (N + TW - 1) / TW, rb, ct);
-  const int steps = K / 32 / KS, s0 = kh * steps;  // this wave's k-steps: s0 .. s0 + steps
-  const int r16 = lane & 15, kq = 8 * (lane >> 4);
-  const int n0 = ct * TW + cb * 16;  // this wave's column block
-  const bool live = n0 < N;
-
-  // 1. the wave's weight fragments for its K range, in flight during the prologue
-  dl_u32x4 wa[MS];
-  {
-    const bf16* wp = w + (size_t)min(n0 + r16, N - 1) * K + kq + s0 * 32;
+  dl_tile(blockIdx.x, (M + 15) / 16, (N + 31) / 32, rb, ct);
+  const int r16 = lane & 15, kq = 8 * (lane >> 4), cb = wid & 1, kh = wid >> 1;
+  const int m = rb * 16 + r16, n = ct * 32 + cb * 16 + 4 * (lane >> 4);
+  uint2 bias_v{0u, 0u};
+  if (wid >= 4) {
+    const unsigned base = lds_addr_of(wt);
+    for (int p = wid - 4; p < 4 * subs; p += 4) {  // 8 rows of a sub-slice
+      const int row = (p & 3) * 8 + (lane >> 3), k = (p >> 2) * 64 + 8 * ((lane & 7) ^ ((row >> 1) & 7));
+      const bf16* src = w + (size_t)min(ct * 32 + row, N - 1) * K + k;
+      glds16(k < K ? (const void*)src : (const void*)g_zero16, __builtin_amdgcn_readfirstlane(base + p * 1024));
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  } else {
+    // LayerNorm of rows wid + 4i (fp32 two-pass on the register copy)
+    float v[4][4][4];
 #pragma unroll
-    for (int s = 0; s < MS; ++s)
-      if (s < steps && live && !(flags & 2)) wa[s] = *reinterpret_cast<const dl_u32x4*>(wp + s * 32);
-  }
-
-  // the epilogue's bias terms, fetched now (not a memory round trip after the MFMAs)
-  const int m = rb * 16 + r16, n = n0 + 4 * (lane >> 4);
-  float bv[4] = {0.f, 0.f, 0.f, 0.f};
-  if (bias && live) {
-    const uint2 u = *reinterpret_cast<const uint2*>(bias + n);
-    bv[0] = __uint_as_float(u.x << 16); bv[1] = __uint_as_float(u.x & 0xffff0000u);
-    bv[2] = __uint_as_float(u.y << 16); bv[3] = __uint_as_float(u.y & 0xffff0000u);
-  }
-
-  // 2. LayerNorm of rows rb*16 + wid + 4i (fp32 two-pass on the register copy) -> bf16 LDS
-  float v[4][4][4];
+    for (int i = 0; i < 4; ++i) {
+      const int row = rb * 16 + wid + 4 * i;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = rb * 16 + wid + 4 * i;
+      for (int j = 0; j < 4; ++j) {
+        const int c = 4 * (lane + 64 * j);
+        if (row < M && c < K) {
+          const float4_t r = *reinterpret_cast<const float4_t*>(resid + (size_t)row * K + c);
+          v[i][j][0] = r[0]; v[i][j][1] = r[1]; v[i][j][2] = r[2]; v[i][j][3] = r[3];
+        } else {
+          v[i][j][0] = v[i][j][1] = v[i][j][2] = v[i][j][3] = 0.f;
+        }
+      }
+    }
+    float4_t g[4], b[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int c = 4 * (lane + 64 * j);
-      if (m < M && c < K && !(flags & 1)) {
-        const float4_t r = *reinterpret_cast<const float4_t*>(resid + (size_t)m * K + c);
-        v[i][j][0] = r[0]; v[i][j][1] = r[1]; v[i][j][2] = r[2]; v[i][j][3] = r[3];
-      } else {
-        v[i][j][0] = v[i][j][1] = v[i][j][2] = v[i][j][3] = 0.f;
+      if (c < K) {
+        g[j] = *reinterpret_cast<const float4_t*>(gamma + c);
+        b[j] = *reinterpret_cast<const float4_t*>(beta + c);
+      }
+    }
+    // the epilogue's bias terms, fetched now (not a memory round trip after the MFMAs)
+    if (bias && kh == 0 && n < N) bias_v = *reinterpret_cast<const uint2*>(bias + n);
+    const float inv_k = 1.f / (float)K;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int lr = wid + 4 * i;
+      bf16* xr = xs + lr * LDX;
+      float s = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s += (v[i][j][0] + v[i][j][1]) + (v[i][j][2] + v[i][j][3]);
+      const float mean = wave_sum(s) * inv_k;
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (4 * (lane + 64 * j) < K)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const float d = v[i][j][k] - mean;
+            ss += d * d;
+          }
+      const float rstd = rsqrtf(wave_sum(ss) * inv_k + eps);
+      const bool row_ok = rb * 16 + lr < M;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int c = 4 * (lane + 64 * j);
+        if (c >= K) continue;
+        uint2 pk{0u, 0u};
+        if (row_ok)
+          pk = uint2{pack_bf16x2((v[i][j][0] - mean) * rstd * g[j][0] + b[j][0], (v[i][j][1] - mean) * rstd * g[j][1] + b[j][1]),
+                     pack_bf16x2((v[i][j][2] - mean) * rstd * g[j][2] + b[j][2], (v[i][j][3] - mean) * rstd * g[j][3] + b[j][3])};
+        *reinterpret_cast<uint2*>(xr + c) = pk;
       }
     }
   }
-  float4_t g[4], b[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int c = 4 * (lane + 64 * j);
-    if (c < K) {
-      g[j] = *reinterpret_cast<const float4_t*>(gamma + c);
-      b[j] = *reinterpret_cast<const float4_t*>(beta + c);
-    }
-  }
-  const float inv_k = 1.f / (float)K;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if (flags & 8) break;
-    const int lr = wid + 4 * i;  // local row
-    bf16* xr = xs + lr * LDX;
-    float s = 0.f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) s += (v[i][j][0] + v[i][j][1]) + (v[i][j][2] + v[i][j][3]);
-    const float mean = wave_sum(s) * inv_k;
-    float ss = 0.f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (4 * (lane + 64 * j) < K)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const float d = v[i][j][k] - mean;
-          ss += d * d;
-        }
-    const float rstd = rsqrtf(wave_sum(ss) * inv_k + eps);
-    const bool row_ok = rb * 16 + lr < M;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int c = 4 * (lane + 64 * j);
-      if (c >= K) continue;
-      uint2 pk{0u, 0u};
-      if (row_ok)
-        pk = uint2{pack_bf16x2((v[i][j][0] - mean) * rstd * g[j][0] + b[j][0], (v[i][j][1] - mean) * rstd * g[j][1] + b[j][1]),
-                   pack_bf16x2((v[i][j][2] - mean) * rstd * g[j][2] + b[j][2], (v[i][j][3] - mean) * rstd * g[j][3] + b[j][3])};
-      *reinterpret_cast<uint2*>(xr + c) = pk;
-    }
-  }
   __syncthreads();
-  if (KS == 1 && !live) return;
-  if (flags & 2) {
-#pragma unroll
-    for (int s = 0; s < MS; ++s) wa[s] = dl_u32x4{0u, 0u, 0u, 0u};
-  }
 
-  // 3. MFMA over the wave's K range, x fragments from LDS
   dl_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  const bf16* xl = xs + r16 * LDX + kq + s0 * 32;
-#pragma unroll
-  for (int s = 0; s < MS; ++s) {
-    if (s < steps && live && !(flags & 16)) {
-      const dl_u32x4 xb = *reinterpret_cast<const dl_u32x4*>(xl + s * 32);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dl_bf16x8, wa[s]),
-                                                    __builtin_bit_cast(dl_bf16x8, xb), acc, 0, 0, 0);
-    }
+  const int wrow = cb * 16 + r16;
+  const char* wl = wt + wrow * 128;
+  const bf16* xl = xs + r16 * LDX + kq;
+  const int s1 = steps * (kh + 1) / 4;
+#pragma unroll 4
+  for (int s = steps * kh / 4; s < s1; ++s) {
+    const int ch = (4 * (s & 1) + (lane >> 4)) ^ ((wrow >> 1) & 7);
+    const dl_u32x4 wa = *reinterpret_cast<const dl_u32x4*>(wl + (s >> 1) * 4096 + (ch << 4));
+    const dl_u32x4 xb = *reinterpret_cast<const dl_u32x4*>(xl + s * 32);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dl_bf16x8, wa), __builtin_bit_cast(dl_bf16x8, xb), acc,
+                                                  0, 0, 0);
   }
-  if constexpr (KS > 1) {  // the K parts of a column block meet in LDS (every wave reaches the barrier)
-    if (kh > 0) kred[((kh - 1) * NCB + cb) * 64 + lane] = acc;
-    __syncthreads();
-    if (kh > 0 || !live) return;
+  if (kh > 0) kred[((kh - 1) * 2 + cb) * 64 + lane] = acc;
+  __syncthreads();
+  if (kh > 0 || n >= N || m >= M) return;
 #pragma unroll
-    for (int p = 0; p < KS - 1; ++p) acc += kred[(p * NCB + cb) * 64 + lane];
-  }
+  for (int p = 0; p < 3; ++p) acc += kred[(p * 2 + cb) * 64 + lane];
 
-  // 4. bias (+ GELU on the bf16-rounded linear output, the unfused pair's rounding point)
-  if (m >= M || (flags & 4)) return;
+  // bias (+ GELU on the bf16-rounded linear output, the unfused pair's rounding point)
+  const float bv[4] = {__uint_as_float(bias_v.x << 16), __uint_as_float(bias_v.x & 0xffff0000u), __uint_as_float(bias_v.y << 16),
+                       __uint_as_float(bias_v.y & 0xffff0000u)};
   float y[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -188,62 +170,7 @@ __global__ void __launch_bounds__(256) decode_ln_gemm_kernel(const float* __rest
   *reinterpret_cast<uint2*>(out + (size_t)m * o_rs + n) = uint2{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
 }
 
-// grid = ceil(M/16) * (N/16), block 256; waves split K, partial tiles reduced through LDS.
-__global__ void __launch_bounds__(256) decode_gemm_acc_kernel(const bf16* __restrict__ x, int64_t x_rs,
-                                                              const bf16* __restrict__ w, const bf16* __restrict__ bias,
-                                                              float* __restrict__ resid, int M, int N, int K, int flags) {
-  __shared__ __attribute__((aligned(16))) dl_f32x4 red[3 * 64];
-  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
-  int rb, ct;
-  dl_tile(blockIdx.x, (M + 15) / 16, N / 16, rb, ct);
-  const int steps = K / 32;
-  const int s0 = steps * wid / 4, s1 = steps * (wid + 1) / 4;
-  const int r16 = lane & 15, kq = 8 * (lane >> 4);
-  const int n0 = ct * 16;
-  const bf16* wp = w + (size_t)(n0 + r16) * K + kq;
-  const int mx = rb * 16 + r16;
-  const bf16* xp = x + (size_t)(mx < M ? mx : 0) * x_rs + kq;  // rows past M feed unstored outputs
-  // the epilogue's operands (this lane's 4 residual values and bias terms, wave 0 only) are
-  // fetched now, so the tail is LDS reduce + one store instead of two more memory round trips
-  const int m = rb * 16 + r16, n = n0 + 4 * (lane >> 4);
-  const bool owner = wid == 0 && m < M && !(flags & 4);
-  float4_t cur = {0.f, 0.f, 0.f, 0.f}, bv = {0.f, 0.f, 0.f, 0.f};
-  if (owner) {
-    cur = *reinterpret_cast<const float4_t*>(resid + (size_t)m * N + n);
-    if (bias) {
-      const uint2 u = *reinterpret_cast<const uint2*>(bias + n);
-      bv = float4_t{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
-                    __uint_as_float(u.y & 0xffff0000u)};
-    }
-  }
-  dl_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int s = s0; s < s1; s += kDlGroup) {  // one pass for K <= 4096: every load in flight at once
-    dl_u32x4 wa[kDlGroup], xb[kDlGroup];
-#pragma unroll
-    for (int u = 0; u < kDlGroup; ++u) {
-      if (s + u < s1) {
-        const size_t ko = (size_t)(s + u) * 32;
-        wa[u] = (flags & 2) ? dl_u32x4{0u, 0u, 0u, 0u} : *reinterpret_cast<const dl_u32x4*>(wp + ko);
-        xb[u] = (flags & 1) ? dl_u32x4{0u, 0u, 0u, 0u} : *reinterpret_cast<const dl_u32x4*>(xp + ko);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kDlGroup; ++u)
-      if (s + u < s1)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dl_bf16x8, wa[u]),
-                                                      __builtin_bit_cast(dl_bf16x8, xb[u]), acc, 0, 0, 0);
-  }
-  if (wid) red[(wid - 1) * 64 + lane] = acc;
-  __syncthreads();
-  if (!owner) return;
-  acc += red[lane] + red[64 + lane] + red[128 + lane];
-  float4_t* rp = reinterpret_cast<float4_t*>(resid + (size_t)m * N + n);
-#pragma unroll
-  for (int r = 0; r < 4; ++r) cur[r] += acc[r] + bv[r];
-  *rp = cur;
-}
-
-// out[M, N] = x · Wᵀ (bf16) — decode_gemm_acc's tiling (16 rows × 16 columns per workgroup, the 4
+// out[M, N] = x · Wᵀ (bf16) (16 rows × 16 columns per workgroup, the 4
 // waves split K, partial tiles reduced through LDS; every load of a wave's k-range in flight at
 // once) with a plain store, or with GATED the packed [gate; up] weight [2I, K]: a workgroup takes
 // gate columns n0..n0+15 and the matching up columns I + n0.., out[m, n] = bf16(act(bf16(g)) ·
@@ -690,10 +617,8 @@ static const bf16* dl_bias(const c10::optional<torch::Tensor>& bias, int N, cons
 }
 
 // out[M, N] = act(LayerNorm(resid) · wᵀ + bias); act 0 none, 1 GELU (erf), 2 GELU (tanh).
-// flags (timing ablations only, outputs wrong when set): 1 no residual reads, 2 no weight reads,
-// 4 no stores, 8 no LayerNorm (LDS image unwritten), 16 no MFMA
 void decode_ln_gemm(torch::Tensor resid, torch::Tensor gamma, torch::Tensor beta, double eps, torch::Tensor w,
-                    c10::optional<torch::Tensor> bias, torch::Tensor out, int64_t act, int64_t flags) {
+                    c10::optional<torch::Tensor> bias, torch::Tensor out, int64_t act) {
   TORCH_CHECK(resid.is_cuda() && resid.scalar_type() == torch::kFloat32 && resid.dim() == 2 && resid.is_contiguous(),
               "decode_ln_gemm: fp32 contiguous resid [M, K]");
   const int M = resid.size(0), K = resid.size(1);
@@ -708,41 +633,11 @@ void decode_ln_gemm(torch::Tensor resid, torch::Tensor gamma, torch::Tensor beta
               "decode_ln_gemm: bf16 out [M, N], rows 8-B aligned");
   TORCH_CHECK(act >= 0 && act <= 2, "decode_ln_gemm: act 0 (none), 1 (GELU erf), 2 (GELU tanh)");
   const bf16* bp = dl_bias(bias, N, "decode_ln_gemm");
-  // K halves (KS = 2) by default: GPT-2 decode B = 16 / 32 / 64 0.567 / 0.584 / 0.636 -> 0.532 /
-  // 0.550 / 0.620 ms/step; quarters (KS = 4) lost: 0.55 / 0.74 / 0.96 — every workgroup repeats the
-  // LayerNorm of its 16 rows (profiles/decode_r5.md). PENROZ_DECODE_LN_KSPLIT=1: 64-column tiles.
-  static const int ks_env = [] {
-    const char* e = std::getenv("PENROZ_DECODE_LN_KSPLIT");
-    return e && e[0] == '1' ? 1 : 2;
-  }();
-  const int ks = ks_env == 2 && (K / 32) % 2 == 0 ? 2 : 1;
-  const int tw = 64 / ks;
-  const int grid = ((M + 15) / 16) * ((N + tw - 1) / tw);
-  hipLaunchKernelGGL(ks == 2 ? decode_ln_gemm_kernel<2> : decode_ln_gemm_kernel<1>,
-                     dim3(grid), dim3(256), 0, at::hip::getCurrentHIPStream(), resid.data_ptr<float>(), gamma.data_ptr<float>(),
-                     beta.data_ptr<float>(), (float)eps, reinterpret_cast<const bf16*>(w.data_ptr()), bp,
-                     reinterpret_cast<bf16*>(out.data_ptr()), (int64_t)out.stride(0), M, N, K, (int)act, (int)flags);
-}
-
-// resid[M, N] += x · wᵀ + bias (fp32 residual, in place). flags: timing ablations (1 no x reads,
-// 2 no weight reads, 4 no stores)
-void decode_gemm_acc(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias, torch::Tensor resid,
-                     int64_t flags) {
-  TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kBFloat16 && x.dim() == 2 && x.stride(1) == 1 &&
-                  x.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
-              "decode_gemm_acc: bf16 x [M, K], rows 16-B aligned");
-  const int M = x.size(0), K = x.size(1);
-  TORCH_CHECK(M >= 1 && K % 32 == 0, "decode_gemm_acc: K % 32 == 0");
-  dl_check_w(w, K, "decode_gemm_acc");
-  const int N = w.size(0);
-  TORCH_CHECK(resid.scalar_type() == torch::kFloat32 && resid.is_contiguous() && resid.dim() == 2 &&
-                  resid.size(0) == M && resid.size(1) == N,
-              "decode_gemm_acc: fp32 contiguous resid [M, N]");
-  const bf16* bp = dl_bias(bias, N, "decode_gemm_acc");
-  const int grid = ((M + 15) / 16) * (N / 16);
-  hipLaunchKernelGGL(decode_gemm_acc_kernel, dim3(grid), dim3(256), 0, at::hip::getCurrentHIPStream(),
-                     reinterpret_cast<const bf16*>(x.data_ptr()), (int64_t)x.stride(0),
-                     reinterpret_cast<const bf16*>(w.data_ptr()), bp, resid.data_ptr<float>(), M, N, K, (int)flags);
+  const int grid = ((M + 15) / 16) * ((N + 31) / 32), lds = (K + 63) / 64 * 4096 + 16 * (K + 8) * 2;
+  hipFuncSetAttribute(reinterpret_cast<const void*>(decode_ln_gemm_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  hipLaunchKernelGGL(decode_ln_gemm_kernel, dim3(grid), dim3(512), lds, at::hip::getCurrentHIPStream(), resid.data_ptr<float>(),
+                     gamma.data_ptr<float>(), beta.data_ptr<float>(), (float)eps, reinterpret_cast<const bf16*>(w.data_ptr()),
+                     bp, reinterpret_cast<bf16*>(out.data_ptr()), (int64_t)out.stride(0), M, N, K, (int)act);
 }
 
 // out[M, N] = x · Wᵀ (kind < 0), or with the packed [gate; up] weight [2I, K] out[M, I] =

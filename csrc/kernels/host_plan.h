@@ -117,15 +117,17 @@ inline int plan_wgrad_group(const int* M, const int* N, int n, int K, int n_cu) 
 }
 
 // The tile of rows_gemm.hip for x [M, K] · W [N, K]ᵀ, or 0 for the library: the smallest tile that one round of workgroups on 256
-// CUs holds. 1: 32×32 (in order two to a CU, else the columns split over the waves), 2: 32×64 with split columns, 3: 64×64 (beyond
-// K = 2048 it is 5 to 9 % slower than the library), 4: 64×64 in a ring of two stages, two to a CU, 5: 64×128, two to a CU (both only
-// for K <= 1024, where their shorter rings do not wait; 5 with more than 64 rows is level with the library, 7 % slower to 6 % faster,
-// at a fifth of its host time). Larger products are the library's, whose tiles of 256 read less. M x N x K, here / library:
-// 256 x 1536 x 1024 5.8 (1, in order) / 8.6 us, 64 x 8192 x 2048 11.3 (2) / 13.3, 512 x 2304 x 768 7.7 (4) / 8.5, 1024 x 3072 x 768
-// 11.2 (5) / 11.4, 2048 x 3072 x 768 18 (5) / 15.7, 64 x 32768 x 1024 15.6 (5) / 16.9, 256 x 12288 x 2048 35 (3) / 27.
+// CUs holds. 6: 16×16 and 1: 32×32 with the columns split over the waves (1 in order: two to a CU), 2: 32×64 with split columns,
+// 3: 64×64 (beyond K = 2048 it is 5 to 9 % slower than the library), 4: 64×64 in a ring of two stages, two to a CU, 5: 64×128, two
+// to a CU (both only for K <= 1024, where their shorter rings do not wait; 5 with more than 64 rows is level with the library, 7 %
+// slower to 6 % faster, at a fifth of its host time). Larger products are the library's, whose tiles of 256 read less. M x N x K,
+// here / library, us: 64 x 768 x 3072 5.5 (6; 1: 7.4) / 9.8, 16 x 2048 x 2048 4.6 (6; 1: 5.7) / 8.1, 256 x 1536 x 1024 5.8 (1, in
+// order) / 8.6, 64 x 8192 x 2048 11.3 (2) / 13.3, 512 x 2304 x 768 7.7 (4) / 8.5, 1024 x 3072 x 768 11.2 (5) / 11.4, 2048 x 3072 x
+// 768 18 (5) / 15.7, 64 x 32768 x 1024 15.6 (5) / 16.9, 256 x 12288 x 2048 35 (3) / 27.
 inline int rows_gemm_plan(int64_t M, int64_t N, int64_t K, bool in_order) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 8 != 0 || M > 1 << 20 || N > 1 << 20 || K > 1 << 20) return 0;
   auto tiles = [&](int64_t tm, int64_t tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
+  if (!in_order && tiles(16, 16) <= 256) return 6;
   if (tiles(32, 32) <= (in_order ? 512 : 256)) return 1;
   if (!in_order && tiles(32, 64) <= 256) return 2;
   if (tiles(64, 64) <= 256 && K <= 2048) return 3;

@@ -3,14 +3,15 @@
 // Below products that fill the card with tiles of 256 lie the short steps: batches of up to 64 sequences, 256 training tokens,
 // prompts of a few hundred rows. Their products need 1 to 5 us of memory or matrix time; what bounds them is how many bytes the
 // card has on the way (about 1.1 us a trip, the ring's 96 KB per CU), so the tile is the largest that still gives nearly every CU
-// one (rows_gemm_plan, host_plan.h). A workgroup of 4 waves owns 32×32, 32×64, 64×64 or 64×128 outputs; stages of 64 to 256 columns
+// one (rows_gemm_plan, host_plan.h). A workgroup of 4 waves owns 16×16 to 64×128 outputs; stages of 64 to 256 columns
 // arrive by LDS-DMA in a ring (128-byte row pieces, whole cache lines, chunks permuted on the source side so that a fragment read
 // covers all banks); the waves split the tile (WM × WN) or the columns of a stage (WK, added through LDS at the end, in order).
 // Tiles that share weights run on one XCD. In order (WK = 1) a sum is one chain of MFMAs over k, as in the library's unsplit
 // kernels, and bit for bit theirs at K = 768: training steps take that form, where a rounding that falls otherwise changes every
-// later layer's. With the columns split, 64 x 2048 x 2048 takes 6.1 us instead of 7.0, 64 x 768 x 3072 7.4 instead of 9.0. us, library / here (weights from memory): 64 x 768 x 768 7.1 / 3.8, 64 x 2048 x 2048
+// later layer's. With the columns split, 64 x 2048 x 2048 takes 6.1 us instead of 7.0. decode_gemm_acc adds to an fp32
+// residual in place (64 x 768 x 3072: 8.3 us in a kernel whose waves read their operands directly, 6.0 here). us, library / here (weights from memory): 64 x 768 x 768 7.1 / 3.3, 64 x 2048 x 2048
 // 8.9 / 6.1, 64 x 2048 x 6144 19.0 / 16.3, 256 x 2304 x 768 7.7 / 6.5, 1024 x 1152 x 1024 9.7 / 9.2; at 16 rows, skinny_gemm / here:
-// 768 x 768 9.7 / 3.6, 2048 x 2048 7.1 / 5.7, 7232 x 2048 12.3 / 8.2. A call costs the host 4 us, the library's 19. Tiles of 128×128
+// 768 x 768 9.7 / 3.3, 2048 x 2048 7.1 / 4.6, 7232 x 2048 12.3 / 8.2. A call costs the host 4 us, the library's 19. Tiles of 128×128
 // in rings of two to four stages were no faster than the library anywhere.
 #include "common.h"
 #include "host_plan.h"
@@ -22,6 +23,9 @@ namespace {
 
 typedef __bf16 rg_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float rg_f32x4 __attribute__((ext_vector_type(4)));
+
+// what becomes of a sum: it is the output, is added to it (fp32), or its gelu (erf form) is
+enum { kRgPlain = 0, kRgAdd = 1, kRgGelu = 2 };
 
 template <int P, int LEFT>
 __device__ __forceinline__ void wait_stages(int left) {  // all but the newest `left` stages of P loads have landed
@@ -39,7 +43,8 @@ __device__ __forceinline__ void wait_stages(int left) {  // all but the newest `
 template <int FM, int FN, int WM, int WN, int WK, int KS, int NBUF, typename OUT>
 __global__ void __launch_bounds__(64 * WM * WN * WK) rows_gemm_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
                                                                       const bf16* __restrict__ bias, OUT* __restrict__ out, int M,
-                                                                      int N, int K, int ldx, int ldw, int ldo, int tiles_m) {
+                                                                      int N, int K, int ldx, int ldw, int ldo, int tiles_m,
+                                                                      int end) {
   constexpr int TM = 16 * FM * WM, TN = 16 * FN * WN, NW = WM * WN * WK;
   constexpr int SUB = (TM + TN) * 128, STAGE = WK * KS * SUB;  // a sub-slice of 64 columns: x rows, then W rows
   constexpr int COLS = 64 * WK * KS, PIECES = STAGE / 1024 / NW, PER_SUB = SUB / 1024;
@@ -126,15 +131,20 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) rows_gemm_kernel(const bf16
     const int cnt = min(4, N - n);
     if (bias != nullptr)
       for (int r = 0; r < cnt; ++r) v[r] += to_f(bias[n + r]);
+    if (end == kRgGelu)  // of the value as it is without the activation
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = gelu_f(to_f(from_f<OUT>(v[r])), 0);
     if (cnt == 4 && (ldo & 3) == 0) {
       if constexpr (sizeof(OUT) == 2) {
         bf16 h[4] = {from_f<bf16>(v[0]), from_f<bf16>(v[1]), from_f<bf16>(v[2]), from_f<bf16>(v[3])};
         *reinterpret_cast<uint2*>(o) = *reinterpret_cast<const uint2*>(h);
       } else {
-        *reinterpret_cast<float4*>(o) = float4{v[0], v[1], v[2], v[3]};
+        float4* f = reinterpret_cast<float4*>(o);
+        float4 c = end == kRgAdd ? *f : float4{0.f, 0.f, 0.f, 0.f};
+        *f = float4{c.x + v[0], c.y + v[1], c.z + v[2], c.w + v[3]};
       }
     } else {
-      for (int r = 0; r < cnt; ++r) o[r] = from_f<OUT>(v[r]);
+      for (int r = 0; r < cnt; ++r) o[r] = from_f<OUT>(end == kRgAdd ? to_f(o[r]) + v[r] : v[r]);
     }
   };
   if constexpr (WK == 1) {
@@ -143,8 +153,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) rows_gemm_kernel(const bf16
 #pragma unroll
       for (int j = 0; j < FN; ++j) store(i, j, acc[i][j]);
   } else {
-    // every wave leaves its sums, then adds FM·FN / WK blocks of all WK slices
-    static_assert(FM * FN % WK == 0, "blocks per wave");
+    // every wave leaves its sums; the blocks, shared out over the waves, are added over the WK slices
     rg_f32x4* red = reinterpret_cast<rg_f32x4*>(smem);
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -169,10 +178,40 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) rows_gemm_kernel(const bf16
 
 using namespace penroz;
 
-// x · wᵀ (+ bias) into out, or (none given) into a new tensor, fp32 or of x's type; in_order: each sum in one chain over k. None where rows_gemm_plan leaves the product to
+static void rg_launch(int tile, bool in_order, const torch::Tensor& x, const torch::Tensor& w, const bf16* bias,
+                      const torch::Tensor& out, int end) {
+  const int64_t M = x.size(0), N = w.size(0), K = x.size(1);
+  auto stream = at::hip::getCurrentHIPStream();
+  auto launch = [&](auto kern, int threads, int lds, int TM, int TN, auto* o) {
+    const int64_t tiles_m = (M + TM - 1) / TM, tiles = tiles_m * ((N + TN - 1) / TN);
+    hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(threads), lds, stream, reinterpret_cast<const bf16*>(x.data_ptr()),
+                       reinterpret_cast<const bf16*>(w.data_ptr()), bias, o, (int)M, (int)N, (int)K, (int)x.stride(0),
+                       (int)w.stride(0), (int)out.stride(0), (int)tiles_m, end);
+  };
+#define PENROZ_RG(FM, FN, WM, WN, WK, KS, NB)                                                                    \
+  launch(rows_gemm_kernel<FM, FN, WM, WN, WK, KS, NB, OUT>, 64 * WM * WN * WK,                                   \
+         NB * WK * KS * 128 * 16 * (FM * WM + FN * WN), 16 * FM * WM, 16 * FN * WN, o)
+  auto typed = [&](auto* o) {
+    using OUT = std::remove_pointer_t<decltype(o)>;
+    if (tile == 6) PENROZ_RG(1, 1, 1, 1, 4, 1, 6);
+    else if (tile == 1 && in_order) PENROZ_RG(1, 1, 2, 2, 1, 2, 4);
+    else if (tile == 1) PENROZ_RG(2, 2, 1, 1, 4, 1, 4);
+    else if (tile == 2) PENROZ_RG(2, 4, 1, 1, 4, 1, 3);
+    else if (tile == 3) PENROZ_RG(2, 2, 2, 2, 1, 2, 4);
+    else if (tile == 4) PENROZ_RG(2, 2, 2, 2, 1, 2, 2);
+    else PENROZ_RG(2, 4, 2, 2, 1, 1, 3);
+  };
+#undef PENROZ_RG
+  if (out.scalar_type() == torch::kFloat32) typed(out.data_ptr<float>());
+  else typed(reinterpret_cast<bf16*>(out.data_ptr()));
+}
+
+// x · wᵀ (+ bias) into out, or (none given) into a new tensor, fp32 or of x's type; in_order: each sum in one chain over k; gelu: its gelu (erf form). None
+// where rows_gemm_plan leaves the product to
 // the library or a row is not of 16-byte pieces.
 c10::optional<torch::Tensor> rows_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
-                                       c10::optional<torch::Tensor> out_opt, bool fp32, bool in_order) {
+                                       c10::optional<torch::Tensor> out_opt, bool fp32, bool in_order, bool gelu) {
   const bool given = out_opt.has_value() && out_opt->defined(), has_bias = bias.has_value() && bias->defined();
   if (!(x.is_cuda() && w.is_cuda() && x.get_device() == w.get_device() && x.scalar_type() == torch::kBFloat16 &&
         w.scalar_type() == torch::kBFloat16 && x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1)))
@@ -195,30 +234,33 @@ c10::optional<torch::Tensor> rows_gemm(torch::Tensor x, torch::Tensor w, c10::op
   }
   torch::Tensor out = given ? *out_opt : torch::empty({M, N}, x.options().dtype(fp32 ? torch::kFloat32 : torch::kBFloat16));
   const bf16* bp = has_bias ? reinterpret_cast<const bf16*>(bias->data_ptr()) : nullptr;
-  auto stream = at::hip::getCurrentHIPStream();
-  auto launch = [&](auto kern, int threads, int lds, int TM, int TN, auto* o) {
-    const int64_t tiles_m = (M + TM - 1) / TM, tiles = tiles_m * ((N + TN - 1) / TN);
-    hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(threads), lds, stream, reinterpret_cast<const bf16*>(x.data_ptr()),
-                       reinterpret_cast<const bf16*>(w.data_ptr()), bp, o, (int)M, (int)N, (int)K, (int)x.stride(0),
-                       (int)w.stride(0), (int)out.stride(0), (int)tiles_m);
-  };
-#define PENROZ_RG(FM, FN, WM, WN, WK, KS, NB)                                                                    \
-  launch(rows_gemm_kernel<FM, FN, WM, WN, WK, KS, NB, OUT>, 64 * WM * WN * WK,                                   \
-         NB * WK * KS * 128 * 16 * (FM * WM + FN * WN), 16 * FM * WM, 16 * FN * WN, o)
-  auto typed = [&](auto* o) {
-    using OUT = std::remove_pointer_t<decltype(o)>;
-    if (tile == 1 && in_order) PENROZ_RG(1, 1, 2, 2, 1, 2, 4);
-    else if (tile == 1) PENROZ_RG(2, 2, 1, 1, 4, 1, 4);
-    else if (tile == 2) PENROZ_RG(2, 4, 1, 1, 4, 1, 3);
-    else if (tile == 3) PENROZ_RG(2, 2, 2, 2, 1, 2, 4);
-    else if (tile == 4) PENROZ_RG(2, 2, 2, 2, 1, 2, 2);
-    else PENROZ_RG(2, 4, 2, 2, 1, 1, 3);
-  };
-#undef PENROZ_RG
-  if (fp32) typed(out.data_ptr<float>());
-  else typed(reinterpret_cast<bf16*>(out.data_ptr()));
+  rg_launch(tile, in_order, x, w, bp, out, gelu ? kRgGelu : kRgPlain);
   return out;
 }
 
 int64_t rows_gemm_tile(int64_t M, int64_t N, int64_t K, bool in_order) { return rows_gemm_plan(M, N, K, in_order); }
+
+// resid[M, N] += x · wᵀ + bias (fp32 residual, in place)
+void decode_gemm_acc(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias, torch::Tensor resid) {
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kBFloat16 && x.dim() == 2 && x.stride(1) == 1 &&
+                  x.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
+              "decode_gemm_acc: bf16 x [M, K], rows 16-B aligned");
+  const int64_t M = x.size(0), K = x.size(1);
+  TORCH_CHECK(M >= 1 && K >= 32 && K % 32 == 0, "decode_gemm_acc: K % 32 == 0");
+  TORCH_CHECK(w.is_cuda() && w.scalar_type() == torch::kBFloat16 && w.dim() == 2 && w.is_contiguous() && w.size(1) == K &&
+                  w.size(0) % 16 == 0 && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
+              "decode_gemm_acc: bf16 contiguous 16-B aligned W [N, K], N % 16 == 0");
+  const int64_t N = w.size(0);
+  TORCH_CHECK(resid.is_cuda() && resid.scalar_type() == torch::kFloat32 && resid.is_contiguous() && resid.dim() == 2 &&
+                  resid.size(0) == M && resid.size(1) == N && reinterpret_cast<uintptr_t>(resid.data_ptr()) % 16 == 0,
+              "decode_gemm_acc: fp32 contiguous resid [M, N]");
+  const bf16* bp = nullptr;
+  if (bias.has_value() && bias->defined()) {
+    TORCH_CHECK(bias->scalar_type() == torch::kBFloat16 && bias->is_contiguous() && bias->numel() == N,
+                "decode_gemm_acc: bf16 bias [N]");
+    bp = reinterpret_cast<const bf16*>(bias->data_ptr());
+  }
+  if (N == 0) return;
+  const int tile = rows_gemm_plan(M, N, K, false);
+  rg_launch(tile ? tile : 3, false, x, w, bp, resid, kRgAdd);
+}

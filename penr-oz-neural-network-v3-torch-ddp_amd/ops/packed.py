@@ -283,8 +283,10 @@ def gelu_mlp(x: Tensor, up: Tensor, down: Tensor) -> Tensor:
             u = torch.empty(x.shape[0], up.shape[0], dtype=x.dtype, device=x.device)
             kernels().decode_gemv(x, None, None, None, None, None, None, 0.0, up, None, u, 1)
         else:
-            u = linear(x, up)
-            kernels().gelu_rows(u)
+            u = gemm_ops.rows_linear(x, up, gelu=True)
+            if u is None:
+                u = linear(x, up)
+                kernels().gelu_rows(u)
     else:
         u = torch.nn.functional.gelu(torch.mm(x, up.t()).float()).to(x.dtype)
     return linear(u, down)

@@ -6,19 +6,20 @@ from penroz.ops import _ext, gemm
 
 
 @pytest.mark.skipif(not _ext.available("penroz_serve"), reason="HIP extension not built")
-@pytest.mark.parametrize("M,N,K,tile", [(1, 8, 8, 1), (64, 768, 768, 1), (256, 1024, 1024, 1), (257, 1024, 1024, 2),
+@pytest.mark.parametrize("M,N,K,tile", [(1, 8, 8, 6), (64, 768, 768, 6), (65, 832, 768, 1), (256, 1024, 1024, 1), (257, 1024, 1024, 2),
                                         (64, 8192, 2048, 2), (256, 3072, 768, 3), (64, 12288, 2048, 3), (65, 12288, 2048, 0),
                                         (512, 3072, 768, 4), (1024, 3072, 768, 5), (64, 32768, 2048, 5), (4096, 3072, 768, 0),
                                         (64, 768, 772, 0), (0, 768, 768, 0), (64, 1 << 21, 768, 0)])
 def test_rows_gemm_rule(M, N, K, tile):
     assert _ext.kernels().rows_gemm_tile(M, N, K) == tile
     in_order = _ext.kernels().rows_gemm_tile(M, N, K, True)
-    assert in_order == {(257, 1024, 1024): 1, (64, 8192, 2048): 1}.get((M, N, K), tile)
+    assert in_order == (1 if tile in (2, 6) else tile)
 
 
 # every tile: less than one, its edges, ragged rows and columns; K of less than a stage, whole stages, ragged ones
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,tile", [(1, 8, 1), (31, 33, 1), (33, 250, 1), (256, 1024, 1), (300, 1026, 2), (17, 9001, 2),
+@pytest.mark.parametrize("M,N,tile", [(1, 8, 6), (31, 33, 6), (33, 250, 6), (64, 1022, 6), (70, 1001, 1),
+                                      (256, 1024, 1), (300, 1026, 2), (17, 9001, 2),
                                       (200, 3001, 3), (64, 12288, 3), (500, 3001, 4), (700, 3100, 5), (64, 40000, 5)])
 @pytest.mark.parametrize("K", [8, 56, 64, 72, 256, 264, 760, 1024])
 def test_rows_gemm(M, N, tile, K):
@@ -32,18 +33,27 @@ def test_rows_gemm(M, N, tile, K):
     # fp32 sums of K products: in blocks of 32 in the MFMA, K / 32 of them
     assert full.dtype == torch.float32
     assert torch.linalg.norm(full.double() - want) <= 2.0 ** -24 * (K / 32 + 32) ** 0.5 * torch.linalg.norm(want)
+    act = gemm.rows_linear(x, w, bias, gelu=True)
+    lin = gemm.rows_linear(x, w, bias).double()
+    assert ((act.double() - torch.nn.functional.gelu(lin)).abs() <= 2.0 ** -8 * lin.abs() + 1e-6).all()  # one rounding to bf16
     for b, in_order in ((None, True), (None, False), (bias, True), (bias, False)):
         ref = want if b is None else want + b.double()
         got = gemm.rows_linear(x, w, b, in_order=in_order)
         if got is None:
             assert in_order and tile == 2
-            continue
+            got = gemm.rows_linear(x, w, b)
         assert got.dtype == torch.bfloat16
         # half a step of bf16 at each value, and the sums' own error where they cancel
         assert ((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -18 * K ** 0.5).all()
     buf = torch.full((M, N + 8), 7.0, device="cuda", dtype=torch.bfloat16)  # rows of a wider buffer
     assert gemm.rows_linear(x, w, bias, buf[:, :N]) is not None
     assert torch.equal(buf[:, :N], got) and (buf[:, N:] == 7.0).all()
+    if K % 32 == 0 and N % 16 == 0:  # added to an fp32 residual
+        w = w.contiguous()
+        resid = torch.randn(M, N, generator=g, device="cuda")
+        ref = resid.double() + want + bias.double()
+        _ext.kernels().decode_gemm_acc(x, w, bias, resid)
+        assert torch.linalg.norm(resid.double() - ref) <= 2.0 ** -24 * (K / 32 + 32) ** 0.5 * torch.linalg.norm(ref)
 
 
 @pytest.mark.gpu
