@@ -93,8 +93,8 @@ void gemm_nt(torch::Tensor a, torch::Tensor b, c10::optional<torch::Tensor> bias
 // gemm_wgrad.hip
 void wgrad_gemm(torch::Tensor dy, torch::Tensor x, torch::Tensor grad, int64_t tile, int64_t variant, bool accumulate);
 void wgrad_group(std::vector<torch::Tensor> dys, std::vector<torch::Tensor> xs, std::vector<torch::Tensor> grads,
-                 std::vector<bool> accumulate, int64_t variant);
-int64_t wgrad_group_tile(std::vector<int64_t> Ms, std::vector<int64_t> Ns, int64_t K, int64_t n_cu);
+                 std::vector<bool> accumulate, int64_t variant, bool shared);
+int64_t wgrad_group_tile(std::vector<int64_t> Ms, std::vector<int64_t> Ns, int64_t K, int64_t n_cu, bool shared);
 // flash_attn.hip
 void flash_attn_fwd(torch::Tensor qkv, torch::Tensor out, torch::Tensor lse, int64_t H, int64_t Hkv, int64_t D,
                     double scale, double p_drop, int64_t seed);
@@ -209,8 +209,10 @@ PYBIND11_MODULE(penroz_kernels, m) {
         pybind11::arg("act") = pybind11::none(), pybind11::arg("approx") = 0, pybind11::arg("group_m") = 0,
         pybind11::arg("grid") = 0, pybind11::arg("ablate") = 0,
         "out = a·bᵀ (+ bias) (bf16, both operands reduction-contiguous); with act: act = GELU(out)");
-  m.def("wgrad_group", &wgrad_group);
-  m.def("wgrad_group_tile", &wgrad_group_tile);
+  m.def("wgrad_group", &wgrad_group, pybind11::arg("dys"), pybind11::arg("xs"), pybind11::arg("grads"),
+        pybind11::arg("accumulate"), pybind11::arg("variant"), pybind11::arg("shared") = false);
+  m.def("wgrad_group_tile", &wgrad_group_tile, pybind11::arg("Ms"), pybind11::arg("Ns"), pybind11::arg("K"),
+        pybind11::arg("n_cu"), pybind11::arg("shared") = false);
   m.def("wgrad_gemm", &wgrad_gemm, pybind11::arg("dy"), pybind11::arg("x"), pybind11::arg("grad"),
         pybind11::arg("tile") = 256, pybind11::arg("variant") = 8, pybind11::arg("accumulate") = true,
         "grad (+)= dyᵀ·x (fp32 gradient, bf16 operands); accumulate=False overwrites grad");

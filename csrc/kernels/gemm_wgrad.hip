@@ -868,9 +868,10 @@ void wgrad_gemm(torch::Tensor dy, torch::Tensor x, torch::Tensor grad, int64_t t
 }
 
 // grads[i][M_i][N_i] (+)= dys[i]ᵀ·xs[i]: in one launch where plan_wgrad_group says that this is faster, else (and for more than 8
-// products, several K, or operands that are not 16-byte aligned) one after the other by wgrad_gemm's 256-tile kernel.
+// products, several K, or operands that are not 16-byte aligned) one after the other by wgrad_gemm's 256-tile kernel. shared:
+// another stream has work for the CUs too.
 void wgrad_group(std::vector<torch::Tensor> dys, std::vector<torch::Tensor> xs, std::vector<torch::Tensor> grads,
-                 std::vector<bool> accumulate, int64_t variant) {
+                 std::vector<bool> accumulate, int64_t variant, bool shared) {
   const size_t n = dys.size();
   TORCH_CHECK(xs.size() == n && grads.size() == n && accumulate.size() == n, "wgrad_group: one of each per product");
   if (n == 0) return;
@@ -885,7 +886,7 @@ void wgrad_group(std::vector<torch::Tensor> dys, std::vector<torch::Tensor> xs, 
     if (together) Ms[i] = dys[i].size(1), Ns[i] = xs[i].size(1);
   }
   const int K = dys[0].size(0);
-  const int TN = 128, TM = together ? plan_wgrad_group(Ms, Ns, (int)n, K, cu_count(dys[0].get_device())) : 0;
+  const int TN = 128, TM = together ? plan_wgrad_group(Ms, Ns, (int)n, K, cu_count(dys[0].get_device()), shared) : 0;
   if (TM == 0) {
     for (size_t i = 0; i < n; ++i) wgrad_gemm(dys[i], xs[i], grads[i], 256, variant, accumulate[i]);
     return;
@@ -914,8 +915,8 @@ void wgrad_group(std::vector<torch::Tensor> dys, std::vector<torch::Tensor> xs, 
 }
 
 // the tile that plan_wgrad_group takes for products [Ms[i], Ns[i]] over K (0: each by itself)
-int64_t wgrad_group_tile(std::vector<int64_t> Ms, std::vector<int64_t> Ns, int64_t K, int64_t n_cu) {
+int64_t wgrad_group_tile(std::vector<int64_t> Ms, std::vector<int64_t> Ns, int64_t K, int64_t n_cu, bool shared) {
   std::vector<int> m(Ms.begin(), Ms.end()), k(Ns.begin(), Ns.end());
   TORCH_CHECK(m.size() == k.size());
-  return plan_wgrad_group(m.data(), k.data(), (int)m.size(), (int)K, (int)n_cu);
+  return plan_wgrad_group(m.data(), k.data(), (int)m.size(), (int)K, (int)n_cu, shared);
 }

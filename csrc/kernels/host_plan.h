@@ -89,7 +89,9 @@ inline WgradPlan plan_wgrad(int M, int N, int K, int tile, int n_cu, int bk) {
 // CU), 0.6 to 0.75 in the split kernel, which costs 20 whatever its size; outputs are written at 5.5 TB/s. Measured, one by one /
 // together: GPT-2's layer 99 / 14 at 256 tokens, 134 / 62 at 3885, 275 / 243 at 16384; Gemma's 117 / 38, 302 / 239, 886 / 953; a
 // head of 50304 x 768 119 / 104 at 1024, 176 / 189 at 2048; a layer of width 256 104 / 81 at 8192, 120 / 154 at 16384.
-inline int plan_wgrad_group(const int* M, const int* N, int n, int K, int n_cu) {
+// shared: beside another stream's kernels a launch of several rounds holds every CU until its last round (Gemma-3 1B on two streams,
+// 6 x 1024 tokens: 58.2 ms a step together, 55.8 one by one; GPT-2, whose layer is one round, 9.6 and 9.9).
+inline int plan_wgrad_group(const int* M, const int* N, int n, int K, int n_cu, bool shared) {
   if (n <= 0 || K <= 0) return 0;
   const double steps = (double)(((int64_t)K + 31) / 32);
   const int64_t cus = std::max(1, n_cu);
@@ -113,7 +115,9 @@ inline int plan_wgrad_group(const int* M, const int* N, int n, int K, int n_cu) 
                       (1.0 + std::max(0, K - 4096) / 32768.0);  // operands from beyond the XCD's L2
   const double t256 = steps * 0.43 * (double)((large + cus - 1) / cus);
   if (std::min(t128, t256) + store + 6 >= single) return 0;
-  return t128 <= t256 ? 128 : 256;
+  const int tile = t128 <= t256 ? 128 : 256;
+  if (shared && (tile == 128 ? small > 2 * cus : large > cus)) return 0;
+  return tile;
 }
 
 // The tile of rows_gemm.hip for x [M, K] · W [N, K]ᵀ, or 0 for the library: the smallest tile that one round of workgroups on 256

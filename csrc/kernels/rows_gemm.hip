@@ -2,17 +2,17 @@
 //
 // Below products that fill the card with tiles of 256 lie the short steps: batches of up to 64 sequences, 256 training tokens,
 // prompts of a few hundred rows. Their products need 1 to 5 us of memory or matrix time; what bounds them is how many bytes the
-// card has on the way (about 1.1 us a trip, the ring's 96 KB per CU), so the tile is the largest that still gives nearly every CU
-// one (rows_gemm_plan, host_plan.h). A workgroup of 4 waves owns 16×16 to 64×128 outputs; stages of 64 to 256 columns
-// arrive by LDS-DMA in a ring (128-byte row pieces, whole cache lines, chunks permuted on the source side so that a fragment read
-// covers all banks); the waves split the tile (WM × WN) or the columns of a stage (WK, added through LDS at the end, in order).
-// Tiles that share weights run on one XCD. In order (WK = 1) a sum is one chain of MFMAs over k, as in the library's unsplit
-// kernels, and bit for bit theirs at K = 768: training steps take that form, where a rounding that falls otherwise changes every
-// later layer's. With the columns split, 64 x 2048 x 2048 takes 6.1 us instead of 7.0. decode_gemm_acc adds to an fp32
-// residual in place (64 x 768 x 3072: 8.3 us in a kernel whose waves read their operands directly, 6.0 here). us, library / here (weights from memory): 64 x 768 x 768 7.1 / 3.3, 64 x 2048 x 2048
-// 8.9 / 6.1, 64 x 2048 x 6144 19.0 / 16.3, 256 x 2304 x 768 7.7 / 6.5, 1024 x 1152 x 1024 9.7 / 9.2; at 16 rows, skinny_gemm / here:
-// 768 x 768 9.7 / 3.3, 2048 x 2048 7.1 / 4.6, 7232 x 2048 12.3 / 8.2. A call costs the host 4 us, the library's 19. Tiles of 128×128
-// in rings of two to four stages were no faster than the library anywhere.
+// card has on the way (about 1.1 us a trip, the ring's 96 KB per CU), so the tile is the smallest that one round of workgroups
+// holds (rows_gemm_plan, host_plan.h). A workgroup of 4 waves owns 16×16 to 64×128 outputs; stages of 64 to 256 columns arrive by
+// LDS-DMA in a ring (128-byte row pieces, whole cache lines, chunks permuted on the source side so that a fragment read covers all
+// banks); the waves split the tile (WM × WN) or the columns of a stage (WK, added through LDS at the end, in order). Tiles that
+// share weights run on one XCD. In order (WK = 1) a sum is one chain of MFMAs over k, as in the library's unsplit kernels, and bit
+// for bit theirs at K = 768: training steps take that form, where a rounding that falls otherwise changes every later layer's. With
+// the columns split, 64 x 2048 x 2048 takes 6.1 us instead of 7.0. decode_gemm_acc adds to an fp32 residual in place (64 x 768 x
+// 3072: 8.3 us in a kernel whose waves read their operands directly, 6.0 here). us, library / here (weights from memory): 64 x 768
+// x 768 7.1 / 3.3, 64 x 2048 x 2048 8.9 / 6.1, 64 x 2048 x 6144 19.0 / 16.3, 256 x 2304 x 768 7.7 / 6.5, 1024 x 1152 x 1024 9.7 / 9.2;
+// at 16 rows, skinny_gemm / here: 768 x 768 9.7 / 3.3, 2048 x 2048 7.1 / 4.6, 7232 x 2048 12.3 / 8.2. A call costs the host 4 us, the
+// library's 19. Tiles of 128×128 in rings of two to four stages were no faster than the library anywhere.
 #include "common.h"
 #include "host_plan.h"
 #include <torch/extension.h>

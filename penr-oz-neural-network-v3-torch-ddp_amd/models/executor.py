@@ -758,15 +758,14 @@ class GPTExecutor:
         self._side_stream = self._side  # what _plan_step chooses for large enough steps
         self._buf_free = {}
 
-    # The side stream costs the host an event and a wait on either stream per weight gradient: it takes 0.75 to 0.85 ms
-    # per layer to enqueue a step on two streams, whatever its size, and the card has nothing to do meanwhile unless the
-    # step is long enough. On one stream a step lasts about 0.45 ms per layer, 6 ms per 1e9 parameters (AdamW) and
-    # 1 ms per 1.1e12 operations, 6 · tokens · parameters; two streams from where that is more than the host's time. ms
-    # per step, two streams / one: GPT-2 124M (12 layers, 163e6 parameters with its own head) 256 tokens 9.0 / 5.2, 2048
-    # 9.3 / 7.2, 4096 9.7 / 9.4, 6144 11.1 / 11.7, 65536 62.0 / 63.7; 4 of its layers 1024 3.4 / 2.7, 3072 3.8 / 4.0;
-    # 24 layers, 406e6 2048 18.1 / 15.9, 5120 24.0 / 24.3; 48 layers, 1638e6 512 34.7 / 32.1, 1024 36.2 / 39.0; 6 layers,
-    # 17e6 8192 4.9 / 3.6; Gemma-3 1B (26 layers, 1302e6) 256 20.6 / 19.4, 512 20.9 / 22.2; 18 layers, 436e6 1024
-    # 14.5 / 12.4, 3072 15.8 / 17.3; 8 layers, 819e6 64 7.8 / 8.1.
+    # The side stream costs the host an event and a wait on either stream per weight gradient, and it pays from where a step is
+    # long enough for both streams to fill the card; two streams from where a step of one lasts longer than the host's time for
+    # two, 1 ms per 1.1e12 operations (6 · tokens · parameters). ms per step, two streams / one: GPT-2 124M (12 layers, 163e6
+    # parameters with its own head) 1024 tokens 5.9 / 4.4, 2048 6.7 / 5.3, 4096 7.5 / 7.5, 6144 9.6 / 10.1, 16384 18.9 / 19.0,
+    # 65536 62.0 / 63.7; Gemma-3 1B (26 layers, 1302e6) 256 17.1 / 16.5, 512 18.9 / 19.3, 1024 24.0 / 24.0, 4096 43.0 / 43.6,
+    # 6144 55.8 / 57.9, 8192 64.7 / 67.8. With each weight gradient a launch of its own: 4 of GPT-2's layers 1024 3.4 / 2.7, 3072
+    # 3.8 / 4.0; 24 layers, 406e6 2048 18.1 / 15.9, 5120 24.0 / 24.3; 48 layers, 1638e6 512 34.7 / 32.1, 1024 36.2 / 39.0; 6 layers,
+    # 17e6 8192 4.9 / 3.6; 18 layers, 436e6 1024 14.5 / 12.4, 3072 15.8 / 17.3; 8 layers, 819e6 64 7.8 / 8.1.
     SIDE_MIN_FLOPS = None  # operations of the smallest step on two streams; None: side_min_flops
 
     @staticmethod
@@ -807,7 +806,8 @@ class GPTExecutor:
         queue, self._wgrad_queue = getattr(self, "_wgrad_queue", None), None
         if queue:
             dys, xs, grads, accumulate = zip(*queue)
-            self._side_call(dys, lambda: gemm_ops.wgrad_group(dys, xs, grads, accumulate))
+            shared = getattr(self, "_side", None) is not None
+            self._side_call(dys, lambda: gemm_ops.wgrad_group(dys, xs, grads, accumulate, shared))
 
     def _emit_wgrad(self, dy: Tensor, x: Tensor, g: Tensor, accumulate: bool):
         queue = getattr(self, "_wgrad_queue", None)

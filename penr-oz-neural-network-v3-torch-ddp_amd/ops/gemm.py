@@ -67,11 +67,11 @@ def wgrad(dy: Tensor, x: Tensor, grad: Tensor, accumulate: bool = True) -> None:
         reference_wgrad(dy, x, grad, accumulate)
 
 
-def wgrad_group(dys, xs, grads, accumulate) -> None:
+def wgrad_group(dys, xs, grads, accumulate, shared: bool = False) -> None:
     """:func:`wgrad` for each of several products over the same tokens, in one launch where that is faster (the rule,
-    ``plan_wgrad_group`` in ``csrc/kernels/host_plan.h``, knows their sizes)."""
+    ``plan_wgrad_group`` in ``csrc/kernels/host_plan.h``, knows their sizes; ``shared``: another stream works beside)."""
     if not WGRAD_VARIANT and all(_native_wgrad(dy, x) for dy, x in zip(dys, xs)):
-        kernels().wgrad_group(list(dys), list(xs), list(grads), list(accumulate), _wgrad_variant(dys[0].shape[0]))
+        kernels().wgrad_group(list(dys), list(xs), list(grads), list(accumulate), _wgrad_variant(dys[0].shape[0]), shared)
         return
     for args in zip(dys, xs, grads, accumulate):
         wgrad(*args)

@@ -13,6 +13,8 @@ GPT2 = [(768, 3072), (3072, 768), (768, 768), (2304, 768)]
                                            ([(0, 768)], 64, 0), ([(768, 768)] * 9, 64, 128)])
 def test_wgrad_group_rule(shapes, K, tile):
     assert _ext.kernels().wgrad_group_tile([m for m, _ in shapes], [n for _, n in shapes], K, 256) == tile
+    beside = 0 if shapes[0][0] == 50304 else tile  # several rounds of workgroups: not beside another stream
+    assert _ext.kernels().wgrad_group_tile([m for m, _ in shapes], [n for _, n in shapes], K, 256, True) == beside
 
 
 def _products(shapes, K, seed=0):
