@@ -811,10 +811,12 @@ class GPTExecutor:
 
     def _emit_wgrad(self, dy: Tensor, x: Tensor, g: Tensor, accumulate: bool):
         queue = getattr(self, "_wgrad_queue", None)
-        if queue is None:
-            self._side_call(dy, lambda: gemm_ops.wgrad(dy, x, g, accumulate))
-        else:
+        if queue is not None:
             queue.append((dy, x, g, accumulate))
+        elif getattr(self, "_side", None) is None:
+            gemm_ops.wgrad(dy, x, g, accumulate)
+        else:  # (the kernel's rule knows of the other stream, for one product as for several)
+            self._side_call(dy, lambda: gemm_ops.wgrad_group([dy], [x], [g], [accumulate], True))
 
     def _wgrad(self, dy: Tensor, x: Tensor, p: Tensor):
         self._wgrad_into(id(p), dy, x, self.grad(p))

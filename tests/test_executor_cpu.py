@@ -285,3 +285,32 @@ def test_the_stream_rule_counts_the_models_own_parameters():
     with torch.device("meta"):
         m = _model(bench.gpt2_layers())
     assert sum(p.numel() for p in m.parameters()) == SIDE_STREAM_MS[0][1]
+
+
+@pytest.mark.parametrize("gathered", [False, True])
+@pytest.mark.parametrize("two", [False, True])
+def test_weight_gradients_beside_a_second_stream_are_planned_so(monkeypatch, gathered, two):
+    """The rule of the weight gradients' kernel is told of the main stream's work, whether a layer's products are gathered
+    or go out one by one."""
+    import contextlib
+    from types import SimpleNamespace
+
+    import torch
+    from penroz.models import executor as E
+    from penroz.ops import gemm
+    seen = []
+    monkeypatch.setattr(gemm, "_native_wgrad", lambda dy, x: True)
+    monkeypatch.setattr(gemm, "kernels", lambda: SimpleNamespace(
+        wgrad_group=lambda dys, xs, grads, accumulate, variant, shared=False: seen.append((len(dys), shared))))
+    event = SimpleNamespace(record=lambda stream: None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: None)
+    monkeypatch.setattr(torch.cuda, "Event", lambda: event)
+    monkeypatch.setattr(torch.cuda, "stream", lambda stream: contextlib.nullcontext())
+    ex = object.__new__(E.GPTExecutor)
+    ex.device, ex._buf_free = None, {}
+    ex._side = SimpleNamespace(wait_event=lambda e: None) if two else None
+    ex._wgrad_queue = [] if gathered else None
+    for _ in range(2):
+        ex._emit_wgrad(torch.empty(4, 8), torch.empty(4, 8), torch.empty(8, 8), True)
+    ex._flush_wgrads()
+    assert seen == ([(2, two)] if gathered else [(1, two)] * 2)
