@@ -90,9 +90,11 @@ inline WgradPlan plan_wgrad(int M, int N, int K, int tile, int n_cu, int bk) {
 // together: GPT-2's layer 99 / 14 at 256 tokens, 134 / 62 at 3885, 275 / 243 at 16384; Gemma's 117 / 38, 302 / 239, 886 / 953; a
 // head of 50304 x 768 119 / 104 at 1024, 176 / 189 at 2048; a layer of width 256 104 / 81 at 8192, 120 / 154 at 16384.
 // shared: beside another stream's kernels a launch of several rounds holds every CU until its last round (Gemma-3 1B on two streams,
-// 6 x 1024 tokens: 58.2 ms a step together, 55.8 one by one; GPT-2, whose layer is one round, 9.6 and 9.9).
+// 6 x 1024 tokens: 58.2 ms a step together, 55.8 one by one; GPT-2, whose layer is one round, 9.6 and 9.9). A single product is
+// then the split kernel's, whose fewer workgroups leave the other stream CUs (Gemma-3 1B, each product as it comes, 1024 tokens:
+// 24.6 ms a step with the grouped kernel, 22.4 with the split one; 1536 28.4 / 27.0, 2048 28.4 / 28.6).
 inline int plan_wgrad_group(const int* M, const int* N, int n, int K, int n_cu, bool shared) {
-  if (n <= 0 || K <= 0) return 0;
+  if (n <= 0 || K <= 0 || (shared && n == 1)) return 0;
   const double steps = (double)(((int64_t)K + 31) / 32);
   const int64_t cus = std::max(1, n_cu);
   double single = 0, store = 0;

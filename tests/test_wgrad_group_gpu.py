@@ -17,6 +17,13 @@ def test_wgrad_group_rule(shapes, K, tile):
     assert _ext.kernels().wgrad_group_tile([m for m, _ in shapes], [n for _, n in shapes], K, 256, True) == beside
 
 
+@pytest.mark.skipif(not _ext.available(), reason="HIP extension not built")
+@pytest.mark.parametrize("shape", [*GPT2, (1152, 6912), (1536, 1152), (64, 64)])
+@pytest.mark.parametrize("K", [64, 1024, 4096])
+def test_a_product_by_itself_beside_a_second_stream_is_the_split_kernels(shape, K):
+    assert _ext.kernels().wgrad_group_tile([shape[0]], [shape[1]], K, 256, True) == 0
+
+
 def _products(shapes, K, seed=0):
     g = torch.Generator(device="cuda").manual_seed(seed)
     out = []
