@@ -798,9 +798,33 @@ class GPTExecutor:
     # 243; longer ones fill the card each and start as soon as their operand is there)
     WGRAD_GROUP_TOKENS = 16384
 
-    def _gather_wgrads(self, tokens: int):
-        """From here to :meth:`_flush_wgrads` weight gradients are gathered; their operands stay untouched until then."""
-        self._wgrad_queue = [] if tokens <= self.WGRAD_GROUP_TOKENS else None
+    # Beside a second stream, products that no single launch takes start as soon as their operands are there in steps of fewer
+    # tokens than this, in others at the layer's end: always so here. ms a step, at once / at the end: width 1024 (24 layers)
+    # 4096 tokens 20.2 / 19.1, 8192 28.8 / 28.0, 14336 42.2 / 42.1; 1280 (36 layers) 2048 27.3 / 26.9, 4096 36.9 / 36.3, 8192
+    # 58.6 / 56.8. (An event and a wait per product are host time.)
+    WGRAD_AT_ONCE_TOKENS = 0
+
+    @staticmethod
+    def _wgrad_shapes(b) -> tuple:
+        """The weight gradients of a layer, [m, n] each."""
+        return tuple(tuple(lin.weight.shape) for lin in (b.fc2, b.fc, b.proj, b.qkv))
+
+    def _layer_shapes(self) -> list:
+        shapes = getattr(self, "_shapes_by_layer", None)
+        if shapes is None:
+            shapes = self._shapes_by_layer = [self._wgrad_shapes(b) for b in self.spec.blocks]
+        return shapes
+
+    def _gather_wgrads(self, l: int, tokens: int):
+        """From here to :meth:`_flush_wgrads` the weight gradients of layer ``l`` are gathered; their operands stay
+        untouched until then."""
+        self._wgrad_queue = None
+        if tokens > self.WGRAD_GROUP_TOKENS:
+            return
+        if (getattr(self, "_side", None) is not None and tokens < self.WGRAD_AT_ONCE_TOKENS
+                and not gemm_ops.wgrad_together(self._layer_shapes()[l], tokens, self.device, True)):
+            return
+        self._wgrad_queue = []
 
     def _flush_wgrads(self):
         queue, self._wgrad_queue = getattr(self, "_wgrad_queue", None), None
@@ -992,7 +1016,7 @@ class GPTExecutor:
             layer_range = trace_range(f"backward.block{l}")
             layer_range.__enter__()
             b = s.blocks[l]
-            self._gather_wgrads(N)
+            self._gather_wgrads(l, N)
             d_f, dqkv = self._reuse(self.d_f2[l & 1]), self._reuse(self.dqkv2[l & 1])
             dres_bf = self.dresid_bf2[rb]
             # ---- MLP branch

@@ -239,11 +239,14 @@ class GemmaExecutor(GPTExecutor):
             self._tw[key] = (f, self.shadow_t[off:off + n].view(w.shape[1], w.shape[0]))
             off += n
 
-    # AdamW's 28 bytes per parameter beside the main stream's memory-bound kernels slow both: two streams from 2500 tokens on.
-    # Gemma-3 1B, ms per step, two / one: 1024 tokens 24.0 / 24.0, 2048 31.5 / 30.4, 4096 43.0 / 43.6, 6144 55.8 / 57.9.
-    @staticmethod
-    def side_min_flops(layers: int, parameters: int) -> float:
-        return max(GPTExecutor.side_min_flops(layers, parameters), 6 * 2500 * parameters)
+    # ms a step on two streams, at once / at the layer's end (on one stream), of width x feed-forward x layers: 1152 x 6912 x
+    # 26 (Gemma-3 1B) 1024 tokens 22.4 / 22.3 (23.6), 1536 27.0 / 26.9 (28.3), 1792 27.9 / 29.1 (30.2), 2048 28.6 / 29.5
+    # (30.1), 3072 35.8 / 35.6 (37.5), 4096 42.2 / 42.5 (44.0), 8192 66.9 / 66.4 (69.1); 2048 x 8192 x 12 1024 14.4 / 14.7
+    # (14.2), 2048 18.5 / 18.8 (19.0), 3072 22.6 / 23.1 (23.6), 8192 42.5 / 42.6 (42.7); 1536 x 6144 x 16 1024 14.0 / 13.7
+    # (13.4), 2048 16.9 / 18.4 (17.7), 4096 26.3 / 26.4 (26.6), 6144 33.6 / 33.5 (34.4); 896 x 4864 x 20 2048 15.0 / 15.0
+    # (14.9), 3072 17.2 / 18.2 (17.3), 4096 20.4 / 20.9 (21.0), 8192 31.4 / 31.4 (32.0). (640 x 2048 x 18, one launch: 1024
+    # 10.5 (10.7), 2048 12.5 (13.1), 8192 25.6 (26.6).)
+    WGRAD_AT_ONCE_TOKENS = 4096
 
     def _refresh_transposed(self):
         if not self._tw:
@@ -357,6 +360,11 @@ class GemmaExecutor(GPTExecutor):
             inv = a._inv_freq(b.D, self.device)
             tab = self._rope_tables[key] = rope_ops.rope_table(inv, 0, T, self.device)
         return tab
+
+    @staticmethod
+    def _wgrad_shapes(b) -> tuple:
+        gate = b.mlp.gate_proj.weight
+        return (*(tuple(lin.weight.shape) for lin in (b.mlp.down_proj, b.o, b.qkv)), (2 * gate.shape[0], gate.shape[1]))
 
     def _mm(self, x: Tensor, w: Tensor, out: Tensor) -> Tensor:
         return gemm_ops.train_linear(x, w, None, out)
@@ -523,7 +531,7 @@ class GemmaExecutor(GPTExecutor):
             layer_range = trace_range(f"backward.block{l}")
             layer_range.__enter__()
             b = s.blocks[l]
-            self._gather_wgrads(N)
+            self._gather_wgrads(l, N)
             H, Hkv, D = b.H, b.Hkv, b.D
             QKV = (H + 2 * Hkv) * D
             db = self.d_branch2[rb]

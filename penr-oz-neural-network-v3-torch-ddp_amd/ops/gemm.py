@@ -10,6 +10,7 @@
 """
 from __future__ import annotations
 
+import functools
 import os
 
 import torch
@@ -75,6 +76,18 @@ def wgrad_group(dys, xs, grads, accumulate, shared: bool = False) -> None:
         return
     for args in zip(dys, xs, grads, accumulate):
         wgrad(*args)
+
+
+@functools.lru_cache(maxsize=256)
+def _wgrad_tile(shapes: tuple, tokens: int, cus: int, shared: bool) -> int:
+    return kernels().wgrad_group_tile([m for m, _ in shapes], [n for _, n in shapes], tokens, cus, shared)
+
+
+def wgrad_together(shapes: tuple, tokens: int, device: torch.device, shared: bool = False) -> bool:
+    """Whether :func:`wgrad_group` takes products [m, n] of these ``shapes`` over ``tokens`` in one launch."""
+    if WGRAD_VARIANT or NATIVE_WGRAD == "0":
+        return False
+    return _wgrad_tile(shapes, tokens, torch.cuda.get_device_properties(device).multi_processor_count, shared) != 0
 
 
 # ---- linear layers of short steps (csrc/kernels/rows_gemm.hip) ------------------------------

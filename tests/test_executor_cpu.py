@@ -314,3 +314,43 @@ def test_weight_gradients_beside_a_second_stream_are_planned_so(monkeypatch, gat
         ex._emit_wgrad(torch.empty(4, 8), torch.empty(4, 8), torch.empty(8, 8), True)
     ex._flush_wgrads()
     assert seen == ([(2, two)] if gathered else [(1, two)] * 2)
+
+
+@pytest.mark.parametrize("tokens,two,one", [(256, 16.3, 16.0), (512, 18.5, 18.6), (1024, 22.4, 23.6), (1536, 27.0, 28.3),
+                                            (2048, 28.6, 30.1), (4096, 42.5, 44.0), (8192, 66.4, 69.1)])
+def test_gemma_steps_take_the_streams_measured_faster(tokens, two, one):
+    import torch
+    from penroz.models.gemma_executor import GemmaExecutor
+    ex = GemmaExecutor.__new__(GemmaExecutor)  # Gemma-3 1B
+    ex.L, ex._side_stream, ex.flat = 26, "side", torch.empty(1301862528, device="meta")
+    ex._plan_step(tokens)
+    assert (ex._side is not None) == (two < one)
+
+
+def test_gemma_products_that_no_launch_takes_together_start_at_once(monkeypatch):
+    """On two streams, in steps of up to 4096 tokens; one stream, larger steps and products of one launch: gathered."""
+    from penroz.models import executor as E
+    from penroz.models.gemma_executor import GemmaExecutor
+    shapes = ((8, 8), (16, 8))
+    monkeypatch.setattr(E.gemm_ops, "wgrad_together", lambda sh, tokens, device, shared: (sh, shared) == ("one", True))
+    ex = GemmaExecutor.__new__(GemmaExecutor)
+    ex.device, ex._shapes_by_layer = None, [shapes, "one"]
+    for side, l, tokens, gathered in [("side", 0, 2048, False), ("side", 1, 2048, True), (None, 0, 2048, True),
+                                      ("side", 0, 4095, False), ("side", 0, 4096, True), (None, 0, 16384, True),
+                                      (None, 0, 16385, False)]:
+        ex._side = side
+        ex._gather_wgrads(l, tokens)
+        assert (ex._wgrad_queue is not None) == gathered
+
+
+def test_gemma_layer_shapes_are_those_of_its_weight_gradients():
+    from types import SimpleNamespace
+
+    from penroz.models.gemma_executor import GemmaExecutor
+    cfg = SimpleNamespace(model_type="gemma3_text", vocab_size=64, hidden_size=64, intermediate_size=128, num_hidden_layers=1,
+                          num_attention_heads=2, num_key_value_heads=1, head_dim=64, rms_norm_eps=1e-6,
+                          rope_theta=10000.0, attention_dropout=0.0, hidden_activation="gelu_pytorch_tanh")
+    spec = GemmaExecutor.match(NeuralNetworkModel("g", Mapper(Mapper.from_hf_config(cfg), {"adamw": {"lr": 1e-3}})))
+    assert GemmaExecutor._wgrad_shapes(spec.blocks[0]) == ((64, 128), (64, 128), (256, 64), (256, 64))
+    gpt = GPTExecutor.match(_model(bench.gpt2_layers(V=128, C=128, L=1, H=2, P=64)))
+    assert GPTExecutor._wgrad_shapes(gpt.blocks[0]) == ((128, 512), (512, 128), (128, 128), (384, 128))
