@@ -4,17 +4,18 @@
 // The rows of one KV head are (tq, head of its group), tq-major: a workgroup takes 64 of them, a wave 16, and goes
 // over the cache in tiles of KT keys, so that a key or value is read once per 64 rows. (decode_kernel's workgroup per
 // query row reads the whole cache for each.) us, decode_kernel / this one: 64 prompts of 64 tokens, 12 heads of 64
-// 177 / 7.7, of 512 tokens 3217 / 130; one of 64 6.3 / 4.2, of 512 60 / 13.6; 4 query heads of 256 on one key head,
-// 3 prompts of 200 tokens 38.6 / 19.8, 64 of 100 169 / 16.5, 64 of 512 2352 / 132, one of 9 9.0 / 6.7; 8 on 2 of 128,
-// 4 prompts of 300 66 / 16.4; 8 of 512, 2 of 100 132 / 43. What bounds it: at few workgroups a tile's chain (load, barrier,
-// scores, softmax, values: 1.2 us at D = 64, 2.3 at 256), at many the LDS reads of V for two products per weight.
+// 171 / 7.6, of 512 tokens 3220 / 114; one of 64 6.5 / 4.5, of 512 59 / 14.0; 4 query heads of 256 on one key head,
+// 64 prompts of 100 tokens 171 / 16.9, 64 of 512 2366 / 113; 8 on 2 of 128, 4 prompts of 300 65 / 16.8; 8 of 512, 8 of 100
+// 477 / 48.9. What bounds it: at few workgroups a tile's chain (load, barrier, scores, softmax, values: 1.2 us at D = 64,
+// 2.3 at 256), at many the LDS reads of V and three products per weight.
 //   * K and V tiles go through registers (the next tile's loads are on their way during this one's products) into
 //     LDS, 16-byte chunks XOR-swizzled by row so that neither the row reads of K nor the column reads of V
 //     (ds_read_b64_tr_b16) meet in a bank;
 //   * scores are formed transposed, K times Qt with v_mfma_f32_16x16x32_bf16: a lane holds keys of ONE query row, the
 //     softmax needs two exchanges across the wave per tile, and the weights are already the B operand of Vt times Pt;
-//   * the weights stay as exact as fp32 ones of 16 bits: they enter that product as a bf16 value and its bf16
-//     remainder (against float64 the result is as far off as with fp32 weights, to 7 digits);
+//   * the weights are fp32 ones, every bit: they enter that product as three bf16 parts of 8 bits each. (As two parts, 16
+//     bits, values that cancel leave 2^-18 of their size as an error instead of 2^-23; 64 prompts of 64 tokens 7.4 us, 64 of
+//     512 102.)
 //   * a value that is not finite would reach rows whose weight for it is zero (0 times inf): a tile that holds one is
 //     multiplied on the vector unit, by the rows that see it.
 // Where the row tiles leave CUs idle and the cache is long, the key tiles are split over workgroups and
@@ -168,12 +169,15 @@ __global__ void __launch_bounds__(256, D <= 256 ? 2 : 1) prompt_attn_kernel(
 #pragma unroll
         for (int n = 0; n < NB; n += 2) {
           // k = 8 g4 + j of the product is key 16 n + 4 g4 + j (j < 4), 16 (n + 1) + 4 g4 + j - 4
-          pa_u32x4 hi, lo;
+          pa_u32x4 hi, mid, lo;
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const float a = p[n + (j >> 1)][2 * (j & 1)], d = p[n + (j >> 1)][2 * (j & 1) + 1];
+            float a = p[n + (j >> 1)][2 * (j & 1)], d = p[n + (j >> 1)][2 * (j & 1) + 1];
             hi[j] = pack_bf16x2(a, d);
-            lo[j] = pack_bf16x2(a - __uint_as_float(hi[j] << 16), d - __uint_as_float(hi[j] & 0xffff0000u));
+            a -= __uint_as_float(hi[j] << 16), d -= __uint_as_float(hi[j] & 0xffff0000u);
+            mid[j] = pack_bf16x2(a, d);
+            a -= __uint_as_float(mid[j] << 16), d -= __uint_as_float(mid[j] & 0xffff0000u);
+            lo[j] = pack_bf16x2(a, d);
           }
           const char* vp = vt + (16 * n + 4 * g4 + (c16 >> 2)) * (2 * D) + 8 * (lane & 3);
 #pragma unroll
@@ -184,6 +188,7 @@ __global__ void __launch_bounds__(256, D <= 256 ? 2 : 1) prompt_attn_kernel(
             const uint2 ux = __builtin_bit_cast(uint2, x), uy = __builtin_bit_cast(uint2, y);
             const pa_u32x4 a = {ux.x, ux.y, uy.x, uy.y};
             o[i] = pa_mfma(a, hi, o[i]);
+            o[i] = pa_mfma(a, mid, o[i]);
             o[i] = pa_mfma(a, lo, o[i]);
           }
         }

@@ -81,3 +81,21 @@ def test_rows_off_sixteen_bytes_and_repeat():
     wide[..., 1:129] = q.reshape(2, 20, 128)
     a = attend(wide[..., 1:129].unflatten(-1, (2, 64)), k, v, 4)
     assert torch.equal(a, attend(q, k, v, 4)) and torch.equal(a, attend(q, k, v, 4))
+
+
+@pytest.mark.parametrize("D", [64, 128, 256, 512])
+def test_weights_keep_all_of_fp32(D):
+    """Values of the last three keys that cancel the others' sum, to bf16 each: what is left of it is the weights' own error."""
+    B, T, H, Hkv = (512 if D > 128 else 24), 2, 4, 1
+    g = torch.Generator(device="cuda").manual_seed(D)
+    q = torch.randn(B, T, H, D, generator=g, device="cuda").bfloat16()
+    q[:] = q[:, :, :1].clone()  # the heads of the group weigh alike, so that one value cancels for all of them
+    k, v = (torch.randn(B, Hkv, 6, D, generator=g, device="cuda").bfloat16() for _ in range(2))
+    k[:, :, 3:], v[:, :, 3:] = 0, 0
+    p = torch.matmul(q[:, 1, :1].double().unsqueeze(1), k.double().transpose(2, 3).contiguous()).div(math.sqrt(D)).softmax(-1)
+    for c in (3, 4, 5):
+        v[:, :, c] = (-torch.matmul(p, v.double())[:, :, 0] / p[:, :, 0, c:c + 1]).bfloat16()
+    ref, size = torch.matmul(p, v.double())[:, 0], torch.matmul(p, v.double().abs())[:, 0]
+    out = attend(q, k, v, 4).view(B, T, H, D)[:, 1].double()
+    # fp32 exponentials and sums of six values: a few steps of 2^-24 each; weights of 16 bits are off by up to 2^-18
+    assert ((out - ref).abs() <= 2.0 ** -20 * size + 2.0 ** -8 * ref.abs()).all()
