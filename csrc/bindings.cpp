@@ -74,6 +74,10 @@ torch::Tensor decode_attn(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, c
                           c10::optional<torch::Tensor> k_new, c10::optional<torch::Tensor> v_new,
                           c10::optional<torch::Tensor> counters, c10::optional<torch::Tensor> rope_cos,
                           c10::optional<torch::Tensor> rope_sin);
+namespace penroz {
+bool prompt_attn_applies(int64_t B, int64_t Tq, int64_t H, int64_t Hkv, int64_t D, int64_t keys);
+int prompt_attn_splits(int64_t items, int64_t rows, int64_t keys, int D, int part_keys);
+}
 bool decode_small_applies(int64_t B, int64_t Tq, int64_t H, int64_t Hkv, int64_t D, int64_t S);
 // elementwise.hip (deferred.h)
 void set_deferred_reduce_stream(int64_t stream, int64_t device);
@@ -194,6 +198,10 @@ PYBIND11_MODULE(penroz_kernels, m) {
         pybind11::arg("seq_len_dev") = pybind11::none(), pybind11::arg("k_new") = pybind11::none(),
         pybind11::arg("v_new") = pybind11::none(), pybind11::arg("counters") = pybind11::none(),
         pybind11::arg("rope_cos") = pybind11::none(), pybind11::arg("rope_sin") = pybind11::none());
+  m.def("prompt_attn_applies", &penroz::prompt_attn_applies,
+        "decode_attn takes the kernel for several query rows per sequence (B, Tq, H, Hkv, D, keys)");
+  m.def("prompt_attn_splits", &penroz::prompt_attn_splits, pybind11::arg("items"), pybind11::arg("rows"), pybind11::arg("keys"),
+        pybind11::arg("D"), pybind11::arg("part_keys") = 0, "parts that it splits the keys into");
   m.def("decode_small_applies", &decode_small_applies, "decode_attn takes the kernel for few heads and short contexts");
   m.def("set_deferred_reduce_stream", &set_deferred_reduce_stream);
   m.def("get_deferred_reduce_stream", &get_deferred_reduce_stream);

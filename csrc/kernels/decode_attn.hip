@@ -884,14 +884,11 @@ torch::Tensor decode_attn(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, c
 #undef PENROZ_DSMALL
     return out;
   }
-  // several query rows per sequence (prompts): 64 of them share each key and value that is read. Wide heads from 1024
-  // tokens: below, the gain is small beside the rest of a prompt of the models that have them (one of 9 tokens 9.0 / 6.7
-  // us, 3 of 200 38.6 / 19.8 in a layer of 190), and their bf16 residual stream turns another rounding of one value into
-  // a difference of 3 % in the logits of a few rows: those keep the results they had.
-  const bool prompt = Tq > 1 && !quant && q.scalar_type() == torch::kBFloat16 && sdev == nullptr && D >= 64 &&
-                      (D <= 128 || (int64_t)B * Tq >= 1024);
+  // several query rows per sequence (prompts): 64 of them share each key and value that is read
+  const bool prompt = !quant && q.scalar_type() == torch::kBFloat16 && sdev == nullptr &&
+                      prompt_attn_applies(B, Tq, H, Hkv, D, q_offset + Tq);
   if (prompt) {
-    splits = prompt_attn_splits((int64_t)B * Hkv, (int64_t)Tq * (H / Hkv), q_offset + Tq, D);
+    splits = prompt_attn_splits((int64_t)B * Hkv, (int64_t)Tq * (H / Hkv), q_offset + Tq, D, split_keys_env);
     if (q_rs % 8 != 0 || reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 != 0) {  // it reads 16 bytes at a time
       q = q.clone(at::MemoryFormat::Contiguous);
       q_rs = (int64_t)H * D;

@@ -244,13 +244,31 @@ __global__ void __launch_bounds__(256, D <= 256 ? 2 : 1) prompt_attn_kernel(
 
 }  // namespace
 
-int prompt_attn_splits(int64_t items, int64_t rows, int64_t keys, int D) {
+// Where a round of decode_kernel's workgroups (a query row of a KV head each) or two hold all rows and the keys are few, a row on a
+// CU of its own is sooner done than 64 together: with one head per KV head, and at 512 columns with more. us, decode_kernel / this
+// one, 2 rows of 8 heads of 64 at 102 keys 4.7 / 5.8, 402 7.6 / 11.1, 1002 13.6 / 13.0; of 128 at 2 4.4 / 5.9, 102 5.8 / 8.6, 402
+// 14.7 / 15.7, 1002 28.6 / 17.1; of 256 at 2 5.0 / 7.4, 202 14.5 / 20.6, 402 23.9 / 16.9; of 512 at 2 8.1 / 18.3, 202 54 / 70,
+// 402 100 / 51. 280 to 512 workgroups: of 64 at 34 keys 5.0 / 4.5, 207 6.9 / 9.0; of 128 at 207 11.4 / 13.8, 404 24.2 / 16.4; of
+// 256 at 57 7.7 / 9.8, 104 15.8 / 14.5; of 512 at 7 15.6 / 19.3, 34 30.6 / 28.1. 8 heads on 2: of 64 at 2 6.0 / 4.2, of 128
+// 6.5 / 5.8, of 256 9.0 / 7.2, 102 15.6 / 13.8; of 512 at 2 13.8 / 18.4, 32 23.2 / 18.3. Gemma-3 1B's logits of 1 to 17 prompts of
+// 9 to 500 tokens are 3.17 % off float64 with it, 3.18 % with decode_kernel (the bf16 residual's own error; 13 runs).
+bool prompt_attn_applies(int64_t B, int64_t Tq, int64_t H, int64_t Hkv, int64_t D, int64_t keys) {
+  if (Tq <= 1 || D < 64 || Hkv <= 0) return false;
+  const int64_t G = H / Hkv, wgs = B * Hkv * Tq;
+  if (G > 1) return !(D == 512 && wgs <= 256 && G * keys * D <= 40960);
+  if (wgs <= 256) return keys * D > (D == 512 ? 122880 : 61440);
+  if (wgs <= 512) return keys * D > (D == 512 ? 8192 : 32768) || (D == 64 && keys < 96);
+  return true;
+}
+
+int prompt_attn_splits(int64_t items, int64_t rows, int64_t keys, int D, int part_keys) {
   // parts of 192 keys (128 of wide heads), as long as there are not two workgroups per CU without: a shorter part costs
   // more in its start and in the launch that adds the parts. 12 heads of 64, 4 rows at 1000 keys, one part / 512 / 256 /
   // 192 keys 22 / 16.3 / 14.0 / 12.2 us; 4 heads of 256, 16 rows at 900 keys, 4 sequences, 512 / 128 / 64 keys
   // 64 / 21.4 / 21.0; 2 rows at 4000 keys 44.7 / 28.2 / 38.7.
   const int64_t wgs = items * ((rows + kPaRows - 1) / kPaRows);
-  return (int)std::max<int64_t>(1, std::min<int64_t>(512 / std::max<int64_t>(1, wgs), keys / (D > 128 ? 128 : 192)));
+  const int64_t parts = part_keys > 0 ? (keys + part_keys - 1) / part_keys : keys / (D > 128 ? 128 : 192);
+  return (int)std::max<int64_t>(1, std::min<int64_t>(512 / std::max<int64_t>(1, wgs), parts));
 }
 
 void prompt_attn_launch(const bf16* q, const bf16* kc, const bf16* vc, bf16* out, float* ws_o, float* ws_ml, int B,

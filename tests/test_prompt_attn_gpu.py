@@ -1,5 +1,5 @@
-"""Attention of several query rows per sequence over a bf16 cache (csrc/kernels/prompt_attn.hip) against float64, and
-against the general decode kernel through a device-side length, which takes it one query row at a time."""
+"""Attention of several query rows per sequence over a bf16 cache (csrc/kernels/prompt_attn.hip, and decode_kernel where the
+rows are few) against float64."""
 import math
 
 import pytest
@@ -99,3 +99,34 @@ def test_weights_keep_all_of_fp32(D):
     out = attend(q, k, v, 4).view(B, T, H, D)[:, 1].double()
     # fp32 exponentials and sums of six values: a few steps of 2^-24 each; weights of 16 bits are off by up to 2^-18
     assert ((out - ref).abs() <= 2.0 ** -20 * size + 2.0 ** -8 * ref.abs()).all()
+
+
+# D, B, Tq, H, Hkv, keys -> the kernel of many rows (True) or a workgroup per row
+@pytest.mark.parametrize("sizes,many", [
+    ((64, 1, 64, 12, 12, 64), True), ((64, 1, 16, 12, 12, 416), False), ((64, 1, 16, 12, 12, 1016), True),
+    ((64, 64, 4, 12, 12, 40), True), ((64, 16, 4, 8, 8, 100), False), ((64, 1, 2, 8, 2, 2), True),
+    ((128, 1, 2, 8, 8, 402), False), ((128, 1, 2, 8, 8, 1002), True), ((128, 16, 4, 8, 8, 404), True),
+    ((256, 1, 2, 8, 8, 240), False), ((256, 1, 2, 8, 8, 241), True), ((256, 3, 200, 4, 1, 200), True),
+    ((256, 1, 9, 4, 1, 9), True), ((512, 1, 2, 8, 8, 202), False), ((512, 1, 2, 8, 8, 402), True),
+    ((512, 1, 2, 8, 2, 20), False), ((512, 1, 2, 8, 2, 32), True), ((512, 8, 100, 8, 8, 100), True),
+    ((32, 8, 100, 8, 8, 100), False), ((64, 8, 1, 8, 8, 100), False)])
+def test_rule_of_rows_and_keys(sizes, many):
+    D, B, Tq, H, Hkv, keys = sizes
+    assert _ext.kernels().prompt_attn_applies(B, Tq, H, Hkv, D, keys) == many
+
+
+def test_keys_of_a_part_as_asked_for():
+    splits = _ext.kernels().prompt_attn_splits
+    assert splits(12, 64, 1000, 64) == 5 and splits(12, 64, 1000, 64, 64) == 16 and splits(12, 64, 1000, 64, 4096) == 1
+    assert splits(600, 64, 1000, 64, 64) == 1 and splits(256, 64, 1000, 64, 64) == 2
+
+
+@pytest.mark.parametrize("D", [64, 128, 256, 512])
+@pytest.mark.parametrize("B,T,H,Hkv,off", [(260, 2, 2, 2, 0), (65, 16, 2, 2, 5), (33, 17, 3, 1, 0), (9, 63, 1, 1, 1),
+                                           (130, 3, 2, 2, 130), (20, 33, 4, 4, 31)])
+def test_prompt_attention_of_many_sequences(D, B, T, H, Hkv, off):
+    assert _ext.kernels().prompt_attn_applies(B, T, H, Hkv, D, off + T)
+    q, k, v = make(B, T, H, Hkv, D, off, off + T + 3)
+    ref = exact(q, k, v, off)
+    bound = 2 ** -7.9 * ref.abs() + 2 ** -16 * v[:, :, :off + T].abs().max().double()
+    assert ((attend(q, k, v, off).double() - ref).abs() <= bound).all()
