@@ -24,8 +24,9 @@ namespace {
 typedef __bf16 rg_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float rg_f32x4 __attribute__((ext_vector_type(4)));
 
-// what becomes of a sum: it is the output, is added to it (fp32), or its gelu (erf form) is
-enum { kRgPlain = 0, kRgAdd = 1, kRgGelu = 2 };
+// what becomes of a sum: it is the output, is added to it (fp32), or its gelu (erf form) is; kRgNarrow beside it: the output is
+// not of 16-byte pieces
+enum { kRgPlain = 0, kRgAdd = 1, kRgGelu = 2, kRgNarrow = 4 };
 
 template <int P, int LEFT>
 __device__ __forceinline__ void wait_stages(int left) {  // all but the newest `left` stages of P loads have landed
@@ -123,6 +124,8 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) rows_gemm_kernel(const bf16
     __syncthreads();
     buf = buf + 1 == NBUF ? 0 : buf + 1;
   }
+  const bool wide = (ldo & 3) == 0 && !(end & kRgNarrow);
+  end &= ~kRgNarrow;
   // a lane holds row m = r16 of a block, columns 4·kq .. + 3
   auto store = [&](int i, int j, rg_f32x4 v) {
     const int m = m0 + 16 * (FM * wm + i) + r16, n = n0 + 16 * (FN * wn + j) + 4 * kq;
@@ -134,7 +137,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) rows_gemm_kernel(const bf16
     if (end == kRgGelu)  // of the value as it is without the activation
 #pragma unroll
       for (int r = 0; r < 4; ++r) v[r] = gelu_f(to_f(from_f<OUT>(v[r])), 0);
-    if (cnt == 4 && (ldo & 3) == 0) {
+    if (cnt == 4 && wide) {
       if constexpr (sizeof(OUT) == 2) {
         bf16 h[4] = {from_f<bf16>(v[0]), from_f<bf16>(v[1]), from_f<bf16>(v[2]), from_f<bf16>(v[3])};
         *reinterpret_cast<uint2*>(o) = *reinterpret_cast<const uint2*>(h);
@@ -246,13 +249,13 @@ void decode_gemm_acc(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tens
                   x.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
               "decode_gemm_acc: bf16 x [M, K], rows 16-B aligned");
   const int64_t M = x.size(0), K = x.size(1);
-  TORCH_CHECK(M >= 1 && K >= 32 && K % 32 == 0, "decode_gemm_acc: K % 32 == 0");
+  TORCH_CHECK(M >= 1 && K % 32 == 0, "decode_gemm_acc: K % 32 == 0");
   TORCH_CHECK(w.is_cuda() && w.scalar_type() == torch::kBFloat16 && w.dim() == 2 && w.is_contiguous() && w.size(1) == K &&
                   w.size(0) % 16 == 0 && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
               "decode_gemm_acc: bf16 contiguous 16-B aligned W [N, K], N % 16 == 0");
   const int64_t N = w.size(0);
   TORCH_CHECK(resid.is_cuda() && resid.scalar_type() == torch::kFloat32 && resid.is_contiguous() && resid.dim() == 2 &&
-                  resid.size(0) == M && resid.size(1) == N && reinterpret_cast<uintptr_t>(resid.data_ptr()) % 16 == 0,
+                  resid.size(0) == M && resid.size(1) == N,
               "decode_gemm_acc: fp32 contiguous resid [M, N]");
   const bf16* bp = nullptr;
   if (bias.has_value() && bias->defined()) {
@@ -261,6 +264,8 @@ void decode_gemm_acc(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tens
     bp = reinterpret_cast<const bf16*>(bias->data_ptr());
   }
   if (N == 0) return;
+  if (x.stride(0) >= (int64_t)1 << 30) x = x.contiguous();  // the kernel takes strides of 32 bits
   const int tile = rows_gemm_plan(M, N, K, false);
-  rg_launch(tile ? tile : 3, false, x, w, bp, resid, kRgAdd);
+  const bool narrow = reinterpret_cast<uintptr_t>(resid.data_ptr()) % 16 != 0;
+  rg_launch(tile ? tile : 3, false, x, w, bp, resid, narrow ? kRgAdd | kRgNarrow : kRgAdd);
 }

@@ -83,3 +83,24 @@ def test_rows_gemm_propagates_what_is_not_finite():
     got, ref = gemm.rows_linear(x, w), torch.mm(x.float(), w.float().t())
     assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(got[3, :5], ref[3, :5].bfloat16())
     assert torch.equal(got[7, :5], ref[7, :5].bfloat16())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["residual off 16 bytes", "no columns", "rows far apart"])
+def test_residual_products_of_every_form(form):
+    g = torch.Generator(device="cuda").manual_seed(1)
+    M, N, K = 5, 768, 96
+    x, w = torch.randn(M, K, generator=g, device="cuda").bfloat16(), torch.randn(N, K, generator=g, device="cuda").bfloat16()
+    bias, resid = torch.randn(N, generator=g, device="cuda").bfloat16(), torch.randn(M, N, generator=g, device="cuda")
+    if form == "residual off 16 bytes":
+        flat = torch.zeros(M * N + 3, device="cuda")
+        resid = flat[3:].view(M, N).copy_(resid)
+    elif form == "no columns":
+        x, w = x[:, :0], w[:, :0].contiguous()
+    else:  # a row stride beyond 32 bits
+        M, resid = 2, resid[:2].contiguous()
+        far = torch.empty((1 << 31) + K, dtype=torch.bfloat16, device="cuda").as_strided((2, K), (1 << 31, 1))
+        x = far.copy_(x[:2])
+    ref = resid.double() + x.double() @ w.double().t() + bias.double()
+    _ext.kernels().decode_gemm_acc(x, w, bias, resid)
+    assert torch.linalg.norm(resid.double() - ref) <= 2.0 ** -24 * 6 * torch.linalg.norm(ref)
