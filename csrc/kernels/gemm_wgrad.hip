@@ -868,8 +868,8 @@ void wgrad_gemm(torch::Tensor dy, torch::Tensor x, torch::Tensor grad, int64_t t
 }
 
 // grads[i][M_i][N_i] (+)= dys[i]ᵀ·xs[i]: in one launch where plan_wgrad_group says that this is faster, else (and for more than 8
-// products, several K, or operands that are not 16-byte aligned) one after the other by wgrad_gemm's 256-tile kernel. shared:
-// another stream has work for the CUs too.
+// products, several K, operands that are not 16-byte aligned, or gradients that share memory, whose order counts) one after the
+// other by wgrad_gemm's 256-tile kernel. shared: another stream has work for the CUs too.
 void wgrad_group(std::vector<torch::Tensor> dys, std::vector<torch::Tensor> xs, std::vector<torch::Tensor> grads,
                  std::vector<bool> accumulate, int64_t variant, bool shared) {
   const size_t n = dys.size();
@@ -884,6 +884,11 @@ void wgrad_group(std::vector<torch::Tensor> dys, std::vector<torch::Tensor> xs, 
                dys[i].stride(0) >= dys[i].size(1) && xs[i].stride(0) >= xs[i].size(1) && aligned(dys[i]) && aligned(xs[i]) &&
                aligned(grads[i]);
     if (together) Ms[i] = dys[i].size(1), Ns[i] = xs[i].size(1);
+    const char* g = static_cast<const char*>(grads[i].data_ptr());
+    for (size_t j = 0; j < i && together; ++j) {
+      const char* o = static_cast<const char*>(grads[j].data_ptr());
+      together = g + grads[i].nbytes() <= o || o + grads[j].nbytes() <= g;
+    }
   }
   const int K = dys[0].size(0);
   const int TN = 128, TM = together ? plan_wgrad_group(Ms, Ns, (int)n, K, cu_count(dys[0].get_device()), shared) : 0;

@@ -73,3 +73,18 @@ def test_wgrad_group_of_other_forms():
     off = flat[1:].view(64, 64)
     off.copy_(g)
     _check(None, 32, [True], [(dy, x, off)])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [(0, 128), (64, 192)])  # the same gradient, half of it
+def test_gradients_that_share_memory_are_written_in_order(rows):
+    g = torch.Generator(device="cuda").manual_seed(0)
+    dys = [torch.randn(96, 128, generator=g, device="cuda").bfloat16() for _ in range(2)]
+    xs = [torch.randn(96, 64, generator=g, device="cuda").bfloat16() for _ in range(2)]
+    buf = torch.randn(192, 64, generator=g, device="cuda")
+    assert _ext.kernels().wgrad_group_tile([128, 128], [64, 64], 96, 256) == 128  # apart they go in one launch
+    want = buf.double()
+    want[:128] = dys[0].double().t() @ xs[0].double()
+    want[rows[0]:rows[1]] += dys[1].double().t() @ xs[1].double()
+    gemm.wgrad_group(dys, xs, [buf[:128], buf[rows[0]:rows[1]]], [False, True])
+    assert torch.linalg.norm(buf.double() - want) <= 2.0 ** -24 * 8 * torch.linalg.norm(want)
