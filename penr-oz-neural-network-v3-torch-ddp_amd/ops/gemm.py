@@ -114,15 +114,18 @@ def linear(x: Tensor, w: Tensor, bias: Tensor | None = None, out: Tensor | None 
     return torch.mm(x, w.t(), out=out) if bias is None else torch.addmm(bias, x, w.t(), out=out)
 
 
-# Training steps take the kernel where its sums are the library's bit for bit: up to this many columns the library does not
-# split them (17 to 1100 rows measured; of 2304 and 3072 columns it splits the sums of some row counts and not of others). A
-# rounding that falls otherwise is as good, but AdamW's first steps carry it through every weight.
-TRAIN_ROWS_MAX_K = 1024
+# Training steps take the kernel where its results are the library's bit for bit (tests/test_rows_gemm_gpu.py): up to this many
+# columns the library does not split the sums (of 2304 and 3072 it splits those of some row counts and not of others), from this
+# many rows on (32 to 3000 measured, of 64 to 1024 columns; of 1 to 24 rows its other kernels round one value in 1e4 otherwise).
+# A rounding that falls otherwise is as good, but AdamW's first steps carry it through every weight.
+TRAIN_ROWS_MAX_K, TRAIN_ROWS_MIN = 1024, 32
 
 
 def train_linear(x: Tensor, w: Tensor, bias: Tensor | None = None, out: Tensor | None = None) -> Tensor:
     """x [M, K] · wᵀ (+ bias) of a training step's forward or data gradient."""
-    y = rows_linear(x, w, bias, out, in_order=True) if x.shape[1] <= TRAIN_ROWS_MAX_K else None
+    y = None
+    if x.shape[1] <= TRAIN_ROWS_MAX_K and x.shape[0] >= TRAIN_ROWS_MIN:
+        y = rows_linear(x, w, bias, out, in_order=True)
     if y is not None:
         return y
     return torch.mm(x, w.t(), out=out) if bias is None else torch.addmm(bias, x, w.t(), out=out)

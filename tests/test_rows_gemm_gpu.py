@@ -104,3 +104,29 @@ def test_residual_products_of_every_form(form):
     ref = resid.double() + x.double() @ w.double().t() + bias.double()
     _ext.kernels().decode_gemm_acc(x, w, bias, resid)
     assert torch.linalg.norm(resid.double() - ref) <= 2.0 ** -24 * 6 * torch.linalg.norm(ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [64, 256, 640, 768, 832, 1024])
+def test_sums_in_order_are_the_librarys_bits(K):
+    """What training steps rest on: from 32 rows on, of up to 1024 columns (GPT-2's and Gemma's outputs, ragged rows)."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    taken = 0
+    for N in (256, 768, 1024, 1152, 2304, 3072):
+        w = torch.randn(N, K, generator=g, device="cuda").bfloat16()
+        bias = torch.randn(N, generator=g, device="cuda").bfloat16()
+        for M in (gemm.TRAIN_ROWS_MIN, 33, 64, 100, 255, 256, 257, 513, 1000, 1100, 2048):
+            x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+            for b, want in ((None, torch.mm(x, w.t())), (bias, torch.addmm(bias, x, w.t()))):
+                got = gemm.rows_linear(x, w, b, in_order=True)
+                if got is not None:
+                    taken += 1
+                    assert torch.equal(got, want), (M, N, b is not None)
+    assert taken >= 100
+
+
+@pytest.mark.gpu
+def test_training_products_of_few_rows_are_the_librarys():
+    for M in (1, 5, 16, 31):
+        x, w = torch.randn(M, 768, device="cuda").bfloat16(), torch.randn(768, 768, device="cuda").bfloat16()
+        assert torch.equal(gemm.train_linear(x, w), torch.mm(x, w.t()))
