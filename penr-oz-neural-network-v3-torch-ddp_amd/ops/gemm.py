@@ -96,12 +96,12 @@ ROWS_GEMM = os.environ.get("PENROZ_ROWS_GEMM", "1") != "0"  # "0": the library (
 
 def rows_linear(x: Tensor, w: Tensor, bias: Tensor | None = None, out: Tensor | None = None,
                 fp32: bool = False, in_order: bool = False, gelu: bool = False) -> Tensor | None:
-    """x [M, K] · wᵀ (+ bias), bf16 (``fp32``: the sums themselves; ``in_order``: each sum in one chain over k; ``gelu``:
-    the erf gelu of the bf16 result), by the kernel of short steps; None for what its rule (``rows_gemm_plan`` in ``csrc/kernels/host_plan.h``) leaves to the
-    library."""
+    """x [M, K] · wᵀ (+ bias), bf16 (``fp32``: the sums themselves; ``in_order``: each sum in one chain over k; ``gelu``: the
+    erf gelu of the bf16 result), by the kernel of short steps; None for what its rule (``rows_gemm_plan`` in
+    ``csrc/kernels/host_plan.h``) leaves to the library."""
     if not (ROWS_GEMM and x.is_cuda and x.dtype == torch.bfloat16 and use_kernels(x)):
         return None
-    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
+    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, w, bias)):
         return None
     return kernels().rows_gemm(x, w, bias, out, fp32, in_order, gelu)
 

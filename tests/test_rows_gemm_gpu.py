@@ -130,3 +130,13 @@ def test_training_products_of_few_rows_are_the_librarys():
     for M in (1, 5, 16, 31):
         x, w = torch.randn(M, 768, device="cuda").bfloat16(), torch.randn(768, 768, device="cuda").bfloat16()
         assert torch.equal(gemm.train_linear(x, w), torch.mm(x, w.t()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", ["x", "w", "bias"])
+def test_operands_that_need_gradients_go_to_the_library(which):
+    t = {"x": torch.randn(64, 256, device="cuda").bfloat16(), "w": torch.randn(128, 256, device="cuda").bfloat16(),
+         "bias": torch.randn(128, device="cuda").bfloat16()}
+    t[which].requires_grad_()
+    gemm.linear(**t).sum().backward()
+    assert t[which].grad is not None and t[which].grad.any()
