@@ -67,6 +67,42 @@ int main() {
     const int s = penroz::reduce_slices(g);
     EXPECT(s >= 1 && (long long)s * s >= g && (long long)(s - 1) * (s - 1) < (g > 1 ? g : 2));
   }
+  // several weight gradients in one launch: a tile of 128 or 256 rows, or each by itself; any size, none of it overflowing
+  const int gsizes[] = {-1, 0, 1, 8, 127, 128, 129, 768, 50304, 1 << 20, 1 << 30};
+  for (int m : gsizes)
+    for (int n : gsizes)
+      for (int k : gsizes)
+        for (int cus : {0, 1, 256})
+          for (bool shared : {false, true}) {
+            const int Ms[8] = {m, m, 768, m, 8, m, m, m}, Ns[8] = {n, 768, n, n, 8, n, n, n};
+            for (int count : {0, 1, 2, 8}) {
+              const int t = penroz::plan_wgrad_group(Ms, Ns, count, k, cus, shared);
+              EXPECT(t == 0 || t == 128 || t == 256);
+              if (count == 0 || k <= 0 || m <= 0 || n <= 0 || (shared && count == 1)) EXPECT(t == 0);
+            }
+          }
+  {  // GPT-2's layer: together at every length up to 16384 tokens, beside a second stream as well; Gemma-3 1B's beside it never
+    const int m[] = {768, 3072, 768, 2304}, n[] = {3072, 768, 768, 768};
+    const int gm[] = {1152, 13824, 1152, 1536}, gn[] = {6912, 1152, 1024, 1152};
+    for (int k : {1, 256, 3885, 16384}) {
+      EXPECT(penroz::plan_wgrad_group(m, n, 4, k, 256, false) != 0 && penroz::plan_wgrad_group(m, n, 4, k, 256, true) != 0);
+      EXPECT(penroz::plan_wgrad_group(gm, gn, 4, k, 256, true) == 0);
+    }
+    EXPECT(penroz::plan_wgrad_group(m, n, 4, 65536, 256, false) == 0);
+  }
+  // rows_gemm: a tile or the library; no size, odd column count or size beyond 2^20 has one, and every tile's grid fits its rule
+  const int64_t rsizes[] = {-8, 0, 1, 8, 16, 17, 64, 65, 768, 772, 1024, 1152, 6912, 1 << 20, (1 << 20) + 8, (int64_t)1 << 40};
+  for (int64_t m : rsizes)
+    for (int64_t n : rsizes)
+      for (int64_t k : rsizes)
+        for (bool in_order : {false, true}) {
+          const int t = penroz::rows_gemm_plan(m, n, k, in_order);
+          EXPECT(t >= 0 && t <= 6);
+          if (m <= 0 || n <= 0 || k <= 0 || k % 8 || m > 1 << 20 || n > 1 << 20 || k > 1 << 20) EXPECT(t == 0);
+          if (in_order) EXPECT(t != 2 && t != 6);  // their waves split the columns
+          const int64_t tm[] = {1, 32, 32, 64, 64, 64, 16}, tn[] = {1, 32, 64, 64, 64, 128, 16};
+          if (t) EXPECT(((m + tm[t] - 1) / tm[t]) * ((n + tn[t] - 1) / tn[t]) <= 512);
+        }
   std::printf("host_plan_test: %s (%d failures)\n", fails ? "FAILED" : "ok", fails);
   return fails ? 1 : 0;
 }
