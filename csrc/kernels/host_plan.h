@@ -122,14 +122,20 @@ inline int plan_wgrad_group(const int* M, const int* N, int n, int K, int n_cu, 
   return tile;
 }
 
-// The tile of rows_gemm.hip for x [M, K] · W [N, K]ᵀ, or 0 for the library: the smallest tile that one round of workgroups on 256
-// CUs holds. 6: 16×16 and 1: 32×32 with the columns split over the waves (1 in order: two to a CU), 2: 32×64 with split columns,
-// 3: 64×64 (beyond K = 2048 it is 5 to 9 % slower than the library), 4: 64×64 in a ring of two stages, two to a CU, 5: 64×128, two
-// to a CU (both only for K <= 1024, where their shorter rings do not wait; 5 with more than 64 rows is level with the library, 7 %
-// slower to 6 % faster, at a fifth of its host time). Larger products are the library's, whose tiles of 256 read less. M x N x K,
-// here / library, us: 64 x 768 x 3072 5.5 (6; 1: 7.4) / 9.8, 16 x 2048 x 2048 4.6 (6; 1: 5.7) / 8.1, 256 x 1536 x 1024 5.8 (1, in
-// order) / 8.6, 64 x 8192 x 2048 11.3 (2) / 13.3, 512 x 2304 x 768 7.7 (4) / 8.5, 1024 x 3072 x 768 11.2 (5) / 11.4, 2048 x 3072 x
-// 768 18 (5) / 15.7, 64 x 32768 x 1024 15.6 (5) / 16.9, 256 x 12288 x 2048 35 (3) / 27.
+// The tile of rows_gemm.hip for x [M, K] · W [N, K]ᵀ, or 0 for the library: the smallest tile that one round of workgroups on the
+// MI355X's 256 CUs holds. 6: 16×16 and 1: 32×32 with the columns split over the waves (1 in order: two to a CU), 2: 32×64 with split
+// columns, 3: 64×64, 4: 64×64 in a ring of two stages, two to a CU, 5: 64×128, two to a CU. Larger products are the library's, whose
+// tiles of 256 read less. M x N x K, here / library, us:
+//   * 6 64 x 768 x 3072 5.5 (1: 7.4) / 9.8, 16 x 2048 x 2048 4.6 (1: 5.7) / 8.1. One block beyond its round 1 is faster than two
+//     rounds of it: 64 x 1152 x 6912 17.3 (6: 18.1) / 20.0, 64 x 1152 x 1024 4.3 (6: 5.6) / 8.4, 96 x 768 x 3072 7.3 (6: 9.3) /
+//     7.6, 96 x 1152 x 6912 17.2 / 17.1. (A tile of 32×16, not built, takes 13.2, 4.0, 6.4 and 13.1.)
+//   * 1 in order 256 x 1536 x 1024 5.8 / 8.6; 2 64 x 8192 x 2048 11.3 / 13.3, 256 x 1152 x 6912 23.9 / 24.2
+//   * 3 beyond K = 2048 is 5 to 9 % slower than the library (256 x 12288 x 2048 35 / 27); 256 x 3072 x 2048 12.5 / 12.9, 400 x 1536 x
+//     1152 8.0 / 9.6, but 400 x 2048 x 2048 11.9 / 11.0 and 1024 x 576 x 2048 11.9 / 10.5, at a fifth of its host time
+//   * 4 and 5 only for K <= 1024, where their shorter rings do not wait: 512 x 2304 x 768 7.7 (4) / 8.5, 1024 x 3072 x 768
+//     11.2 (5) / 11.4, 700 x 4096 x 1024 12.6 (5) / 11.8 (again a fifth of the host time), 2048 x 3072 x 768 18 (5) / 15.7
+//   * 5 of up to 64 rows also to K = 2048: 16 x 32768 x 2048 36.4, skinny_gemm 41.7; of up to 8 rows that is faster (5 rows 32.8,
+//     here 36.5)
 inline int rows_gemm_plan(int64_t M, int64_t N, int64_t K, bool in_order) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 8 != 0 || M > 1 << 20 || N > 1 << 20 || K > 1 << 20) return 0;
   auto tiles = [&](int64_t tm, int64_t tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
@@ -138,7 +144,7 @@ inline int rows_gemm_plan(int64_t M, int64_t N, int64_t K, bool in_order) {
   if (!in_order && tiles(32, 64) <= 256) return 2;
   if (tiles(64, 64) <= 256 && K <= 2048) return 3;
   if (tiles(64, 64) <= 512 && K <= 1024) return 4;
-  if ((tiles(64, 128) <= 384 && K <= 1024) || (M <= 64 && tiles(64, 128) <= 512 && K <= 2048)) return 5;
+  if ((tiles(64, 128) <= 384 && K <= 1024) || (M <= 64 && tiles(64, 128) <= 512 && K <= (M > 8 ? 2048 : 1024))) return 5;
   return 0;
 }
 

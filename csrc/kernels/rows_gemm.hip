@@ -6,9 +6,9 @@
 // holds (rows_gemm_plan, host_plan.h). A workgroup of 4 waves owns 16×16 to 64×128 outputs; stages of 64 to 256 columns arrive by
 // LDS-DMA in a ring (128-byte row pieces, whole cache lines, chunks permuted on the source side so that a fragment read covers all
 // banks); the waves split the tile (WM × WN) or the columns of a stage (WK, added through LDS at the end, in order). Tiles that
-// share weights run on one XCD. In order (WK = 1) a sum is one chain of MFMAs over k, as in the library's unsplit kernels, and bit
-// for bit theirs at K = 768: training steps take that form, where a rounding that falls otherwise changes every later layer's. With
-// the columns split, 64 x 2048 x 2048 takes 6.1 us instead of 7.0. decode_gemm_acc adds to an fp32 residual in place (64 x 768 x
+// share weights run on one XCD. In order (WK = 1) a sum is one chain of MFMAs over k, as in the library's unsplit kernels, and from 32
+// rows on bit for bit theirs up to K = 1024: training steps take that form there, where a rounding that falls otherwise changes every
+// later layer's. With the columns split, 64 x 2048 x 2048 takes 6.1 us instead of 7.0. decode_gemm_acc adds to an fp32 residual in place (64 x 768 x
 // 3072: 8.3 us in a kernel whose waves read their operands directly, 6.0 here). us, library / here (weights from memory): 64 x 768
 // x 768 7.1 / 3.3, 64 x 2048 x 2048 8.9 / 6.1, 64 x 2048 x 6144 19.0 / 16.3, 256 x 2304 x 768 7.7 / 6.5, 1024 x 1152 x 1024 9.7 / 9.2;
 // at 16 rows, skinny_gemm / here: 768 x 768 9.7 / 3.3, 2048 x 2048 7.1 / 4.6, 7232 x 2048 12.3 / 8.2. A call costs the host 4 us, the
@@ -210,9 +210,8 @@ static void rg_launch(int tile, bool in_order, const torch::Tensor& x, const tor
   else typed(reinterpret_cast<bf16*>(out.data_ptr()));
 }
 
-// x · wᵀ (+ bias) into out, or (none given) into a new tensor, fp32 or of x's type; in_order: each sum in one chain over k; gelu: its gelu (erf form). None
-// where rows_gemm_plan leaves the product to
-// the library or a row is not of 16-byte pieces.
+// x · wᵀ (+ bias) into out, or (none given) into a new tensor, fp32 or of x's type; in_order: each sum in one chain over k; gelu: its
+// gelu (erf form). None where rows_gemm_plan leaves the product to the library or a row is not of 16-byte pieces.
 c10::optional<torch::Tensor> rows_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
                                        c10::optional<torch::Tensor> out_opt, bool fp32, bool in_order, bool gelu) {
   const bool given = out_opt.has_value() && out_opt->defined(), has_bias = bias.has_value() && bias->defined();

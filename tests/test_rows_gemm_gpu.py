@@ -16,6 +16,13 @@ def test_rows_gemm_rule(M, N, K, tile):
     assert in_order == (1 if tile in (2, 6) else tile)
 
 
+@pytest.mark.skipif(not _ext.available("penroz_serve"), reason="HIP extension not built")
+@pytest.mark.parametrize("M,N,K,tile", [(5, 32768, 2048, 0), (8, 32768, 2048, 0), (9, 32768, 2048, 5), (5, 50304, 768, 5)])
+def test_wide_outputs_of_few_rows(M, N, K, tile):
+    """Up to 8 rows of more than 1024 columns skinny_gemm is faster."""
+    assert _ext.kernels().rows_gemm_tile(M, N, K) == tile
+
+
 # every tile: less than one, its edges, ragged rows and columns; K of less than a stage, whole stages, ragged ones
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,tile", [(1, 8, 6), (31, 33, 6), (33, 250, 6), (64, 1022, 6), (70, 1001, 1),
