@@ -1,7 +1,6 @@
 """Batched decode linears (csrc/kernels/decode_linear.hip) at GPT-2 124M decode shapes: µs per
 launch inside a replayed graph, 12 weight copies cycled (the 12 layers: weights stream from HBM /
-Infinity Cache as in a real step), with timing ablations (flags: 1 no activation reads, 2 no weight
-reads, 4 no stores; LN GEMM also 8 no LayerNorm, 16 no MFMA) and hipBLASLt (torch.mm) at the same shape for reference.
+Infinity Cache as in a real step), and hipBLASLt (torch.mm) at the same shape for reference.
 
     python bench/decode_linear_bench.py [--rows 64]
 """

@@ -551,9 +551,9 @@ class GemmaDecodeProgram:
 
 
 # 17-32 rows: decode_linear.hip decode_gemm (16 rows × 16 columns per workgroup, K split over its
-# waves) instead of hipBLASLt, whose picks for these skinny shapes ran 36-216 workgroups
-# (profiles/notes_r6.md §13); up to this many output columns (the lm_head keeps hipBLASLt).
-# PENROZ_DECODE_GEMM=0: hipBLASLt (A/B)
+# waves) for gated projections, and for the plain ones that rows_gemm leaves (more than 2048 columns in and 16384 out), instead of
+# hipBLASLt, whose picks for these skinny shapes ran 36-216 workgroups (profiles/notes_r6.md §13); up to this many output
+# columns. PENROZ_DECODE_GEMM=0: hipBLASLt (A/B)
 DECODE_GEMM = os.environ.get("PENROZ_DECODE_GEMM", "1") != "0"
 DECODE_GEMM_MAX_ROWS, DECODE_GEMM_MAX_N = 32, 32768
 

@@ -5,8 +5,11 @@
   ``csrc/kernels/gemm_wgrad.hip`` (256×256 tile, LDS-DMA staging, transposed LDS reads,
   wave-quantisation-aware split-K, deterministic slab reduction fused with the accumulate).
   Measured at GPT-2 124M shapes (K = 65 536 tokens, profiles/kernel_bench_r1_wgrad_ring16.log): 800–1100 TF
-  vs hipBLASLt's 270–950 TF on the same calls. Forward / dgrad GEMMs stay on hipBLASLt through
-  ``torch.addmm``/``torch.mm`` (measured ≈0.9–1.4 PF at these shapes).
+  vs hipBLASLt's 270–950 TF on the same calls; a layer's gradients together: ``wgrad_group``.
+* ``train_linear`` — the forward / dgrad GEMMs of training steps: hipBLASLt through ``torch.addmm``/``torch.mm``
+  (≈0.9–1.4 PF at the headline shapes), in short steps ``csrc/kernels/rows_gemm.hip`` where its bits are the same.
+* ``rows_linear`` / ``linear`` / ``linear_fp32`` — linear layers of short steps (decode, prompts): ``rows_gemm.hip`` by the
+  rule of its sizes, else the library.
 """
 from __future__ import annotations
 
@@ -138,8 +141,8 @@ def linear_fp32(x: Tensor, w: Tensor) -> Tensor:
 
 
 # ---- library GEMM solution choice (hipBLASLt / rocBLAS through torch) -----------------------
-# The forward / dgrad GEMMs stay library calls; which hipBLASLt (or rocBLAS) solution runs each
-# shape is measured, not left to the heuristic: bench/tune_gemms.sh runs PyTorch TunableOp's
+# The forward / dgrad GEMMs of steps beyond rows_gemm's sizes are library calls; which hipBLASLt (or rocBLAS) solution runs
+# each shape is measured, not left to the heuristic: bench/tune_gemms.sh runs PyTorch TunableOp's
 # solution search over every GEMM the executor issues at the GPT-2 headline shapes (and the HF
 # import layout) and ops/tuned/tunableop_gfx950.csv ships the winners (validated against the
 # PyTorch / HIP / hipBLASLt / rocBLAS versions and the gfx950 arch at load; a mismatch is refused
@@ -207,7 +210,7 @@ def guard_tuned_gemms(run_steps, steps: int = 3, rounds: int = 2, margin: float 
 # persistent MFMA GEMM with a bias/GELU epilogue and a 4-wave deferred-epilogue GEMM whose
 # stores (and GELU' / bias-column work) stream inside the next tile. Both lost on every GPT-2
 # shape and on the headline step (profiles/gemm_epi_r4.log, profiles/native_gemm_r4.md), so the
-# forward / dgrad GEMMs are hipBLASLt and the GELU work stays in elementwise.hip.
+# forward / dgrad GEMMs are plain ones (train_linear) and the GELU work stays in elementwise.hip.
 def linear_gelu(x: Tensor, w: Tensor, bias: Tensor, pre: Tensor, act: Tensor, approximate: str = "none"):
     """pre = x·wᵀ + bias (:func:`train_linear`), act = GELU(pre) (bf16; ``approximate`` "none" = erf,
     "tanh" = gelu_new; the HIP GELU kernel)."""
