@@ -35,12 +35,14 @@ inline void reduce_partials_auto(const torch::Tensor& part, int A, int G, int C,
                 "deferred reduce: event ordering failed");
     hipEventDestroy(e);  // released once the wait has been satisfied
     auto hs = c10::hip::getStreamFromExternal(d.stream, (c10::DeviceIndex)d.device);
-    mid = torch::empty({A, reduce_slices(G), C}, part.options());
     c10::hip::HIPCachingAllocator::recordStream(part.storage().data_ptr(), hs);
-    c10::hip::HIPCachingAllocator::recordStream(mid.storage().data_ptr(), hs);
+    if (reduce_in_two(G)) {
+      mid = torch::empty({A, reduce_slices(G), C}, part.options());
+      c10::hip::HIPCachingAllocator::recordStream(mid.storage().data_ptr(), hs);
+    }
     rs = d.stream;
   }
-  reduce_partials_add(part.data_ptr<float>(), A, G, C, outs, rs, mid.defined() ? mid.data_ptr<float>() : nullptr);
+  reduce_partials_add(part.data_ptr<float>(), A, G, C, outs, rs, rs != cur, mid.defined() ? mid.data_ptr<float>() : nullptr);
 }
 
 }  // namespace penroz

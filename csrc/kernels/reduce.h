@@ -1,15 +1,18 @@
 // Deterministic column reduction of per-workgroup partial rows: out[a][c] += Σ_g part[a][g][c].
 //
 // The G rows are taken in S slices of up to sqrt(G) rows, and the slices' sums are added in slice order. Fixed order => bitwise
-// reproducible, and the same bits in both forms:
+// reproducible, and the same bits in every form:
 //   * on a stream that has the card to itself one launch: a workgroup takes 32 columns and 32 of the slices at a time, a thread a
 //     slice of a column (its loads independent); the sums meet in LDS. As two launches the 972 rows of GPT-2's norms at 3885
 //     tokens take 9.8 + 9.2 us, the 64 of a step of 256 tokens 3.9 + 4.1, beside two launches' host time;
-//   * beside a second stream's work two launches, one row at a time: a workgroup per 256 columns and slice, then one per 256
-//     columns. Gemma-3 1B on two streams, 1024 / 1536 / 2048 tokens: 22.5 / 26.9 / 29.7 ms a step so, 23.7 / 27.2 / 31.0 with one
-//     launch whose workgroups walk 8 slices at a time (C / 32 of them: every load waits behind the other stream's), 23.6 / 27.4 /
-//     31.2 as two launches with eight rows' loads in flight (whose CUs the streams' products and AdamW then want at once).
-//     GPT-2, 64 x 1024 tokens: level (63.4 ms as two launches, 63.2 as one of 8 slices at a time, 63.7 of 32).
+//   * beside a second stream's work, of fewer than 1024 rows (up to 3072 tokens of a Gemma step), two launches, one row at a
+//     time: a workgroup per 256 columns and slice, then one per 256 columns. Gemma-3 1B on two streams, 1024 / 1536 / 2048 / 3072
+//     tokens: 22.8 / 27.3 / 29.1 / 36.1 ms a step so, 24.5 / 28.3 / 29.5 / 36.0 with one launch of 8 slices at a time. (Eight rows'
+//     loads in flight give the CUs to the next kernels of both streams at once: with a layer's products at its end 1024 / 1536 / 2048
+//     tokens take 23.6 / 27.7 / 31.3 so, 22.8 / 27.7 / 30.2 with one row at a time.)
+//   * beside a second stream's work, of more rows, one launch of 8 slices at a time, in workgroups of 4 waves: Gemma-3 1B,
+//     4096 / 6144 / 8192 tokens 42.1 / 56.2 / 65.9 ms a step so, 42.9 / 56.6 / 66.2 as two launches; GPT-2, 64 x 1024 61.1 / 61.4
+//     (one launch of 32 slices, whose 16 waves rarely find room on a CU: 0.5 more); 24 layers of 1024, 8192 tokens 27.5 / 27.8.
 #pragma once
 #include <hip/hip_runtime.h>
 #include "host_plan.h"
@@ -21,17 +24,16 @@ struct OutPtrs {
   float* p[3];
 };
 
-constexpr int kReduceSlices = 32;
-
-__global__ void __launch_bounds__(32 * kReduceSlices) reduce_columns_kernel(const float* __restrict__ part, int G, int C, int S,
-                                                                            OutPtrs outs) {
-  __shared__ float sums[kReduceSlices][32];
+// NS slices at a time
+template <int NS>
+__global__ void __launch_bounds__(32 * NS) reduce_columns_kernel(const float* __restrict__ part, int G, int C, int S, OutPtrs outs) {
+  __shared__ float sums[NS][32];
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const int c = blockIdx.x * 32 + tx, a = blockIdx.y;
   const int per = (G + S - 1) / S;
   const float* p = part + (size_t)a * G * C + c;
   float acc = 0.f;
-  for (int s0 = 0; s0 < S; s0 += kReduceSlices) {
+  for (int s0 = 0; s0 < S; s0 += NS) {
     const int s = s0 + ty, g1 = s < S && c < C ? min(G, (s + 1) * per) : 0;
     float v = 0.f;
 #pragma unroll 8
@@ -39,7 +41,7 @@ __global__ void __launch_bounds__(32 * kReduceSlices) reduce_columns_kernel(cons
     sums[ty][tx] = v;
     __syncthreads();
     if (ty == 0)
-      for (int j = 0; j < min(kReduceSlices, S - s0); ++j) acc += sums[j][tx];
+      for (int j = 0; j < min(NS, S - s0); ++j) acc += sums[j][tx];
     __syncthreads();
   }
   if (ty == 0 && c < C) outs.p[a][c] += acc;
@@ -64,19 +66,25 @@ __global__ void __launch_bounds__(256) reduce_sums_kernel(const float* __restric
   outs.p[a][c] += acc;
 }
 
-// part: [A][G][C] fp32 (A <= 3); outs[a] fp32 [C] (accumulated into); mid: null, or room for A·S·C floats where another stream
-// has work for the CUs too (S = reduce_slices(G))
+// whether rows beside another stream's work are summed in two launches
+inline bool reduce_in_two(int G) { return G < 1024; }
+
+// part: [A][G][C] fp32 (A <= 3); outs[a] fp32 [C] (accumulated into); shared: another stream has work for the CUs too; mid: then, if
+// reduce_in_two(G), room for A·S·C floats (S = reduce_slices(G))
 inline void reduce_partials_add(const float* part, int A, int G, int C, float* const* outs, hipStream_t stream,
-                                float* mid = nullptr) {
+                                bool shared = false, float* mid = nullptr) {
   OutPtrs o{};
   for (int a = 0; a < A; ++a) o.p[a] = outs[a];
   const int S = reduce_slices(G);
-  if (mid == nullptr) {
-    hipLaunchKernelGGL(reduce_columns_kernel, dim3((C + 31) / 32, A), dim3(32 * kReduceSlices), 0, stream, part, G, C, S, o);
-    return;
+  const dim3 grid((C + 31) / 32, A);
+  if (!shared) {
+    hipLaunchKernelGGL(reduce_columns_kernel<32>, grid, dim3(1024), 0, stream, part, G, C, S, o);
+  } else if (mid == nullptr) {
+    hipLaunchKernelGGL(reduce_columns_kernel<8>, grid, dim3(256), 0, stream, part, G, C, S, o);
+  } else {
+    hipLaunchKernelGGL(reduce_slices_kernel, dim3((C + 255) / 256, S, A), dim3(256), 0, stream, part, G, C, S, mid);
+    hipLaunchKernelGGL(reduce_sums_kernel, dim3((C + 255) / 256, A), dim3(256), 0, stream, mid, C, S, o);
   }
-  hipLaunchKernelGGL(reduce_slices_kernel, dim3((C + 255) / 256, S, A), dim3(256), 0, stream, part, G, C, S, mid);
-  hipLaunchKernelGGL(reduce_sums_kernel, dim3((C + 255) / 256, A), dim3(256), 0, stream, mid, C, S, o);
 }
 
 }  // namespace

@@ -27,3 +27,10 @@ def test_column_reduction(rows, cols):
         K.set_deferred_reduce_stream(0, 0)
     torch.cuda.current_stream().wait_stream(side)
     assert torch.equal(main, beside)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cols", [40, 3072])
+def test_column_reduction_of_many_rows(cols):
+    """1024 partial rows and more: one launch on either stream, of 32 slices or of 8 at a time, the same bits."""
+    test_column_reduction(16500, cols)
