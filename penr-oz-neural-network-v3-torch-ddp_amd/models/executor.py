@@ -762,8 +762,8 @@ class GPTExecutor:
     # long enough for both streams to fill the card; two streams from where a step of one lasts longer than the host's time for
     # two, 1 ms per 1.1e12 operations (6 · tokens · parameters). ms per step, two streams / one: GPT-2 124M (12 layers, 163e6
     # parameters with its own head) 1024 tokens 5.9 / 4.4, 2048 6.7 / 5.3, 4096 7.5 / 7.5, 6144 9.6 / 10.1, 16384 18.9 / 19.0,
-    # 65536 62.0 / 63.7; Gemma-3 1B (26 layers, 1302e6) 256 17.1 / 16.5, 512 18.9 / 19.3, 1024 24.0 / 24.0, 4096 43.0 / 43.6,
-    # 6144 55.8 / 57.9, 8192 64.7 / 67.8. With each weight gradient a launch of its own: 4 of GPT-2's layers 1024 3.4 / 2.7, 3072
+    # 65536 62.0 / 63.7; Gemma-3 1B (26 layers, 1302e6) 256 16.3 / 16.0, 512 18.5 / 18.6, 1024 22.4 / 23.6, 2048 28.6 / 30.1, 4096
+    # 42.5 / 44.0, 8192 66.4 / 69.1. With each weight gradient a launch of its own: 4 of GPT-2's layers 1024 3.4 / 2.7, 3072
     # 3.8 / 4.0; 24 layers, 406e6 2048 18.1 / 15.9, 5120 24.0 / 24.3; 48 layers, 1638e6 512 34.7 / 32.1, 1024 36.2 / 39.0; 6 layers,
     # 17e6 8192 4.9 / 3.6; 18 layers, 436e6 1024 14.5 / 12.4, 3072 15.8 / 17.3; 8 layers, 819e6 64 7.8 / 8.1.
     SIDE_MIN_FLOPS = None  # operations of the smallest step on two streams; None: side_min_flops
