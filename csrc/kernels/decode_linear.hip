@@ -6,10 +6,10 @@
 // The residual stream stays fp32 and is updated IN PLACE by decode_gemm_acc's epilogue, so
 // the separate "residual add + LayerNorm" kernel between the GEMMs disappears: the next
 // decode_ln_gemm normalises the rows it needs itself. Two choices keep that redundant
-// normalisation cheap (the round-2 fused kernel normalised all 64 rows in every 16-column
-// workgroup and lost at 64 rows, profiles/decode_fused_rows_r2.log):
-//   * a decode_ln_gemm workgroup owns 16 ROWS × 32 columns, so it normalises only its 16 rows;
-//   * four waves bring the weights while the other four normalise.
+// normalisation cheap (a kernel that normalised all 64 rows in every 16-column workgroup lost at 64 rows,
+// profiles/decode_fused_rows_r2.log):
+//   * a decode_ln_gemm workgroup owns up to 16 ROWS × 16 to 64 columns, so it normalises only its rows;
+//   * its weights are on the way meanwhile.
 // Row blocks of one column tile are placed on one XCD (blockIdx % 8 picks the XCD), so the
 // 4 row blocks' weight reads after the first hit that XCD's L2.
 //
@@ -27,7 +27,7 @@ typedef short dl_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float dl_f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t dl_u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kDlMaxSteps = 32;  // decode_ln_gemm: K <= 1024 (16 values of a row per lane)
+constexpr int kDlMaxSteps = 32;  // decode_ln_gemm: K <= 1024 (up to 4 quads of a row per lane)
 constexpr int kDlGroup = 32;     // decode_gemm: k-steps per wave whose loads are issued together
 
 // (row block, column tile) of a workgroup: the nrb row blocks of column tile ct share
@@ -45,120 +45,66 @@ __device__ __forceinline__ void dl_tile(int id, int nrb, int nct, int& rb, int& 
   }
 }
 
-// grid = ceil(M/16) * ceil(N/32), block 512: waves 0-3 normalise 16 rows, 4 each, into LDS ([16][K + 8] bf16) while waves 4-7
-// bring the 32 weight rows by LDS-DMA (sub-slices of 64 columns, 16-byte chunks permuted on the source side: fragment reads cover
-// all banks); then the 8 waves take 2 column blocks × 4 shares of K, which meet in LDS. Bound by the chain launch, loads, two wave
-// sums per row, MFMAs, store: with the weights in the registers of the waves that normalise, their loads (memory) stood before
-// the residual's (L2) in the wave's queue: qkv / fc of GPT-2 at 64 rows 9.1 / 9.7 us so, 7.2 / 7.8 now; at 8 rows 7.0 / 7.5, 5.7 /
-// 6.2. (8 waves that each hold weights and normalise two rows: 12.7 at 64 rows.)
-__global__ void __launch_bounds__(512) decode_ln_gemm_kernel(const float* __restrict__ resid,
-                                                             const float* __restrict__ gamma,
-                                                             const float* __restrict__ beta, float eps,
-                                                             const bf16* __restrict__ w, const bf16* __restrict__ bias,
-                                                             bf16* __restrict__ out, int64_t o_rs, int M, int N, int K,
-                                                             int act) {
-  extern __shared__ __attribute__((aligned(16))) char dl_smem[];
-  __shared__ __attribute__((aligned(16))) dl_f32x4 kred[3 * 2 * 64];
-  const int subs = (K + 63) / 64, steps = K / 32;
-  char* const wt = dl_smem;                                        // [subs][32 rows][128 B]
-  bf16* const xs = reinterpret_cast<bf16*>(dl_smem + subs * 4096);  // [16][LDX]
-  const int LDX = K + 8;  // +16 B per row: a fragment's 16 row reads spread over the banks
-  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int rb, ct;
-  dl_tile(blockIdx.x, (M + 15) / 16, (N + 31) / 32, rb, ct);
-  const int r16 = lane & 15, kq = 8 * (lane >> 4), cb = wid & 1, kh = wid >> 1;
-  const int m = rb * 16 + r16, n = ct * 32 + cb * 16 + 4 * (lane >> 4);
-  uint2 bias_v{0u, 0u};
-  if (wid >= 4) {
-    const unsigned base = lds_addr_of(wt);
-    for (int p = wid - 4; p < 4 * subs; p += 4) {  // 8 rows of a sub-slice
-      const int row = (p & 3) * 8 + (lane >> 3), k = (p >> 2) * 64 + 8 * ((lane & 7) ^ ((row >> 1) & 7));
-      const bf16* src = w + (size_t)min(ct * 32 + row, N - 1) * K + k;
-      glds16(k < K ? (const void*)src : (const void*)g_zero16, __builtin_amdgcn_readfirstlane(base + p * 1024));
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  } else {
-    // LayerNorm of rows wid + 4i (fp32 two-pass on the register copy)
-    float v[4][4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = rb * 16 + wid + 4 * i;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int c = 4 * (lane + 64 * j);
-        if (row < M && c < K) {
-          const float4_t r = *reinterpret_cast<const float4_t*>(resid + (size_t)row * K + c);
-          v[i][j][0] = r[0]; v[i][j][1] = r[1]; v[i][j][2] = r[2]; v[i][j][3] = r[3];
-        } else {
-          v[i][j][0] = v[i][j][1] = v[i][j][2] = v[i][j][3] = 0.f;
-        }
-      }
-    }
-    float4_t g[4], b[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int c = 4 * (lane + 64 * j);
-      if (c < K) {
-        g[j] = *reinterpret_cast<const float4_t*>(gamma + c);
-        b[j] = *reinterpret_cast<const float4_t*>(beta + c);
-      }
-    }
-    // the epilogue's bias terms, fetched now (not a memory round trip after the MFMAs)
-    if (bias && kh == 0 && n < N) bias_v = *reinterpret_cast<const uint2*>(bias + n);
-    const float inv_k = 1.f / (float)K;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int lr = wid + 4 * i;
-      bf16* xr = xs + lr * LDX;
-      float s = 0.f;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) s += (v[i][j][0] + v[i][j][1]) + (v[i][j][2] + v[i][j][3]);
-      const float mean = wave_sum(s) * inv_k;
-      float ss = 0.f;
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (4 * (lane + 64 * j) < K)
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const float d = v[i][j][k] - mean;
-            ss += d * d;
-          }
-      const float rstd = rsqrtf(wave_sum(ss) * inv_k + eps);
-      const bool row_ok = rb * 16 + lr < M;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int c = 4 * (lane + 64 * j);
-        if (c >= K) continue;
-        uint2 pk{0u, 0u};
-        if (row_ok)
-          pk = uint2{pack_bf16x2((v[i][j][0] - mean) * rstd * g[j][0] + b[j][0], (v[i][j][1] - mean) * rstd * g[j][1] + b[j][1]),
-                     pack_bf16x2((v[i][j][2] - mean) * rstd * g[j][2] + b[j][2], (v[i][j][3] - mean) * rstd * g[j][3] + b[j][3])};
-        *reinterpret_cast<uint2*>(xr + c) = pk;
-      }
-    }
-  }
-  __syncthreads();
+// Sums over the wave of R values per lane at once (R 1, 2 or 4): two values share every step of the butterfly, so R of them take
+// little more than one (each by itself: 13 instructions a sum). Afterwards a lane holds the sum of value sum_of<R>(lane).
+template <int R>
+__device__ __forceinline__ int sum_of(int lane) {
+  return R == 1 ? 0 : R == 2 ? lane >> 5 : (lane >> 5) + 2 * ((lane >> 4) & 1);
+}
+template <int R>
+__device__ __forceinline__ float wave_sums(const float (&s)[R]) {
+  static_assert(R == 1 || R == 2 || R == 4, "");
+  auto over32 = [](float a, float b) {  // the lower half gets the sums of a, the upper one those of b
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  };
+  auto over16 = [](float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  };
+  const float lo = over32(s[0], s[R > 1]);
+  float u = over16(lo, R == 4 ? over32(s[R - 2], s[R - 1]) : lo);
+  u += dpp_f32<0xB1>(u);   // quad_perm [1,0,3,2]
+  u += dpp_f32<0x4E>(u);   // quad_perm [2,3,0,1]
+  u += dpp_f32<0x141>(u);  // row_half_mirror
+  u += dpp_f32<0x140>(u);  // row_mirror
+  return u;
+}
+template <int R>
+__device__ __forceinline__ float sum_at(float u, int i) {  // value i's, for every lane
+  return R == 1 ? u : lane_f32(u, R == 2 ? 32 * i : 32 * (i & 1) + 16 * (i >> 1));
+}
 
+__device__ __forceinline__ uint2 ln_quad(const float4_t& d, float rstd, const float4_t& g, const float4_t& b) {
+  return uint2{pack_bf16x2(d[0] * rstd * g[0] + b[0], d[1] * rstd * g[1] + b[1]),
+               pack_bf16x2(d[2] * rstd * g[2] + b[2], d[3] * rstd * g[3] + b[3])};
+}
+
+// A wave's steps s0 .. s1 - 1 of K, its weights in registers. (With every read of x before the first product, and the steps past the
+// wave's own on zeros instead of behind a branch, GPT-2's steps took 1 to 3 % longer.)
+template <int SMAX>
+__device__ __forceinline__ dl_f32x4 ln_products(const dl_u32x4 (&wv)[SMAX], const bf16* xl, int s0, int s1) {
   dl_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  const int wrow = cb * 16 + r16;
-  const char* wl = wt + wrow * 128;
-  const bf16* xl = xs + r16 * LDX + kq;
-  const int s1 = steps * (kh + 1) / 4;
-#pragma unroll 4
-  for (int s = steps * kh / 4; s < s1; ++s) {
-    const int ch = (4 * (s & 1) + (lane >> 4)) ^ ((wrow >> 1) & 7);
-    const dl_u32x4 wa = *reinterpret_cast<const dl_u32x4*>(wl + (s >> 1) * 4096 + (ch << 4));
-    const dl_u32x4 xb = *reinterpret_cast<const dl_u32x4*>(xl + s * 32);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dl_bf16x8, wa), __builtin_bit_cast(dl_bf16x8, xb), acc,
-                                                  0, 0, 0);
-  }
-  if (kh > 0) kred[((kh - 1) * 2 + cb) * 64 + lane] = acc;
-  __syncthreads();
-  if (kh > 0 || n >= N || m >= M) return;
 #pragma unroll
-  for (int p = 0; p < 3; ++p) acc += kred[(p * 2 + cb) * 64 + lane];
+  for (int u = 0; u < SMAX; ++u)
+    if (s0 + u < s1) {
+      const dl_u32x4 xb = *reinterpret_cast<const dl_u32x4*>(xl + 32 * (s0 + u));
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dl_bf16x8, wv[u]), __builtin_bit_cast(dl_bf16x8, xb), acc, 0, 0,
+                                                    0);
+    }
+  return acc;
+}
 
-  // bias (+ GELU on the bf16-rounded linear output, the unfused pair's rounding point)
+// The end of both LayerNorm products: this wave's sums over its share of K (wave: column block cb, share kh of KS) meet those of the
+// others; bias, and GELU on the bf16-rounded linear output (the unfused pair's rounding point).
+template <int NB, int KS>
+__device__ __forceinline__ void ln_end(dl_f32x4 acc, dl_f32x4* kred, int cb, int kh, int lane, uint2 bias_v, bool store,
+                                       bf16* __restrict__ o, int act) {
+  if (kh > 0) kred[((kh - 1) * NB + cb) * 64 + lane] = acc;
+  __syncthreads();
+  if (kh > 0 || !store) return;
+#pragma unroll
+  for (int p = 0; p < KS - 1; ++p) acc += kred[(p * NB + cb) * 64 + lane];
   const float bv[4] = {__uint_as_float(bias_v.x << 16), __uint_as_float(bias_v.x & 0xffff0000u), __uint_as_float(bias_v.y << 16),
                        __uint_as_float(bias_v.y & 0xffff0000u)};
   float y[4];
@@ -167,7 +113,205 @@ __global__ void __launch_bounds__(512) decode_ln_gemm_kernel(const float* __rest
     y[r] = acc[r] + bv[r];
     if (act) y[r] = gelu_f(bf2f(from_f<bf16>(y[r])), act - 1);
   }
-  *reinterpret_cast<uint2*>(out + (size_t)m * o_rs + n) = uint2{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
+  *reinterpret_cast<uint2*>(o) = uint2{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
+}
+
+// out = act(LN(resid) · Wᵀ + bias), 5 rows or more. A workgroup owns 4·RPW rows × 16·NB columns: the first 4 waves normalise RPW rows
+// each (fp32, two passes over the row in registers) into LDS, and all its waves hold their shares of the weights in registers, asked
+// for behind the residual, whose reads (L2) then come back first. JC = ceil(K / 256): quads of a row per lane.
+// Bound by the chain launch, loads, sums, MFMAs, store, and from two workgroups on a CU by what one CU reads (48 KB of residual and
+// 24 KB of weights per 16 columns at K = 768). So NB is the smallest, up to 4, that leaves every workgroup a CU of its own (256 of
+// them; 64 x 2304 x 768 with NB 1 to 4: 6.4, 6.2, 5.0, 5.7 us). us, K 768: N 2304 at 8 / 16 / 32 / 64 rows 3.5 / 4.0 / 4.4 / 5.0,
+// N 3072 4.2 / 4.5 / 4.9 / 5.6; with weights by LDS-DMA beside 4 waves that sum each row by itself, always 32 columns: 5.4 / 5.7 /
+// 5.7 / 6.8 and 5.9 / 6.2 / 6.2 / 7.4. K 1024, N 4096: 4.4 / 4.6 / 5.6 / 7.2, so 6.5 / 7.2 / 7.3 / 12.0.
+template <int JC, int RPW, int NB>
+__global__ void __launch_bounds__(NB == 1 ? 256 : NB == 3 ? 384 : 512) decode_ln_gemm_kernel(
+    const float* __restrict__ resid, const float* __restrict__ gamma, const float* __restrict__ beta, float eps,
+    const bf16* __restrict__ w, const bf16* __restrict__ bias, bf16* __restrict__ out, int64_t o_rs, int M, int N, int K, int act) {
+  constexpr int NW = NB == 1 ? 4 : NB == 3 ? 6 : 8, KS = NW / NB, MB = 4 * RPW, SMAX = 8 * JC / KS;
+  __shared__ __attribute__((aligned(16))) bf16 xs[MB * (256 * JC + 8)];
+  __shared__ __attribute__((aligned(16))) dl_f32x4 kred[(KS - 1) * NB * 64];
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int rb, ct;
+  dl_tile(blockIdx.x, (M + MB - 1) / MB, (N + 16 * NB - 1) / (16 * NB), rb, ct);
+  const int LDX = K + 8, steps = K / 32;  // (+16 B per row: a fragment's row reads spread over the banks)
+  const int r16 = lane & 15, kq = 8 * (lane >> 4), cb = wid % NB, kh = wid / NB;
+  // rows past M and quads past K are read from the last one
+  float4_t r[RPW][JC], g[JC], b[JC];
+  if (wid < 4) {
+#pragma unroll
+    for (int i = 0; i < RPW; ++i)
+#pragma unroll
+      for (int j = 0; j < JC; ++j)
+        r[i][j] = *reinterpret_cast<const float4_t*>(resid + (size_t)min(rb * MB + wid + 4 * i, M - 1) * K +
+                                                     min(4 * lane + 256 * j, K - 4));
+#pragma unroll
+    for (int j = 0; j < JC; ++j) {
+      g[j] = *reinterpret_cast<const float4_t*>(gamma + min(4 * lane + 256 * j, K - 4));
+      b[j] = *reinterpret_cast<const float4_t*>(beta + min(4 * lane + 256 * j, K - 4));
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);  // the loads below stay behind those above
+  const int s0 = steps * kh / KS, s1 = steps * (kh + 1) / KS, nrow = (ct * NB + cb) * 16;
+  const bf16* wp = w + (size_t)min(nrow + r16, N - 1) * K + kq;
+  dl_u32x4 wv[SMAX];
+#pragma unroll
+  for (int s = 0; s < SMAX; ++s) wv[s] = *reinterpret_cast<const dl_u32x4*>(wp + 32 * min(s0 + s, steps - 1));
+  const int m = rb * MB + r16, n = nrow + 4 * (lane >> 4);
+  uint2 bias_v{0u, 0u};
+  if (bias && kh == 0 && n < N) bias_v = *reinterpret_cast<const uint2*>(bias + n);
+  __builtin_amdgcn_sched_barrier(0);
+  if (wid < 4) {
+    const float inv_k = 1.f / (float)K;
+    const bool last = 4 * lane + 256 * (JC - 1) < K;  // the lane's last quad is one of the row
+    float s[RPW], q[RPW];
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      s[i] = 0.f;
+#pragma unroll
+      for (int j = 0; j < JC; ++j) {
+        const float v = (r[i][j][0] + r[i][j][1]) + (r[i][j][2] + r[i][j][3]);
+        s[i] += j < JC - 1 || last ? v : 0.f;
+      }
+    }
+    const float mean = wave_sums<RPW>(s) * inv_k;
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      const float mi = sum_at<RPW>(mean, i);
+      q[i] = 0.f;
+#pragma unroll
+      for (int j = 0; j < JC; ++j) {
+        float v = 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          r[i][j][k] -= mi;
+          v += r[i][j][k] * r[i][j][k];
+        }
+        q[i] += j < JC - 1 || last ? v : 0.f;
+      }
+    }
+    const float rstd = rsqrtf(wave_sums<RPW>(q) * inv_k + eps);
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      const float ri = sum_at<RPW>(rstd, i);
+#pragma unroll
+      for (int j = 0; j < JC; ++j)
+        if (j < JC - 1 || last)
+          *reinterpret_cast<uint2*>(xs + (wid + 4 * i) * LDX + 4 * lane + 256 * j) = ln_quad(r[i][j], ri, g[j], b[j]);
+    }
+  }
+  // a barrier for LDS alone: __syncthreads would wait for the weights as well
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  const dl_f32x4 acc = ln_products<SMAX>(wv, xs + min(r16, MB - 1) * LDX + kq, s0, s1);
+  ln_end<NB, KS>(acc, kred, cb, kh, lane, bias_v, n < N && m < M && r16 < MB, out + (size_t)m * o_rs + n, act);
+}
+
+// The same for up to R = 1, 2 or 4 rows: 16 columns per workgroup of 4 waves, each with 256 columns of all the rows; the waves' sums
+// and squares about their own means meet in LDS (Chan's rule, as exact as two passes over the row). EMB: the residual rows are
+// wte[token] + wpe[position] (the first block of a decode step, embed_fwd_kernel's arithmetic: clamped token, position min(*epos, P -
+// 1)) and are written to `resid`. us at 1 / 2 / 4 rows: N 2304, K 768 2.9 / 3.1 / 3.3, where waves of their own that each normalise all
+// the rows took 3.7 / 5.2 / 7.8; N 3072 3.6 / 3.7 / 4.0, so 3.9 / 5.5 / 8.0; N 4096, K 1024 3.7 / 3.8 / 3.8, so 4.7 / 6.5 / 10.6.
+template <int JC, int R, bool EMB>
+__global__ void __launch_bounds__(256) decode_ln_few_kernel(float* __restrict__ resid, const float* __restrict__ gamma,
+                                                            const float* __restrict__ beta, float eps, const bf16* __restrict__ w,
+                                                            const bf16* __restrict__ bias, bf16* __restrict__ out, int64_t o_rs,
+                                                            int M, int N, int K, int act, const int64_t* __restrict__ eidx,
+                                                            const bf16* __restrict__ ewte, const bf16* __restrict__ ewpe,
+                                                            const int64_t* __restrict__ epos, int eV, int eP) {
+  constexpr int SMAX = 2 * JC;
+  __shared__ __attribute__((aligned(16))) bf16 xs[R * (256 * JC + 8)];
+  __shared__ __attribute__((aligned(16))) float2 part[R][4];
+  __shared__ __attribute__((aligned(16))) dl_f32x4 kred[3 * 64];
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int LDX = K + 8, steps = K / 32, c = 4 * threadIdx.x, cc = min(c, K - 4);
+  const int r16 = lane & 15, kq = 8 * (lane >> 4);
+  float4_t r[R];
+  uint2 te[R], pe{0u, 0u};
+  if constexpr (EMB) {
+    const int64_t p = *epos;
+    pe = *reinterpret_cast<const uint2*>(ewpe + (size_t)(p < eP ? p : eP - 1) * K + cc);
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      int64_t tok = eidx[min(i, M - 1)];
+      tok = tok < 0 ? 0 : tok >= eV ? eV - 1 : tok;
+      te[i] = *reinterpret_cast<const uint2*>(ewte + (size_t)tok * K + cc);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < R; ++i) r[i] = *reinterpret_cast<const float4_t*>(resid + (size_t)min(i, M - 1) * K + cc);
+  }
+  const float4_t g = *reinterpret_cast<const float4_t*>(gamma + cc), b = *reinterpret_cast<const float4_t*>(beta + cc);
+  __builtin_amdgcn_sched_barrier(0);
+  const int s0 = steps * wid / 4, s1 = steps * (wid + 1) / 4, nrow = blockIdx.x * 16;
+  const bf16* wp = w + (size_t)min(nrow + r16, N - 1) * K + kq;
+  dl_u32x4 wv[SMAX];
+#pragma unroll
+  for (int s = 0; s < SMAX; ++s) wv[s] = *reinterpret_cast<const dl_u32x4*>(wp + 32 * min(s0 + s, steps - 1));
+  const int n = nrow + 4 * (lane >> 4);
+  uint2 bias_v{0u, 0u};
+  if (bias && wid == 0 && n < N) bias_v = *reinterpret_cast<const uint2*>(bias + n);
+  __builtin_amdgcn_sched_barrier(0);
+  const bool ok = c < K;
+  if constexpr (EMB) {
+    auto quad = [](uint2 u) {
+      return float4_t{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                      __uint_as_float(u.y & 0xffff0000u)};
+    };
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      r[i] = quad(te[i]) + quad(pe);
+      if (blockIdx.x == 0 && ok && i < M) *reinterpret_cast<float4_t*>(resid + (size_t)i * K + c) = r[i];
+    }
+  }
+  float2 mine{0.f, 0.f};
+  if (256 * wid < K) {
+    const float inv_c = 1.f / (float)min(K - 256 * wid, 256);
+    float s[R], q[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) s[i] = ok ? (r[i][0] + r[i][1]) + (r[i][2] + r[i][3]) : 0.f;
+    mine.x = wave_sums<R>(s);
+    const float mu = mine.x * inv_c;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const float mi = sum_at<R>(mu, i);
+      float v = 0.f;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v += (r[i][k] - mi) * (r[i][k] - mi);
+      q[i] = ok ? v : 0.f;
+    }
+    mine.y = wave_sums<R>(q);
+  }
+  if ((lane & 15) == 0) part[sum_of<R>(lane)][wid] = mine;
+  __builtin_amdgcn_s_waitcnt(0xc07f);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  if (256 * wid < K) {
+    const float inv_k = 1.f / (float)K;
+    const float2* pr = part[sum_of<R>(lane)];
+    float2 p[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) p[x] = pr[x];
+    const float mean = ((p[0].x + p[1].x) + (p[2].x + p[3].x)) * inv_k;
+    float sq = 0.f;
+#pragma unroll
+    for (int x = 0; x < JC; ++x) {
+      const float cnt = (float)min(K - 256 * x, 256), d = p[x].x / cnt - mean;
+      sq += p[x].y + cnt * d * d;
+    }
+    const float rstd = rsqrtf(sq * inv_k + eps);
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const float mi = sum_at<R>(mean, i), ri = sum_at<R>(rstd, i);
+      if (ok) *reinterpret_cast<uint2*>(xs + i * LDX + c) = ln_quad(r[i] - mi, ri, g, b);
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0xc07f);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  const dl_f32x4 acc = ln_products<SMAX>(wv, xs + min(r16, R - 1) * LDX + kq, s0, s1);
+  ln_end<1, 4>(acc, kred, 0, wid, lane, bias_v, n < N && r16 < M && r16 < R, out + (size_t)r16 * o_rs + n, act);
 }
 
 // out[M, N] = x · Wᵀ (bf16) (16 rows × 16 columns per workgroup, the 4
@@ -616,6 +760,58 @@ static const bf16* dl_bias(const c10::optional<torch::Tensor>& bias, int N, cons
   return reinterpret_cast<const bf16*>(bias->data_ptr());
 }
 
+struct LnEmb {  // the residual rows are the step's embeddings
+  const int64_t* idx = nullptr;
+  const bf16 *wte = nullptr, *wpe = nullptr;
+  const int64_t* pos = nullptr;
+  int V = 0, P = 0;
+};
+
+// K % 32 == 0, K <= 1024, N % 16 == 0, rows of out and the bias of 8-byte pieces; emb: up to 4 rows
+static void ln_launch(float* resid, const float* gamma, const float* beta, float eps, const bf16* w, const bf16* bias, bf16* out,
+                      int64_t o_rs, int M, int N, int K, int act, const LnEmb* emb) {
+  auto stream = at::hip::getCurrentHIPStream();
+  auto few = [&](auto jc, auto r, auto e) {
+    constexpr int JC = decltype(jc)::value, R = decltype(r)::value;
+    constexpr bool EMB = decltype(e)::value;
+    const LnEmb none, &m = emb ? *emb : none;
+    hipLaunchKernelGGL((decode_ln_few_kernel<JC, R, EMB>), dim3((N + 15) / 16), dim3(256), 0, stream, resid, gamma, beta, eps, w,
+                       bias, out, o_rs, M, N, K, act, m.idx, m.wte, m.wpe, m.pos, m.V, m.P);
+  };
+  auto rows = [&](auto jc, auto rpw, auto nb) {
+    constexpr int JC = decltype(jc)::value, RPW = decltype(rpw)::value, NB = decltype(nb)::value;
+    const int grid = ((M + 4 * RPW - 1) / (4 * RPW)) * ((N + 16 * NB - 1) / (16 * NB));
+    hipLaunchKernelGGL((decode_ln_gemm_kernel<JC, RPW, NB>), dim3(grid), dim3(NB == 1 ? 256 : NB == 3 ? 384 : 512), 0, stream, resid,
+                       gamma, beta, eps, w, bias, out, o_rs, M, N, K, act);
+  };
+  auto typed = [&](auto jc) {
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    using Four = std::integral_constant<int, 4>;
+    if (M <= 4) {
+      auto by_rows = [&](auto e) {
+        if (M == 1) few(jc, One{}, e);
+        else if (M == 2) few(jc, Two{}, e);
+        else few(jc, Four{}, e);
+      };
+      if (emb) by_rows(std::true_type{});
+      else by_rows(std::false_type{});
+      return;
+    }
+    if (M <= 8) return rows(jc, Two{}, One{});
+    // the smallest tile that leaves each workgroup one of the 256 CUs
+    const int64_t blocks = (int64_t)((M + 15) / 16) * (N / 16);
+    if (blocks <= 256) rows(jc, Four{}, One{});
+    else if (blocks <= 512) rows(jc, Four{}, Two{});
+    else if (blocks <= 768) rows(jc, Four{}, std::integral_constant<int, 3>{});
+    else rows(jc, Four{}, Four{});
+  };
+  if (K <= 256) typed(std::integral_constant<int, 1>{});
+  else if (K <= 512) typed(std::integral_constant<int, 2>{});
+  else if (K <= 768) typed(std::integral_constant<int, 3>{});
+  else typed(std::integral_constant<int, 4>{});
+}
+
 // out[M, N] = act(LayerNorm(resid) · wᵀ + bias); act 0 none, 1 GELU (erf), 2 GELU (tanh).
 void decode_ln_gemm(torch::Tensor resid, torch::Tensor gamma, torch::Tensor beta, double eps, torch::Tensor w,
                     c10::optional<torch::Tensor> bias, torch::Tensor out, int64_t act) {
@@ -633,11 +829,9 @@ void decode_ln_gemm(torch::Tensor resid, torch::Tensor gamma, torch::Tensor beta
               "decode_ln_gemm: bf16 out [M, N], rows 8-B aligned");
   TORCH_CHECK(act >= 0 && act <= 2, "decode_ln_gemm: act 0 (none), 1 (GELU erf), 2 (GELU tanh)");
   const bf16* bp = dl_bias(bias, N, "decode_ln_gemm");
-  const int grid = ((M + 15) / 16) * ((N + 31) / 32), lds = (K + 63) / 64 * 4096 + 16 * (K + 8) * 2;
-  hipFuncSetAttribute(reinterpret_cast<const void*>(decode_ln_gemm_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  hipLaunchKernelGGL(decode_ln_gemm_kernel, dim3(grid), dim3(512), lds, at::hip::getCurrentHIPStream(), resid.data_ptr<float>(),
-                     gamma.data_ptr<float>(), beta.data_ptr<float>(), (float)eps, reinterpret_cast<const bf16*>(w.data_ptr()),
-                     bp, reinterpret_cast<bf16*>(out.data_ptr()), (int64_t)out.stride(0), M, N, K, (int)act);
+  ln_launch(resid.data_ptr<float>(), gamma.data_ptr<float>(), beta.data_ptr<float>(), (float)eps,
+            reinterpret_cast<const bf16*>(w.data_ptr()), bp, reinterpret_cast<bf16*>(out.data_ptr()), out.stride(0), M, N, K, (int)act,
+            nullptr);
 }
 
 // out[M, N] = x · Wᵀ (kind < 0), or with the packed [gate; up] weight [2I, K] out[M, I] =
@@ -760,6 +954,15 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
     TORCH_CHECK(bias->scalar_type() == torch::kBFloat16 && bias->is_contiguous() && bias->numel() == N,
                 "decode_gemv: bf16 bias [N]");
     bp = reinterpret_cast<const bf16*>(bias->data_ptr());
+  }
+  // a LayerNorm product of whole tiles: one workgroup normalises for 16 columns (decode_ln_few_kernel). The vocabulary's many columns
+  // stay with the waves below (50304 x 768, one row: 15.9 us, 77 MB at 4.9 TB/s)
+  if (ln && !dp && rows_per_wave <= 0 && K % 32 == 0 && N % 16 == 0 && N < 16384 && out.stride(0) % 4 == 0 &&
+      reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0 && reinterpret_cast<uintptr_t>(bp) % 8 == 0) {
+    const LnEmb e{eip, ewp, epp, eps_p, eV, eP};
+    ln_launch(emb ? rop : const_cast<float*>(rp), gp, bt, (float)eps, reinterpret_cast<const bf16*>(w.data_ptr()), bp,
+              reinterpret_cast<bf16*>(out.data_ptr()), out.stride(0), M, N, K, (int)act, emb ? &e : nullptr);
+    return;
   }
   const int cpl = (K / 8 + 31) / 32;
   int rpw = (int)rows_per_wave;
