@@ -443,45 +443,19 @@ __device__ __forceinline__ float other_half(float v, int half) {  // lane ^ 32
   return __uint_as_float(half ? r[0] : r[1]);
 }
 
-// EPI (the two half-waves' rows as a pair): 0 — independent rows, act(y + bias); 1 — gated MLP
-// on the packed [gate; up] weight (N = 2I rows): half 0 takes gate row n, half 1 up row I + n,
-// out[n] = act_f(bf16(g), kind) · bf16(u) (skinny_gated's rounding); 2 — RoPE QKV: pair p of head
-// p / (D/2), j = p % (D/2): half 0 row head·D + j, half 1 row + D/2, both rounded to bf16, then
-// rotated by one position's cos / sin [D/2] for the first nrot heads (skinny_qkv_rope's math).
-// In modes 1 / 2 a wave owns RP output pairs.
 // PRO: 0 — x is the bf16 operand; 1 — LN mode (GPT: fp32 residual + delta + dbias, LayerNorm)
-template <int M, int PRO, int RP, int CPL, int EPI = 0>
+template <int M, int PRO, int RP, int CPL>
 __global__ void __launch_bounds__(64) decode_gemv_kernel(
     const float* __restrict__ rin, const bf16* __restrict__ delta, const float* __restrict__ dbias,
     float* __restrict__ rout, const float* __restrict__ gamma, const float* __restrict__ beta, float eps,
     const bf16* __restrict__ x, int64_t x_rs, const bf16* __restrict__ w, const bf16* __restrict__ bias,
-    bf16* __restrict__ out, int64_t o_rs, int N, int K, int act, int D = 0, int nrot = 0,
-    const float* __restrict__ cosv = nullptr, const float* __restrict__ sinv = nullptr,
-    const int64_t* __restrict__ eidx = nullptr, const bf16* __restrict__ ewte = nullptr,
+    bf16* __restrict__ out, int64_t o_rs, int N, int K, int act, const int64_t* __restrict__ eidx = nullptr, const bf16* __restrict__ ewte = nullptr,
     const bf16* __restrict__ ewpe = nullptr, const int64_t* __restrict__ epos = nullptr, int eV = 0, int eP = 0) {
   constexpr bool LN = PRO == 1;
-  // EPI 3 (PRO 0 only): the whole wave on each of its RP rows — lane l reads chunks l, l + 64, …
-  // — twice the workgroups of the half-wave form for the same rows per wave
-  constexpr bool WR = EPI == 3;
-  constexpr int CS = WR ? 64 : 32;  // lanes striding over a row's chunks
-  static_assert(!WR || PRO == 0, "wave-per-row mode reads a bf16 x");
   const int lane = threadIdx.x, h = lane >> 5, l32 = lane & 31;
-  const int cl = WR ? lane : l32;
   const int nc = K / 8;  // 16-B chunks per row
-  const int n0 = blockIdx.x * (EPI == 0 ? 2 * RP : RP);
-  const int npair = N / 2;  // modes 1 / 2: output pairs
-  auto row_of = [&](int rp) -> int {  // this half's weight row for its rp-th row (pair)
-    if constexpr (WR) {
-      return min(n0 + rp, N - 1);
-    } else if constexpr (EPI == 0) {
-      return min(n0 + 2 * rp + h, N - 1);
-    } else if constexpr (EPI == 1) {
-      return min(n0 + rp, npair - 1) + h * npair;
-    } else {
-      const int p = min(n0 + rp, npair - 1), hd = D / 2, head = p / hd;
-      return head * D + (p - head * hd) + h * hd;
-    }
-  };
+  const int n0 = blockIdx.x * 2 * RP;
+  auto row_of = [&](int rp) -> int { return min(n0 + 2 * rp + h, N - 1); };  // this half's rp-th weight row
   // 1. every load first, in the order of use (the vector-memory counter drains in order): the LayerNorm's operands,
   // then the weight chunks of this half's rows, whose flight covers the LayerNorm. Loads are never behind a branch on
   // a lane or behind an earlier load's use: with the residual, delta and bias of each chunk added as they came, and
@@ -493,7 +467,7 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
   constexpr bool EARLY = CPL * (28 + 12 * M + 5 * RP) <= 260;
   int cc[CPL];  // chunks past the row are read from its last one and count as zero
 #pragma unroll
-  for (int i = 0; i < CPL; ++i) cc[i] = min(cl + CS * i, nc - 1);
+  for (int i = 0; i < CPL; ++i) cc[i] = min(l32 + 32 * i, nc - 1);
   uint4 wv[RP][CPL], xb[M][CPL];
   auto weights = [&]() {
 #pragma unroll
@@ -501,20 +475,18 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
       const bf16* wr = w + (size_t)row_of(rp) * K;
 #pragma unroll
       for (int i = 0; i < CPL; ++i) {
-        const int c = cl + CS * i;
+        const int c = l32 + 32 * i;
         wv[rp][i] = c < nc ? *reinterpret_cast<const uint4*>(wr + 8 * c) : uint4{0u, 0u, 0u, 0u};
       }
     }
   };
-  float bias_v[RP];  // (paired rows have none)
+  float bias_v[RP];
 #pragma unroll
   for (int rp = 0; rp < RP; ++rp) bias_v[rp] = 0.f;
   auto biases = [&]() {
-    if constexpr (EPI == 0 || WR) {
-      if (bias) {
+    if (bias) {
 #pragma unroll
-        for (int rp = 0; rp < RP; ++rp) bias_v[rp] = bf2f(bias[row_of(rp)]);
-      }
+      for (int rp = 0; rp < RP; ++rp) bias_v[rp] = bf2f(bias[row_of(rp)]);
     }
   };
   if constexpr (!LN) {
@@ -524,7 +496,7 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
     for (int m = 0; m < M; ++m)
 #pragma unroll
       for (int i = 0; i < CPL; ++i) {
-        const int c = cl + CS * i;
+        const int c = l32 + 32 * i;
         xb[m][i] = c < nc ? *reinterpret_cast<const uint4*>(x + (size_t)m * x_rs + 8 * c) : uint4{0u, 0u, 0u, 0u};
       }
   } else {
@@ -681,54 +653,9 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
       float a = 0.f;
 #pragma unroll
       for (int i = 0; i < CPL; ++i) a = dot8_bf16(wv[rp][i], xb[m][i], a);
-      a = half_sum(a);
-      if constexpr (WR) a += other_half(a, h);
-      acc[rp][m] = a;
+      acc[rp][m] = half_sum(a);
     }
   // 3. epilogue
-  if constexpr (WR) {
-    if (lane != 0) return;
-#pragma unroll
-    for (int rp = 0; rp < RP; ++rp) {
-      const int n = n0 + rp;
-      if (n >= N) continue;
-#pragma unroll
-      for (int m = 0; m < M; ++m) {
-        float y = acc[rp][m] + bias_v[rp];
-        if (act) y = gelu_f(bf2f(from_f<bf16>(y)), act - 1);
-        out[(size_t)m * o_rs + n] = from_f<bf16>(y);
-      }
-    }
-    return;
-  } else if constexpr (EPI != 0) {
-    float other[RP][M];  // the partner half's sums (lane 0 <-> lane 32)
-#pragma unroll
-    for (int rp = 0; rp < RP; ++rp)
-#pragma unroll
-      for (int m = 0; m < M; ++m) other[rp][m] = other_half(acc[rp][m], h);
-    if (l32 != 0) return;
-#pragma unroll
-    for (int rp = 0; rp < RP; ++rp) {
-      const int p = n0 + rp;
-      if (p >= npair) continue;
-#pragma unroll
-      for (int m = 0; m < M; ++m) {
-        const float mine = bf2f(from_f<bf16>(acc[rp][m])), theirs = bf2f(from_f<bf16>(other[rp][m]));
-        if constexpr (EPI == 1) {
-          if (h == 0) out[(size_t)m * o_rs + p] = from_f<bf16>(act_f(mine, act) * theirs);
-        } else {
-          const int hd = D / 2, head = p / hd, j = p - head * hd;
-          float y = mine;
-          if (head < nrot) {
-            const float cs = cosv[j], sn = sinv[j];
-            y = h == 0 ? mine * cs - theirs * sn : mine * cs + theirs * sn;
-          }
-          out[(size_t)m * o_rs + head * D + j + h * hd] = from_f<bf16>(y);
-        }
-      }
-    }
-    return;
-  }
   // a lane per output: one after the other on one lane the activations of 8 rows, 4 of x, take as long as the loads
   static_assert(RP * M <= 32, "");
   float mine = 0.f;
@@ -740,6 +667,169 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
   if (l32 >= RP * M || n >= N) return;
   if (act) mine = gelu_f(bf2f(from_f<bf16>(mine)), act - 1);
   out[(size_t)(l32 % M) * o_rs + n] = from_f<bf16>(mine);
+}
+
+// The decode GEMV of up to 16k outputs: NW waves share the columns of RP weight rows (wave w, lane l: 16-B chunks l + 64 w, l + 64 (w +
+// NW), ...), every load of a wave in flight before the first use, x first. ADD: out (fp32) += the sum, whose old value is fetched with
+// the operands. At one row of x a call costs its weights' way through memory; each further row was read again by the one wave per
+// weight row that there was before, so long rows (K > 4608) are shared out two to a pair of waves: half the reads of x. us before /
+// now at 1, 3 and 4 rows: 1152 x 6912 5.3 / 5.2, 8.6 / 6.2, 9.9 / 6.7 (rows alone in 4 waves 6.8 at 3 rows, 4 rows in 4 waves 6.9, 8
+// in 7 waves 6.3), 768 x 3072 2.8 / 2.7, 3.3 / 3.0, 3.5 / 3.2, 1152 x 1024 2.4 / 2.4, 2.8 / 2.6, 3.0 / 2.7.
+template <int M, int RP, int NW, int CPL, bool ADD>
+__global__ void __launch_bounds__(64 * NW) decode_gemv_rows_kernel(const bf16* __restrict__ x, int64_t x_rs,
+                                                                   const bf16* __restrict__ w, const bf16* __restrict__ bias,
+                                                                   void* __restrict__ out, int64_t o_rs, int N, int K, int act) {
+  __shared__ float red[NW][RP * M];
+  const int t = threadIdx.x, lane = t & 63, wid = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int nc = K / 8, n0 = blockIdx.x * RP;
+  // thread t < RP * M: output row t % M, column n0 + t / M; the others read the last one's
+  const int e = min(t, RP * M - 1), n = n0 + e / M;
+  const bool mine = t < RP * M && n < N;
+  const size_t o = (size_t)(e % M) * o_rs + min(n, N - 1);
+  const uint16_t* bp = reinterpret_cast<const uint16_t*>(bias ? bias : x);  // (a value of x, not used, is as quick)
+  uint32_t bias_v = bp[bias ? min(n, N - 1) : 0];
+  float old = 0.f;
+  if constexpr (ADD) old = reinterpret_cast<const float*>(out)[o];
+  int cc[CPL];  // chunks past the row are read from its last one and count as zero
+#pragma unroll
+  for (int i = 0; i < CPL; ++i) cc[i] = min(lane + 64 * (wid + NW * i), nc - 1);
+  uint4 xb[M][CPL], wv[RP][CPL];
+#pragma unroll
+  for (int m = 0; m < M; ++m)
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) xb[m][i] = *reinterpret_cast<const uint4*>(x + (size_t)m * x_rs + 8 * cc[i]);
+#pragma unroll
+  for (int r = 0; r < RP; ++r)
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) wv[r][i] = *reinterpret_cast<const uint4*>(w + (size_t)min(n0 + r, N - 1) * K + 8 * cc[i]);
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" : "+v"(bias_v), "+v"(old));  // asked for with the others: left to itself, each is fetched where it is needed
+#pragma unroll
+  for (int i = 0; i < CPL; ++i)
+    if (lane + 64 * (wid + NW * i) >= nc)
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        xb[m][i] = uint4{0u, 0u, 0u, 0u};
+        for (int r = 0; m == 0 && r < RP; ++r) wv[r][i] = uint4{0u, 0u, 0u, 0u};  // (0 · inf)
+      }
+  float y = bias ? __uint_as_float(bias_v << 16) : 0.f;
+#pragma unroll
+  for (int r = 0; r < RP; ++r)
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      float a = 0.f;
+#pragma unroll
+      for (int i = 0; i < CPL; ++i) a = dot8_bf16(wv[r][i], xb[m][i], a);
+      a = half_sum(a);
+      a += other_half(a, lane >> 5);
+      if constexpr (NW == 1)
+        y += lane == r * M + m ? a : 0.f;
+      else if (lane == 0)
+        red[wid][r * M + m] = a;
+    }
+  if constexpr (NW > 1) {
+    __syncthreads();
+    if (mine) {
+      float a = 0.f;
+#pragma unroll
+      for (int i = 0; i < NW; ++i) a += red[i][t];
+      y += a;
+    }
+  }
+  if (!mine) return;
+  if (act) y = gelu_f(bf2f(from_f<bf16>(y)), act - 1);
+  if constexpr (ADD)
+    reinterpret_cast<float*>(out)[o] = old + y;
+  else
+    reinterpret_cast<bf16*>(out)[o] = from_f<bf16>(y);
+}
+
+// Pairs of weight rows, a half-wave each, x once per workgroup of 4 waves in LDS (with every wave fetching it, a call of 3 rows of x
+// read more of x than of weights). GATED: on the packed [gate; up] weight (N = 2I rows): half 0 takes gate row n, half 1 up row I + n,
+// out[n] = act_f(bf16(g), kind) · bf16(u) (skinny_gated's rounding). Otherwise RoPE QKV: pair p of head p / (D/2), j = p % (D/2): half
+// 0 row head·D + j, half 1 row + D/2, both rounded to bf16, then rotated by one position's cos / sin [D/2] for the first nrot heads
+// (skinny_qkv_rope's math). A wave owns RP pairs. us before / now at 1, 3 and 4 rows, 2 x 6912 x 1152 gated: 8.0 / 7.3, 10.2 / 7.6,
+// 11.2 / 7.8 (32 MB of weights; 2 pairs per wave 8.1 at 3 rows, 3 8.8, 4 8.1).
+template <int M, int RP, int CPL, bool GATED>
+__global__ void __launch_bounds__(256) decode_gemv_pair_kernel(const bf16* __restrict__ x, int64_t x_rs, const bf16* __restrict__ w,
+                                                               bf16* __restrict__ out, int64_t o_rs, int N, int K, int kind, int D,
+                                                               int nrot, const float* __restrict__ cosv,
+                                                               const float* __restrict__ sinv) {
+  constexpr int XN = M * 32 * CPL, XL = (XN + 255) / 256;
+  static_assert(RP * M <= 32, "a lane per output");
+  __shared__ uint4 xs[XN];
+  const int t = threadIdx.x, lane = t & 63, wid = __builtin_amdgcn_readfirstlane(t >> 6), h = lane >> 5, l32 = lane & 31;
+  const int nc = K / 8, npair = N / 2, hd = D / 2;
+  const int p0 = (blockIdx.x * 4 + wid) * RP;
+  uint4 xt[XL], wv[RP][CPL];  // chunks past a row are read from its last one and count as zero
+#pragma unroll
+  for (int i = 0; i < XL; ++i) {
+    const int e = t + 256 * i;
+    xt[i] = *reinterpret_cast<const uint4*>(x + (size_t)min(e / (32 * CPL), M - 1) * x_rs + 8 * min(e % (32 * CPL), nc - 1));
+  }
+#pragma unroll
+  for (int r = 0; r < RP; ++r) {
+    const int p = min(p0 + r, npair - 1), row = GATED ? p + h * npair : p / hd * D + p % hd + h * hd;
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) wv[r][i] = *reinterpret_cast<const uint4*>(w + (size_t)row * K + 8 * min(l32 + 32 * i, nc - 1));
+  }
+  const int p = p0 + l32 / M;  // this lane's output pair, row l32 % M of x
+  const bool mine = l32 < RP * M && p < npair;
+  float cs = 1.f, sn = 0.f;
+  if constexpr (!GATED) {
+    if (mine && p / hd < nrot) {
+      cs = cosv[p % hd];
+      sn = sinv[p % hd];
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < XL; ++i) launder(xt[i]);  // asked for before the weights, all of them (not where a branch needs one)
+#pragma unroll
+  for (int i = 0; i < XL; ++i) {
+    const int e = t + 256 * i;
+    if (e < XN) xs[e] = e % (32 * CPL) < nc ? xt[i] : uint4{0u, 0u, 0u, 0u};
+  }
+  // a barrier for LDS alone: __syncthreads would wait for the weights as well
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  float acc[RP][M];
+#pragma unroll
+  for (int r = 0; r < RP; ++r)
+#pragma unroll
+    for (int m = 0; m < M; ++m) acc[r][m] = 0.f;
+#pragma unroll
+  for (int i = 0; i < CPL; ++i) {
+    if (l32 + 32 * i >= nc)
+#pragma unroll
+      for (int r = 0; r < RP; ++r) wv[r][i] = uint4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const uint4 xv = xs[m * 32 * CPL + l32 + 32 * i];
+#pragma unroll
+      for (int r = 0; r < RP; ++r) acc[r][m] = dot8_bf16(wv[r][i], xv, acc[r][m]);
+    }
+  }
+  float a = 0.f, b = 0.f;  // this half's row and the other's
+#pragma unroll
+  for (int r = 0; r < RP; ++r)
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const float v = half_sum(acc[r][m]), u = other_half(v, h);
+      a = l32 == r * M + m ? v : a;
+      b = l32 == r * M + m ? u : b;
+    }
+  if (!mine) return;
+  a = bf2f(from_f<bf16>(a));
+  b = bf2f(from_f<bf16>(b));
+  bf16* o = out + (size_t)(l32 % M) * o_rs;
+  if constexpr (GATED) {
+    if (h == 0) o[p] = from_f<bf16>(act_f(a, kind) * b);
+  } else {
+    const float y = p / hd < nrot ? (h == 0 ? a * cs - b * sn : a * cs + b * sn) : a;
+    o[p / hd * D + p % hd + h * hd] = from_f<bf16>(y);
+  }
 }
 
 }  // namespace penroz
@@ -862,6 +952,41 @@ void decode_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64_t ki
                      (int64_t)out.stride(0), M, N, K, (int)(gated ? kind : 0));
 }
 
+// decode_gemv_rows_kernel by the length of a row; M <= 4, K <= 8192
+template <bool ADD>
+static void gemv_rows_launch(const bf16* x, int64_t x_rs, const bf16* w, const bf16* bias, void* out, int64_t o_rs, int M, int N,
+                             int K, int act) {
+  auto stream = at::hip::getCurrentHIPStream();
+  auto go = [&](auto mt, auto rpt, auto nwt, auto cplt) {
+    constexpr int MM = decltype(mt)::value, RP = decltype(rpt)::value, NW = decltype(nwt)::value, CPL = decltype(cplt)::value;
+    hipLaunchKernelGGL((decode_gemv_rows_kernel<MM, RP, NW, CPL, ADD>), dim3((N + RP - 1) / RP), dim3(64 * NW), 0, stream, x, x_rs, w,
+                       bias, out, o_rs, N, K, act);
+  };
+  auto by_len = [&](auto mt) {
+    using C1 = std::integral_constant<int, 1>;
+    using C2 = std::integral_constant<int, 2>;
+    using C3 = std::integral_constant<int, 3>;
+    const int nc = (K + 7) / 8;
+    if (nc <= 64) go(mt, C1{}, C1{}, C1{});
+    else if (nc <= 128) go(mt, C1{}, C1{}, C2{});
+    else if (nc <= 192) go(mt, C1{}, C1{}, C3{});
+    else if (nc <= 384) go(mt, C1{}, C3{}, C2{});
+    else if (nc <= 576) go(mt, C1{}, C3{}, C3{});
+    else if (nc <= 896) go(mt, C2{}, C2{}, std::integral_constant<int, 7>{});
+    else go(mt, C2{}, C2{}, std::integral_constant<int, 8>{});
+  };
+  switch (M) {
+    case 1: by_len(std::integral_constant<int, 1>{}); break;
+    case 2: by_len(std::integral_constant<int, 2>{}); break;
+    case 3: by_len(std::integral_constant<int, 3>{}); break;
+    default: by_len(std::integral_constant<int, 4>{});
+  }
+}
+
+void gemv_add(const bf16* x, int64_t x_rs, const bf16* w, const bf16* bias, float* resid, int M, int N, int K) {
+  gemv_rows_launch<true>(x, x_rs, w, bias, resid, N, M, N, K, 0);
+}
+
 // out[M, N] = act(x · Wᵀ + bias) for M <= 4 decode rows (decode_gemv_kernel). LN mode (x
 // undefined): x = LayerNorm(resid_in + delta + dbias) with γ / β, resid_out receives the sum.
 // act 0 none, 1 GELU (erf), 2 GELU (tanh). rows_per_wave 2, 4 or 8 (0: by N).
@@ -955,40 +1080,33 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
                 "decode_gemv: bf16 bias [N]");
     bp = reinterpret_cast<const bf16*>(bias->data_ptr());
   }
+  static const int rpw_env = [] {
+    const char* e = std::getenv("PENROZ_DECODE_GEMV_RPW");
+    return e ? std::atoi(e) : 0;
+  }();
   // a LayerNorm product of whole tiles: one workgroup normalises for 16 columns (decode_ln_few_kernel). The vocabulary's many columns
   // stay with the waves below (50304 x 768, one row: 15.9 us, 77 MB at 4.9 TB/s)
-  if (ln && !dp && rows_per_wave <= 0 && K % 32 == 0 && N % 16 == 0 && N < 16384 && out.stride(0) % 4 == 0 &&
+  if (ln && !dp && rows_per_wave <= 0 && rpw_env <= 0 && K % 32 == 0 && N % 16 == 0 && N < 16384 && out.stride(0) % 4 == 0 &&
       reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0 && reinterpret_cast<uintptr_t>(bp) % 8 == 0) {
     const LnEmb e{eip, ewp, epp, eps_p, eV, eP};
     ln_launch(emb ? rop : const_cast<float*>(rp), gp, bt, (float)eps, reinterpret_cast<const bf16*>(w.data_ptr()), bp,
               reinterpret_cast<bf16*>(out.data_ptr()), out.stride(0), M, N, K, (int)act, emb ? &e : nullptr);
     return;
   }
+  if (!ln && rows_per_wave <= 0 && N < 16384)
+    return gemv_rows_launch<false>(xp, x_rs, reinterpret_cast<const bf16*>(w.data_ptr()), bp, out.data_ptr(), out.stride(0), M, N, K,
+                                   (int)act);
   const int cpl = (K / 8 + 31) / 32;
   int rpw = (int)rows_per_wave;
   // by shape: the vocabulary projection wants fewer, longer-lived waves (8 rows); behind a LayerNorm 4 rows, since every
   // wave reads and normalises the whole operand again (2 / 4 / 8 rows, us: K 768, N 2304, one row of x 4.8 / 4.2 / 4.3,
-  // four 10.5 / 9.0 / 8.8; K 1024, N 4096 6.7 / 5.3 / 4.9 and 13.8 / 12.1 / 12.0; K 512, N 512 3.1 / 3.2 / 3.3); else 2
-  // rows per wave — the most workgroups in flight. PENROZ_DECODE_GEMV_RPW forces 2 / 4 / 8 below 16k rows (A/B).
-  static const int rpw_env = [] {
-    const char* e = std::getenv("PENROZ_DECODE_GEMV_RPW");
-    return e ? std::atoi(e) : 0;
-  }();
+  // four 10.5 / 9.0 / 8.8; K 1024, N 4096 6.7 / 5.3 / 4.9 and 13.8 / 12.1 / 12.0; K 512, N 512 3.1 / 3.2 / 3.3).
+  // PENROZ_DECODE_GEMV_RPW forces 2 / 4 / 8 there below 16k rows (A/B).
   if (rpw <= 0 && rpw_env > 0 && N < 16384) rpw = rpw_env;
-  if (rpw <= 0) rpw = N >= 16384 ? 8 : ln ? 4 : 2;
+  if (rpw <= 0) rpw = N >= 16384 ? 8 : 4;
   TORCH_CHECK(rpw == 2 || rpw == 4 || rpw == 8, "decode_gemv: rows_per_wave 2, 4 or 8");
   const int RPv = rpw / 2;
-  // wave-per-row form for the bf16-x GEMVs (proj, fc2, Gemma o / down): one row per wave, the
-  // whole wave striding over K — twice the workgroups. Same box: Gemma-3 1B B = 1 1.2626 / 1.2621 ->
-  // 1.2577 / 1.2555 ms, GPT-2 B = 4 0.549 / 0.544 -> 0.544 / 0.542, GPT-2 B = 1 even
-  // (profiles/decode_r5.md). PENROZ_DECODE_GEMV_WAVE_ROW=0: the half-wave form.
-  static const bool wave_row_env = [] {
-    const char* e = std::getenv("PENROZ_DECODE_GEMV_WAVE_ROW");
-    return !(e && e[0] == '0');
-  }();
-  const bool wave_row = wave_row_env && !ln && rows_per_wave <= 0 && N < 16384;
-  const int cpl64 = (K / 8 + 63) / 64;
-  const dim3 grid(wave_row ? N : (N + rpw - 1) / rpw);
+  const dim3 grid((N + rpw - 1) / rpw);
   auto stream = at::hip::getCurrentHIPStream();
   auto wp = reinterpret_cast<const bf16*>(w.data_ptr());
   auto op = reinterpret_cast<bf16*>(out.data_ptr());
@@ -997,8 +1115,7 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
     constexpr int MM = decltype(mt)::value, RR = decltype(rpt)::value, CC = decltype(cplt)::value;
     constexpr int LL = decltype(lnt)::value ? 1 : 0;
     hipLaunchKernelGGL((decode_gemv_kernel<MM, LL, RR, CC>), grid, dim3(64), 0, stream, rp, dp, dbp, rop, gp, bt,
-                       (float)eps, xp, x_rs, wp, bp, op, o_rs, N, K, (int)act, 0, 0, (const float*)nullptr,
-                       (const float*)nullptr, eip, ewp, epp, eps_p, eV, eP);
+                       (float)eps, xp, x_rs, wp, bp, op, o_rs, N, K, (int)act, eip, ewp, epp, eps_p, eV, eP);
   };
   auto by_cpl = [&](auto mt, auto lnt, auto rpt) {
     using I = std::integral_constant<int, 0>;
@@ -1020,19 +1137,6 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
     else by_cpl(mt, lnt, std::integral_constant<int, 4>{});
   };
   auto by_ln = [&](auto mt) {
-    if (wave_row) {  // one row per wave (RP = 1), chunks per lane over 64 lanes
-      auto go = [&](auto cplt) {
-        constexpr int MM = decltype(mt)::value, CC = decltype(cplt)::value;
-        hipLaunchKernelGGL((decode_gemv_kernel<MM, 0, 1, CC, 3>), grid, dim3(64), 0, stream, rp, dp, dbp, rop, gp, bt,
-                           (float)eps, xp, x_rs, wp, bp, op, o_rs, N, K, (int)act);
-      };
-      if (cpl64 <= 2) go(std::integral_constant<int, 2>{});
-      else if (cpl64 <= 4) go(std::integral_constant<int, 4>{});
-      else if (cpl64 <= 7) go(std::integral_constant<int, 7>{});
-      else if (cpl64 <= 16) go(std::integral_constant<int, 16>{});
-      else go(std::integral_constant<int, 16>{});  // K <= 8192 (checked above)
-      return;
-    }
     if (ln) {
       TORCH_CHECK(cpl <= 4, "decode_gemv: LN mode needs K <= 1024");
       auto by_chunks = [&](auto rpt) {  // K <= 1024
@@ -1056,7 +1160,7 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
   }
 }
 
-// Paired-row decode GEMV for 1..4 rows on a bf16 x (decode_gemv_kernel modes 1 / 2):
+// Paired-row decode GEMV for 1..4 rows on a bf16 x (decode_gemv_pair_kernel):
 //   mode 1 (gated): out[M, I] = act_f(x·Wgᵀ, kind) ⊙ (x·Wuᵀ), w = [Wg; Wu] [2I, K];
 //   mode 2 (RoPE QKV): out[M, (H + 2Hkv)·D] = rope(x · Wᵀ) for the first nrot heads, cos / sin [D/2].
 void decode_gemv_pair(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64_t mode, int64_t kind, int64_t D,
@@ -1089,10 +1193,9 @@ void decode_gemv_pair(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64
     cp = cosv->data_ptr<float>();
     sp = sinv->data_ptr<float>();
   }
-  int ppw = (int)pairs_per_wave;
-  if (ppw <= 0) ppw = N / 2 >= 16384 ? 4 : N / 2 <= 1024 ? 1 : 2;
+  const int ppw = pairs_per_wave <= 0 ? 1 : (int)pairs_per_wave;
   TORCH_CHECK(ppw == 1 || ppw == 2 || ppw == 4, "decode_gemv_pair: pairs_per_wave 1, 2 or 4");
-  const dim3 grid((N / 2 + ppw - 1) / ppw);
+  const dim3 grid((N / 2 + 4 * ppw - 1) / (4 * ppw));
   auto stream = at::hip::getCurrentHIPStream();
   auto xp = reinterpret_cast<const bf16*>(x.data_ptr());
   auto wp = reinterpret_cast<const bf16*>(w.data_ptr());
@@ -1100,10 +1203,8 @@ void decode_gemv_pair(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64
   const int64_t x_rs = x.stride(0), o_rs = out.stride(0);
   auto launch = [&](auto mt, auto rpt, auto cplt, auto et) {
     constexpr int MM = decltype(mt)::value, RR = decltype(rpt)::value, CC = decltype(cplt)::value;
-    constexpr int EE = decltype(et)::value;
-    hipLaunchKernelGGL((decode_gemv_kernel<MM, 0, RR, CC, EE>), grid, dim3(64), 0, stream, nullptr, nullptr,
-                       nullptr, nullptr, nullptr, nullptr, 0.f, xp, x_rs, wp, nullptr, op, o_rs, N, K,
-                       EE == 1 ? (int)kind : 0, (int)D, (int)nrot, cp, sp);
+    hipLaunchKernelGGL((decode_gemv_pair_kernel<MM, RR, CC, decltype(et)::value>), grid, dim3(256), 0, stream, xp, x_rs, wp, op, o_rs,
+                       N, K, (int)kind, mode == 1 ? 2 : (int)D, (int)nrot, cp, sp);
   };
   auto by_cpl = [&](auto mt, auto rpt, auto et) {
     if (cpl <= 3) launch(mt, rpt, std::integral_constant<int, 3>{}, et);
@@ -1117,8 +1218,8 @@ void decode_gemv_pair(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64
     else by_cpl(mt, std::integral_constant<int, 4>{}, et);
   };
   auto by_mode = [&](auto mt) {
-    if (mode == 1) by_rp(mt, std::integral_constant<int, 1>{});
-    else by_rp(mt, std::integral_constant<int, 2>{});
+    if (mode == 1) by_rp(mt, std::true_type{});
+    else by_rp(mt, std::false_type{});
   };
   switch (M) {
     case 1: by_mode(std::integral_constant<int, 1>{}); break;

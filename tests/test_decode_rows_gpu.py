@@ -1,5 +1,5 @@
-"""Decode products of a few rows (csrc/kernels/decode_linear.hip): the LayerNorm products at the edges of
-their tiles and shares, against fp32 torch."""
+"""Decode products of a few rows (csrc/kernels/decode_linear.hip): the LayerNorm products, the GEMV whose waves share a row,
+the paired rows, at the edges of their tiles, shares and lengths, against fp32 torch."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -70,3 +70,57 @@ def test_ln_product_of_embeddings(M, K):
     s = wte[idx.clamp(max=8)].float() + wpe[8].float()
     assert torch.equal(rows, s)
     _near(out, *_ln_ref(s, gamma, beta, w, b))
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("K", [8, 512, 520, 1024, 1032, 1536, 1544, 3072, 3080, 4608, 4616, 7168, 7176, 8192])
+@pytest.mark.parametrize("N", [1, 33])
+def test_gemv_rows(M, K, N):
+    """Every length class of the GEMV, exact and one chunk over; a last workgroup with one row of its two."""
+    torch.manual_seed(M + K + N)
+    x = torch.randn(M, K + 8, device=DEV).to(torch.bfloat16)[:, :K]
+    w = (torch.randn(N, K, device=DEV) / K ** 0.5).to(torch.bfloat16)
+    b = torch.randn(N, device=DEV).to(torch.bfloat16)
+    big = torch.full((M + 1, N + 3), 7.0, device=DEV, dtype=torch.bfloat16)
+    _ext.kernels().decode_gemv(x, None, None, None, None, None, None, 0.0, w, b, big[:M, :N], 0)
+    ref = x.float() @ w.float().t() + b.float()
+    _near(big[:M, :N], ref, 0 * ref)
+    assert (big[M] == 7).all() and (big[:, N:] == 7).all()
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("K", [32, 768, 3072, 4640, 8192, 8224])
+def test_gemv_adds_to_the_residual(M, K):
+    """decode_gemm_acc around the GEMV's limits (4 rows, 8192 columns): fp32 sums of exact products, so within K roundings."""
+    torch.manual_seed(M + K)
+    N = 48
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=DEV) / K ** 0.5).to(torch.bfloat16)
+    b = torch.randn(N, device=DEV).to(torch.bfloat16)
+    old = torch.randn(M, N, device=DEV)
+    got = old.clone()
+    _ext.kernels().decode_gemm_acc(x, w, b, got)
+    ref = old.double() + x.double() @ w.double().t() + b.double()
+    bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + old.double().abs() + b.double().abs())
+    assert torch.all((got.double() - ref).abs() <= bound)
+
+
+@pytest.mark.parametrize("M", [1, 3, 4])
+@pytest.mark.parametrize("K,I", [(8, 1), (256, 5), (768, 4), (1032, 17), (1792, 3)])
+@pytest.mark.parametrize("ppw", [0, 2, 4])
+def test_gemv_pairs_of_few_rows(M, K, I, ppw):
+    """Pairs that end inside a wave and inside a workgroup, columns that end inside a chunk group; infinities stay in their row."""
+    torch.manual_seed(M + K + I)
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    gu = (torch.randn(2 * I, K, device=DEV) / K ** 0.5).to(torch.bfloat16)
+    gu[0, K - 1] = float("inf")
+    big = torch.full((M + 1, I + 3), 7.0, device=DEV, dtype=torch.bfloat16)
+    _ext.kernels().decode_gemv_pair(x, gu, big[:M, :I], 1, 2, pairs_per_wave=ppw)
+    y = (x.float() @ gu.float().t()).to(torch.bfloat16).float()
+    ref = F.silu(y[:, :I]) * y[:, I:]
+    got = big[:M, :I].float()
+    fin = torch.isfinite(ref)
+    assert torch.equal(torch.isfinite(got), fin)
+    # gate and up, rounded from sums of another order, may be a bf16 step apart each; the result is rounded once more
+    assert torch.all((got - ref)[fin].abs() <= 2.0 ** -8 * 4 * (ref.abs() + y[:, :I].abs() + y[:, I:].abs())[fin] + 1e-5)
+    assert (big[M] == 7).all() and (big[:, I:] == 7).all()
