@@ -1,4 +1,4 @@
-// Decode linears. A GPT block's decode step of 5 to 64 rows costs 5 launches instead of 8:
+// Decode linears. A GPT block's decode step of 1 to 64 rows costs 5 launches instead of 8:
 //
 //   decode_ln_gemm : out = act(LN(resid) · Wᵀ + bias)          (QKV; fc + GELU)
 //   decode_gemm_acc: resid += x · Wᵀ + bias                     (proj; fc2; rows_gemm.hip)

@@ -67,23 +67,18 @@ SKINNY_MAX_ROWS = int(os.environ.get("PENROZ_SKINNY_MAX_ROWS", "16"))
 # Gemma program: RoPE and the gated activation in the skinny GEMM epilogues ("1", default) or the
 # separate RoPE / packed-activation kernels after plain skinny GEMMs ("0": same-box A/B switch)
 DECODE_EPILOGUES = os.environ.get("PENROZ_DECODE_EPILOGUES", "1") != "0"
-# GPT decode program: residual add + LayerNorm fused in front of the QKV and fc GEMMs (and GELU
-# behind fc) in one decode-shaped kernel (csrc/kernels/skinny_gemm.hip decode_ln_linear); "0":
-# separate add+LN, GEMM and GELU kernels
-FUSED_LN_LINEAR = os.environ.get("PENROZ_DECODE_FUSED", "1") != "0"
-# ... up to this many decode rows: every workgroup normalises all rows itself, which pays off
-# while the rows are few (batch 1 / 4 / 8: -8 / -10 / -3 %) and loses from 16 rows on (+14 % at 16,
-# +69 % at 64): profiles/decode_fused_rows_r2.log
-FUSED_MAX_ROWS = int(os.environ.get("PENROZ_DECODE_FUSED_MAX_ROWS", "8"))
-# ... above that: the batched block (csrc/kernels/decode_linear.hip) — 5 kernels per block, the
-# fp32 residual updated in place by the proj / fc2 epilogues, LayerNorm recomputed per 16-row
-# block inside the QKV / fc GEMMs; "0": add+LN, GEMM, GELU kernels (8 per block)
+# GPT decode program, widths that are multiples of 32: 5 kernels per block (csrc/kernels/decode_linear.hip), the fp32
+# residual updated in place by the proj / fc2 epilogues, LayerNorm computed inside the QKV / fc products. Greedy
+# generation at 2 / 4 / 8 rows, against the residual carried along as a second operand (the two programs below):
+# 21.5 / 28.4 / 31.3 -> 17.2 / 18.2 / 23.3 ms for 64 tokens. "0": the programs below, above 8 rows 8 kernels per block
 BATCHED_BLOCK = os.environ.get("PENROZ_DECODE_BATCHED", "1") != "0"
-# ... and up to this many rows (batch 1-4) every linear of the GPT block — the LN-fused QKV and
-# fc(+GELU), proj, fc2 and the lm_head — runs as the one-wave-per-workgroup decode GEMV
-# (csrc/kernels/decode_linear.hip decode_gemv: one memory round trip, no LDS, no barrier, no
-# split-K hand-off); "0": decode_ln_linear + skinny GEMMs
+# ... else up to this many rows every linear of the block as decode_gemv; "0": decode_ln_linear + skinny GEMMs
 GEMV_MAX_ROWS = int(os.environ.get("PENROZ_DECODE_GEMV_MAX_ROWS", "4"))
+# ... and up to FUSED_MAX_ROWS the residual add + LayerNorm in front of the QKV and fc GEMMs (and GELU behind fc) in one
+# kernel (csrc/kernels/skinny_gemm.hip decode_ln_linear), whose workgroups all normalise every row: it loses from 16
+# rows on (profiles/decode_fused_rows_r2.log); "0": separate add+LN, GEMM and GELU kernels
+FUSED_LN_LINEAR = os.environ.get("PENROZ_DECODE_FUSED", "1") != "0"
+FUSED_MAX_ROWS = int(os.environ.get("PENROZ_DECODE_FUSED_MAX_ROWS", "8"))
 # decode_gemv's reduction limit (256 lanes × 32 values, decode_linear.hip); wider linears take the
 # skinny GEMM
 GEMV_MAX_K = 8192
@@ -219,7 +214,7 @@ class GPTDecodeProgram:
 
     def _batched_ok(self, rows: int) -> bool:
         sp = self.spec
-        return (BATCHED_BLOCK and rows > FUSED_MAX_ROWS and sp.C % 32 == 0 and sp.C <= 1024
+        return (BATCHED_BLOCK and sp.C % 32 == 0 and sp.C <= 1024
                 and sp.blocks[0].fc.out_features % 32 == 0 and sp.gelu_approx in ("none", "tanh")
                 and _ext.available())
 
@@ -227,13 +222,15 @@ class GPTDecodeProgram:
         """idx [rows, 1] -> logits [rows, V] (bf16); appends this step's K/V at cache.pos_t."""
         sp = self.spec
         rows, C, H, D = idx.shape[0], sp.C, sp.H, sp.D
-        if (rows == 1 and self._gemv_ok(rows) and sp.wte.weight.dtype == torch.bfloat16
-                and sp.wpe.weight.dtype == torch.bfloat16):
-            # the first block's LN + QKV GEMV reads the embedding row itself (no embedding kernel):
+        if rows == 1 and (self._batched_ok(rows) or self._gemv_ok(rows)):
+            # the first block's LN + QKV product reads the embedding row itself (no embedding kernel):
             # B = 1 0.3548 / 0.3564 -> 0.3520 / 0.3544 ms; at 4 rows every workgroup's four-row
             # gather cost more than the launch it saves (0.535 -> 0.551), profiles/decode_r5.md
             x = torch.empty(rows, C, dtype=torch.float32, device=idx.device)
-            return self._forward_gemv(x, torch.empty_like(x), rows, cache, emb=(idx.reshape(-1).contiguous(), cache.pos_t))
+            emb = (idx.reshape(-1).contiguous(), cache.pos_t)
+            if self._batched_ok(rows):
+                return self._forward_batched(x, rows, cache, emb=emb)
+            return self._forward_gemv(x, torch.empty_like(x), rows, cache, emb=emb)
         x = fused_ops.embedding_fwd(idx, sp.wte.weight, sp.wpe.weight, 0, pos_dev=cache.pos_t)  # fp32 [rows, C]
         if self._batched_ok(rows):
             return self._forward_batched(x, rows, cache)
@@ -303,7 +300,7 @@ class GPTDecodeProgram:
 
 
     def _forward_gemv(self, x: Tensor, x2: Tensor, rows: int, cache, emb=None) -> Tensor:
-        """Batch 1-4, per block: [add + LN1 + QKV GEMV + bias] → decode attention (K/V append fused)
+        """Widths off 32, batch 1-4, per block: [add + LN1 + QKV GEMV + bias] → decode attention (K/V append fused)
         → proj GEMV → [add + proj bias + LN2 + fc GEMV + bias + GELU] → fc2 GEMV; then the final
         add + LN and the lm_head GEMV — every linear one decode_gemv launch. ``emb`` = (token ids,
         device position): the first GEMV builds the residual rows wte[tok] + wpe[pos] itself and
@@ -343,10 +340,11 @@ class GPTDecodeProgram:
         K.decode_gemv(None, x, delta, dbias, x2, wf, bf, ef, sp.head.weight, None, logits, 0)
         return logits
 
-    def _forward_batched(self, x: Tensor, rows: int, cache) -> Tensor:
-        """Per block: [LN1 + QKV GEMM + bias] → decode attention (K/V append fused) → [proj GEMM +
-        bias, added into the fp32 residual in place] → [LN2 + fc GEMM + bias + GELU] → [fc2 GEMM +
-        bias, added into the residual]: 5 kernels instead of 8."""
+    def _forward_batched(self, x: Tensor, rows: int, cache, emb=None) -> Tensor:
+        """Per block: [LN1 + QKV product + bias] → decode attention (K/V append fused) → [proj product +
+        bias, added into the residual in place] → [LN2 + fc product + bias + GELU] → [fc2 product +
+        bias, added into the residual]: 5 kernels instead of 8. ``emb`` = (token ids, device position): the
+        first product builds the residual rows wte[tok] + wpe[pos] itself and writes them to ``x``."""
         sp = self.spec
         K = _ext.kernels()
         C, H, D = sp.C, sp.H, sp.D
@@ -354,7 +352,11 @@ class GPTDecodeProgram:
         for l, blk in enumerate(sp.blocks):
             w1, b1, e1, w2, b2, e2 = self.ln[l]
             qkv = torch.empty(rows, 3 * C, dtype=torch.bfloat16, device=x.device)
-            K.decode_ln_gemm(x, w1, b1, e1, blk.qkv.weight, blk.qkv.bias, qkv, 0)
+            if l == 0 and emb is not None:
+                K.decode_gemv(None, None, None, None, x, w1, b1, e1, blk.qkv.weight, blk.qkv.bias, qkv, 0,
+                              emb_idx=emb[0], emb_wte=sp.wte.weight, emb_wpe=sp.wpe.weight, emb_pos=emb[1])
+            else:
+                K.decode_ln_gemm(x, w1, b1, e1, blk.qkv.weight, blk.qkv.bias, qkv, 0)
             qkv = qkv.view(rows, 1, 3 * C)
             q = qkv[:, :, :C].view(rows, 1, H, D)
             k = qkv[:, :, C:2 * C].view(rows, 1, H, D)
@@ -365,6 +367,14 @@ class GPTDecodeProgram:
             K.decode_ln_gemm(x, w2, b2, e2, blk.fc.weight, blk.fc.bias, h, act)
             K.decode_gemm_acc(h, blk.fc2.weight, blk.fc2.bias, x)
         wf, bf, ef = self.lnf
+        if rows <= 4:  # one row: LN in front of the product, whose waves all repeat it; more rows: once
+            logits = torch.empty(rows, sp.head.weight.shape[0], dtype=torch.bfloat16, device=x.device)
+            if rows == 1:
+                K.decode_gemv(None, x, None, None, None, wf, bf, ef, sp.head.weight, None, logits, 0)
+            else:
+                y, _, _ = norm_ops.ln_fwd(x, wf, bf, ef)
+                K.decode_gemv(y, None, None, None, None, None, None, 0.0, sp.head.weight, None, logits, 0)
+            return logits
         y, _, _ = norm_ops.ln_fwd(x, wf, bf, ef)
         return self._linear(y, sp.head)
 
