@@ -405,22 +405,26 @@ __global__ void __launch_bounds__(256) decode_kernel(const TQ* __restrict__ q, c
   }
 }
 
-// Small-batch decode attention (bf16 cache, one query row, query group G <= 16): D / DC workgroups
-// per (batch, KV head), each for DC of the output columns — no split-K launch, no hand-over between
-// workgroups, no barrier inside the key loop. Each computes all the scores; its 8 waves own a
-// contiguous eighth of the keys. Per 16-key block a wave computes the scores of all G heads with
-// v_mfma_f32_16x16x32_bf16 (A = 16 K rows straight from global memory, B = the group's queries,
+// Decode attention of short contexts (bf16 cache, one query row, query group G <= 16): D / DC · REP workgroups
+// per (batch, KV head), each for G / REP heads of the group and DC of the output columns — no split-K launch, no hand-over
+// between workgroups, no barrier inside the key loop. Each computes all its heads' scores; its 8 waves own a
+// contiguous eighth of the keys. Per 16-key block a wave computes the scores of its heads with
+// v_mfma_f32_16x16x32_bf16 (A = 16 K rows, B = the queries,
 // held in registers), runs the online softmax per head with two cross-lane exchanges, parks P in
 // its own LDS slice and accumulates P·V on the VALU: a lane takes 4 columns of every quarter of the
 // block's keys, the quarters meet after the last block. The next block's K and V rows are issued
-// before this block's math. The waves' (m, l, O) merge through LDS at the end.
+// before this block's softmax. The waves' (m, l, O) merge through LDS at the end.
 // Bound by what one CU can read and by a wave's blocks one after the other, so the keys go over 8
 // waves and V over D / 64 workgroups, whose K rows meet in the L2 of one XCD (they are 8 apart in
-// the grid). 232 keys, D = 256, G = 4, 3 rows: 12.6 us with
-// one workgroup of 4 waves per item, 11.4 with 8 waves, 9.0 so. 128 columns where 64 would make more workgroups than
+// the grid). A fragment's lanes lie a row apart, and read straight from memory each of a row's pieces costs a cache line: 16 bytes a
+// clock, 120 KB of keys in 3 us. From D = 128 on (KLDS) the keys come by LDS-DMA instead, whole lines, into the wave's own 16 rows,
+// and are read from there. The heads of a group go to workgroups of their own while those are no more than half the CUs: less to
+// do one after the other. us at a 1024-slot cache, D = 256, G = 4: 3 items, 40 / 232 / 1000 keys 4.0 / 7.6 / 20.0 before, 4.3 /
+// 6.5 / 14.5 with the keys in LDS, 3.6 / 5.9 / 13.0 with single heads as well; 16 items 4.1 / 7.8 / 21.2 before, 4.2 / 6.3 / 15.7 with
+// pairs of heads (single ones, 256 workgroups: 4.2 / 6.5 / 15.9); 64 items 4.4 / 8.2 / 22.8 before, 4.6 / 7.2 / 19.1 with all four.
+// D = 64 through LDS: the same time. 128 columns where 64 would make more workgroups than
 // CUs (D = 512, more than 32 items; G <= 4, for the registers): 64 items, 200 keys, G = 1 16.1 us with one workgroup of
-// 4 waves per item, 19.8 / 12.1 with 64 / 128 columns. Made for the batch-1 GQA shapes where the
-// general kernel's thread-per-key loop is serial (Gemma-3 1B: G = 4, D = 256 — 19 µs per layer).
+// 4 waves per item, 19.8 / 12.1 with 64 / 128 columns.
 // Fused append as in decode_kernel: key S-1 comes from k_new / v_new and is written to the cache.
 // rc / rs (optional, fp32 [D/2]: this step's RoPE cos / sin): the query and the new key arrive
 // unrotated and are rotated here (rotate-half pairs d, d + D/2, rope_vec_kernel's arithmetic), so the
@@ -429,10 +433,10 @@ __global__ void __launch_bounds__(256) decode_kernel(const TQ* __restrict__ q, c
 // ROPE is a template flag so the default instantiations compile exactly as without it (as a run-time
 // branch it cost the D = 512 kernels 320 B/lane of scratch).
 constexpr int kSmallWaves = 8;
-// GMAX: the exact query-group size H / Hkv; DC: output columns per workgroup
+// GMAX: the heads of a workgroup; DC: its output columns
 template <int D, int GMAX, bool ROPE = false, int DC = 64>
 __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf16* __restrict__ q, bf16* __restrict__ kc,
-                                                           bf16* __restrict__ vc, bf16* __restrict__ out, int items,
+                                                           bf16* __restrict__ vc, bf16* __restrict__ out, int items, int log_rep,
                                                            int H, int Hkv, int cap, int S, float scale,
                                                            const int64_t* __restrict__ S_dev, int64_t q_rs,
                                                            const bf16* __restrict__ k_new,
@@ -446,10 +450,14 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
   typedef float f32x4_t __attribute__((ext_vector_type(4)));
   constexpr int G = GMAX, NW = kSmallWaves;
   const int item = blockIdx.x / (8 * CG) * 8 + blockIdx.x % 8, cg = blockIdx.x / 8 % CG;
-  if (item >= items) return;
-  const int g = item % Hkv, b = item / Hkv;
+  if (item >= items << log_rep) return;
+  const int kv = item >> log_rep, hs = item - (kv << log_rep), b = kv / Hkv, g = kv - b * Hkv;
+  const int h0 = ((g << log_rep) + hs) * GMAX;  // of H / Hkv = GMAX << log_rep
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const int r16 = lane & 15, qd = lane >> 4;
+  constexpr bool KLDS = D >= 128;
+  constexpr int CH = D / 8;                  // 16-byte chunks of a K row
+  __shared__ __attribute__((aligned(16))) char kt[KLDS ? NW : 1][KLDS ? 32 * D : 16];  // a wave's 16 K rows, chunks permuted by row
   __shared__ float pl[NW][16][16];           // a wave's P block [key][head]
   __shared__ float wm[NW][GMAX], wl[NW][GMAX];
   __shared__ float wo[NW][GMAX][DC];
@@ -463,7 +471,7 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
   uint4 qf[KS];
   {
     const bool ok = r16 < G;
-    const bf16* qp = q + (size_t)b * q_rs + (size_t)(g * G + (ok ? r16 : 0)) * D + 8 * qd;
+    const bf16* qp = q + (size_t)b * q_rs + (size_t)(h0 + (ok ? r16 : 0)) * D + 8 * qd;
 #pragma unroll
     for (int s2 = 0; s2 < KS; ++s2) qf[s2] = ok ? *reinterpret_cast<const uint4*>(qp + 32 * s2) : uint4{0u, 0u, 0u, 0u};
   }
@@ -506,14 +514,25 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
 
   uint4 kf[KS];
   uint2 vraw[4][CL];  // this lane's quads of bf16 of its 4 V rows
+  const unsigned kbase = __builtin_amdgcn_readfirstlane(lds_addr_of(kt[KLDS ? w : 0]));
   auto load_block = [&](int kb) {
-    const int key = min(kb + r16, S - 1);
-    const bool fresh = k_new != nullptr && key == S - 1;
-    const bf16* kr = fresh ? k_new + new_off : kc + (head_base + key) * D;
+    if constexpr (KLDS) {
 #pragma unroll
-    for (int s2 = 0; s2 < KS; ++s2) kf[s2] = *reinterpret_cast<const uint4*>(kr + 32 * s2 + 8 * qd);
-    if constexpr (ROPE) {
-      if (fresh) rotate(kf);
+      for (int p = 0; p < KS; ++p) {  // 1 KiB: the wave's next 64 chunks
+        const int row = (64 * p + lane) / CH, ch = (64 * p + lane) % CH ^ row;
+        const int key = min(kb + row, S - 1);
+        const bool fresh = k_new != nullptr && key == S - 1;
+        glds16((fresh ? k_new + new_off : kc + (head_base + key) * D) + 8 * ch, kbase + 1024 * p);
+      }
+    } else {
+      const int key = min(kb + r16, S - 1);
+      const bool fresh = k_new != nullptr && key == S - 1;
+      const bf16* kr = fresh ? k_new + new_off : kc + (head_base + key) * D;
+#pragma unroll
+      for (int s2 = 0; s2 < KS; ++s2) kf[s2] = *reinterpret_cast<const uint4*>(kr + 32 * s2 + 8 * qd);
+      if constexpr (ROPE) {
+        if (fresh) rotate(kf);
+      }
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -525,7 +544,7 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
     }
   };
   // fused append: the wave holding key S-1 writes this step's K / V row into the cache (no workgroup reads it there)
-  if (cg == 0 && k_new != nullptr && k0 < k1 && S - 1 >= k0 && S - 1 < k1) {
+  if (cg == 0 && hs == 0 && k_new != nullptr && k0 < k1 && S - 1 >= k0 && S - 1 < k1) {
     const bf16* ks = k_new + new_off;
     const bf16* vs = v_new + new_off;
     bf16* kd = kc + (head_base + S - 1) * D;
@@ -549,6 +568,15 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
   }
   if (k0 < k1) load_block(k0);
   for (int kb = k0; kb < k1; kb += 16) {
+    if constexpr (KLDS) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * CL) : "memory");  // the keys; the values behind them may be on the way
+#pragma unroll
+      for (int s2 = 0; s2 < KS; ++s2)
+        kf[s2] = *reinterpret_cast<const uint4*>(kt[w] + r16 * 2 * D + (((4 * s2 + qd) ^ r16) << 4));
+      if constexpr (ROPE) {
+        if (k_new != nullptr && kb + r16 >= S - 1) rotate(kf);
+      }
+    }
     f32x4_t sacc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s2 = 0; s2 < KS; ++s2)
@@ -567,6 +595,7 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
         vf[j][4 * c4 + 2] = __uint_as_float(u.y << 16);
         vf[j][4 * c4 + 3] = __uint_as_float(u.y & 0xffff0000u);
       }
+    if constexpr (KLDS) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (this block's keys are in registers)
     if (kb + 16 < k1) load_block(kb + 16);
     // scores of keys kb + 4qd + r for head r16 (masked past the wave's range)
     float sc[4], bmax = -INFINITY;
@@ -649,7 +678,7 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
       O += e * wo[x][i][d];
       L += e * wl[x][i];
     }
-    out[((size_t)b * H + g * G + i) * D + DC * cg + d] = from_f<bf16>(L > 0.f ? O / L : 0.f);
+    out[((size_t)b * H + h0 + i) * D + DC * cg + d] = from_f<bf16>(L > 0.f ? O / L : 0.f);
   }
 }
 
@@ -722,7 +751,7 @@ bool decode_small_applies(int64_t B, int64_t Tq, int64_t H, int64_t Hkv, int64_t
   // PENROZ_DECODE_SMALL_ITEMS: the largest B·Hkv it takes (0 disables)
   static const int small_items = [] {
     const char* e = std::getenv("PENROZ_DECODE_SMALL_ITEMS");
-    return e ? std::atoi(e) : 64;
+    return e ? std::atoi(e) : -1;
   }();
   static const int split_keys_env = [] {
     const char* e = std::getenv("PENROZ_DECODE_SPLIT_KEYS");
@@ -732,13 +761,17 @@ bool decode_small_applies(int64_t B, int64_t Tq, int64_t H, int64_t Hkv, int64_t
   if (Hkv <= 0 || H % Hkv) return false;
   const int64_t G0 = H / Hkv;
   // decode_small takes contexts up to 1024 keys (a workgroup goes over the whole cache, so longer ones keep the
-  // key-split grid) and up to 64 items. General / small kernel, us per launch at a 1024-slot cache, 40, 200, 500 and 1000
-  // keys: D = 64, G = 1, 12 items 4.9 / 4.0, 5.7 / 5.1, 9.2 / 6.5, 9.9 / 9.8, 64 items 4.9 / 4.0, 6.3 / 5.1, 13.1 / 7.5,
-  // 15.1 / 10.4; D = 256, G = 4, 64 items 11.1 / 5.1, 29.8 / 8.5, .., 47.5 / 23.7; D = 512, G = 1, 64 items 17.6 / 6.0,
-  // 56.8 / 12.1, .., 81.1 / 45.5. Of D 64 to 512, G 1 to 16, 1 to 64 items only D = 256, G = 1 with 1 to 4 items is
-  // slower at 1000 keys (19.0 / 20.2), and faster up to 500 (18.5 / 11.8).
+  // key-split grid), whatever the number of items, but for D = 256 with G 1, 4 or 8, where decode_kernel has loops of its own and is
+  // ahead from 512 items on. General / small kernel, us per launch at a 1024-slot cache, 40, 200, 500 and 1000
+  // keys: D = 64, G = 1, 128 items 5.3 / 3.3, 7.3 / 5.2, 18.6 / 7.3, 19.7 / 10.4, 512 items 5.5 / 4.0, 8.5 / 7.9, 18.8 / 17.3, 30.9 /
+  // 27.9, 1024 items 7.3 / 5.9, 12.7 / 12.4, 30.4 / 28.7, 55.8 / 50.5; D = 128, G = 1, 512 items 6.6 / 6.0, 14.0 / 12.1, 33 / 28, 59
+  // / 49, G = 8 13.8 / 14.4, 26.7 / 24.1, 51 / 41, 93 / 64; D = 256, G = 4, 256 items 13.7 / 14.4, 36.5 / 23.2, 64 / 42, 98 / 69, 512 items
+  // 14.3 / 27.4, 41 / 47, 80 / 77, 148 / 131, G = 1, 512 items 9.1 / 13.7, 29.4 / 30.3, 61 / 62, 108 / 117, G = 2 23 / 15, 80 / 31, 171 /
+  // 64, 331 / 117; D = 512, G = 1, 1024 items 68 / 65, 235 / 134, 537 / 276, 1049 / 470. At 40 keys and 64 items or fewer the
+  // keys' way through LDS is 0.1 to 0.3 us slower than straight reads (D = 128, G = 1, 64 items 3.3, here 3.5; D = 256 3.8, 4.1).
   const int64_t small_keys = split_keys_env ? split_keys_env : 1024;
-  return Tq == 1 && B * Hkv <= small_items && S <= small_keys &&
+  const int64_t most = small_items >= 0 ? small_items : D == 256 && (G0 == 1 || G0 == 4 || G0 == 8) ? 256 : INT64_MAX;
+  return Tq == 1 && B * Hkv <= most && S <= small_keys &&
          (G0 == 1 || G0 == 2 || G0 == 4 || G0 == 8 || G0 == 16) && (D == 64 || D == 128 || D == 256 || D == 512) &&
          G0 * D <= 4096;
 }
@@ -844,44 +877,43 @@ torch::Tensor decode_attn(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, c
     bf16* op = reinterpret_cast<bf16*>(out.data_ptr());
     const bf16* knp = fuse ? reinterpret_cast<const bf16*>(k_new->data_ptr()) : nullptr;
     const bf16* vnp = fuse ? reinterpret_cast<const bf16*>(v_new->data_ptr()) : nullptr;
-#define PENROZ_DSMALL(DD, GG)                                                                                   \
-  do {                                                                                                          \
-    const dim3 grid((items + 7) / 8 * 8 * (DD / 64));                                                           \
-    if (rope && DD <= 256)                                                                                      \
-      hipLaunchKernelGGL((decode_small_kernel<DD, GG, true>), grid, dim3(64 * kSmallWaves), 0, stream, qp, kp,  \
-                         vp, op, items, H, Hkv, cap, (int)S, (float)scale, sdev, q_rs, knp, vnp, kv_rs, rcp, rsp); \
-    else                                                                                                        \
-      hipLaunchKernelGGL((decode_small_kernel<DD, GG, false>), grid, dim3(64 * kSmallWaves), 0, stream, qp, kp, \
-                         vp, op, items, H, Hkv, cap, (int)S, (float)scale, sdev, q_rs, knp, vnp, kv_rs, nullptr, \
-                         nullptr);                                                                              \
-  } while (0)
-#define PENROZ_DSMALL_G(DD)                      \
-  switch (G0) {                                   \
-    case 1: PENROZ_DSMALL(DD, 1); break;          \
-    case 2: PENROZ_DSMALL(DD, 2); break;          \
-    case 4: PENROZ_DSMALL(DD, 4); break;          \
-    case 8: PENROZ_DSMALL(DD, 8); break;          \
-    default: PENROZ_DSMALL(DD, 16);               \
-  }
-    if (D == 64) PENROZ_DSMALL_G(64)
-    else if (D == 128) PENROZ_DSMALL_G(128)
-    else if (D == 256) PENROZ_DSMALL_G(256)
-    else if (items > 32 && G0 <= 4) {  // more workgroups of 64 columns than CUs: of 128
-      auto wide = [&](auto g0) {
-        hipLaunchKernelGGL((decode_small_kernel<512, decltype(g0)::value, false, 128>), dim3((items + 7) / 8 * 8 * 4),
-                           dim3(64 * kSmallWaves), 0, stream, qp, kp, vp, op, items, H, Hkv, cap, (int)S, (float)scale,
-                           sdev, q_rs, knp, vnp, kv_rs, nullptr, nullptr);
+    auto launch = [&](auto dd, auto gg, auto dc) {
+      constexpr int DD = decltype(dd)::value, GG = decltype(gg)::value, DC = decltype(dc)::value;
+      int log_rep = 0;  // G0 / GG, both powers of two
+      while ((GG << log_rep) < G0) ++log_rep;
+      const dim3 grid(((items << log_rep) + 7) / 8 * 8 * (DD / DC));
+      auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, grid, dim3(64 * kSmallWaves), 0, stream, qp, kp, vp, op, items, log_rep, H, Hkv, cap, (int)S,
+                           (float)scale, sdev, q_rs, knp, vnp, kv_rs, rcp, rsp);
       };
-      if (G0 == 1) wide(std::integral_constant<int, 1>{});
-      else if (G0 == 2) wide(std::integral_constant<int, 2>{});
-      else wide(std::integral_constant<int, 4>{});
+      if constexpr (DD <= 256) {
+        if (rope) return go(decode_small_kernel<DD, GG, true, DC>);
+      }
+      go(decode_small_kernel<DD, GG, false, DC>);
+    };
+    // heads of a workgroup: all of the group's, or as many fewer as at most 128 workgroups allow
+    auto by_heads = [&](auto dd) {
+      using C64 = std::integral_constant<int, 64>;
+      constexpr int DD = decltype(dd)::value;
+      int64_t gh = G0;
+      while (gh > 1 && (int64_t)items * (DD / 64) * (2 * G0 / gh) <= 128) gh /= 2;
+      if (gh == 1) launch(dd, std::integral_constant<int, 1>{}, C64{});
+      else if (gh == 2) launch(dd, std::integral_constant<int, 2>{}, C64{});
+      else if (gh == 4) launch(dd, std::integral_constant<int, 4>{}, C64{});
+      else if (gh == 8) launch(dd, std::integral_constant<int, 8>{}, C64{});
+      else if constexpr (DD <= 256) launch(dd, std::integral_constant<int, 16>{}, C64{});
+    };
+    if (D == 64) by_heads(std::integral_constant<int, 64>{});
+    else if (D == 128) by_heads(std::integral_constant<int, 128>{});
+    else if (D == 256) by_heads(std::integral_constant<int, 256>{});
+    else if (items > 32 && G0 <= 4) {  // more workgroups of 64 columns than CUs: of 128
+      using D5 = std::integral_constant<int, 512>;
+      using C128 = std::integral_constant<int, 128>;
+      if (G0 == 1) launch(D5{}, std::integral_constant<int, 1>{}, C128{});
+      else if (G0 == 2) launch(D5{}, std::integral_constant<int, 2>{}, C128{});
+      else launch(D5{}, std::integral_constant<int, 4>{}, C128{});
     }
-    else if (G0 == 1) PENROZ_DSMALL(512, 1);
-    else if (G0 == 2) PENROZ_DSMALL(512, 2);
-    else if (G0 == 4) PENROZ_DSMALL(512, 4);
-    else PENROZ_DSMALL(512, 8);
-#undef PENROZ_DSMALL_G
-#undef PENROZ_DSMALL
+    else by_heads(std::integral_constant<int, 512>{});
     return out;
   }
   // several query rows per sequence (prompts): 64 of them share each key and value that is read
