@@ -26,6 +26,11 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
 void decode_gemv_pair(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64_t mode, int64_t kind, int64_t D,
                       int64_t nrot, c10::optional<torch::Tensor> cosv, c10::optional<torch::Tensor> sinv,
                       int64_t pairs_per_wave);
+void decode_norm_pair(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> a, c10::optional<torch::Tensor> w1, torch::Tensor w2,
+                      int64_t step, double eps1, double eps2, c10::optional<torch::Tensor> h, torch::Tensor w, torch::Tensor out,
+                      int64_t mode, int64_t kind, int64_t D, int64_t nrot, c10::optional<torch::Tensor> cosv,
+                      c10::optional<torch::Tensor> sinv, c10::optional<torch::Tensor> tok, c10::optional<torch::Tensor> table,
+                      double scale);
 void decode_gemm_acc(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias, torch::Tensor resid);
 void decode_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64_t kind);
 // rows_gemm.hip
@@ -148,6 +153,12 @@ PYBIND11_MODULE(penroz_serve, m) {
         pybind11::arg("cos") = pybind11::none(), pybind11::arg("sin") = pybind11::none(),
         pybind11::arg("pairs_per_wave") = 0,
         "paired-row decode GEMV for 1..4 rows: gated MLP (mode 1) or RoPE QKV (mode 2) epilogue");
+  m.def("decode_norm_pair", &decode_norm_pair, pybind11::arg("x"), pybind11::arg("a"), pybind11::arg("w1"), pybind11::arg("w2"),
+        pybind11::arg("step"), pybind11::arg("eps1"), pybind11::arg("eps2"), pybind11::arg("h"), pybind11::arg("w"),
+        pybind11::arg("out"), pybind11::arg("mode"), pybind11::arg("kind") = 0, pybind11::arg("D") = 0, pybind11::arg("nrot") = 0,
+        pybind11::arg("cos") = pybind11::none(), pybind11::arg("sin") = pybind11::none(), pybind11::arg("tok") = pybind11::none(),
+        pybind11::arg("table") = pybind11::none(), pybind11::arg("scale") = 1.0,
+        "decode_gemv_pair behind the residual add and norms of a Gemma block (rms_residual), for 1..4 rows");
   m.def("rows_gemm", &rows_gemm, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("bias"), pybind11::arg("out"),
         pybind11::arg("fp32") = false, pybind11::arg("in_order") = false, pybind11::arg("gelu") = false);
   m.def("rows_gemm_tile", &rows_gemm_tile, pybind11::arg("M"), pybind11::arg("N"), pybind11::arg("K"),

@@ -744,51 +744,149 @@ __global__ void __launch_bounds__(64 * NW) decode_gemv_rows_kernel(const bf16* _
     reinterpret_cast<bf16*>(out)[o] = from_f<bf16>(y);
 }
 
-// Pairs of weight rows, a half-wave each, x once per workgroup of 4 waves in LDS (with every wave fetching it, a call of 3 rows of x
+// What stands in front of a pair product: nothing, or the step between two sublayers of a Gemma block (rms_residual_kernel's math and
+// rounding points): v = rms(x + a)·w1 (mode 0), x + rms(a)·w1 (1), x + a (2) or x alone (3); h = v, the product's x = rms(v)·w2. In
+// mode 3 with token ids x is their rows of `table`, times `scale`.
+struct PairNorm {
+  const bf16 *x, *a, *w1, *w2;
+  bf16* h;
+  int mode;
+  float eps1, eps2;
+  const int64_t* tok;
+  const bf16* table;
+  int64_t vocab;
+  float scale;
+};
+
+// Pairs of weight rows, a half-wave each, x once per workgroup in LDS (with every wave fetching it, a call of 3 rows of x
 // read more of x than of weights). GATED: on the packed [gate; up] weight (N = 2I rows): half 0 takes gate row n, half 1 up row I + n,
 // out[n] = act_f(bf16(g), kind) · bf16(u) (skinny_gated's rounding). Otherwise RoPE QKV: pair p of head p / (D/2), j = p % (D/2): half
 // 0 row head·D + j, half 1 row + D/2, both rounded to bf16, then rotated by one position's cos / sin [D/2] for the first nrot heads
 // (skinny_qkv_rope's math). A wave owns RP pairs. us before / now at 1, 3 and 4 rows, 2 x 6912 x 1152 gated: 8.0 / 7.3, 10.2 / 7.6,
 // 11.2 / 7.8 (32 MB of weights; 2 pairs per wave 8.1 at 3 rows, 3 8.8, 4 8.1).
-template <int M, int RP, int CPL, bool GATED>
-__global__ void __launch_bounds__(256) decode_gemv_pair_kernel(const bf16* __restrict__ x, int64_t x_rs, const bf16* __restrict__ w,
-                                                               bf16* __restrict__ out, int64_t o_rs, int N, int K, int kind, int D,
-                                                               int nrot, const float* __restrict__ cosv,
-                                                               const float* __restrict__ sinv) {
-  constexpr int XN = M * 32 * CPL, XL = (XN + 255) / 256;
-  static_assert(RP * M <= 32, "a lane per output");
+// NORM: the first M waves each make a row of x from nm, while the weights are on their way; workgroup 0 writes h. Gated, 8 waves and
+// 2 pairs a wave, so that each CU repeats the rows' work at most twice, in 128 registers, so that it holds two (one with 132: 12.1 us).
+// In steps of Gemma-3 1B, 3 rows: step and QKV 4.0 + 3.5 us as two kernels, 5.4 as one, step and gate|up 4.0 + 8.6, 10.9 as one.
+template <int M, int RP, int CPL, int NW, bool GATED, bool NORM>
+__global__ void __launch_bounds__(64 * NW, NORM && CPL <= 5 ? 4 : 1) decode_gemv_pair_kernel(const bf16* __restrict__ x, int64_t x_rs,
+                                                                   const bf16* __restrict__ w, bf16* __restrict__ out, int64_t o_rs,
+                                                                   int N, int K, int kind, int D, int nrot,
+                                                                   const float* __restrict__ cosv, const float* __restrict__ sinv,
+                                                                   PairNorm nm) {
+  constexpr int T = 64 * NW, XN = M * 32 * CPL, XL = (XN + T - 1) / T, NV = (CPL + 1) / 2;
+  static_assert(RP * M <= 32 && M <= NW, "a lane per output, a wave per row");
   __shared__ uint4 xs[XN];
   const int t = threadIdx.x, lane = t & 63, wid = __builtin_amdgcn_readfirstlane(t >> 6), h = lane >> 5, l32 = lane & 31;
   const int nc = K / 8, npair = N / 2, hd = D / 2;
-  const int p0 = (blockIdx.x * 4 + wid) * RP;
-  uint4 xt[XL], wv[RP][CPL];  // chunks past a row are read from its last one and count as zero
+  const int p0 = (blockIdx.x * NW + wid) * RP;
+  uint4 wv[RP][CPL];  // chunks past a row are read from its last one and count as zero
+  auto weights = [&]() {
 #pragma unroll
-  for (int i = 0; i < XL; ++i) {
-    const int e = t + 256 * i;
-    xt[i] = *reinterpret_cast<const uint4*>(x + (size_t)min(e / (32 * CPL), M - 1) * x_rs + 8 * min(e % (32 * CPL), nc - 1));
-  }
+    for (int r = 0; r < RP; ++r) {
+      const int p = min(p0 + r, npair - 1), row = GATED ? p + h * npair : p / hd * D + p % hd + h * hd;
 #pragma unroll
-  for (int r = 0; r < RP; ++r) {
-    const int p = min(p0 + r, npair - 1), row = GATED ? p + h * npair : p / hd * D + p % hd + h * hd;
-#pragma unroll
-    for (int i = 0; i < CPL; ++i) wv[r][i] = *reinterpret_cast<const uint4*>(w + (size_t)row * K + 8 * min(l32 + 32 * i, nc - 1));
-  }
+      for (int i = 0; i < CPL; ++i) wv[r][i] = *reinterpret_cast<const uint4*>(w + (size_t)row * K + 8 * min(l32 + 32 * i, nc - 1));
+    }
+  };
   const int p = p0 + l32 / M;  // this lane's output pair, row l32 % M of x
   const bool mine = l32 < RP * M && p < npair;
   float cs = 1.f, sn = 0.f;
-  if constexpr (!GATED) {
-    if (mine && p / hd < nrot) {
-      cs = cosv[p % hd];
-      sn = sinv[p % hd];
+  auto angles = [&]() {
+    if constexpr (!GATED) {
+      if (mine && p / hd < nrot) {
+        cs = cosv[p % hd];
+        sn = sinv[p % hd];
+      }
     }
-  }
-  __builtin_amdgcn_sched_barrier(0);
+  };
+  if constexpr (NORM) {
+    uint4 rx[NV], ra[NV], r1[NV], r2[NV];
+    if (wid < M) {
+      const bf16* xr = nm.x + (size_t)wid * K;
+      if (nm.tok) {
+        int64_t tok = nm.tok[wid];
+        tok = tok < 0 ? 0 : tok >= nm.vocab ? nm.vocab - 1 : tok;
+        xr = nm.table + (size_t)tok * K;
+      }
 #pragma unroll
-  for (int i = 0; i < XL; ++i) launder(xt[i]);  // asked for before the weights, all of them (not where a branch needs one)
+      for (int i = 0; i < NV; ++i) rx[i] = *reinterpret_cast<const uint4*>(xr + 8 * min(lane + 64 * i, nc - 1));
+      if (nm.mode != 3)
 #pragma unroll
-  for (int i = 0; i < XL; ++i) {
-    const int e = t + 256 * i;
-    if (e < XN) xs[e] = e % (32 * CPL) < nc ? xt[i] : uint4{0u, 0u, 0u, 0u};
+        for (int i = 0; i < NV; ++i) ra[i] = *reinterpret_cast<const uint4*>(nm.a + (size_t)wid * K + 8 * min(lane + 64 * i, nc - 1));
+      if (nm.mode < 2)
+#pragma unroll
+        for (int i = 0; i < NV; ++i) r1[i] = *reinterpret_cast<const uint4*>(nm.w1 + 8 * min(lane + 64 * i, nc - 1));
+#pragma unroll
+      for (int i = 0; i < NV; ++i) r2[i] = *reinterpret_cast<const uint4*>(nm.w2 + 8 * min(lane + 64 * i, nc - 1));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    weights();
+    angles();
+    __builtin_amdgcn_sched_barrier(0);
+    if (wid < M) {
+      auto rounded = [](float f) { return bf2f(from_f<bf16>(f)); };
+      float v[NV][8], xv[NV][8];
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const bool ok = lane + 64 * i < nc;
+        Vec8<bf16>::load(reinterpret_cast<const bf16*>(&rx[i]), xv[i]);
+        if (nm.mode != 3) Vec8<bf16>::load(reinterpret_cast<const bf16*>(&ra[i]), v[i]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if (nm.mode == 3) v[i][e] = nm.tok ? rounded(xv[i][e] * nm.scale) : xv[i][e];
+          else if (nm.mode != 1) v[i][e] = rounded(xv[i][e] + v[i][e]);
+          if (nm.mode < 2 && ok) ss += v[i][e] * v[i][e];
+        }
+      }
+      if (nm.mode < 2) {
+        const float r = rsqrtf(wave_sum(ss) / K + nm.eps1);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+          float w1v[8];
+          Vec8<bf16>::load(reinterpret_cast<const bf16*>(&r1[i]), w1v);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float n = rounded(rounded(v[i][e] * r) * w1v[e]);
+            v[i][e] = nm.mode == 0 ? n : rounded(xv[i][e] + n);
+          }
+        }
+      }
+      ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        if (lane + 64 * i < nc)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) ss += v[i][e] * v[i][e];
+      const float r = rsqrtf(wave_sum(ss) / K + nm.eps2);
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int j = lane + 64 * i;
+        if (nm.h != nullptr && blockIdx.x == 0 && j < nc) Vec8<bf16>::store(nm.h + (size_t)wid * K + 8 * j, v[i]);
+        float w2v[8];
+        Vec8<bf16>::load(reinterpret_cast<const bf16*>(&r2[i]), w2v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[i][e] = j < nc ? rounded(v[i][e] * r) * w2v[e] : 0.f;
+        if (j < 32 * CPL) Vec8<bf16>::store(reinterpret_cast<bf16*>(xs + wid * 32 * CPL + j), v[i]);
+      }
+    }
+  } else {
+    uint4 xt[XL];
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+      const int e = t + T * i;
+      xt[i] = *reinterpret_cast<const uint4*>(x + (size_t)min(e / (32 * CPL), M - 1) * x_rs + 8 * min(e % (32 * CPL), nc - 1));
+    }
+    weights();
+    angles();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < XL; ++i) launder(xt[i]);  // asked for before the weights, all of them (not where a branch needs one)
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+      const int e = t + T * i;
+      if (e < XN) xs[e] = e % (32 * CPL) < nc ? xt[i] : uint4{0u, 0u, 0u, 0u};
+    }
   }
   // a barrier for LDS alone: __syncthreads would wait for the weights as well
   __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
@@ -1160,66 +1258,70 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
   }
 }
 
-// Paired-row decode GEMV for 1..4 rows on a bf16 x (decode_gemv_pair_kernel):
+// Paired-row decode GEMV for 1..4 rows (decode_gemv_pair_kernel):
 //   mode 1 (gated): out[M, I] = act_f(x·Wgᵀ, kind) ⊙ (x·Wuᵀ), w = [Wg; Wu] [2I, K];
 //   mode 2 (RoPE QKV): out[M, (H + 2Hkv)·D] = rope(x · Wᵀ) for the first nrot heads, cos / sin [D/2].
-void decode_gemv_pair(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64_t mode, int64_t kind, int64_t D,
-                      int64_t nrot, c10::optional<torch::Tensor> cosv, c10::optional<torch::Tensor> sinv,
-                      int64_t pairs_per_wave) {
+// x is given, or nm makes it.
+static void gemv_pair_launch(const bf16* xp, int64_t x_rs, const PairNorm* nm, int M, const torch::Tensor& w, const torch::Tensor& out,
+                             int64_t mode, int64_t kind, int64_t D, int64_t nrot, const c10::optional<torch::Tensor>& cosv,
+                             const c10::optional<torch::Tensor>& sinv, int64_t pairs_per_wave, const char* who) {
   const int N = w.size(0), K = w.size(1);
-  TORCH_CHECK(mode == 1 || mode == 2, "decode_gemv_pair: mode 1 (gated) or 2 (RoPE)");
+  TORCH_CHECK(mode == 1 || mode == 2, who, ": mode 1 (gated) or 2 (RoPE)");
   TORCH_CHECK(w.is_cuda() && w.scalar_type() == torch::kBFloat16 && w.dim() == 2 && w.is_contiguous() &&
                   reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 && K % 8 == 0 && N % 2 == 0,
-              "decode_gemv_pair: bf16 contiguous 16-B aligned W [N, K], K % 8 == 0, N even");
-  TORCH_CHECK(x.scalar_type() == torch::kBFloat16 && x.dim() == 2 && x.size(1) == K && x.stride(1) == 1 &&
-                  x.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
-              "decode_gemv_pair: bf16 x [M, K], rows 16-B aligned");
-  const int M = x.size(0);
-  TORCH_CHECK(M >= 1 && M <= 4, "decode_gemv_pair: 1..4 rows");
+              who, ": bf16 contiguous 16-B aligned W [N, K], K % 8 == 0, N even");
+  TORCH_CHECK(M >= 1 && M <= 4, who, ": 1..4 rows");
   const int cpl = (K / 8 + 31) / 32;
-  TORCH_CHECK(cpl <= 7, "decode_gemv_pair: K <= 1792");
+  TORCH_CHECK(cpl <= 7, who, ": K <= 1792");
   const int Nout = mode == 1 ? N / 2 : N;
   TORCH_CHECK(out.scalar_type() == torch::kBFloat16 && out.dim() == 2 && out.size(0) == M && out.size(1) == Nout &&
-                  out.stride(1) == 1, "decode_gemv_pair: bf16 out [M, N/2] (gated) or [M, N] (RoPE)");
+                  out.stride(1) == 1, who, ": bf16 out [M, N/2] (gated) or [M, N] (RoPE)");
   const float *cp = nullptr, *sp = nullptr;
   if (mode == 1) {
-    TORCH_CHECK(kind >= 0 && kind <= 2, "decode_gemv_pair: kind 0 gelu, 1 gelu_tanh, 2 silu");
+    TORCH_CHECK(kind >= 0 && kind <= 2, who, ": kind 0 gelu, 1 gelu_tanh, 2 silu");
   } else if (mode == 2) {
-    TORCH_CHECK(D >= 2 && D % 2 == 0 && N % D == 0 && nrot >= 0 && nrot <= N / D, "decode_gemv_pair: RoPE geometry");
+    TORCH_CHECK(D >= 2 && D % 2 == 0 && N % D == 0 && nrot >= 0 && nrot <= N / D, who, ": RoPE geometry");
     TORCH_CHECK(cosv.has_value() && sinv.has_value() && cosv->is_cuda() && sinv->is_cuda() &&
                     cosv->scalar_type() == torch::kFloat32 && sinv->scalar_type() == torch::kFloat32 &&
                     cosv->numel() >= D / 2 && sinv->numel() >= D / 2 && cosv->is_contiguous() && sinv->is_contiguous(),
-                "decode_gemv_pair: fp32 cos / sin [D/2]");
+                who, ": fp32 cos / sin [D/2]");
     cp = cosv->data_ptr<float>();
     sp = sinv->data_ptr<float>();
   }
   const int ppw = pairs_per_wave <= 0 ? 1 : (int)pairs_per_wave;
-  TORCH_CHECK(ppw == 1 || ppw == 2 || ppw == 4, "decode_gemv_pair: pairs_per_wave 1, 2 or 4");
-  const dim3 grid((N / 2 + 4 * ppw - 1) / (4 * ppw));
+  TORCH_CHECK(ppw == 1 || ppw == 2 || ppw == 4, who, ": pairs_per_wave 1, 2 or 4");
   auto stream = at::hip::getCurrentHIPStream();
-  auto xp = reinterpret_cast<const bf16*>(x.data_ptr());
   auto wp = reinterpret_cast<const bf16*>(w.data_ptr());
   auto op = reinterpret_cast<bf16*>(out.data_ptr());
-  const int64_t x_rs = x.stride(0), o_rs = out.stride(0);
-  auto launch = [&](auto mt, auto rpt, auto cplt, auto et) {
+  const int64_t o_rs = out.stride(0);
+  auto launch = [&](auto mt, auto rpt, auto cplt, auto et, auto nt) {
     constexpr int MM = decltype(mt)::value, RR = decltype(rpt)::value, CC = decltype(cplt)::value;
-    hipLaunchKernelGGL((decode_gemv_pair_kernel<MM, RR, CC, decltype(et)::value>), grid, dim3(256), 0, stream, xp, x_rs, wp, op, o_rs,
-                       N, K, (int)kind, mode == 1 ? 2 : (int)D, (int)nrot, cp, sp);
+    constexpr bool GATED = decltype(et)::value, NORM = decltype(nt)::value;
+    constexpr int NW = NORM && GATED ? 8 : 4;
+    const dim3 grid((N / 2 + NW * RR - 1) / (NW * RR));
+    hipLaunchKernelGGL((decode_gemv_pair_kernel<MM, RR, CC, NW, GATED, NORM>), grid, dim3(64 * NW), 0, stream, xp, x_rs, wp, op, o_rs,
+                       N, K, (int)kind, mode == 1 ? 2 : (int)D, (int)nrot, cp, sp, nm ? *nm : PairNorm{});
   };
-  auto by_cpl = [&](auto mt, auto rpt, auto et) {
-    if (cpl <= 3) launch(mt, rpt, std::integral_constant<int, 3>{}, et);
-    else if (cpl <= 4) launch(mt, rpt, std::integral_constant<int, 4>{}, et);
-    else if (cpl <= 5) launch(mt, rpt, std::integral_constant<int, 5>{}, et);
-    else launch(mt, rpt, std::integral_constant<int, 7>{}, et);
-  };
-  auto by_rp = [&](auto mt, auto et) {
-    if (ppw == 1) by_cpl(mt, std::integral_constant<int, 1>{}, et);
-    else if (ppw == 2) by_cpl(mt, std::integral_constant<int, 2>{}, et);
-    else by_cpl(mt, std::integral_constant<int, 4>{}, et);
+  auto by_cpl = [&](auto mt, auto rpt, auto et, auto nt) {
+    if (cpl <= 3) launch(mt, rpt, std::integral_constant<int, 3>{}, et, nt);
+    else if (cpl <= 4) launch(mt, rpt, std::integral_constant<int, 4>{}, et, nt);
+    else if (cpl <= 5) launch(mt, rpt, std::integral_constant<int, 5>{}, et, nt);
+    else launch(mt, rpt, std::integral_constant<int, 7>{}, et, nt);
   };
   auto by_mode = [&](auto mt) {
-    if (mode == 1) by_rp(mt, std::true_type{});
-    else by_rp(mt, std::false_type{});
+    using C1 = std::integral_constant<int, 1>;
+    using C2 = std::integral_constant<int, 2>;
+    auto by_rp = [&](auto et) {
+      if (nm != nullptr) {
+        if constexpr (decltype(et)::value) by_cpl(mt, C2{}, et, std::true_type{});
+        else by_cpl(mt, C1{}, et, std::true_type{});
+      }
+      else if (ppw == 1) by_cpl(mt, C1{}, et, std::false_type{});
+      else if (ppw == 2) by_cpl(mt, C2{}, et, std::false_type{});
+      else by_cpl(mt, std::integral_constant<int, 4>{}, et, std::false_type{});
+    };
+    if (mode == 1) by_rp(std::true_type{});
+    else by_rp(std::false_type{});
   };
   switch (M) {
     case 1: by_mode(std::integral_constant<int, 1>{}); break;
@@ -1227,4 +1329,64 @@ void decode_gemv_pair(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64
     case 3: by_mode(std::integral_constant<int, 3>{}); break;
     default: by_mode(std::integral_constant<int, 4>{});
   }
+}
+
+void decode_gemv_pair(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64_t mode, int64_t kind, int64_t D,
+                      int64_t nrot, c10::optional<torch::Tensor> cosv, c10::optional<torch::Tensor> sinv,
+                      int64_t pairs_per_wave) {
+  TORCH_CHECK(w.dim() == 2 && x.scalar_type() == torch::kBFloat16 && x.dim() == 2 && x.size(1) == w.size(1) && x.stride(1) == 1 &&
+                  x.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
+              "decode_gemv_pair: bf16 x [M, K], rows 16-B aligned");
+  gemv_pair_launch(reinterpret_cast<const bf16*>(x.data_ptr()), x.stride(0), nullptr, (int)x.size(0), w, out, mode, kind, D, nrot, cosv,
+                   sinv, pairs_per_wave, "decode_gemv_pair");
+}
+
+// decode_gemv_pair of x' = rms(v)·w2 with v of `step` (PairNorm's modes 0 to 3); h [M, K] receives v (optional in mode 3 without
+// tokens, where it is x)
+void decode_norm_pair(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> a, c10::optional<torch::Tensor> w1, torch::Tensor w2,
+                      int64_t step, double eps1, double eps2, c10::optional<torch::Tensor> h, torch::Tensor w, torch::Tensor out,
+                      int64_t mode, int64_t kind, int64_t D, int64_t nrot, c10::optional<torch::Tensor> cosv,
+                      c10::optional<torch::Tensor> sinv, c10::optional<torch::Tensor> tok, c10::optional<torch::Tensor> table,
+                      double scale) {
+  const char* who = "decode_norm_pair";
+  TORCH_CHECK(w.dim() == 2 && step >= 0 && step <= 3, who, ": W [N, K], step 0 to 3");
+  const int64_t K = w.size(1);
+  auto given = [](const c10::optional<torch::Tensor>& t) { return t.has_value() && t->defined(); };
+  const bool emb = given(tok);
+  TORCH_CHECK(!emb || (step == 3 && given(table) && given(h)), who, ": tokens with step 3, a table and h");
+  TORCH_CHECK(emb != given(x) && given(a) == (step != 3) && (step >= 2 || given(w1)), who, ": operands of the step");
+  PairNorm nm{};
+  int64_t M;
+  if (emb) {
+    TORCH_CHECK(tok->is_cuda() && tok->scalar_type() == torch::kInt64 && tok->is_contiguous(), who, ": int64 tokens");
+    M = tok->numel();
+  } else {
+    TORCH_CHECK(x->dim() == 2, who, ": x [M, K]");
+    M = x->size(0);
+  }
+  auto rows = [&](const torch::Tensor& t, int64_t n) {
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kBFloat16 && t.is_contiguous() && t.numel() == n * K &&
+                    reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, who, ": bf16 contiguous rows of K values, 16-B aligned");
+    return reinterpret_cast<bf16*>(t.data_ptr());
+  };
+  if (given(x)) nm.x = rows(*x, M);
+  if (given(a)) nm.a = rows(*a, M);
+  if (step < 2) nm.w1 = rows(*w1, 1);
+  nm.w2 = rows(w2, 1);
+  if (given(h)) {
+    nm.h = rows(*h, M);
+    TORCH_CHECK(nm.h != nm.x && nm.h != nm.a, who, ": h apart from x and a (other workgroups still read them)");
+  }
+  TORCH_CHECK(step == 3 || nm.h != nullptr, who, ": h");
+  nm.mode = (int)step;
+  nm.eps1 = (float)eps1;
+  nm.eps2 = (float)eps2;
+  if (emb) {
+    TORCH_CHECK(table->dim() == 2, who, ": table [V, K]");
+    nm.tok = tok->data_ptr<int64_t>();
+    nm.vocab = table->size(0);
+    nm.table = rows(*table, nm.vocab);
+    nm.scale = (float)scale;
+  }
+  gemv_pair_launch(nullptr, 0, &nm, (int)M, w, out, mode, kind, D, nrot, cosv, sinv, 0, who);
 }

@@ -17,6 +17,8 @@ from penroz.ops._ext import use_kernels, kernels
 def rope_table(inv_freq: Tensor, offset: int, T: int, device, offset_dev: Tensor | None = None) -> tuple[Tensor, Tensor]:
     """cos / sin [T, D/2] for positions offset..offset+T-1; ``offset_dev`` (device int64 [1])
     supplies the offset at run time instead (graph-replayed decode)."""
+    if offset_dev is not None and use_kernels(offset_dev) and inv_freq.device == offset_dev.device:
+        return tuple(kernels().rope_table(inv_freq.float().contiguous(), offset_dev, T))
     if offset_dev is not None:
         t = offset_dev.to(torch.float32) + torch.arange(T, device=device, dtype=torch.float32)
     else:

@@ -124,3 +124,72 @@ def test_gemv_pairs_of_few_rows(M, K, I, ppw):
     # gate and up, rounded from sums of another order, may be a bf16 step apart each; the result is rounded once more
     assert torch.all((got - ref)[fin].abs() <= 2.0 ** -8 * 4 * (ref.abs() + y[:, :I].abs() + y[:, I:].abs())[fin] + 1e-5)
     assert (big[M] == 7).all() and (big[:, I:] == 7).all()
+
+
+def _step_ref(x, a, w1, w2, mode, eps1, eps2):
+    """rms_residual's step in fp32 with its bf16 rounding points, from 64-bit sums."""
+    b16 = lambda t: t.to(torch.bfloat16).float()
+    rms = lambda t, eps: b16(t * torch.rsqrt(t.double().square().mean(-1, keepdim=True) + eps).float())
+    x = x.float()
+    if mode == 0:
+        v = b16(rms(b16(x + a.float()), eps1) * w1.float())
+    elif mode == 1:
+        v = b16(x + b16(rms(a.float(), eps1) * w1.float()))
+    else:
+        v = b16(x + a.float()) if mode == 2 else x
+    return v, b16(rms(v, eps2) * w2.float())
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("K", [8, 264, 768, 1032, 1152, 1792])
+@pytest.mark.parametrize("mode", [0, 1, 2, 3])
+@pytest.mark.parametrize("gated", [True, False])
+def test_norm_pair(M, K, mode, gated):
+    """The step between two sublayers in front of a pair product: its residual row by row, its product against the product of
+    the reference's rows; pairs that end inside a wave and a workgroup."""
+    torch.manual_seed(M + K + mode)
+    k = _ext.kernels()
+    x, a = (torch.randn(M, K, device=DEV).to(torch.bfloat16) for _ in range(2))
+    w1, w2 = ((1 + 0.1 * torch.randn(K, device=DEV)).to(torch.bfloat16) for _ in range(2))
+    D, N = 16, 2 * 37 if gated else 5 * 16
+    w = (torch.randn(N, K, device=DEV) / K ** 0.5).to(torch.bfloat16)
+    big = torch.full((M + 1, N + 3), 7.0, device=DEV, dtype=torch.bfloat16)
+    out = big[:M, :N // 2 if gated else N]
+    h = torch.empty(M, K, device=DEV, dtype=torch.bfloat16)
+    ang = torch.rand(D // 2, device=DEV) * 6
+    cs, sn = ang.cos(), ang.sin()
+    if mode == 3:
+        table, idx = torch.randn(9, K, device=DEV).to(torch.bfloat16), torch.tensor([8, 0, 3, 5][:M], device=DEV)
+        x = (table[idx] * 3.5)
+        k.decode_norm_pair(None, None, None, w2, 3, 0.0, 1e-6, h, w, out, 1 if gated else 2, 2, D, 4, cs, sn, idx, table, 3.5)
+    else:
+        k.decode_norm_pair(x, a, w1, w2, mode, 1e-6, 1e-5, h, w, out, 1 if gated else 2, 2, D, 4, cs, sn)
+    v, y = _step_ref(x, a, w1, w2, mode, 1e-6, 1e-6 if mode == 3 else 1e-5)
+    # a value near a tie may be rounded apart at each of the step's four roundings
+    assert torch.all((h.float() - v).abs() <= 4 * 2.0 ** -8 * (v.abs() + x.float().abs()) + 1e-6)
+    z = (y @ w.float().t())
+    slack = 2.0 ** -8 * (z.abs() + 4 * (y.square() @ w.float().square().t()).sqrt())
+    if gated:
+        I = N // 2
+        ref = F.silu(z[:, :I]) * z[:, I:]
+        # |silu'| <= 1.1
+        bound = slack[:, :I] * 1.1 * z[:, I:].abs() + F.silu(z[:, :I]).abs() * slack[:, I:] + slack[:, :I] * slack[:, I:]
+        bound = bound + 2.0 ** -8 * ref.abs() + 1e-5
+    else:
+        zz, s2 = z.view(M, 5, D), slack.view(M, 5, D)
+        lo, hi = zz[..., :D // 2], zz[..., D // 2:]
+        rot = torch.cat([lo * cs - hi * sn, hi * cs + lo * sn], -1)
+        ref = torch.cat([rot[:, :4], zz[:, 4:]], 1).view(M, N)
+        both = s2[..., :D // 2] + s2[..., D // 2:]
+        bound = torch.cat([both, both], -1).view(M, N) + 2.0 ** -8 * ref.abs() + 1e-5
+    assert torch.all((out.float() - ref).abs() <= bound), float(((out.float() - ref).abs() / bound).max())
+    assert (big[M] == 7).all() and (big[:, out.shape[1]:] == 7).all()
+
+
+@pytest.mark.parametrize("T,n,pos", [(1, 128, 0), (1, 4, 8191), (5, 33, 1000)])
+def test_rope_table_at_a_device_position(T, n, pos):
+    from penroz.ops import rope
+    inv = 1.0 / (1e6 ** (torch.arange(n, device=DEV, dtype=torch.float32) / n))
+    got = rope.rope_table(inv, 0, T, DEV, offset_dev=torch.tensor([pos], device=DEV))
+    for g, r in zip(got, rope.rope_table(inv, pos, T, DEV)):
+        assert g.shape == r.shape and torch.all((g - r).abs() <= 2.0 ** -22)
