@@ -33,6 +33,47 @@ __global__ void __launch_bounds__(256) rms_fwd_kernel(const TX* __restrict__ x, 
   if (lane == 0) rstd_out[row] = r;
 }
 
+// The same for rows of 16-byte pieces and one type, up to 6144 wide: a row in registers (NV 8-value vectors per lane), read once, 16 bytes
+// at a time, the weights with it. us in bf16, a value at a time / so: 3 x 1152 4.6 / 2.1,
+// 600 x 1152 5.3 / 2.5, 4096 x 1152 7.3 / 4.5, 8192 x 2304 25.6 / 12.4.
+template <int NV, typename T>
+__global__ void __launch_bounds__(256) rms_fwd_vec_kernel(const T* __restrict__ x, const T* __restrict__ w, T* __restrict__ y,
+                                                          float* __restrict__ rstd_out, int N, int C, float eps) {
+  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= N) return;
+  const int nvec = C / 8;
+  struct alignas(16) Raw {
+    T v[8];
+  };
+  Raw rx[NV], rw[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) rx[i] = *reinterpret_cast<const Raw*>(x + (size_t)row * C + 8 * min(lane + 64 * i, nvec - 1));
+#pragma unroll
+  for (int i = 0; i < NV; ++i) rw[i] = *reinterpret_cast<const Raw*>(w + 8 * min(lane + 64 * i, nvec - 1));
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    float v[8];
+    Vec8<T>::load(rx[i].v, v);
+    if (lane + 64 * i < nvec)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+  }
+  const float r = rsqrtf(wave_sum(ss) / C + eps);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int j = lane + 64 * i;
+    float v[8], wv[8];
+    Vec8<T>::load(rx[i].v, v);
+    Vec8<T>::load(rw[i].v, wv);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = to_f(from_f<T>(v[e] * r)) * wv[e];  // (x*norm).to(x.dtype)
+    if (j < nvec) Vec8<T>::store(y + (size_t)row * C + 8 * j, v);
+  }
+  if (lane == 0) rstd_out[row] = r;
+}
+
 // One wave per row; lane l owns columns l + 64·k (k < NPL), so each row's x / dy stay in registers
 // between the two passes and the dγ partial sums accumulate in registers across the wave's rows
 // (no LDS atomics); the 4 waves' partials are combined through LDS into one row of `part`.
@@ -231,6 +272,27 @@ std::vector<torch::Tensor> rmsnorm_fwd(torch::Tensor x, torch::Tensor w, double 
   if (N == 0) return {y, rstd};
   auto wc = w.contiguous();
   auto stream = at::hip::getCurrentHIPStream();
+  const auto aligned = [](const torch::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+  if (x.scalar_type() == w.scalar_type() && C % 8 == 0 && C >= 8 && C <= 6144 && aligned(x) && aligned(wc)) {
+    auto launch = [&](auto tag) {
+      using T = decltype(tag);
+      auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((N + 3) / 4), dim3(256), 0, stream, reinterpret_cast<const T*>(x.data_ptr()),
+                           reinterpret_cast<const T*>(wc.data_ptr()), reinterpret_cast<T*>(y.data_ptr()), rstd.data_ptr<float>(), N,
+                           C, (float)eps);
+      };
+      const int nv = (C / 8 + 63) / 64;
+      if (nv <= 1) go(rms_fwd_vec_kernel<1, T>);
+      else if (nv <= 2) go(rms_fwd_vec_kernel<2, T>);
+      else if (nv <= 3) go(rms_fwd_vec_kernel<3, T>);
+      else if (nv <= 4) go(rms_fwd_vec_kernel<4, T>);
+      else if (nv <= 6) go(rms_fwd_vec_kernel<6, T>);
+      else if (nv <= 8) go(rms_fwd_vec_kernel<8, T>);
+      else go(rms_fwd_vec_kernel<12, T>);
+    };
+    RMS_TYPES(x.scalar_type(), T, launch(T{}))
+    return {y, rstd};
+  }
   RMS_TYPES(x.scalar_type(), TX, RMS_TYPES(w.scalar_type(), TW, RMS_TYPES(out_t, TY,
     hipLaunchKernelGGL((rms_fwd_kernel<TX, TW, TY>), dim3((N + 3) / 4), dim3(256), 0, stream,
                        reinterpret_cast<const TX*>(x.data_ptr()), reinterpret_cast<const TW*>(wc.data_ptr()),
