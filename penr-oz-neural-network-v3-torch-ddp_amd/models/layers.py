@@ -22,6 +22,7 @@ from torch import Tensor
 import torch.nn as nn
 
 from penroz.ops import attention as attn_ops
+from penroz.ops import gemm as gemm_ops
 from penroz.ops import norms as norm_ops
 from penroz.ops import activations as act_ops
 from penroz.ops import packed as packed_ops
@@ -179,6 +180,9 @@ class LayerNorm(nn.LayerNorm):
         return c[1], c[2]
 
 
+Linear = gemm_ops.Linear
+
+
 class GELU(nn.GELU):
     """``nn.GELU`` (erf or tanh) whose GPU path is the vectorised HIP GELU kernel."""
 
@@ -204,9 +208,9 @@ class GatedMLP(nn.Module):
     def __init__(self, in_features: int, intermediate_size: int,
                  bias: bool = False, activation: str = "gelu_pytorch_tanh"):
         super().__init__()
-        self.gate_proj = nn.Linear(in_features, intermediate_size, bias=bias)
-        self.up_proj = nn.Linear(in_features, intermediate_size, bias=bias)
-        self.down_proj = nn.Linear(intermediate_size, in_features, bias=bias)
+        self.gate_proj = Linear(in_features, intermediate_size, bias=bias)
+        self.up_proj = Linear(in_features, intermediate_size, bias=bias)
+        self.down_proj = Linear(intermediate_size, in_features, bias=bias)
         if activation in ("silu", "swish"):
             self.act_kind = "silu"
             self.act = nn.SiLU()

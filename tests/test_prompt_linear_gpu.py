@@ -1,0 +1,66 @@
+"""Linear layers of prompts: inference mode on bf16 takes the kernel of short steps, every other call the library."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from penroz.models import layers as L
+from penroz.ops import gemm as gemm_ops
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+
+def _layer(K, N, bias, dtype=BF):
+    torch.manual_seed(K + N)
+    lin = L.Linear(K, N, bias=bias).to("cuda", dtype)
+    return lin
+
+
+@pytest.fixture
+def taken(monkeypatch):
+    calls, inner = [], gemm_ops.rows_linear
+
+    def spy(*a, **k):
+        y = inner(*a, **k)
+        calls.append(y is not None)
+        return y
+
+    monkeypatch.setattr(gemm_ops, "rows_linear", spy)
+    return calls
+
+
+@pytest.mark.parametrize("shape,N,bias", [((1, 1, 8), 1, True), ((1, 7, 768), 2304, True), ((3, 200, 1152), 1536, False),
+                                          ((64, 776), 130, True), ((2, 3, 5, 64), 96, False), ((1, 512, 768), 50304, False)])
+def test_prompt_products(shape, N, bias, taken):
+    lin = _layer(shape[-1], N, bias)
+    wide = torch.randn(*shape[:-1], 2 * shape[-1], device="cuda", dtype=BF)
+    x = wide[..., :shape[-1]]  # rows of a wider buffer
+    with torch.inference_mode():
+        y = lin(x)
+        t = lin(x.movedim(0, -2))  # leading axes that reshape has to copy
+    want = F.linear(x.double(), lin.weight.double(), lin.bias.double() if bias else None)
+    mass = F.linear(x.double().abs(), lin.weight.double().abs(), lin.bias.double().abs() if bias else None)
+    # one bf16 rounding of the result and K fp32 additions
+    bound = want.abs() * 2.0 ** -8 + mass * shape[-1] * 2.0 ** -24 + 1e-30
+    assert y.shape == (*shape[:-1], N) and y.dtype == BF
+    assert ((y.double() - want).abs() <= bound).all()
+    assert ((t.double() - want.movedim(0, -2)).abs() <= bound.movedim(0, -2)).all()
+    assert len(taken) == 2 and (N == 50304 or taken[0])
+
+
+def test_other_calls_keep_the_library(taken):
+    lin = _layer(64, 96, True)
+    x = torch.randn(4, 64, device="cuda", dtype=BF)
+    lin(x.requires_grad_()).sum().backward()
+    assert x.grad is not None and lin.weight.grad is not None
+    with torch.no_grad():
+        lin(x)
+    with torch.inference_mode():
+        torch.func.vmap(lin)(x.detach()[None])
+        lin(x[0])
+        lin(x[:0])
+        lin.float()(x.float())
+        lin.to(BF)
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert lin(x).dtype == torch.float16
+    assert taken == []
