@@ -43,6 +43,8 @@ void embedding_fwd(torch::Tensor idx, torch::Tensor wte, torch::Tensor wpe, int6
 void embedding_bwd(torch::Tensor dout, torch::Tensor idx, torch::Tensor dwte, torch::Tensor dwpe, int64_t off,
                    double dropout_p, int64_t dropout_seed);
 std::vector<torch::Tensor> rope_table(torch::Tensor inv_freq, torch::Tensor pos, int64_t T);
+c10::optional<torch::Tensor> prompt_kv(torch::Tensor qkv, c10::optional<torch::Tensor> inv_freq, torch::Tensor kc, torch::Tensor vc,
+                                       int64_t pos, int64_t H, int64_t Hkv);
 torch::Tensor rope_qkv(torch::Tensor qkv, torch::Tensor cosv, torch::Tensor sinv, int64_t H, int64_t Hkv, int64_t D,
                        bool inverse, c10::optional<torch::Tensor> out);
 void kv_quantize(torch::Tensor x, torch::Tensor q, torch::Tensor scale, int64_t pos);
@@ -178,6 +180,8 @@ PYBIND11_MODULE(penroz_kernels, m) {
         pybind11::arg("dwpe"), pybind11::arg("off"), pybind11::arg("dropout_p") = 0.0,
         pybind11::arg("dropout_seed") = 0);
   m.def("rope_table", &rope_table, pybind11::arg("inv_freq"), pybind11::arg("pos"), pybind11::arg("T"));
+  m.def("prompt_kv", &prompt_kv, pybind11::arg("qkv"), pybind11::arg("inv_freq"), pybind11::arg("kc"), pybind11::arg("vc"),
+        pybind11::arg("pos"), pybind11::arg("H"), pybind11::arg("Hkv"));
   m.def("rope_qkv", &rope_qkv, pybind11::arg("qkv"), pybind11::arg("cosv"), pybind11::arg("sinv"), pybind11::arg("H"),
         pybind11::arg("Hkv"), pybind11::arg("D"), pybind11::arg("inverse"), pybind11::arg("out") = pybind11::none());
   m.def("kv_quantize", &kv_quantize);

@@ -373,6 +373,57 @@ __global__ void __launch_bounds__(256) rope_vec_kernel(const T* __restrict__ in,
   }
 }
 
+// A prompt's new keys and values from qkv [B, T, (H + 2 Hkv) * D] into the caches [B, Hkv, cap, D] at pos.., and with ROPE the
+// rotated queries into q [B, T, H, D] (keys rotated on the way, angles in the arithmetic of rope_table_kernel). Bound by the
+// host: a layer's pass was the table (7 launches of 5 us of host time each), the rotation, two strided copies. A workgroup takes
+// `per_wg` tokens, whose angles it computes once for all heads into LDS; an item is 8 rotated pairs or 16 bytes copied. 3 x 200
+// tokens, 4 + 1 heads of 256: 5.1 us of the device for the former 25.
+template <bool ROPE, typename F>
+__global__ void __launch_bounds__(256) prompt_kv_kernel(const __hip_bfloat16* __restrict__ in, const F* __restrict__ inv,
+                                                        __hip_bfloat16* __restrict__ q, __hip_bfloat16* __restrict__ kc,
+                                                        __hip_bfloat16* __restrict__ vc, int64_t tokens, int per_wg, int T,
+                                                        int H, int Hkv, int D, int64_t cap, int pos) {
+  extern __shared__ float angles[];  // [per_wg][cos D/2, sin D/2]
+  const int half = D / 2, h8 = half / 8, d8 = D / 8;
+  const int64_t row0 = blockIdx.x * (int64_t)per_wg, W = (int64_t)(H + 2 * Hkv) * D;
+  const int n = (int)(tokens - row0 < per_wg ? tokens - row0 : per_wg);
+  if (ROPE) {
+    for (int i = threadIdx.x; i < n * half; i += 256) {
+      const int r = i / half, j = i - r * half;
+      const float a = (float)(pos + (int)((row0 + r) % T)) * to_f(inv[j]);
+      angles[r * D + j] = cosf(a);
+      angles[r * D + half + j] = sinf(a);
+    }
+    __syncthreads();
+  }
+  const int nrot = ROPE ? (H + Hkv) * h8 : 0, ncopy = (ROPE ? Hkv : 2 * Hkv) * d8, per = nrot + ncopy;
+  for (int i = threadIdx.x; i < n * per; i += 256) {
+    const int r = i / per, k = i - r * per;
+    const int64_t row = row0 + r, b = row / T, slot = pos + row - b * T;
+    const __hip_bfloat16* src = in + row * W;
+    if (ROPE && k < nrot) {
+      const int head = k / h8, j0 = 8 * (k - head * h8);
+      const float *cs = angles + r * D + j0, *sn = cs + half;
+      float x1[8], x2[8], o1[8], o2[8];
+      Vec8<__hip_bfloat16>::load(src + (int64_t)head * D + j0, x1);
+      Vec8<__hip_bfloat16>::load(src + (int64_t)head * D + half + j0, x2);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        o1[e] = x1[e] * cs[e] - x2[e] * sn[e];
+        o2[e] = x2[e] * cs[e] + x1[e] * sn[e];
+      }
+      __hip_bfloat16* dst = head < H ? q + (row * H + head) * D : kc + ((b * Hkv + head - H) * cap + slot) * D;
+      Vec8<__hip_bfloat16>::store(dst + j0, o1);
+      Vec8<__hip_bfloat16>::store(dst + half + j0, o2);
+    } else {
+      const int c = k - nrot, head = c / d8, j0 = 8 * (c - head * d8), kv = ROPE ? head + Hkv : head;  // kv: of the k heads, then v
+      const uint4 x = *reinterpret_cast<const uint4*>(src + (int64_t)(H + kv) * D + j0);
+      __hip_bfloat16* dst = (kv < Hkv ? kc : vc) + ((b * Hkv + (kv < Hkv ? kv : kv - Hkv)) * cap + slot) * D;
+      *reinterpret_cast<uint4*>(dst + j0) = x;
+    }
+  }
+}
+
 // ------------------------------------------------------------------------------ int8 KV quant
 // x [B, T, Hkv, D] -> q [B, Hkv, cap, D] int8 at pos.., scale [B, Hkv, cap] f32 (absmax/127)
 template <typename T>
@@ -703,6 +754,41 @@ std::vector<torch::Tensor> rope_table(torch::Tensor inv_freq, torch::Tensor pos,
                      at::hip::getCurrentHIPStream(), inv_freq.data_ptr<float>(), pos.data_ptr<int64_t>(), cosv.data_ptr<float>(),
                      sinv.data_ptr<float>(), (int)T, (int)n);
   return {cosv, sinv};
+}
+
+// qkv's keys and values into the caches at pos (inv_freq given: q and k rotated); q [B, T, H, D], a view of qkv without rotation.
+// None where it is not bf16 in rows of 16-byte pieces throughout.
+c10::optional<torch::Tensor> prompt_kv(torch::Tensor qkv, c10::optional<torch::Tensor> inv_freq, torch::Tensor kc, torch::Tensor vc,
+                                       int64_t pos, int64_t H, int64_t Hkv) {
+  TORCH_CHECK(qkv.dim() == 3 && kc.dim() == 4 && kc.sizes() == vc.sizes() && H >= 1 && Hkv >= 1, "prompt_kv: shapes");
+  const int64_t B = qkv.size(0), T = qkv.size(1), D = kc.size(3), cap = kc.size(2);
+  TORCH_CHECK(qkv.size(2) == (H + 2 * Hkv) * D && kc.size(0) == B && kc.size(1) == Hkv && pos >= 0 && pos + T <= cap,
+              "prompt_kv: sizes");
+  auto aligned = [](const torch::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+  for (const auto* t : {&qkv, &kc, &vc})
+    if (!(t->is_cuda() && t->get_device() == qkv.get_device() && t->scalar_type() == torch::kBFloat16 && t->is_contiguous() &&
+          aligned(*t)))
+      return c10::nullopt;
+  const bool rope = inv_freq.has_value() && inv_freq->defined();
+  if (D % 16 != 0 || D > 1024 || H + 2 * Hkv > 4096 || B * T < 1 || B * T > (int64_t)1 << 30 || pos + T > 1 << 24) return c10::nullopt;
+  if (rope && !(inv_freq->is_cuda() && inv_freq->get_device() == qkv.get_device() && inv_freq->is_contiguous() &&
+                inv_freq->dim() == 1 && inv_freq->numel() == D / 2 &&
+                (inv_freq->scalar_type() == torch::kFloat32 || inv_freq->scalar_type() == torch::kBFloat16)))
+    return c10::nullopt;
+  auto q = rope ? torch::empty({B, T, H, D}, qkv.options())
+                : qkv.as_strided({B, T, H, D}, {qkv.stride(0), qkv.stride(1), D, 1}, qkv.storage_offset());
+  const int64_t items = rope ? (H + Hkv) * (D / 16) + Hkv * (D / 8) : 2 * Hkv * (D / 8);
+  const int per_wg = (int)std::min<int64_t>(4, std::max<int64_t>(1, 256 / items));
+  auto bp = [](const torch::Tensor& t) { return reinterpret_cast<__hip_bfloat16*>(t.data_ptr()); };
+  auto launch = [&](auto kernel, auto* inv) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((B * T + per_wg - 1) / per_wg)), dim3(256), rope ? per_wg * D * sizeof(float) : 0,
+                       at::hip::getCurrentHIPStream(), bp(qkv), inv, bp(q), bp(kc), bp(vc), B * T, per_wg, (int)T, (int)H,
+                       (int)Hkv, (int)D, cap, (int)pos);
+  };
+  if (!rope) launch(prompt_kv_kernel<false, float>, (const float*)nullptr);
+  else if (inv_freq->scalar_type() == torch::kFloat32) launch(prompt_kv_kernel<true, float>, (const float*)inv_freq->data_ptr());
+  else launch(prompt_kv_kernel<true, __hip_bfloat16>, (const __hip_bfloat16*)inv_freq->data_ptr());
+  return q;
 }
 
 // out (optional): a preallocated contiguous tensor of qkv's shape and dtype (not aliasing qkv)

@@ -115,6 +115,9 @@ class _GraphMode:
         return self._attend_graph(layer_idx, q, k, v)
 
 
+kvc._STORES_AS_GIVEN.add(_GraphMode.attend)
+
+
 class StaticKVCache(_GraphMode, kvc.KVCache):
     def _attend_graph(self, l: int, q: Tensor, k: Tensor, v: Tensor) -> Tensor:
         # k, v, q are views into this layer's fused QKV rows: one kernel appends K/V at pos_t,

@@ -26,6 +26,7 @@ import numpy as np
 import torch
 from torch import Tensor
 
+from penroz.ops._ext import kernels, plain_call
 from penroz.ops import attention as attn_ops
 from penroz.ops import packed as packed_ops
 from penroz.ops import sampling as samp_ops
@@ -146,6 +147,32 @@ class KVCache:
         n = self._write(layer_idx, k, v)
         self._record(t0, k.shape[1], raw, raw)
         return attn_ops.decode_attention(q, self._k[layer_idx], self._v[layer_idx], n)
+
+    def attend_qkv(self, layer_idx: int, qkv: Tensor, H: int, Hkv: int, D: int, inv_freq: Tensor | None,
+                   offset: int) -> Tensor | None:
+        """``attend`` of the fused projection [B, T, (H + 2 Hkv) * D] at position ``offset``, rotated on the way
+        (``inv_freq``): one kernel in place of table, rotation and two copies. None, and nothing stored, where that kernel
+        does not apply."""
+        cls = type(self)
+        if not (cls.attend in _STORES_AS_GIVEN and cls._write is KVCache._write and qkv.dtype == torch.bfloat16 and plain_call(qkv)):
+            return None
+        t0 = time.monotonic()
+        B, T, _ = qkv.shape
+        self._ensure(layer_idx, qkv, B, Hkv, D, T)
+        kc, vc, pos = self._k[layer_idx], self._v[layer_idx], self._len[layer_idx]
+        if pos != offset or kc.dtype != qkv.dtype:
+            return None
+        q = kernels().prompt_kv(qkv, inv_freq, kc, vc, pos, H, Hkv)
+        if q is None:
+            return None
+        self._len[layer_idx] = pos + T
+        raw = 2 * B * T * Hkv * D * qkv.element_size()
+        self._record(t0, T, raw, raw)
+        return attn_ops.decode_attention(q, kc, vc, pos + T)
+
+
+# the ``attend`` methods that ``attend_qkv`` may stand in for (a subclass's own is always called)
+_STORES_AS_GIVEN = {KVCache.attend}
 
 
 class TurboQuantKVCache(KVCache):

@@ -21,6 +21,7 @@ import torch
 from torch import Tensor
 import torch.nn as nn
 
+from penroz.models.kv_cache import KVCache
 from penroz.ops import attention as attn_ops
 from penroz.ops import gemm as gemm_ops
 from penroz.ops import norms as norm_ops
@@ -75,8 +76,13 @@ class CausalSelfAttention(nn.Module):
         cache = self._kv_cache
         offset = cache.seq_len(self._layer_idx) if cache is not None else 0
 
-        if self.rope_theta is not None:
-            inv_freq = self._inv_freq(head_dim, query_key_value.device)
+        inv_freq = None if self.rope_theta is None else self._inv_freq(head_dim, query_key_value.device)
+        if isinstance(cache, KVCache) and not getattr(cache, "graph_mode", False):
+            out = cache.attend_qkv(self._layer_idx, query_key_value, self.num_heads, self.num_kv_heads, head_dim, inv_freq, offset)
+            if out is not None:
+                return out
+
+        if inv_freq is not None:
             # graph-replayed decode: positions come from the cache's device counter (one table per
             # (theta, head_dim) and step, shared by the layers)
             table = (cache.rope_table((self.rope_theta, head_dim), inv_freq, block_size)

@@ -19,7 +19,7 @@ import os
 import torch
 from torch import Tensor
 
-from penroz.ops._ext import use_kernels, kernels
+from penroz.ops._ext import use_kernels, kernels, plain_call
 
 # "auto"/"1": the native kernel (faster than hipBLASLt on every measured GPT-2 shape);
 # "0": hipBLASLt (A/B switch for benchmarking).
@@ -134,16 +134,6 @@ def train_linear(x: Tensor, w: Tensor, bias: Tensor | None = None, out: Tensor |
     return torch.mm(x, w.t(), out=out) if bias is None else torch.addmm(bias, x, w.t(), out=out)
 
 
-def _plain_call(x: Tensor, w: Tensor) -> bool:
-    """Nothing but the product's value is asked of ``x · wᵀ``: inference mode (no backward, no tangents), no trace, transform,
-    mode or autocast that has to see a library operator, bf16 tensors of no subclass."""
-    return (torch.is_inference_mode_enabled() and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda
-            and type(x) is Tensor and type(w) is torch.nn.Parameter and x.dim() >= 2 and x.numel() > 0
-            and not torch.is_autocast_enabled("cuda") and torch._C._get_tracing_state() is None
-            and not torch.compiler.is_compiling() and torch._C._functorch.peek_interpreter_stack() is None
-            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0)
-
-
 class Linear(torch.nn.Linear):
     """``nn.Linear`` whose prompts (inference mode, bf16 on the GPU) take :func:`rows_linear` where its rule does. A short
     prompt's pass is bound by the host, and the library's call costs it 19 µs against 4: GPT-2's pass over one prompt of 64
@@ -151,7 +141,7 @@ class Linear(torch.nn.Linear):
 
     def forward(self, x: Tensor) -> Tensor:
         w = self.weight
-        if _plain_call(x, w):
+        if x.dtype == torch.bfloat16 and x.dim() >= 2 and type(w) is torch.nn.Parameter and plain_call(x):
             y = rows_linear(x.reshape(-1, x.shape[-1]), w, self.bias)
             if y is not None:
                 return y.view(*x.shape[:-1], w.shape[0])
