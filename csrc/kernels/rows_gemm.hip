@@ -10,7 +10,7 @@
 // rows on bit for bit theirs up to K = 1024: training steps take that form there, where a rounding that falls otherwise changes every
 // later layer's. With the columns split, 64 x 2048 x 2048 takes 6.1 us instead of 7.0. decode_gemm_acc adds to an fp32 residual in place (64 x 768 x
 // 3072: 8.3 us in a kernel whose waves read their operands directly, 6.0 here). us, library / here (weights from memory): 64 x 768
-// x 768 7.1 / 3.3, 64 x 2048 x 2048 8.9 / 6.1, 64 x 2048 x 6144 19.0 / 16.3, 256 x 2304 x 768 7.7 / 6.5, 1024 x 1152 x 1024 9.7 / 9.2;
+// x 768 7.1 / 3.3, 64 x 2048 x 2048 8.9 / 6.1, 64 x 2048 x 6144 19.0 / 16.3 (32×32; 32×16 since: 13.3), 256 x 2304 x 768 7.7 / 6.5, 1024 x 1152 x 1024 9.7 / 9.2;
 // at 16 rows, skinny_gemm / here: 768 x 768 9.7 / 3.3, 2048 x 2048 7.1 / 4.6, 7232 x 2048 12.3 / 8.2. A call costs the host 4 us, the
 // library's 19. Tiles of 128×128 in rings of two to four stages were no faster than the library anywhere.
 #include "common.h"
@@ -199,6 +199,7 @@ static void rg_launch(int tile, bool in_order, const torch::Tensor& x, const tor
     using OUT = std::remove_pointer_t<decltype(o)>;
     if (tile == 6) PENROZ_RG(1, 1, 1, 1, 4, 1, 6);
     else if (tile == 1 && in_order) PENROZ_RG(1, 1, 2, 2, 1, 2, 4);
+    else if (tile == 1 && rows_gemm_narrow(M, N)) PENROZ_RG(2, 1, 1, 1, 4, 1, 6);
     else if (tile == 1) PENROZ_RG(2, 2, 1, 1, 4, 1, 4);
     else if (tile == 2) PENROZ_RG(2, 4, 1, 1, 4, 1, 3);
     else if (tile == 3) PENROZ_RG(2, 2, 2, 2, 1, 2, 4);
