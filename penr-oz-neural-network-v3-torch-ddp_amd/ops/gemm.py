@@ -139,13 +139,16 @@ class Linear(torch.nn.Linear):
     prompt's pass is bound by the host, and the library's call costs it 19 µs against 4: GPT-2's pass over one prompt of 64
     tokens 2.60 -> 1.71 ms, of 512 2.64 -> 1.79, Gemma 3 1B's over 3 of 200 7.6 -> 7.0."""
 
-    def forward(self, x: Tensor) -> Tensor:
+    def rows(self, x: Tensor) -> Tensor | None:
         w = self.weight
-        if x.dtype == torch.bfloat16 and x.dim() >= 2 and type(w) is torch.nn.Parameter and plain_call(x):
-            y = rows_linear(x.reshape(-1, x.shape[-1]), w, self.bias)
-            if y is not None:
-                return y.view(*x.shape[:-1], w.shape[0])
-        return torch.nn.functional.linear(x, w, self.bias)
+        if not (x.dtype == torch.bfloat16 and x.dim() >= 2 and type(w) is torch.nn.Parameter and plain_call(x)):
+            return None
+        y = rows_linear(x.reshape(-1, x.shape[-1]), w, self.bias)
+        return None if y is None else y.view(*x.shape[:-1], w.shape[0])
+
+    def forward(self, x: Tensor) -> Tensor:
+        y = self.rows(x)
+        return torch.nn.functional.linear(x, self.weight, self.bias) if y is None else y
 
 
 def linear_fp32(x: Tensor, w: Tensor) -> Tensor:
@@ -325,8 +328,8 @@ def skinny_qkv_rope(x: Tensor, w: Tensor, cos: Tensor, sin: Tensor, D: int, nrot
 
 
 class decode_gemms:
-    """Context: the ``nn.Linear`` modules of ``model`` run decode-shaped inputs through the skinny
-    kernel (others keep ``F.linear``). Entered by the graph decoder around the captured step of a
+    """Context: the ``nn.Linear`` modules of ``model`` run decode-shaped inputs that ``Linear`` itself leaves to the
+    library through the skinny kernel (others keep ``F.linear``). Entered by the graph decoder around the captured step of a
     model without a decode program. Only that model's own Linear instances are re-routed (an
     instance-level ``forward``, removed on exit): other models, and other threads serving them,
     are untouched; the serving lock keeps concurrent requests off the same model."""
@@ -345,6 +348,9 @@ class decode_gemms:
                 continue
 
             def forward(x, mod=mod):
+                y = mod.rows(x) if type(mod) is Linear else None  # as outside of the capture
+                if y is not None:
+                    return y
                 if (x.numel() <= max_rows * x.shape[-1] and skinny_ok(x, mod.weight)
                         and (mod.bias is None or mod.bias.is_contiguous())):
                     return skinny_linear(x, mod.weight, mod.bias)

@@ -64,3 +64,14 @@ def test_other_calls_keep_the_library(taken):
         with torch.autocast("cuda", dtype=torch.float16):
             assert lin(x).dtype == torch.float16
     assert taken == []
+
+
+@pytest.mark.parametrize("rows", [1, 5, 64])
+def test_a_captured_step_takes_the_same_kernel(rows, taken):
+    model = torch.nn.Sequential(_layer(128, 384, True), _layer(384, 128, False))
+    x = torch.randn(rows, 1, 128, device="cuda", dtype=BF)
+    with torch.inference_mode():
+        want = model(x)
+        with gemm_ops.decode_gemms(model):
+            got = model(x)
+    assert torch.equal(got, want) and taken == [True] * 4
