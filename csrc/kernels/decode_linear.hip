@@ -948,6 +948,17 @@ static const bf16* dl_bias(const c10::optional<torch::Tensor>& bias, int N, cons
   return reinterpret_cast<const bf16*>(bias->data_ptr());
 }
 
+// act(0 + bias) in every row of out: a product over no columns. The kernels clamp their loads to a row's last piece, which
+// rows of no columns do not have.
+static void no_columns(const c10::optional<torch::Tensor>& bias, const torch::Tensor& out, int64_t act) {
+  if (!bias.has_value() || !bias->defined()) {
+    out.zero_();  // (the activations' value at 0)
+    return;
+  }
+  torch::Tensor y = bias->view({1, -1});
+  out.copy_(act ? at::gelu(y.to(torch::kFloat32), act == 2 ? "tanh" : "none") : y);
+}
+
 struct LnEmb {  // the residual rows are the step's embeddings
   const int64_t* idx = nullptr;
   const bf16 *wte = nullptr, *wpe = nullptr;
@@ -1017,6 +1028,7 @@ void decode_ln_gemm(torch::Tensor resid, torch::Tensor gamma, torch::Tensor beta
               "decode_ln_gemm: bf16 out [M, N], rows 8-B aligned");
   TORCH_CHECK(act >= 0 && act <= 2, "decode_ln_gemm: act 0 (none), 1 (GELU erf), 2 (GELU tanh)");
   const bf16* bp = dl_bias(bias, N, "decode_ln_gemm");
+  if (K == 0) return no_columns(bias, out, act);
   ln_launch(resid.data_ptr<float>(), gamma.data_ptr<float>(), beta.data_ptr<float>(), (float)eps,
             reinterpret_cast<const bf16*>(w.data_ptr()), bp, reinterpret_cast<bf16*>(out.data_ptr()), out.stride(0), M, N, K, (int)act,
             nullptr);
@@ -1178,6 +1190,7 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
                 "decode_gemv: bf16 bias [N]");
     bp = reinterpret_cast<const bf16*>(bias->data_ptr());
   }
+  if (K == 0) return no_columns(bias, out, act);
   static const int rpw_env = [] {
     const char* e = std::getenv("PENROZ_DECODE_GEMV_RPW");
     return e ? std::atoi(e) : 0;
@@ -1290,6 +1303,10 @@ static void gemv_pair_launch(const bf16* xp, int64_t x_rs, const PairNorm* nm, i
   }
   const int ppw = pairs_per_wave <= 0 ? 1 : (int)pairs_per_wave;
   TORCH_CHECK(ppw == 1 || ppw == 2 || ppw == 4, who, ": pairs_per_wave 1, 2 or 4");
+  if (K == 0) {  // (as in no_columns; both forms of nothing are 0)
+    out.zero_();
+    return;
+  }
   auto stream = at::hip::getCurrentHIPStream();
   auto wp = reinterpret_cast<const bf16*>(w.data_ptr());
   auto op = reinterpret_cast<bf16*>(out.data_ptr());
@@ -1349,7 +1366,7 @@ void decode_norm_pair(c10::optional<torch::Tensor> x, c10::optional<torch::Tenso
                       c10::optional<torch::Tensor> sinv, c10::optional<torch::Tensor> tok, c10::optional<torch::Tensor> table,
                       double scale) {
   const char* who = "decode_norm_pair";
-  TORCH_CHECK(w.dim() == 2 && step >= 0 && step <= 3, who, ": W [N, K], step 0 to 3");
+  TORCH_CHECK(w.dim() == 2 && w.size(1) > 0 && step >= 0 && step <= 3, who, ": W [N, K], step 0 to 3");
   const int64_t K = w.size(1);
   auto given = [](const c10::optional<torch::Tensor>& t) { return t.has_value() && t->defined(); };
   const bool emb = given(tok);

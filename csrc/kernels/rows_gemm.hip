@@ -267,6 +267,10 @@ void decode_gemm_acc(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tens
     bp = reinterpret_cast<const bf16*>(bias->data_ptr());
   }
   if (N == 0) return;
+  if (K == 0) {  // gemv_add clamps its loads to a row's last piece
+    if (bp != nullptr) resid.add_(*bias);
+    return;
+  }
   if (M <= 4 && K <= 8192 && N < 16384)
     return gemv_add(reinterpret_cast<const bf16*>(x.data_ptr()), x.stride(0), reinterpret_cast<const bf16*>(w.data_ptr()), bp,
                     resid.data_ptr<float>(), (int)M, (int)N, (int)K);
