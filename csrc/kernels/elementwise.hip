@@ -770,7 +770,7 @@ c10::optional<torch::Tensor> prompt_kv(torch::Tensor qkv, c10::optional<torch::T
           aligned(*t)))
       return c10::nullopt;
   const bool rope = inv_freq.has_value() && inv_freq->defined();
-  if (D % 16 != 0 || D > 1024 || H + 2 * Hkv > 4096 || B * T < 1 || B * T > (int64_t)1 << 30 || pos + T > 1 << 24) return c10::nullopt;
+  if (D < 16 || D % 16 != 0 || D > 1024 || H + 2 * Hkv > 4096 || B * T < 1 || B * T > (int64_t)1 << 30 || pos + T > 1 << 24) return c10::nullopt;
   if (rope && !(inv_freq->is_cuda() && inv_freq->get_device() == qkv.get_device() && inv_freq->is_contiguous() &&
                 inv_freq->dim() == 1 && inv_freq->numel() == D / 2 &&
                 (inv_freq->scalar_type() == torch::kFloat32 || inv_freq->scalar_type() == torch::kBFloat16)))

@@ -52,3 +52,8 @@ def test_other_products_over_no_columns(M):
         assert (out == 0).all()
     with pytest.raises(RuntimeError):  # its norms are over the columns
         k.decode_norm_pair(x, None, None, torch.empty(0, device=DEV, dtype=BF), 3, 0.0, 1e-6, None, w, out, 2, 0, D, 2, cs, cs)
+
+
+def test_prompt_rows_of_no_width():
+    qkv, cache = torch.empty(1, 2, 0, device=DEV, dtype=BF), torch.empty(1, 1, 4, 0, device=DEV, dtype=BF)
+    assert _ext.kernels().prompt_kv(qkv, None, cache, cache, 0, 1, 1) is None
