@@ -226,12 +226,13 @@ c10::optional<torch::Tensor> rows_gemm(torch::Tensor x, torch::Tensor w, c10::op
   };
   const int tile = rows_gemm_plan(M, N, K, in_order);
   if (tile == 0 || !rows_ok(x) || !rows_ok(w)) return c10::nullopt;
-  if (has_bias && !(bias->is_cuda() && bias->scalar_type() == torch::kBFloat16 && bias->is_contiguous() && bias->numel() == N))
+  if (has_bias && !(bias->is_cuda() && bias->get_device() == x.get_device() && bias->scalar_type() == torch::kBFloat16 &&
+                    bias->is_contiguous() && bias->numel() == N))
     return c10::nullopt;
   if (given) {
     const torch::Tensor& o = *out_opt;
-    if (!(o.is_cuda() && o.scalar_type() == (fp32 ? torch::kFloat32 : torch::kBFloat16) && o.dim() == 2 && o.size(0) == M &&
-          o.size(1) == N && o.stride(1) == 1 && o.stride(0) >= N && o.stride(0) < (int64_t)1 << 30 &&
+    if (!(o.is_cuda() && o.get_device() == x.get_device() && o.scalar_type() == (fp32 ? torch::kFloat32 : torch::kBFloat16) &&
+          o.dim() == 2 && o.size(0) == M && o.size(1) == N && o.stride(1) == 1 && o.stride(0) >= N && o.stride(0) < (int64_t)1 << 30 &&
           (o.stride(0) % 4 != 0 || reinterpret_cast<uintptr_t>(o.data_ptr()) % (4 * o.element_size()) == 0)))
       return c10::nullopt;
   }

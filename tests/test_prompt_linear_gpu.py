@@ -4,6 +4,7 @@ import torch
 import torch.nn.functional as F
 
 from penroz.models import layers as L
+from penroz.ops import _ext
 from penroz.ops import gemm as gemm_ops
 
 pytestmark = pytest.mark.gpu
@@ -75,3 +76,12 @@ def test_a_captured_step_takes_the_same_kernel(rows, taken):
         with gemm_ops.decode_gemms(model):
             got = model(x)
     assert torch.equal(got, want) and taken == [True] * 4
+
+
+def test_an_input_on_another_device_is_the_librarys(monkeypatch):
+    """The kernels start on the current device; the library goes to its operands' own."""
+    x = torch.randn(4, 64, device="cuda", dtype=BF)
+    with torch.inference_mode():
+        assert _ext.plain_call(x)
+        monkeypatch.setattr(torch.cuda, "current_device", lambda: x.get_device() + 1)
+        assert not _ext.plain_call(x)
