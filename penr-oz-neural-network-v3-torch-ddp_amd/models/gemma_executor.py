@@ -112,7 +112,7 @@ class GemmaExecutor(GPTExecutor):
         if len(ls) < 4 or type(ls[0]) is not L.ScaledEmbedding or type(ls[-2]) is not L.RMSNorm:
             return None
         head = ls[-1]
-        if type(head) not in (nn.Linear, L.Linear) or head.bias is not None:
+        if type(head) is not nn.Linear or head.bias is not None:
             return None
         emb = ls[0]
         if head.weight is emb.weight:  # a tied head would be one parameter in two flat slots
@@ -126,8 +126,8 @@ class GemmaExecutor(GPTExecutor):
             if type(blk) is not L.TransformerBlock:
                 return None
             ab, mb = list(blk.attn_block), list(blk.mlp_block)
-            if not (len(ab) == 4 and type(ab[0]) is L.RMSNorm and type(ab[1]) in (nn.Linear, L.Linear)
-                    and type(ab[2]) is L.CausalSelfAttention and type(ab[3]) in (nn.Linear, L.Linear)
+            if not (len(ab) == 4 and type(ab[0]) is L.RMSNorm and type(ab[1]) is nn.Linear
+                    and type(ab[2]) is L.CausalSelfAttention and type(ab[3]) is nn.Linear
                     and len(mb) == 2 and type(mb[0]) is L.RMSNorm and type(mb[1]) is L.GatedMLP):
                 return None
             in_norm, qkv, attn, o = ab

@@ -23,7 +23,7 @@ import torch.nn as nn
 
 from penroz.models.kv_cache import KVCache
 from penroz.ops import attention as attn_ops
-from penroz.ops import gemm as gemm_ops
+from penroz.ops.gemm import apply
 from penroz.ops import norms as norm_ops
 from penroz.ops import activations as act_ops
 from penroz.ops import packed as packed_ops
@@ -150,7 +150,10 @@ class ResidualConnection(nn.Sequential):
 
     def forward(self, forwarded: Tensor) -> Tensor:
         for layer in self:
-            forwarded = forwarded + layer(forwarded)
+            if torch.jit.is_scripting():
+                forwarded = forwarded + layer(forwarded)
+            else:
+                forwarded = forwarded + apply(layer, forwarded)
         return forwarded
 
 
@@ -186,9 +189,6 @@ class LayerNorm(nn.LayerNorm):
         return c[1], c[2]
 
 
-Linear = gemm_ops.Linear
-
-
 class GELU(nn.GELU):
     """``nn.GELU`` (erf or tanh) whose GPU path is the vectorised HIP GELU kernel."""
 
@@ -214,9 +214,9 @@ class GatedMLP(nn.Module):
     def __init__(self, in_features: int, intermediate_size: int,
                  bias: bool = False, activation: str = "gelu_pytorch_tanh"):
         super().__init__()
-        self.gate_proj = Linear(in_features, intermediate_size, bias=bias)
-        self.up_proj = Linear(in_features, intermediate_size, bias=bias)
-        self.down_proj = Linear(intermediate_size, in_features, bias=bias)
+        self.gate_proj = nn.Linear(in_features, intermediate_size, bias=bias)
+        self.up_proj = nn.Linear(in_features, intermediate_size, bias=bias)
+        self.down_proj = nn.Linear(intermediate_size, in_features, bias=bias)
         if activation in ("silu", "swish"):
             self.act_kind = "silu"
             self.act = nn.SiLU()
@@ -228,7 +228,7 @@ class GatedMLP(nn.Module):
             self.act = nn.GELU()
 
     def forward(self, x: Tensor) -> Tensor:
-        return self.down_proj(act_ops.gated_act(self.gate_proj(x), self.up_proj(x), self.act_kind))
+        return apply(self.down_proj, act_ops.gated_act(apply(self.gate_proj, x), apply(self.up_proj, x), self.act_kind))
 
 
 class ScaledEmbedding(nn.Embedding):
@@ -260,7 +260,10 @@ class TransformerBlock(nn.Module):
         self.post_norm_on_residual = post_norm_on_residual
 
     def forward(self, x: Tensor) -> Tensor:
-        attn_out = self.attn_block(x)
+        if torch.jit.is_scripting():
+            attn_out = self.attn_block(x)
+        else:
+            attn_out = apply(self.attn_block, x)
         if self.post_attn_norm is not None and not self.post_norm_on_residual:
             attn_out = self.post_attn_norm(attn_out)
         h = x + attn_out
@@ -268,7 +271,10 @@ class TransformerBlock(nn.Module):
             h = self.post_attn_norm(h)
         if self.mlp_block is None:
             return h
-        mlp_out = self.mlp_block(h)
+        if torch.jit.is_scripting():
+            mlp_out = self.mlp_block(h)
+        else:
+            mlp_out = apply(self.mlp_block, h)
         if self.post_mlp_norm is not None and not self.post_norm_on_residual:
             mlp_out = self.post_mlp_norm(mlp_out)
         out = h + mlp_out

@@ -10,8 +10,8 @@ Differences on purpose:
   * the config is never mutated (the reference compiles ``transformerblock`` by writing
     ``nn.Module`` objects back into the caller's dict, so modules end up pickled in the
     checkpoint — SURVEY §7.4 bug 14);
-  * ``linear`` / ``layernorm`` / ``gelu`` compile to subclasses whose GPU path is a HIP kernel (same
-    parameters and keys as ``nn.Linear`` / ``nn.LayerNorm`` / ``nn.GELU``);
+  * ``layernorm`` / ``gelu`` compile to subclasses whose GPU path is a HIP kernel (same
+    parameters and keys as ``nn.LayerNorm`` / ``nn.GELU``);
   * ``adam`` / ``adamw`` compile to fused-kernel subclasses of ``torch.optim.Adam/AdamW``
     (identical ``state_dict`` format, one multi-tensor HIP launch per step on GPU).
 """
@@ -34,7 +34,7 @@ log = logging.getLogger(__name__)
 class Mapper:
     _algo_to_func = {
         "embedding": nn.Embedding,
-        "linear": L.Linear,
+        "linear": nn.Linear,
         "flatten": nn.Flatten,
         "batchnorm1d": nn.BatchNorm1d,
         "relu": nn.ReLU,

@@ -44,6 +44,7 @@ from penroz.models.layers import CausalSelfAttention, PositionEmbedding, Softmax
 from penroz.models.mapper import Mapper
 from penroz.ops import sampling as samp_ops
 from penroz.ops import fused as fused_ops
+from penroz.ops.gemm import apply
 from penroz.parallel import dist as ddp
 from penroz.parallel.launcher import maybe_inject_fault
 from penroz.utils import checkpoint as ckpt
@@ -303,7 +304,7 @@ class NeuralNetworkModel(nn.Module):
         layers = self.layers[:-1] if skip_softmax and self._is_softmax_last else self.layers
         for layer in layers:
             prev = x
-            x = layer(prev)
+            x = apply(layer, prev)
             activations.append(x)
         if target is None:
             cost = torch.empty(0)

@@ -19,7 +19,8 @@ import os
 import torch
 from torch import Tensor
 
-from penroz.ops._ext import use_kernels, kernels, plain_call
+from penroz.ops import _ext
+from penroz.ops._ext import use_kernels, kernels
 
 # "auto"/"1": the native kernel (faster than hipBLASLt on every measured GPT-2 shape);
 # "0": hipBLASLt (A/B switch for benchmarking).
@@ -134,21 +135,33 @@ def train_linear(x: Tensor, w: Tensor, bias: Tensor | None = None, out: Tensor |
     return torch.mm(x, w.t(), out=out) if bias is None else torch.addmm(bias, x, w.t(), out=out)
 
 
-class Linear(torch.nn.Linear):
-    """``nn.Linear`` whose prompts (inference mode, bf16 on the GPU) take :func:`rows_linear` where its rule does. A short
-    prompt's pass is bound by the host, and the library's call costs it 19 µs against 4: GPT-2's pass over one prompt of 64
-    tokens 2.60 -> 1.71 ms, of 512 2.64 -> 1.79, Gemma 3 1B's over 3 of 200 7.6 -> 7.0."""
+def _bare(mod: torch.nn.Module) -> bool:
+    """A call of ``mod`` is its class's forward and nothing else: no hooks, no forward of its own (but for ``decode_gemms``'s)."""
+    f = mod.__dict__.get("forward")
+    return ((f is None or getattr(f, "of_decode_gemms", False)) and mod._compiled_call_impl is None
+            and not (mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks
+                     or torch.nn.modules.module._has_any_global_hook()))
 
-    def rows(self, x: Tensor) -> Tensor | None:
-        w = self.weight
-        if not (x.dtype == torch.bfloat16 and x.dim() >= 2 and type(w) is torch.nn.Parameter and plain_call(x)):
-            return None
-        y = rows_linear(x.reshape(-1, x.shape[-1]), w, self.bias)
-        return None if y is None else y.view(*x.shape[:-1], w.shape[0])
 
-    def forward(self, x: Tensor) -> Tensor:
-        y = self.rows(x)
-        return torch.nn.functional.linear(x, self.weight, self.bias) if y is None else y
+def apply(mod: torch.nn.Module, x: Tensor) -> Tensor:
+    """``mod(x)``, where the ``nn.Linear`` layers of prompts (inference mode, bf16 on the GPU; ``mod`` itself or in the
+    ``nn.Sequential`` that it is) take :func:`rows_linear` where its rule does. The model and its containers call their
+    children so, and the layers stay ``nn.Linear`` for whatever traces, compiles or replaces them. A short prompt's pass is
+    bound by the host, and the library's call costs it 19 µs against 4: GPT-2's pass over one prompt of 64 tokens
+    2.60 -> 1.71 ms, of 512 2.64 -> 1.79, Gemma 3 1B's over 3 of 200 7.6 -> 7.0."""
+    kind = type(mod)
+    if kind is torch.nn.Sequential:
+        if _ext.plain_call(x) and _bare(mod):
+            for m in mod:
+                x = apply(m, x)
+            return x
+    elif kind is torch.nn.Linear and _ext.plain_call(x) and x.dtype == torch.bfloat16 and x.dim() >= 2 and _bare(mod):
+        w, b = mod.weight, mod.bias
+        if type(w) is torch.nn.Parameter and (b is None or type(b) is torch.nn.Parameter):
+            y = rows_linear(x.reshape(-1, x.shape[-1]), w, b)
+            if y is not None:
+                return y.view(*x.shape[:-1], w.shape[0])
+    return mod(x)
 
 
 def linear_fp32(x: Tensor, w: Tensor) -> Tensor:
@@ -328,8 +341,8 @@ def skinny_qkv_rope(x: Tensor, w: Tensor, cos: Tensor, sin: Tensor, D: int, nrot
 
 
 class decode_gemms:
-    """Context: the ``nn.Linear`` modules of ``model`` run decode-shaped inputs that ``Linear`` itself leaves to the
-    library through the skinny kernel (others keep ``F.linear``). Entered by the graph decoder around the captured step of a
+    """Context: the ``nn.Linear`` modules of ``model`` run decode-shaped inputs that :func:`apply` leaves to them through the
+    skinny kernel (others keep ``F.linear``). Entered by the graph decoder around the captured step of a
     model without a decode program. Only that model's own Linear instances are re-routed (an
     instance-level ``forward``, removed on exit): other models, and other threads serving them,
     are untouched; the serving lock keeps concurrent requests off the same model."""
@@ -344,18 +357,16 @@ class decode_gemms:
             return self
         max_rows = self.max_rows
         for mod in self.model.modules():
-            if type(mod) not in (torch.nn.Linear, Linear) or "forward" in mod.__dict__:
+            if type(mod) is not torch.nn.Linear or "forward" in mod.__dict__:
                 continue
 
             def forward(x, mod=mod):
-                y = mod.rows(x) if type(mod) is Linear else None  # as outside of the capture
-                if y is not None:
-                    return y
                 if (x.numel() <= max_rows * x.shape[-1] and skinny_ok(x, mod.weight)
                         and (mod.bias is None or mod.bias.is_contiguous())):
                     return skinny_linear(x, mod.weight, mod.bias)
                 return torch.nn.functional.linear(x, mod.weight, mod.bias)
 
+            forward.of_decode_gemms = True
             mod.forward = forward
             self._patched.append(mod)
         return self

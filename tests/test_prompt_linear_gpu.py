@@ -3,9 +3,9 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from penroz.models import layers as L
 from penroz.ops import _ext
 from penroz.ops import gemm as gemm_ops
+from penroz.ops.gemm import apply
 
 pytestmark = pytest.mark.gpu
 BF = torch.bfloat16
@@ -13,7 +13,7 @@ BF = torch.bfloat16
 
 def _layer(K, N, bias, dtype=BF):
     torch.manual_seed(K + N)
-    lin = L.Linear(K, N, bias=bias).to("cuda", dtype)
+    lin = torch.nn.Linear(K, N, bias=bias).to("cuda", dtype)
     return lin
 
 
@@ -37,8 +37,8 @@ def test_prompt_products(shape, N, bias, taken):
     wide = torch.randn(*shape[:-1], 2 * shape[-1], device="cuda", dtype=BF)
     x = wide[..., :shape[-1]]  # rows of a wider buffer
     with torch.inference_mode():
-        y = lin(x)
-        t = lin(x.movedim(0, -2))  # leading axes that reshape has to copy
+        y = apply(lin, x)
+        t = apply(lin, x.movedim(0, -2))  # leading axes that reshape has to copy
     want = F.linear(x.double(), lin.weight.double(), lin.bias.double() if bias else None)
     mass = F.linear(x.double().abs(), lin.weight.double().abs(), lin.bias.double().abs() if bias else None)
     # one bf16 rounding of the result and K fp32 additions
@@ -52,19 +52,39 @@ def test_prompt_products(shape, N, bias, taken):
 def test_other_calls_keep_the_library(taken):
     lin = _layer(64, 96, True)
     x = torch.randn(4, 64, device="cuda", dtype=BF)
-    lin(x.requires_grad_()).sum().backward()
+    apply(lin, x.requires_grad_()).sum().backward()
     assert x.grad is not None and lin.weight.grad is not None
     with torch.no_grad():
-        lin(x)
+        apply(lin, x)
     with torch.inference_mode():
-        torch.func.vmap(lin)(x.detach()[None])
-        lin(x[0])
-        lin(x[:0])
-        lin.float()(x.float())
+        lin(x)  # the layer by itself
+        torch.func.vmap(lambda t: apply(lin, t))(x.detach()[None])
+        apply(lin, x[0])
+        apply(lin, x[:0])
+        apply(lin.float(), x.float())
         lin.to(BF)
         with torch.autocast("cuda", dtype=torch.float16):
-            assert lin(x).dtype == torch.float16
+            assert apply(lin, x).dtype == torch.float16
     assert taken == []
+
+
+def test_hooks_are_called(taken):
+    """A layer, or a sequence of layers, that does more than its class's forward is called as a module."""
+    seen = []
+    for hook in ("register_forward_hook", "register_forward_pre_hook"):
+        model = torch.nn.Sequential(_layer(64, 96, True))
+        x = torch.randn(4, 64, device="cuda", dtype=BF)
+        with torch.inference_mode():
+            for mod in (model[0], model):
+                handle = getattr(mod, hook)(lambda *a: seen.append(a[0]))
+                apply(model, x)
+                handle.remove()
+                assert seen.pop() is mod and not seen
+            assert taken == [True]  # the hooked sequence's own call reaches its layer without apply
+            taken.clear()
+    model[0].forward = lambda t: seen.append(t)
+    with torch.inference_mode():
+        assert apply(model, x) is None and len(seen) == 1 and taken == []
 
 
 @pytest.mark.parametrize("rows", [1, 5, 64])
@@ -72,9 +92,9 @@ def test_a_captured_step_takes_the_same_kernel(rows, taken):
     model = torch.nn.Sequential(_layer(128, 384, True), _layer(384, 128, False))
     x = torch.randn(rows, 1, 128, device="cuda", dtype=BF)
     with torch.inference_mode():
-        want = model(x)
+        want = apply(model, x)
         with gemm_ops.decode_gemms(model):
-            got = model(x)
+            got = apply(model, x)
     assert torch.equal(got, want) and taken == [True] * 4
 
 
