@@ -471,6 +471,12 @@ class GemmaDecodeProgram:
         return (1 <= rows <= min(4, GEMV_MAX_ROWS) and C % 8 == 0 and C <= 1792 and _ext.available()
                 and all(b["o"].shape[1] <= GEMV_MAX_K and b["down"].shape[1] <= GEMV_MAX_K for b in self.blocks))
 
+    def _norm_pair_ok(self) -> bool:
+        """decode_norm_pair reads the embedding's rows and the norms' weights 16 bytes at a time; views of other offsets
+        or strides take the kernels that step and product are by themselves."""
+        norms = [n for b in self.blocks for n in (b["in_norm"], b["post_attn"], b["pre_mlp"], b["post_mlp"]) if n is not None]
+        return all(m.weight.is_contiguous() and m.weight.data_ptr() % 16 == 0 for m in [self.emb, *norms])
+
     def forward(self, idx: Tensor, cache) -> Tensor:
         """idx [rows, 1] -> logits [rows, V] (bf16); appends this step's K/V at cache.pos_t."""
         K = _ext.kernels()
@@ -485,7 +491,7 @@ class GemmaDecodeProgram:
             return _linear(x, w)
 
         if gemv and DECODE_EPILOGUES and all(b["attn"].rope_theta is not None and b["attn"].head_dim % 2 == 0
-                                             for b in self.blocks):
+                                             for b in self.blocks) and self._norm_pair_ok():
             return self._forward_gemv(K, rows, idx, cache)
         x = torch.nn.functional.embedding(idx.view(rows), self.emb.weight) * self.emb.scale
         first = self.blocks[0]["in_norm"]
