@@ -219,7 +219,14 @@ class GPTDecodeProgram:
         sp = self.spec
         return (BATCHED_BLOCK and sp.C % 32 == 0 and sp.C <= 1024
                 and sp.blocks[0].fc.out_features % 32 == 0 and sp.gelu_approx in ("none", "tanh")
-                and _ext.available())
+                and (rows > FUSED_MAX_ROWS or self._whole()) and _ext.available())
+
+    def _whole(self) -> bool:
+        """decode_ln_gemm stores 4 outputs with their biases at a time, decode_gemm_acc reads its weight in pieces of 16 bytes
+        and its bias as it lies. Up to FUSED_MAX_ROWS rows the programs below take others too."""
+        return all(b.qkv.bias.data_ptr() % 8 == 0 and b.fc.bias.data_ptr() % 8 == 0
+                   and all(l.bias.is_contiguous() and l.weight.is_contiguous() and l.weight.data_ptr() % 16 == 0
+                           for l in (b.proj, b.fc2)) for b in self.spec.blocks)
 
     def forward(self, idx: Tensor, cache) -> Tensor:
         """idx [rows, 1] -> logits [rows, V] (bf16); appends this step's K/V at cache.pos_t."""
@@ -303,7 +310,7 @@ class GPTDecodeProgram:
 
 
     def _forward_gemv(self, x: Tensor, x2: Tensor, rows: int, cache, emb=None) -> Tensor:
-        """Widths off 32, batch 1-4, per block: [add + LN1 + QKV GEMV + bias] → decode attention (K/V append fused)
+        """Where ``_batched_ok`` does not hold, batch 1-4, per block: [add + LN1 + QKV GEMV + bias] → decode attention (K/V append fused)
         → proj GEMV → [add + proj bias + LN2 + fc GEMV + bias + GELU] → fc2 GEMV; then the final
         add + LN and the lm_head GEMV — every linear one decode_gemv launch. ``emb`` = (token ids,
         device position): the first GEMV builds the residual rows wte[tok] + wpe[pos] itself and

@@ -3,7 +3,7 @@ import pytest
 import torch
 
 from penroz.models import graph_decode as gd
-from test_graph_decode_gpu import _gemma_model
+from test_graph_decode_gpu import _gemma_model, _model
 
 pytestmark = pytest.mark.gpu
 
@@ -44,4 +44,28 @@ def test_gemma_norms_and_table(rows, what):
     got = _step(m, rows)
     # the same products behind the same norms, whose row sums run in another order in the kernel by itself: roundings of
     # the bf16 residual stream, as test_gemma_program_step_matches_module_step's bound has them
+    assert (got - want).norm() / want.norm() < 2e-2
+
+
+@pytest.mark.parametrize("rows,what", [(r, w) for r in (1, 4, 5, 8) for w in ("qkv", "fc", "proj", "fc2")] +
+                         [(r, w) for r in (5, 8) for w in ("proj.weight", "fc2.weight")])
+def test_gpt_biases_and_weights(rows, what):
+    m = _model(torch.bfloat16)
+    blocks = gd.GPTDecodeProgram.build(m).spec.blocks
+    for b in blocks:  # (they are zero at first)
+        for lin in (b.qkv, b.proj, b.fc, b.fc2):
+            torch.nn.init.normal_(lin.bias, std=0.1)
+    want = _step(m, rows)
+    for b in blocks:
+        lin = getattr(b, what.split(".")[0])
+        if what.endswith("weight"):
+            _shift(lin.weight)
+        elif what in ("qkv", "fc"):
+            _shift(lin.bias)
+        else:  # every second element of a longer one
+            view = torch.zeros(2 * lin.bias.numel(), device="cuda", dtype=torch.bfloat16)[::2]
+            view.copy_(lin.bias.data)
+            lin.bias.data = view
+    got = _step(m, rows)
+    # bf16 operands in sums of another order: test_decode_program_step_matches_module_step's bound
     assert (got - want).norm() / want.norm() < 2e-2
