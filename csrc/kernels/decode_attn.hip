@@ -433,8 +433,8 @@ __global__ void __launch_bounds__(256) decode_kernel(const TQ* __restrict__ q, c
 // ROPE is a template flag so the default instantiations compile exactly as without it (as a run-time
 // branch it cost the D = 512 kernels 320 B/lane of scratch).
 constexpr int kSmallWaves = 8;
-// GMAX: the heads of a workgroup; DC: its output columns
-template <int D, int GMAX, bool ROPE = false, int DC = 64>
+// GMAX: the heads of a workgroup; DC: its output columns; KLDS: keys through LDS
+template <int D, int GMAX, bool ROPE = false, int DC = 64, bool KLDS = (D >= 128)>
 __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf16* __restrict__ q, bf16* __restrict__ kc,
                                                            bf16* __restrict__ vc, bf16* __restrict__ out, int items, int log_rep,
                                                            int H, int Hkv, int cap, int S, float scale,
@@ -455,7 +455,6 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
   const int h0 = ((g << log_rep) + hs) * GMAX;  // of H / Hkv = GMAX << log_rep
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const int r16 = lane & 15, qd = lane >> 4;
-  constexpr bool KLDS = D >= 128;
   constexpr int CH = D / 8;                  // 16-byte chunks of a K row
   __shared__ __attribute__((aligned(16))) char kt[KLDS ? NW : 1][KLDS ? 32 * D : 16];  // a wave's 16 K rows, chunks permuted by row
   __shared__ float pl[NW][16][16];           // a wave's P block [key][head]
@@ -852,9 +851,12 @@ torch::Tensor decode_attn(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, c
   const float* vsp = quant ? v_scale->data_ptr<float>() : nullptr;
   auto stream = at::hip::getCurrentHIPStream();
   // small batches, bf16, one query row: the wave-parallel MFMA kernel (decode_small_kernel)
-  const bool small = !quant && q.scalar_type() == torch::kBFloat16 && decode_small_applies(B, Tq, H, Hkv, D, S) &&
-                     (!fuse || kv_rs % 8 == 0);
   const bool rope = rope_cos.has_value() && rope_cos->defined();
+  // LDS-DMA takes keys from 16-byte pieces: a cache that is a view off them is left to the general kernel, or read
+  // straight with the in-kernel RoPE that only this one has
+  const bool lines = D < 128 || reinterpret_cast<uintptr_t>(kc.data_ptr()) % 16 == 0;
+  const bool small = !quant && q.scalar_type() == torch::kBFloat16 && decode_small_applies(B, Tq, H, Hkv, D, S) &&
+                     (!fuse || kv_rs % 8 == 0) && (lines || rope);
   if (rope) {
     TORCH_CHECK(small && fuse && D <= 256, "in-kernel RoPE: the small decode kernel with the fused append, "
                 "head_dim <= 256 only (check decode_small_applies first)");
@@ -887,7 +889,7 @@ torch::Tensor decode_attn(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, c
                            (float)scale, sdev, q_rs, knp, vnp, kv_rs, rcp, rsp);
       };
       if constexpr (DD <= 256) {
-        if (rope) return go(decode_small_kernel<DD, GG, true, DC>);
+        if (rope) return lines ? go(decode_small_kernel<DD, GG, true, DC>) : go(decode_small_kernel<DD, GG, true, DC, false>);
       }
       go(decode_small_kernel<DD, GG, false, DC>);
     };

@@ -44,3 +44,40 @@ def test_decode_small(D, G, B, Hkv, S):
     assert torch.all((out.double() - ref).abs() <= bound), float(((out.double() - ref).abs() / bound).max())
     for t, f in zip((kc, vc), full):
         assert torch.equal(t.view(torch.int16), f.view(torch.int16)), "cache"
+
+
+@pytest.mark.parametrize("D,G,rope", [(128, 8, False), (128, 2, True), (256, 4, False), (256, 4, True), (512, 2, False)])
+@pytest.mark.parametrize("S", [1, 40, 200])
+def test_cache_off_16_bytes(D, G, rope, S):
+    """A cache that is a view at an odd offset: read without LDS-DMA, by another kernel or straight, the same answer."""
+    torch.manual_seed(D + G + S)
+    B, Hkv, cap = 2, 1, 256
+    H = G * Hkv
+
+    def cache():
+        return torch.randn(B * Hkv * cap * D + 1, device=DEV).to(torch.bfloat16)[1:].view(B, Hkv, cap, D)
+
+    kc, vc = cache(), cache()
+    qkv = torch.randn(B, 1, (H + 2 * Hkv) * D, device=DEV).to(torch.bfloat16)
+    q = qkv[:, :, :H * D].view(B, 1, H, D)
+    k, v = (qkv[:, :, (H + i * Hkv) * D:(H + (i + 1) * Hkv) * D].view(B, 1, Hkv, D) for i in (0, 1))
+    ang = torch.rand(D // 2, device=DEV) * 6
+    cos, sin = ang.cos(), ang.sin()
+
+    def turn(x):  # rotate-half in fp32, rounded to bf16 as the kernel keeps it
+        if not rope:
+            return x
+        a, b = x.float().split(D // 2, -1)
+        return torch.cat([a * cos - b * sin, b * cos + a * sin], -1).to(torch.bfloat16)
+
+    full = [t.clone() for t in (kc, vc)]
+    full[0][:, :, S - 1], full[1][:, :, S - 1] = turn(k)[:, 0], v[:, 0]
+    ref = _reference(turn(q)[:, 0], full[0][:, :, :S], full[1][:, :, :S], D ** -0.5).view(B, 1, H * D)
+    out = _ext.kernels().decode_attn(q, kc, vc, None, None, cap, cap - 1, D ** -0.5, torch.tensor([S], device=DEV), k, v, None,
+                                     *((cos, sin) if rope else (None, None)))
+    # as above; a fused multiply-add in the rotation may round a query or the new key to its other neighbour: 2^-9 of each of D
+    # products of a score, whose spread is 1
+    bound = 2.0 ** -8 * ref.abs() + (2.0 ** -5 if rope else 2.0 ** -14)
+    assert torch.all((out.double() - ref).abs() <= bound), float(((out.double() - ref).abs() / bound).max())
+    assert torch.equal(vc, full[1]) and torch.equal(kc[:, :, :S - 1], full[0][:, :, :S - 1]) and torch.equal(kc[:, :, S:], full[0][:, :, S:])
+    assert torch.all((kc[:, :, S - 1].float() - full[0][:, :, S - 1].float()).abs() <= 2.0 ** -7 * full[0][:, :, S - 1].float().abs() + 2.0 ** -14)
