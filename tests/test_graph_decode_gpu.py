@@ -100,10 +100,12 @@ def test_decode_program_graph_replay_matches_eager_program(monkeypatch, rows):
     assert graphed == eager
 
 
+@pytest.mark.parametrize("batched", [True, False])
 @pytest.mark.parametrize("rows", [1, 3, 6, 24, 64])
-def test_decode_program_step_matches_module_step(rows):
-    """One decode-program step vs the module forward: rows 1 and 3 run the decode GEMV path, 6 the
-    fused LN-linear path, 24 and 64 the batched block (decode_ln_gemm / decode_gemm_acc)."""
+def test_decode_program_step_matches_module_step(monkeypatch, rows, batched):
+    """One decode-program step vs the module forward: the block of 5 kernels (decode_ln_gemm / decode_gemm_acc); without
+    it rows 1 and 3 run decode_gemv throughout, 6 decode_ln_linear, 24 and 64 separate norms, products and GELU."""
+    monkeypatch.setattr(gd, "BATCHED_BLOCK", batched)
     m = _model(torch.bfloat16)
     cap = 32
     dec = gd.GraphDecoder(m, rows, cap, 0.0, None)

@@ -9,8 +9,8 @@ DEV = "cuda"
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("E,top", [(1, 1), (16, 16), (17, 3), (33, 4), (48, 48), (63, 6), (64, 6), (64, 64), (79, 5), (80, 6)])
-@pytest.mark.parametrize("C,gate", [(8, False), (520, True), (2048, True), (2056, False), (4104, True)])
+@pytest.mark.parametrize("E,top", [(1, 1), (16, 16), (17, 3), (33, 4), (48, 48), (63, 6), (64, 6), (64, 64), (79, 5), (80, 6), (129, 7)])
+@pytest.mark.parametrize("C,gate", [(8, False), (520, True), (2048, True), (2056, False), (4104, True), (1023, False)])
 def test_router_rounds(dt, E, top, C, gate):
     torch.manual_seed(E + C)
     h = torch.randn(3, C, device=DEV).to(dt)
