@@ -145,7 +145,8 @@ __device__ __forceinline__ Piece<T, V> piece(const T* p) {
 // The same row with one 4-channel vector per thread (C <= 4096, parts of a multiple of 4): everything the
 // row needs is loaded, and the state's share of the convolution summed, before the norm's barrier. As in residual_norm_kernel the
 // loads are issued before any is waited for, the expert rows KT at a time, the state's 3; KT and CONV are
-// template arguments for the registers that the simpler forms save (plain rows would lose 9 % to them). Rows of 2048, one load waited
+// template arguments for the registers that the simpler forms save (plain rows would lose 9 % to them; with the convolution, KT 8
+// leaves one workgroup of 1024 threads per CU: 512 x 4096, 6 experts, one tap 14.4 us, KT 4 12.6). Rows of 2048, one load waited
 // for at a time / here, us: 64 rows of 6 experts with the convolution 6.1 / 5.2, 8192 of 6 experts 69 / 59 (5.3 TB/s), 8192 plain
 // 33.4 / 32.5; 2000 rows of 1024, 4 experts 8.6 / 7.9.
 template <typename T, int KT, bool CONV>
@@ -496,9 +497,11 @@ __device__ __forceinline__ float2 block_sum2(float a, float b, float2* red) {
 
 // V channels per thread and pass, I passes: blockDim.x · V · I >= C. A decode step's few rows are bound by the chain of memory trips,
 // so every load that does not follow from another is issued before the first is waited for: the norm weights ahead of the sums
-// that they scale, the expert rows 8 (or 4) at a time. Rows of 2048, one load waited for at a time / here, us: 16 rows of 6 experts and a shared one
-// 4.2 / 3.8, 64 of them 4.9 / 4.0, 8192 of them 78 / 64 (4.9 TB/s); 16 of two normed outputs 3.8 / 3.5, 4096 of them 26 / 24.
-template <typename T, int V, int I>
+// that they scale, the expert rows up to KM at a time. Rows of 2048, one load waited for at a time / here, us: 16 rows of 6 experts and a shared one
+// 4.2 / 3.8, 64 of them 4.9 / 4.0, 8192 of them 78 / 64 (4.9 TB/s); 16 of two normed outputs 3.8 / 3.5, 4096 of them 26 / 24. One or two
+// experts' rows are not read as four (one expert, 512 x 2048: 6.4 us, here 5.9). KM 4 for fp32 rows of more than 2048 values, whose
+// 1024 threads are the only workgroup of a CU with the registers of KM 8 (two normed outputs, 4096 x 4096: 92 us, here 68).
+template <typename T, int V, int I, int KM>
 __global__ void __launch_bounds__(1024) residual_norm_kernel(ResidualArgs<T> a) {
   __shared__ float2 red[2][16];
   const int row = blockIdx.x, t = threadIdx.x, C = a.C;
@@ -573,7 +576,9 @@ __global__ void __launch_bounds__(1024) residual_norm_kernel(ResidualArgs<T> a) 
             for (int k = 0; k < KT; ++k) add(wk[k], r[k], k0 + k < a.top);
           }
         };
-        if (I > 1 || a.top <= 4) rows(std::integral_constant<int, 4>{});
+        if (a.top == 1) rows(std::integral_constant<int, 1>{});
+        else if (a.top == 2) rows(std::integral_constant<int, 2>{});
+        else if (KM == 4 || a.top <= 4) rows(std::integral_constant<int, 4>{});
         else rows(std::integral_constant<int, 8>{});
         add(ws, rs, a.ys != nullptr);
       } else {
@@ -743,8 +748,10 @@ void row_norm_add(c10::optional<torch::Tensor> tok, c10::optional<torch::Tensor>
       constexpr int KT = decltype(kt)::value;
       cw.has_value() ? run(row_norm_add4_kernel<T, KT, true>, wide, 0) : run(row_norm_add4_kernel<T, KT, false>, wide, 0);
     };
+    // a single expert's row is not read as four (1 x 4096: 3.5 us, so 3.1); rows of more than 512 threads: see the kernel's registers
     if (vec && !(y.has_value() && pw.has_value() && top > 0)) conv(std::integral_constant<int, 0>{});
-    else if (vec && top <= 4) conv(std::integral_constant<int, 4>{});
+    else if (vec && top == 1) conv(std::integral_constant<int, 1>{});
+    else if (vec && (top <= 4 || (C > 2048 && cw.has_value()))) conv(std::integral_constant<int, 4>{});
     else if (vec) conv(std::integral_constant<int, 8>{});
     else run(row_norm_add_kernel<T>, kPrThreads, lds);
   });
@@ -939,13 +946,11 @@ void residual_norm(c10::optional<torch::Tensor> tok, c10::optional<torch::Tensor
                       (const float*)ptr(wa), (const float*)ptr(wb), (float)coef, (float)yeps, (const float*)ptr(pw),
                       (int)top, (int)pws, (const T*)ptr(ys), (const float*)ptr(nw), (float)eps, (int*)ptr(pos),
                       advance ? 1 : 0, (T*)ptr(h), (int)C};
-    auto run = [&](auto v, auto i) {
-      hipLaunchKernelGGL((residual_norm_kernel<T, decltype(v)::value, decltype(i)::value>), dim3(N), dim3(threads), 0,
-                         at::hip::getCurrentHIPStream(), a);
-    };
-    using I1 = std::integral_constant<int, 1>;
-    using I4 = std::integral_constant<int, 4>;
-    if (vec) groups <= 1024 ? run(I4{}, I1{}) : run(I4{}, I4{});
-    else groups <= 1024 ? run(I1{}, I1{}) : run(I1{}, I4{});
+    auto run = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(N), dim3(threads), 0, at::hip::getCurrentHIPStream(), a); };
+    if (vec && groups > 1024) run(residual_norm_kernel<T, 4, 4, 4>);
+    else if (vec && sizeof(T) == 4 && groups > 512) run(residual_norm_kernel<T, 4, 1, 4>);
+    else if (vec) run(residual_norm_kernel<T, 4, 1, 8>);
+    else if (groups <= 1024) run(residual_norm_kernel<T, 1, 1, 8>);
+    else run(residual_norm_kernel<T, 1, 4, 4>);
   });
 }

@@ -7,8 +7,8 @@ from penroz.ops import _ext
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("top", [1, 4, 5, 8, 9, 17])
-@pytest.mark.parametrize("C", [7, 100, 2048, 4100])
+@pytest.mark.parametrize("top", [1, 2, 3, 4, 5, 8, 9, 17])
+@pytest.mark.parametrize("C", [7, 100, 2048, 2052, 4096, 4100])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("shared", [False, True])
 def test_weighted_rows(top, C, dt, shared):
@@ -34,7 +34,7 @@ def test_weighted_rows(top, C, dt, shared):
 
 @pytest.mark.parametrize("top", [0, 1, 4, 5, 9])  # 0: one plain row
 @pytest.mark.parametrize("taps", [0, 1, 2, 4, 5, 16])
-@pytest.mark.parametrize("C,dt", [(96, torch.bfloat16), (2048, torch.bfloat16), (4096, torch.float32)])
+@pytest.mark.parametrize("C,dt", [(96, torch.bfloat16), (2048, torch.bfloat16), (4096, torch.float32), (2056, torch.bfloat16)])
 def test_rows_with_a_convolution(top, taps, C, dt):
     g = torch.Generator(device="cuda").manual_seed(top * C + taps)
     N, groups, eps = 4, 2, 1e-5
