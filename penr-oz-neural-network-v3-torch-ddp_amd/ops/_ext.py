@@ -84,12 +84,17 @@ def use_kernels(*tensors) -> bool:
     return False
 
 
-def plain_call(x) -> bool:
-    """Nothing but the value is asked of an op on ``x``: inference mode (no backward, no tangents), no trace, transform, mode or
-    autocast that has to see the operators themselves, a GPU tensor of no subclass that holds something, on the current device
-    (the kernels start there, whatever device their operands are on)."""
+def plain_mode() -> bool:
+    """Nothing but values is asked of ops: inference mode (no backward, no tangents), no trace, transform, mode or autocast
+    that has to see the operators themselves."""
     return (not torch.compiler.is_compiling()  # first: a compiler's trace cannot ask for the others
-            and torch.is_inference_mode_enabled() and type(x) is torch.Tensor and x.is_cuda and x.numel() > 0
-            and x.get_device() == torch.cuda.current_device() and not torch.is_autocast_enabled("cuda")
+            and torch.is_inference_mode_enabled() and not torch.is_autocast_enabled("cuda")
             and torch._C._get_tracing_state() is None and torch._C._functorch.peek_interpreter_stack() is None
-            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0 and use_kernels(x))
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0 and not FORCE_TORCH)
+
+
+def plain_call(x) -> bool:
+    """:func:`plain_mode`, and ``x`` is a GPU tensor of no subclass that holds something, on the current device (the kernels
+    start there, whatever device their operands are on)."""
+    return (plain_mode() and type(x) is torch.Tensor and x.is_cuda and x.numel() > 0
+            and x.get_device() == torch._C._cuda_getDevice())

@@ -135,12 +135,18 @@ def train_linear(x: Tensor, w: Tensor, bias: Tensor | None = None, out: Tensor |
     return torch.mm(x, w.t(), out=out) if bias is None else torch.addmm(bias, x, w.t(), out=out)
 
 
+def _rows_sized(M: int, N: int, K: int) -> bool:
+    """``rows_gemm_plan`` (``csrc/kernels/host_plan.h``) may have a tile for these sizes: what it certainly leaves to the library
+    is not asked for, at 5 µs of the host a layer."""
+    n = M * N
+    return n <= 1 << 19 or (n <= 1 << 22 and K <= 1024) or (K <= 2048 and (n <= 1 << 20 or (M <= 64 and n <= 1 << 22)))
+
+
 def _bare(mod: torch.nn.Module) -> bool:
     """A call of ``mod`` is its class's forward and nothing else: no hooks, no forward of its own (but for ``decode_gemms``'s)."""
     f = mod.__dict__.get("forward")
     return ((f is None or getattr(f, "of_decode_gemms", False)) and mod._compiled_call_impl is None
-            and not (mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks
-                     or torch.nn.modules.module._has_any_global_hook()))
+            and not (mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks))
 
 
 def apply(mod: torch.nn.Module, x: Tensor) -> Tensor:
@@ -150,17 +156,28 @@ def apply(mod: torch.nn.Module, x: Tensor) -> Tensor:
     bound by the host, and the library's call costs it 19 µs against 4: GPT-2's pass over one prompt of 64 tokens
     2.60 -> 1.71 ms, of 512 2.64 -> 1.79, Gemma 3 1B's over 3 of 200 7.6 -> 7.0."""
     kind = type(mod)
-    if kind is torch.nn.Sequential:
-        if _ext.plain_call(x) and _bare(mod):
-            for m in mod:
-                x = apply(m, x)
-            return x
-    elif kind is torch.nn.Linear and _ext.plain_call(x) and x.dtype == torch.bfloat16 and x.dim() >= 2 and _bare(mod):
-        w, b = mod.weight, mod.bias
-        if type(w) is torch.nn.Parameter and (b is None or type(b) is torch.nn.Parameter):
-            y = rows_linear(x.reshape(-1, x.shape[-1]), w, b)
-            if y is not None:
-                return y.view(*x.shape[:-1], w.shape[0])
+    if ((kind is torch.nn.Sequential or kind is torch.nn.Linear) and _ext.plain_call(x)
+            and not torch.nn.modules.module._has_any_global_hook()):
+        return _apply(mod, x, x.get_device())
+    return mod(x)
+
+
+def _apply(mod: torch.nn.Module, x: Tensor, device: int) -> Tensor:
+    """:func:`apply` where its call is plain: a child leaves the modes as it found them, so they are asked for once."""
+    kind = type(mod)
+    if kind is torch.nn.Linear:
+        if (type(x) is Tensor and x.dtype == torch.bfloat16 and x.get_device() == device and x.dim() >= 2 and x.numel() > 0
+                and _bare(mod)):
+            w, b, K = mod.weight, mod.bias, x.shape[-1]
+            if (type(w) is torch.nn.Parameter and (b is None or type(b) is torch.nn.Parameter)
+                    and _rows_sized(x.numel() // K, w.shape[0], K)):
+                y = rows_linear(x.reshape(-1, K), w, b)
+                if y is not None:
+                    return y.view(*x.shape[:-1], w.shape[0])
+    elif kind is torch.nn.Sequential and _bare(mod):
+        for m in mod:
+            x = _apply(m, x, device)
+        return x
     return mod(x)
 
 

@@ -81,3 +81,15 @@ def test_attn_work_plan_off_and_many_rounds(monkeypatch):
     assert _ext.kernels().attn_work_plan(8, 768, 256, 128, 32, 1024, 256, 2.7)[:2] == [8, 8]
     r = _ext.kernels().attn_work_plan(8, 32, 256, 128, 32, 1024, 256, 2.7)
     assert r[1] < 8  # the Gemma-3 1B B=8 forward grid (one round) is split
+
+
+def test_sizes_not_tried_by_rows_gemm_have_no_tile():
+    """gemm.apply skips the call for sizes that rows_gemm_plan certainly leaves to the library: never for one that has a tile."""
+    import random
+    r, k, skipped = random.Random(1), _ext.kernels(), 0
+    for _ in range(20000):
+        M, N, K = int(2 ** r.uniform(0, 12)), int(2 ** r.uniform(3, 17)), 8 * int(2 ** r.uniform(0, 10.5))
+        if not G._rows_sized(M, N, K):
+            skipped += 1
+            assert k.rows_gemm_tile(M, N, K, False) == 0, (M, N, K)
+    assert skipped > 2000

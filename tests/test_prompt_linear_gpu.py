@@ -46,7 +46,7 @@ def test_prompt_products(shape, N, bias, taken):
     assert y.shape == (*shape[:-1], N) and y.dtype == BF
     assert ((y.double() - want).abs() <= bound).all()
     assert ((t.double() - want.movedim(0, -2)).abs() <= bound.movedim(0, -2)).all()
-    assert len(taken) == 2 and (N == 50304 or taken[0])
+    assert True not in taken if N == 50304 else len(taken) == 2 and taken[0]
 
 
 def test_other_calls_keep_the_library(taken):
@@ -105,5 +105,5 @@ def test_an_input_on_another_device_is_the_librarys(monkeypatch):
     x = torch.randn(4, 64, device="cuda", dtype=BF)
     with torch.inference_mode():
         assert _ext.plain_call(x)
-        monkeypatch.setattr(torch.cuda, "current_device", lambda: x.get_device() + 1)
+        monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: x.get_device() + 1)
         assert not _ext.plain_call(x)
