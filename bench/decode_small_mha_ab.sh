@@ -1,5 +1,5 @@
 # GPT-2 graph decode: MHA head_dim-64 attention through the kernel for few heads and short contexts
-# (PENROZ_DECODE_SMALL_ITEMS=1024: 192 and 768 items, beyond its default of 64) vs the general kernel
+# (PENROZ_DECODE_SMALL_ITEMS=1024: 192 and 768 items, what runs by default) vs the general kernel
 # (PENROZ_DECODE_SMALL_ITEMS=0); batch 16 / 64, same box, 2 passes.
 set -o pipefail
 export TMPDIR=/tmp PYTHONUNBUFFERED=1

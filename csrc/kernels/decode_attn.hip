@@ -418,7 +418,7 @@ __global__ void __launch_bounds__(256) decode_kernel(const TQ* __restrict__ q, c
 // waves and V over D / 64 workgroups, whose K rows meet in the L2 of one XCD (they are 8 apart in
 // the grid). A fragment's lanes lie a row apart, and read straight from memory each of a row's pieces costs a cache line: 16 bytes a
 // clock, 120 KB of keys in 3 us. From D = 128 on (KLDS) the keys come by LDS-DMA instead, whole lines, into the wave's own 16 rows,
-// and are read from there. The heads of a group go to workgroups of their own while those are no more than half the CUs: less to
+// and are read from there (a cache off 16 bytes is not: `lines` below). The heads of a group go to workgroups of their own while those are no more than half the CUs: less to
 // do one after the other. us at a 1024-slot cache, D = 256, G = 4: 3 items, 40 / 232 / 1000 keys 4.0 / 7.6 / 20.0 before, 4.3 /
 // 6.5 / 14.5 with the keys in LDS, 3.6 / 5.9 / 13.0 with single heads as well; 16 items 4.1 / 7.8 / 21.2 before, 4.2 / 6.3 / 15.7 with
 // pairs of heads (single ones, 256 workgroups: 4.2 / 6.5 / 15.9); 64 items 4.4 / 8.2 / 22.8 before, 4.6 / 7.2 / 19.1 with all four.
@@ -568,7 +568,7 @@ __global__ void __launch_bounds__(64 * kSmallWaves) decode_small_kernel(const bf
   if (k0 < k1) load_block(k0);
   for (int kb = k0; kb < k1; kb += 16) {
     if constexpr (KLDS) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * CL) : "memory");  // the keys; the values behind them may be on the way
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * CL) : "memory");  // the keys: the values' loads stand behind theirs
 #pragma unroll
       for (int s2 = 0; s2 < KS; ++s2)
         kf[s2] = *reinterpret_cast<const uint4*>(kt[w] + r16 * 2 * D + (((4 * s2 + qd) ^ r16) << 4));
@@ -766,8 +766,11 @@ bool decode_small_applies(int64_t B, int64_t Tq, int64_t H, int64_t Hkv, int64_t
   // 27.9, 1024 items 7.3 / 5.9, 12.7 / 12.4, 30.4 / 28.7, 55.8 / 50.5; D = 128, G = 1, 512 items 6.6 / 6.0, 14.0 / 12.1, 33 / 28, 59
   // / 49, G = 8 13.8 / 14.4, 26.7 / 24.1, 51 / 41, 93 / 64; D = 256, G = 4, 256 items 13.7 / 14.4, 36.5 / 23.2, 64 / 42, 98 / 69, 512 items
   // 14.3 / 27.4, 41 / 47, 80 / 77, 148 / 131, G = 1, 512 items 9.1 / 13.7, 29.4 / 30.3, 61 / 62, 108 / 117, G = 2 23 / 15, 80 / 31, 171 /
-  // 64, 331 / 117; D = 512, G = 1, 1024 items 68 / 65, 235 / 134, 537 / 276, 1049 / 470. At 40 keys and 64 items or fewer the
-  // keys' way through LDS is 0.1 to 0.3 us slower than straight reads (D = 128, G = 1, 64 items 3.3, here 3.5; D = 256 3.8, 4.1).
+  // 64, 331 / 117; D = 512, G = 1, 1024 items 68 / 65, 235 / 134, 537 / 276, 1049 / 470. Below 64 keys
+  // their way through LDS is slower than straight reads (16 / 40 / 64 keys, straight and here: D = 128, G = 1, 64 items 3.1, 3.6, 4.0 and
+  // 3.3, 3.7, 4.0; D = 256, G = 4, 64 items 4.1, 4.7, 5.1 and 4.5, 5.0, 5.1; D = 512, G = 1, 4 items 3.8, 4.6, 5.1 and 4.5, 4.6, 4.7). The length
+  // is on the device; a second path in the kernel for fewer than 48 keys gained 0.3 us at 16, nothing at 40, and its registers cost
+  // 0.05 us from 64 keys on and 0.25 at 1000 (D = 128, 512 items 14.5 -> 16.4 at 200).
   const int64_t small_keys = split_keys_env ? split_keys_env : 1024;
   const int64_t most = small_items >= 0 ? small_items : D == 256 && (G0 == 1 || G0 == 4 || G0 == 8) ? 256 : INT64_MAX;
   return Tq == 1 && B * Hkv <= most && S <= small_keys &&

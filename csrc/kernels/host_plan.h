@@ -128,7 +128,7 @@ inline int plan_wgrad_group(const int* M, const int* N, int n, int K, int n_cu, 
 // tiles of 256 read less. M x N x K, here / library, us:
 //   * 6 64 x 768 x 3072 5.5 (1: 7.4) / 9.8, 16 x 2048 x 2048 4.6 (1: 5.7) / 8.1. One block beyond its round 1 is faster than two
 //     rounds of it: 64 x 1152 x 6912 17.3 (6: 18.1) / 20.0, 64 x 1152 x 1024 4.3 (6: 5.6) / 8.4, 96 x 768 x 3072 7.3 (6: 9.3) /
-//     7.6, 96 x 1152 x 6912 17.2 / 17.1 (rows_gemm_narrow's tile of 32×16: 13.5, 4.5, 7.5 and 13.4).
+//     7.6, 96 x 1152 x 6912 17.2 / 17.1 (32×32 each; rows_gemm_narrow's tile has these products now).
 //   * 1 in order 256 x 1536 x 1024 5.8 / 8.6; 2 64 x 8192 x 2048 11.3 / 13.3, 256 x 1152 x 6912 23.9 / 24.2
 //   * 3 beyond K = 2048 is 5 to 9 % slower than the library (256 x 12288 x 2048 35 / 27); 256 x 3072 x 2048 12.5 / 12.9, 400 x 1536 x
 //     1152 8.0 / 9.6, but 400 x 2048 x 2048 11.9 / 11.0 and 1024 x 576 x 2048 11.9 / 10.5, at a fifth of its host time
@@ -149,9 +149,9 @@ inline int rows_gemm_plan(int64_t M, int64_t N, int64_t K, bool in_order) {
 }
 
 // Tile 1 with split columns is 32×16 where one round holds that: the same sums in the same order, but more CUs, of which each takes
-// some 22 B a cycle whatever the tile. us, 32×32 / 32×16, weights from memory: 64 x 2048 x 6144 16.8 / 13.3, 64 x 2048 x 2048 7.1 /
-// 6.4, 64 x 1152 x 6912 17.8 / 13.5, 32 x 4096 x 2048 7.8 / 7.5, 256 x 512 x 2048 5.8 / 5.4, 65 x 832 x 768 3.7 / 3.6; two rounds of
-// it are slower (64 x 3648 x 2048 7.7 / 11.3), and so is 16×8 in place of 16×16 (16 x 2048 x 2048 5.2 / 5.5).
+// some 22 B a cycle whatever the tile. us, 32×32 / 32×16, weights from memory, both in turn: 64 x 2048 x 6912 18.5 / 14.5, 64 x 2048 x
+// 2048 7.1 / 6.4, 64 x 1152 x 6912 17.7 / 13.5, 64 x 1152 x 1024 4.9 / 4.6, 96 x 768 x 3072 9.2 / 7.5, 32 x 4096 x 2048 7.8 / 7.0, 256 x
+// 512 x 2048 6.7 / 5.9, 65 x 832 x 768 4.1 / 3.8; of 256 columns the same (3.1). Two rounds of it are slower (64 x 3648 x 2048 7.7 / 11.3), and so is 16×8 in place of 16×16 (16 x 2048 x 2048 5.2 / 5.5).
 inline bool rows_gemm_narrow(int64_t M, int64_t N) { return ((M + 31) / 32) * ((N + 15) / 16) <= 256; }
 
 // Slices of the deterministic column reduction (reduce.h): ~sqrt(G) balances its two steps.

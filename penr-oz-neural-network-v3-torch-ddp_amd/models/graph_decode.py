@@ -22,8 +22,8 @@ replayed. Everything that changes between steps lives on the device:
   non-streaming calls therefore draw identical tokens under the same ``torch.manual_seed``;
 * the step's ``nn.Linear`` GEMMs (M = rows ≤ 64) run on the decode-shaped MFMA kernel
   (``csrc/kernels/skinny_gemm.hip``): called explicitly by the decode programs, or — for the
-  module-forward fallback — through ``ops/gemm.py: decode_gemms(model)``, which re-routes only
-  that model's own ``nn.Linear`` instances for the capture.
+  module-forward fallback — through ``ops/gemm.py: apply`` and ``decode_gemms(model)``, which re-routes
+  only that model's own ``nn.Linear`` instances for the capture.
 
 The host only tracks the cache length (one per replay) to switch to the reference's
 sliding-window re-prefill when the window is full, and copies each burst of tokens back once
@@ -67,12 +67,14 @@ SKINNY_MAX_ROWS = int(os.environ.get("PENROZ_SKINNY_MAX_ROWS", "16"))
 # Gemma program: RoPE and the gated activation in the skinny GEMM epilogues ("1", default) or the
 # separate RoPE / packed-activation kernels after plain skinny GEMMs ("0": same-box A/B switch)
 DECODE_EPILOGUES = os.environ.get("PENROZ_DECODE_EPILOGUES", "1") != "0"
-# GPT decode program, widths that are multiples of 32: 5 kernels per block (csrc/kernels/decode_linear.hip), the fp32
+# GPT decode program, widths up to 1024 that are multiples of 32: 5 kernels per block (csrc/kernels/decode_linear.hip), the fp32
 # residual updated in place by the proj / fc2 epilogues, LayerNorm computed inside the QKV / fc products. Greedy
 # generation at 2 / 4 / 8 rows, against the residual carried along as a second operand (the two programs below):
-# 21.5 / 28.4 / 31.3 -> 17.2 / 18.2 / 23.3 ms for 64 tokens. "0": the programs below, above 8 rows 8 kernels per block
+# 21.5 / 28.4 / 31.3 -> 17.2 / 18.2 / 23.3 ms for 64 tokens. "0", and wider models: 8 kernels per block, but up to 8
+# rows (as with parameters that are views off the kernels' alignment) the two programs below, of up to 1024 columns too
 BATCHED_BLOCK = os.environ.get("PENROZ_DECODE_BATCHED", "1") != "0"
-# ... else up to this many rows every linear of the block as decode_gemv; "0": decode_ln_linear + skinny GEMMs
+# ... up to this many rows (at most 4) every linear of the block as decode_gemv; also Gemma's steps of that many rows, whose
+# products are then decode_gemv and decode_gemv_pair ("0": the skinny kernels)
 GEMV_MAX_ROWS = int(os.environ.get("PENROZ_DECODE_GEMV_MAX_ROWS", "4"))
 # ... and up to FUSED_MAX_ROWS the residual add + LayerNorm in front of the QKV and fc GEMMs (and GELU behind fc) in one
 # kernel (csrc/kernels/skinny_gemm.hip decode_ln_linear), whose workgroups all normalise every row: it loses from 16
@@ -310,9 +312,9 @@ class GPTDecodeProgram:
 
 
     def _forward_gemv(self, x: Tensor, x2: Tensor, rows: int, cache, emb=None) -> Tensor:
-        """Where ``_batched_ok`` does not hold, batch 1-4, per block: [add + LN1 + QKV GEMV + bias] → decode attention (K/V append fused)
-        → proj GEMV → [add + proj bias + LN2 + fc GEMV + bias + GELU] → fc2 GEMV; then the final
-        add + LN and the lm_head GEMV — every linear one decode_gemv launch. ``emb`` = (token ids,
+        """Where ``_batched_ok`` does not hold, batch 1-4, per block: [add + LN1 + QKV GEMV + bias] → decode attention
+        (K/V append fused) → proj GEMV → [add + proj bias + LN2 + fc GEMV + bias + GELU] → fc2 GEMV; then the
+        final add + LN and the lm_head GEMV — every linear one decode_gemv launch. ``emb`` = (token ids,
         device position): the first GEMV builds the residual rows wte[tok] + wpe[pos] itself and
         writes them to ``x`` (one kernel less per token)."""
         sp = self.spec
@@ -470,9 +472,8 @@ class GemmaDecodeProgram:
         return GemmaDecodeProgram(mods[0], mods[1:-2], mods[-2], mods[-1])
 
     def _gemv_ok(self, rows: int, C: int) -> bool:
-        """Batch 1-4: every projection as one decode GEMV (decode_gemv / decode_gemv_pair:
-        one wave per workgroup, one memory round trip; RoPE and the gated activation in the
-        paired-row epilogues)."""
+        """Batch 1-4: every projection as one decode GEMV (decode_gemv / decode_gemv_pair: every load of
+        a workgroup in flight at once; RoPE and the gated activation in the paired-row epilogues)."""
         # decode_gemv reads K <= 8192 (decode_linear.hip); the O and down projections read K = H·D
         # and the intermediate size (12288 on Gemma-4 e2b's KV-shared double-wide MLPs)
         return (1 <= rows <= min(4, GEMV_MAX_ROWS) and C % 8 == 0 and C <= 1792 and _ext.available()
