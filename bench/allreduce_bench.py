@@ -7,7 +7,7 @@ Like ``bench.py`` it launches one rank per GPU itself (parent never touches the 
 launcher already set ``WORLD_SIZE``. Each point: W warm-up + K timed in-place AVG all-reduces of
 one bucket, bracketed by barrier + synchronize, max over ranks. Reported per point:
 ``ms``, ``algbw_GBps`` = bucket bytes / time, ``busbw_GBps`` = algbw · 2(n-1)/n (the per-rank
-link traffic of a ring; compare against 7 xGMI links × ≈153 GB/s per MI355X, SURVEY §2.6).
+link traffic of a ring; compare against 7 xGMI links × ≈153 GB/s per MI355X).
 Transports: ``c10d`` (torch ProcessGroupNCCL = RCCL) and ``native`` (``csrc/comm/rccl_comm.cpp``).
 Also prints the bucket plan the executor would use for GPT-2 124M (652 MB of fp32 gradients)
 and GPT-2 XL (6.55 GB) at the default bucket size, so the sweep can be read against it.

@@ -1,4 +1,4 @@
-# Decode at long contexts (ADVICE r5: the unsplit small kernel / the 1024-key split rule were only
+# Decode at long contexts (the unsplit small kernel / the 1024-key split rule were only
 # measured at prompt 64): default rules vs PENROZ_DECODE_MERGE=0 (no in-launch merge: the combine
 # launch and the 1024-key split rule), two passes. Writes gpurun_out/longctx.log.
 set -e

@@ -106,7 +106,7 @@ template <int D> constexpr int fwd_waves() { return D >= 256 ? 8 : 2; }
 //   version spilled ~90 B per lane and ran fwd at 195 TF);
 //   dQ: the same (8 waves, quarters of Q, dO; partial S, then partial dP exchanged);
 //   dK / dV: fa_roles_bwd_dkdv_kernel below (S-wave / dP-wave roles, every D).
-// (The round-4 design recomputed S over the full D in every column part — forward 2×, dQ 2×,
+// (An earlier design recomputed S over the full D in every column part — forward 2×, dQ 2×,
 // dK / dV 4× — and still spilled 350-560 B per lane: 106 / 64 TF fwd / bwd, slower than SDPA.)
 template <int D> constexpr int fwd_dsplit() { return D >= 512 ? 4 : (D >= 256 ? 2 : 1); }
 template <int D> constexpr int dq_dsplit() { return D >= 512 ? 4 : (D >= 256 ? 2 : 1); }
@@ -375,11 +375,11 @@ __global__ void __launch_bounds__(256) fa_gen_bwd_pre_kernel(const bf16* __restr
 // dKᵀ. Per 32-row query slice the S-wave computes S and P and hands P (fp32) to its dP-wave through
 // LDS; the dP-wave forms dS = P ⊙ (dP − δ). Each wave then runs 32 MFMAs of S or dP and 32 of dV or
 // dK. D = 128 / 256: 32 / 64 operand + 64 / 128 accumulator registers, 3 / 2 waves per SIMD, no
-// recomputation (the round-4 kernel held K and V in every wave and computed both S and dP —
+// recomputation (the earlier kernel held K and V in every wave and computed both S and dP —
 // at D = 256 in both column halves of two workgroups: D = 128 bwd 1855 -> 1502 µs, D = 256
 // 227 -> 177 µs). D = 512: the dVᵀ / dKᵀ columns are split over kv_role_parts = 2 workgroups
 // (virtual heads) — a wave's 256 accumulators for all of D beside its 128 operand registers
-// spilled ~800 B — so S and dP are computed twice (the round-4 kernel: four times).
+// spilled ~800 B — so S and dP are computed twice (the earlier kernel: four times).
 // Query-head split (part != nullptr): each workgroup sweeps ONE query head of its group and writes
 // fp32 partial dK / dV ([G][B·T][K | V][Hkv·D]) that fa_gen_kv_reduce sums (Gemma-3 1B: Hkv = 1).
 template <int D> constexpr int kv_role_parts() { return D >= 512 ? 2 : 1; }

@@ -21,7 +21,7 @@
 //   * the epilogue stores are NOT waited for: vmcnt counts loads, LDS-DMA and stores in issue
 //     order, so the stores are issued right after the k-step's DMA and the next three end-of-step
 //     waits count them among the younger operations (vmcnt(2G + S)) — the stores get three
-//     k-steps to drain before anything waits on them (the round-3/4 designs stalled the next
+//     k-steps to drain before anything waits on them (earlier designs stalled the next
 //     tile's DMA behind the store burst: profiles/native_gemm_r4.md);
 //   * tile order: XCD-aware (the 32 workgroups of one XCD take 32 consecutive tiles per round)
 //     and grouped along M (GROUP_M row tiles × the column tiles), so concurrently running tiles

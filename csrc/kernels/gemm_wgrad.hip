@@ -21,7 +21,7 @@
 //   * XCD-aware bijective block remap: a contiguous chunk of (split, tile) pairs per XCD so
 //     workgroups sharing a k-range and an operand panel share that XCD's L2.
 // wgrad_kernel (128×128, 4 waves, register staging; tile=128) and wgrad256_ring16_kernel
-// (variant 4, the round-1 default) stay selectable for A/B measurement.
+// (variant 4, the first default) stay selectable for A/B measurement.
 #include "common.h"
 #include "host_plan.h"
 #include <cstdlib>
@@ -158,7 +158,7 @@ __global__ void __launch_bounds__(256, 2) wgrad_kernel(const bf16* __restrict__ 
 // 256×256 tile, 8 waves (2 along M × 4 along N, each wave 128×64). Per 32-deep k-step: 32 KiB
 // of operands for 2·256·256·32 FLOP = 128 FLOP/B (the 128² tile's 64 FLOP/B left it
 // L2-bandwidth-bound at 320–500 TF). LDS rows are 512 B. (The 32x32x16 and register-staged
-// 256-tile variants of round 1 measured slower and were removed.)
+// 256-tile variants measured slower and were removed.)
 constexpr int BM2 = 256, BN2 = 256, BK2 = 32;
 
 // ---- 16x16x32 MFMA variant ---------------------------------------------------------------

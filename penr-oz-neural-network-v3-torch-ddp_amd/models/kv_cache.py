@@ -12,7 +12,7 @@ MI355X-first differences:
   * ``attend`` runs the decode-attention HIP kernel directly on the cache — for the int8
     cache the dequantisation is fused into the kernel, so the full cache is never
     materialised in fp32 (the reference dequantises the *whole* cache every step and returns
-    fp32, which also breaks bf16 models — SURVEY §7.4 bug 4);
+    fp32, which also breaks bf16 models);
   * ``seq_len(layer_idx)`` is per layer, so each layer's RoPE offset is its own.
 """
 from __future__ import annotations

@@ -9,7 +9,7 @@ mapping lives in :mod:`penroz.models.hf` and is re-exported here as classmethods
 Differences on purpose:
   * the config is never mutated (the reference compiles ``transformerblock`` by writing
     ``nn.Module`` objects back into the caller's dict, so modules end up pickled in the
-    checkpoint — SURVEY §7.4 bug 14);
+    checkpoint);
   * ``layernorm`` / ``gelu`` compile to subclasses whose GPU path is a HIP kernel (same
     parameters and keys as ``nn.LayerNorm`` / ``nn.GELU``);
   * ``adam`` / ``adamw`` compile to fused-kernel subclasses of ``torch.optim.Adam/AdamW``

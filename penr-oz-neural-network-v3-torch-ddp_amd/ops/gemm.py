@@ -230,7 +230,7 @@ def set_tuned_gemms(on: bool) -> bool:
 
 
 def guard_tuned_gemms(run_steps, steps: int = 3, rounds: int = 2, margin: float = 1.0, agree=None) -> dict:
-    """The shipped table must never cost time (VERDICT r4: it once drifted to 1 ms/step SLOWER than
+    """The shipped table must never cost time (it once drifted to 1 ms/step SLOWER than
     hipBLASLt's heuristic and nothing noticed). Times ``run_steps(steps)`` (returns seconds) with the
     table off and on, ``rounds`` interleaved times each, keeps the table only if its best time is
     <= ``margin`` × the heuristic's best, and leaves that choice switched on. ``agree`` (optional)
@@ -253,7 +253,7 @@ def guard_tuned_gemms(run_steps, steps: int = 3, rounds: int = 2, margin: float 
 
 
 # ---- linear + GELU / GELU backward (library GEMM + the HIP GELU kernels) -------------------
-# Two native fused designs were built and measured against this pair (round 3-4): an 8-phase
+# Two native fused designs were built and measured against this pair: an 8-phase
 # persistent MFMA GEMM with a bias/GELU epilogue and a 4-wave deferred-epilogue GEMM whose
 # stores (and GELU' / bias-column work) stream inside the next tile. Both lost on every GPT-2
 # shape and on the headline step (profiles/gemm_epi_r4.log, profiles/native_gemm_r4.md), so the

@@ -3,7 +3,7 @@
 Reference semantics (``neural_net_model.py:393-405``): temperature 0 → argmax of the last
 position; ``top_k`` → softmax over the top-k logits / T then multinomial; otherwise softmax
 over logits / T then multinomial.  (The reference's top-k runs over every position and its
-non-softmax-model path crashes — bugs 2 and 5 of SURVEY §7.4 — both fixed here.)
+non-softmax-model path crashes — both fixed here.)
 
 GPU: ``csrc/kernels/sampling.hip`` — one workgroup per row: temperature scale, top-k by a
 radix-select threshold in LDS, softmax and inverse-CDF draw from one uniform per row, all in

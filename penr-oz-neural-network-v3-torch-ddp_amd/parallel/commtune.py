@@ -183,7 +183,7 @@ def _probe_native(device, native, channels, proto, algo):
     protocol / algorithm that RCCL cannot serve fails at ENQUEUE time, not at init. The ranks first
     agree (MIN over the c10d group) that EVERY rank enqueued it — a rank whose enqueue failed leaves
     its peers' collective hanging, so they abort the communicator instead of waiting on it
-     — then wait, check the average and agree again; a failed arm is dropped on every
+    — then wait, check the average and agree again; a failed arm is dropped on every
     rank."""
     from penroz.parallel import rccl
     arm = (f"native RCCL arm ({channels or 'default'} channels, protocol {proto or 'default'}, "

@@ -7,7 +7,7 @@ design:
     fork of a GPU-initialised process) with ``RANK / LOCAL_RANK / WORLD_SIZE / MASTER_ADDR /
     MASTER_PORT`` set; ``torch.distributed`` env:// rendezvous uses the TCPStore on rank 0;
   * ``OMP_NUM_THREADS`` is split across CPU workers (the reference's elastic launch left it
-    unset: 7× slower CPU DDP at world_size 2, SURVEY §6);
+    unset: 7× slower CPU DDP at world_size 2);
   * a monitor polls worker exit codes; the first failure tears the group down and is
     *returned* (and reported through ``on_failure``) so the caller can mark the model
     ``Error`` instead of leaving it ``Training`` forever (reference bug 9);

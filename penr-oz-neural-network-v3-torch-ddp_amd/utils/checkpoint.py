@@ -4,7 +4,7 @@ Format parity with the reference (``neural_net_model.py:98-174``): ``torch.save`
 with ``layers, state, optim, optim_state, progress, average_cost, average_cost_history,
 stats, status`` at ``models/model_{id}.pth``, cached under ``{SHM}/models/``.
 
-Fixes (SURVEY §5.2/§7.4 bug 10): every write goes to a temp file + ``os.replace`` (readers
+Fixes: every write goes to a temp file + ``os.replace`` (readers
 never see a torn checkpoint); the disk flush copies atomically on a background *thread*
 (never a fork of a GPU-initialised process); a small JSON sidecar carries progress/status so
 ``/progress`` does not ``torch.load`` a multi-GB file.  Loads use ``weights_only=True``.

@@ -1,4 +1,4 @@
-"""Tracing and profiling hooks (SURVEY §5.1 — the reference has none).
+"""Tracing and profiling hooks (the reference has none).
 
 * ``trace_range(name)`` — a roctx range (ROCm's marker API, loaded from the ROCm runtime with
   ctypes: ``librocprofiler-sdk-roctx`` first, the legacy ``libroctx64`` otherwise). Ranges

@@ -208,7 +208,7 @@ def _probe_worker(rank, world, port, out):
 
 
 def test_native_probe_agrees_on_enqueue_before_waiting(tmp_path):
-    """when one rank's enqueue fails, no rank waits on the probe collective; every rank
+    """When one rank's enqueue fails, no rank waits on the probe collective; every rank
     drops the arm, aborting (not destroying) the communicator."""
     mp.spawn(_probe_worker, args=(2, _port(), str(tmp_path)), nprocs=2, join=True)
     for r in range(2):

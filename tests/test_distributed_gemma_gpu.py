@@ -1,5 +1,5 @@
 """Two ranks of the fused GEMMA executor on ONE MI355X (gloo, GPU buckets staged through host memory): the Gemma analogue of
-tests/test_distributed_gpu.py (VERDICT r3, next-round item 6a). The Gemma executor inherits the
+tests/test_distributed_gpu.py. The Gemma executor inherits the
 bucketed reducer wiring of the GPT executor but its flat-buffer segment order differs (the gate /
 up projections adjacent so their gradient is one [2F, C] slice, optional post-norms per block), so
 the bucket-ready bookkeeping and the rank-0 broadcast are checked on its own layout, with and

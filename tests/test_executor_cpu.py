@@ -126,7 +126,7 @@ def _range_exec(monkeypatch):
 
 
 def test_wgrad_ranges_chunked_after_learning(monkeypatch):
-    """after the ranges are learned, a key that writes sub-ranges (chunked wgrad) must
+    """After the ranges are learned, a key that writes sub-ranges (chunked wgrad) must
     never accumulate onto last step's data — whether its first chunk is a sub-range, the whole
     learned range, or some parts are never written."""
     import torch

@@ -366,7 +366,7 @@ def test_capture_returns_activation_and_gradient_pairs():
 
 
 def test_new_session_after_segment_transposes_uses_fresh_weights(monkeypatch):
-    """the transposed dgrad copies rebuilt after each segment's AdamW pass are marked
+    """The transposed dgrad copies rebuilt after each segment's AdamW pass are marked
     fresh; a new session that rebuilds the shadow from other weights (loaded after training) must
     rebuild them too, or its first step's data gradients use the old weights. Gradients of the
     first step after the reload == an executor without transposed copies (PENROZ_DGRAD_T=0)."""

@@ -194,7 +194,7 @@ def test_gemma_program_step_matches_module_step(monkeypatch, model_type, rows, r
 @pytest.mark.parametrize("rows", [1, 3])
 def test_gemma_program_wide_mlp_falls_back_from_gemv(rows):
     """An intermediate size above decode_gemv's K <= 8192 (Gemma-4 e2b's double-wide MLPs are
-    12288): the program must not take the GEMV path for the down projection (ADVICE r5)."""
+    12288): the program must not take the GEMV path for the down projection."""
     m = _gemma_model(64, intermediate_size=8192 + 256)
     dec = gd.GraphDecoder(m, rows, 32, 0.0, None)
     assert isinstance(dec.program, gd.GemmaDecodeProgram)

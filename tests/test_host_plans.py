@@ -1,6 +1,6 @@
 """Host-side launch plans of the HIP extension (no GPU needed: the built extension imports on the
 CPU runner): the fused decode QKV + RoPE kernel's split-K plan is exported by the kernel's own
-source and the Python admission check reads it instead of re-deriving the rule (ADVICE r3)."""
+source and the Python admission check reads it instead of re-deriving the rule."""
 import pytest
 
 from penroz.ops import _ext, gemm as G

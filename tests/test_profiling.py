@@ -1,4 +1,4 @@
-"""Tracing / profiling hooks (SURVEY §5.1): roctx ranges and the torch.profiler step wrapper."""
+"""Tracing / profiling hooks: roctx ranges and the torch.profiler step wrapper."""
 import os
 
 import torch

@@ -150,7 +150,7 @@ def _prow(tr, mb, bw, ok=True, wire="fp32", ch=None, proto="", algo=""):
 
 
 def test_comm_plan_judges_each_transport_at_its_own_bucket():
-    """the transport is compared at each arm's own chosen bucket size, not at a fixed 64 MB."""
+    """The transport is compared at each arm's own chosen bucket size, not at a fixed 64 MB."""
     from penroz.parallel.commtune import plan
     rows = [_prow("c10d", 16, 100), _prow("c10d", 64, 104),
             _prow("native", 16, 70, ch=0), _prow("native", 64, 130, ch=0)]
@@ -164,7 +164,7 @@ def test_comm_plan_judges_each_transport_at_its_own_bucket():
 
 
 def test_comm_plan_picks_channel_count():
-    """The channel count comes with the winning native arm (SURVEY §5.8: NCCL_MIN/MAX_NCHANNELS)."""
+    """The channel count comes with the winning native arm (NCCL_MIN/MAX_NCHANNELS)."""
     from penroz.parallel.commtune import plan
     rows = [_prow("c10d", 64, 100), _prow("native", 64, 110, ch=0), _prow("native", 64, 160, ch=16),
             _prow("native", 64, 140, ch=32), _prow("native", 32, 170, ok=False, ch=8)]
@@ -209,8 +209,8 @@ def test_comm_plan_picks_algorithm():
 
 def test_comm_plan_bf16_wire_only_when_exposed():
     """bf16 wire recommended only when the predicted fp32 all-reduce of the whole gradient exceeds
-    the backward and the bf16 arm is correct and clearly faster; APPLIED only with auto_bf16 (ADVICE
-    r4: the default wire stays the reference DDP's fp32)."""
+    the backward and the bf16 arm is correct and clearly faster; APPLIED only with auto_bf16
+    (the default wire stays the reference DDP's fp32)."""
     from penroz.parallel.commtune import plan
     rows = [_prow("c10d", 64, 100), _prow("c10d", 64, 100, wire="bf16")]
     g = 6550 * 2**20  # GPT-2 XL fp32 gradients
@@ -243,7 +243,7 @@ def test_parse_rccl_log_nranks_and_channels():
 
 
 def test_sweep_arms_default_is_rccl_only(monkeypatch):
-    """the forced channel / protocol / algorithm arms are opt-in."""
+    """The forced channel / protocol / algorithm arms are opt-in."""
     from penroz.parallel import commtune
     monkeypatch.delenv("PENROZ_COMM_SWEEP_ARMS", raising=False)
     assert commtune.sweep_arms() == ((0,), ("",), ("",))
@@ -369,7 +369,7 @@ def test_bench_gemma4_config_shapes():
 
 
 def test_gemm_table_guard_keeps_only_a_faster_table(monkeypatch):
-    """the shipped GEMM table is timed against hipBLASLt's heuristic before the
+    """The shipped GEMM table is timed against hipBLASLt's heuristic before the
     timed region and dropped when slower; the choice is left switched on."""
     import torch.cuda.tunable as tunable
     from penroz.ops import gemm as G
@@ -389,7 +389,7 @@ def test_gemm_table_guard_keeps_only_a_faster_table(monkeypatch):
 @pytest.mark.slow
 @pytest.mark.parametrize("world", [4, 8])
 def test_bench_multi_rank_cpu_matches_single_process(world):
-    """the data-parallel bench at 4 and 8 ranks (gloo on the CPU, tiny model).
+    """The data-parallel bench at 4 and 8 ranks (gloo on the CPU, tiny model).
     Every rank agrees on the first-contact plan and builds the same gradient buckets, and the
     rank-averaged loss and the parameters after the run equal one process training on the
     concatenated batches (``--data-ranks``)."""
