@@ -1136,7 +1136,7 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
     TORCH_CHECK(emb_idx->is_cuda() && emb_idx->scalar_type() == torch::kInt64 && emb_idx->is_contiguous(),
                 "decode_gemv: int64 token ids");
     for (const torch::Tensor* t : {&*emb_wte, &*emb_wpe})
-      TORCH_CHECK(t->scalar_type() == torch::kBFloat16 && t->dim() == 2 && t->is_contiguous() && t->size(1) == K &&
+      TORCH_CHECK(t->scalar_type() == torch::kBFloat16 && t->dim() == 2 && t->is_contiguous() && t->size(1) == K && t->size(0) > 0 &&
                       reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "decode_gemv: bf16 contiguous wte / wpe [*, K]");
     TORCH_CHECK(emb_pos->is_cuda() && emb_pos->scalar_type() == torch::kInt64 && emb_pos->numel() == 1, "decode_gemv: int64 pos [1]");
     TORCH_CHECK(K <= 1024, "decode_gemv: LN mode needs K <= 1024");
@@ -1399,7 +1399,7 @@ void decode_norm_pair(c10::optional<torch::Tensor> x, c10::optional<torch::Tenso
   nm.eps1 = (float)eps1;
   nm.eps2 = (float)eps2;
   if (emb) {
-    TORCH_CHECK(table->dim() == 2, who, ": table [V, K]");
+    TORCH_CHECK(table->dim() == 2 && table->size(0) > 0, who, ": table [V, K]");
     nm.tok = tok->data_ptr<int64_t>();
     nm.vocab = table->size(0);
     nm.table = rows(*table, nm.vocab);

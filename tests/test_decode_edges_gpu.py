@@ -57,3 +57,17 @@ def test_other_products_over_no_columns(M):
 def test_prompt_rows_of_no_width():
     qkv, cache = torch.empty(1, 2, 0, device=DEV, dtype=BF), torch.empty(1, 1, 4, 0, device=DEV, dtype=BF)
     assert _ext.kernels().prompt_kv(qkv, None, cache, cache, 0, 1, 1) is None
+
+
+def test_tables_of_no_rows_are_refused():
+    """Token and position are held to the table's rows, of which the last would be -1."""
+    k, C, N = _ext.kernels(), 64, 128
+    z = lambda *s, dt=BF: torch.zeros(*s, device=DEV, dtype=dt)
+    tok, pos, out, w = z(1, dt=torch.int64), z(1, dt=torch.int64), z(1, N), z(N, C)
+    f = torch.float32
+    for wte, wpe in ((z(0, C), z(4, C)), (z(4, C), z(0, C))):
+        with pytest.raises(RuntimeError):
+            k.decode_gemv(None, None, None, None, z(1, C, dt=f), z(C, dt=f), z(C, dt=f), 1e-5, w, None, out, 0, emb_idx=tok, emb_wte=wte,
+                          emb_wpe=wpe, emb_pos=pos)
+    with pytest.raises(RuntimeError):
+        k.decode_norm_pair(None, None, None, z(C), 3, 0.0, 1e-6, z(1, C), w, out[:, :N // 2], 1, 2, tok=tok, table=z(0, C))
