@@ -1,0 +1,44 @@
+"""Experts of few pairs (csrc/kernels/experts.hip): weights by whole lines, each width's kernel and the one for any width, against
+float64."""
+import pytest
+import torch
+
+from penroz.ops import packed as P
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _chosen(N, E, top, spread):
+    """ids [N, top]: ``spread`` experts share all pairs, each row's are distinct."""
+    if top == 1:
+        return torch.randint(0, spread, (N, 1))
+    return torch.stack([torch.randperm(spread)[:top] for _ in range(N)])
+
+
+# pairs per expert: 8, 9, 16, 17 and many; pairs fewer than experts (and several of one), as many, more; blocks of 16 and 32 rows
+@pytest.mark.parametrize("N,E,top,spread", [(1, 1, 1, 1), (8, 1, 1, 1), (9, 4, 1, 1), (16, 1, 1, 1), (17, 2, 1, 1), (100, 3, 2, 2),
+                                            (1, 64, 6, 64), (5, 64, 3, 4), (16, 48, 3, 48), (60, 16, 4, 16), (260, 20, 3, 20),
+                                            (512, 64, 2, 64)])
+# widths: every kernel of 256 columns per step, and widths in between, off 64 columns, and above
+@pytest.mark.parametrize("kind,C,F", [(P.UNGATED, 256, 512), (1, 512, 256), (1, 768, 1024), (P.UNGATED, 1024, 768), (1, 1536, 32),
+                                      (P.UNGATED, 2048, 1536), (0, 2304, 96), (P.UNGATED, 32, 2048), (1, 160, 1280), (0, 2080, 64)])
+def test_expert_rows(N, E, top, spread, kind, C, F):
+    torch.manual_seed(N + 31 * E + C)
+    ids = _chosen(N, E, top, spread)
+    h = torch.randn(N, C).bfloat16().to(DEV)
+    g, u = ((torch.randn(E, F, C) * C ** -0.5).bfloat16().to(DEV) for _ in range(2))
+    d = (torch.randn(E, C, F) * F ** -0.5).bfloat16().to(DEV)
+    gated = kind != P.UNGATED
+    w = P.pack_experts(g if gated else None, u, d)
+    y = P.experts(h, ids.int().to(DEV), w, kind, 0.7).view(N, top, C).double()
+    for e in range(spread):
+        r, k = (ids == e).nonzero(as_tuple=True)
+        if not r.numel():
+            continue
+        x = h[r.to(DEV)].double()
+        a = P.expert_activation(x @ g[e].double().t() if gated else None, x @ u[e].double().t(), kind, 0.7)
+        want = a @ d[e].double().t()
+        # the hidden row is rounded to bf16 (2^-9), and the result (2^-9); fp32 sums of C and F terms are far below
+        tol = 2.0 ** -8 * (a.abs() @ d[e].double().abs().t()) + 2.0 ** -8 * want.abs() + 1e-6
+        assert torch.all((y[r.to(DEV), k.to(DEV)] - want).abs() <= tol), (e, r.numel())
