@@ -443,6 +443,17 @@ __device__ __forceinline__ float other_half(float v, int half) {  // lane ^ 32
   return __uint_as_float(half ? r[0] : r[1]);
 }
 
+// 16 bytes of weights. NT: by a load that no cache keeps, 6.4 to 7.2 TB/s from memory where others take 5.7 to 6.3 (200 to 640 MB).
+// The vocabulary's projection, gate | up and long rows (K > 4608) are read so: nothing holds those from one step to the next, and
+// what they leave in the 256 MB in front of the memory is what a step finds there of its other weights. Generation of 64 tokens, GPT-2
+// 124M, one row: 14.95 -> 14.45 ms, but 14.94 with its layers' weights (170 MB) read so too; of 32 tokens, Gemma-3 1B, 3 rows: 34.9 ->
+// 33.4, 33.7 with QKV and output projections too. (A choice at run time costs a kernel 0.3 us.)
+template <bool NT>
+__device__ __forceinline__ uint4 weight16(const bf16* p) {
+  if constexpr (NT) return __builtin_bit_cast(uint4, __builtin_nontemporal_load(reinterpret_cast<const dl_u32x4*>(p)));
+  else return *reinterpret_cast<const uint4*>(p);
+}
+
 // PRO: 0 — x is the bf16 operand; 1 — LN mode (GPT: fp32 residual + delta + dbias, LayerNorm)
 template <int M, int PRO, int RP, int CPL>
 __global__ void __launch_bounds__(64) decode_gemv_kernel(
@@ -468,7 +479,7 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
   int cc[CPL];  // chunks past the row are read from its last one and count as zero
 #pragma unroll
   for (int i = 0; i < CPL; ++i) cc[i] = min(l32 + 32 * i, nc - 1);
-  uint4 wv[RP][CPL], xb[M][CPL];
+  uint4 wv[RP][CPL], xb[M][CPL];  // (8 rows per wave: the vocabulary's)
   auto weights = [&]() {
 #pragma unroll
     for (int rp = 0; rp < RP; ++rp) {
@@ -476,7 +487,7 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
 #pragma unroll
       for (int i = 0; i < CPL; ++i) {
         const int c = l32 + 32 * i;
-        wv[rp][i] = c < nc ? *reinterpret_cast<const uint4*>(wr + 8 * c) : uint4{0u, 0u, 0u, 0u};
+        wv[rp][i] = c < nc ? weight16<RP == 4>(wr + 8 * c) : uint4{0u, 0u, 0u, 0u};
       }
     }
   };
@@ -701,7 +712,7 @@ __global__ void __launch_bounds__(64 * NW) decode_gemv_rows_kernel(const bf16* _
 #pragma unroll
   for (int r = 0; r < RP; ++r)
 #pragma unroll
-    for (int i = 0; i < CPL; ++i) wv[r][i] = *reinterpret_cast<const uint4*>(w + (size_t)min(n0 + r, N - 1) * K + 8 * cc[i]);
+    for (int i = 0; i < CPL; ++i) wv[r][i] = weight16<RP == 2>(w + (size_t)min(n0 + r, N - 1) * K + 8 * cc[i]);
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("" : "+v"(bias_v), "+v"(old));  // asked for with the others: left to itself, each is fetched where it is needed
 #pragma unroll
@@ -785,7 +796,7 @@ __global__ void __launch_bounds__(64 * NW, NORM && CPL <= 5 ? 4 : 1) decode_gemv
     for (int r = 0; r < RP; ++r) {
       const int p = min(p0 + r, npair - 1), row = GATED ? p + h * npair : p / hd * D + p % hd + h * hd;
 #pragma unroll
-      for (int i = 0; i < CPL; ++i) wv[r][i] = *reinterpret_cast<const uint4*>(w + (size_t)row * K + 8 * min(l32 + 32 * i, nc - 1));
+      for (int i = 0; i < CPL; ++i) wv[r][i] = weight16<GATED>(w + (size_t)row * K + 8 * min(l32 + 32 * i, nc - 1));
     }
   };
   const int p = p0 + l32 / M;  // this lane's output pair, row l32 % M of x
@@ -1196,7 +1207,7 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
     return e ? std::atoi(e) : 0;
   }();
   // a LayerNorm product of whole tiles: one workgroup normalises for 16 columns (decode_ln_few_kernel). The vocabulary's many columns
-  // stay with the waves below (50304 x 768, one row: 15.9 us, 77 MB at 4.9 TB/s)
+  // stay with the waves below (50304 x 768, one row: 15.9 us through the caches, 77 MB at 4.9 TB/s)
   if (ln && !dp && rows_per_wave <= 0 && rpw_env <= 0 && K % 32 == 0 && N % 16 == 0 && N < 16384 && out.stride(0) % 4 == 0 &&
       reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0 && reinterpret_cast<uintptr_t>(bp) % 8 == 0) {
     const LnEmb e{eip, ewp, epp, eps_p, eV, eP};
