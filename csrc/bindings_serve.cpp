@@ -85,6 +85,8 @@ void experts_plain(torch::Tensor h, torch::Tensor ids, torch::Tensor wgu, torch:
                    torch::Tensor act, torch::Tensor y);
 void experts_rows(torch::Tensor h, torch::Tensor ids, torch::Tensor wgu, torch::Tensor wd, int64_t kind, double limit,
                   torch::Tensor act, torch::Tensor y);
+bool experts_rows_shared(torch::Tensor h, torch::Tensor ids, torch::Tensor wgu, torch::Tensor wd, double limit, torch::Tensor act,
+                         torch::Tensor y, torch::Tensor up, torch::Tensor down, torch::Tensor sact, torch::Tensor sy);
 void experts_grouped(torch::Tensor h, torch::Tensor ids, torch::Tensor wgu, torch::Tensor wd, int64_t kind, double limit,
                      torch::Tensor act, torch::Tensor y, torch::Tensor perm, torch::Tensor tiles);
 void gelu_rows(torch::Tensor u);
@@ -189,6 +191,7 @@ PYBIND11_MODULE(penroz_serve, m) {
   m.def("latent_flash_ok", &latent_flash_ok, "latent_flash takes these sizes");
   m.def("latent_flash", &latent_flash, "causal attention of packed prompts / portions over expanded keys (MFMA)");
   m.def("experts_rows", &experts_rows, "gated experts of few (token, expert) pairs (MFMA)");
+  m.def("experts_rows_shared", &experts_rows_shared);
   m.def("experts_grouped", &experts_grouped, "gated experts of pairs grouped by expert (MFMA tiles)");
   m.def("gated_rows", &gated_rows, "act(g)·u of packed [g | u] rows");
   m.def("gelu_rows", &gelu_rows, "gelu (erf form) in place");

@@ -103,8 +103,10 @@ class _Experts:
 
     def run(self, h: Tensor, b, st) -> ops.Delta:
         ids, wts = ops.route(h, self.router, **self.rule)
-        y = ops.experts(h, ids, self.w, self.kind, self.limit)
-        return ops.Delta(y, pair_w=wts, shared=None if self.shared is None else ops.gelu_mlp(h, **self.shared))
+        if self.shared is None:
+            return ops.Delta(ops.experts(h, ids, self.w, self.kind, self.limit), pair_w=wts)
+        y, shared = ops.experts_beside_shared(h, ids, self.w, self.kind, self.limit, self.shared)
+        return ops.Delta(y, pair_w=wts, shared=shared)
 
 
 # --------------------------------------------------------------------------- entries

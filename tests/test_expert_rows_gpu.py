@@ -42,3 +42,23 @@ def test_expert_rows(N, E, top, spread, kind, C, F):
         # the hidden row is rounded to bf16 (2^-9), and the result (2^-9); fp32 sums of C and F terms are far below
         tol = 2.0 ** -8 * (a.abs() @ d[e].double().abs().t()) + 2.0 ** -8 * want.abs() + 1e-6
         assert torch.all((y[r.to(DEV), k.to(DEV)] - want).abs() <= tol), (e, r.numel())
+
+
+@pytest.mark.parametrize("N,E,top", [(1, 8, 2), (3, 8, 3), (8, 2, 2), (9, 40, 4), (16, 3, 3), (16, 64, 6), (17, 8, 2)])
+@pytest.mark.parametrize("C,F,S", [(256, 256, 512), (512, 1024, 2048), (1024, 768, 1536), (2048, 512, 1024), (1536, 256, 512),
+                                   (512, 256, 768), (256, 1536, 3072), (288, 256, 512)])
+def test_shared_expert_beside(N, E, top, C, F, S):
+    """The shared expert in the experts' launches, and where it keeps its own (17 rows, other widths)."""
+    torch.manual_seed(N + C + F)
+    ids = _chosen(N, E, top, E).int().to(DEV)
+    h = torch.randn(N, C).bfloat16().to(DEV)
+    u, d = ((torch.randn(E, *s) * s[1] ** -0.5).bfloat16().to(DEV) for s in ((F, C), (C, F)))
+    su, sd = ((torch.randn(*s) * s[1] ** -0.5).bfloat16().to(DEV) for s in ((S, C), (C, S)))
+    w = P.pack_experts(None, u, d)
+    y, out = P.experts_beside_shared(h, ids, w, P.UNGATED, 0.0, {"up": su, "down": sd})
+    assert torch.equal(y, P.experts(h, ids, w, P.UNGATED, 0.0))
+    pre = h.double() @ su.double().t()
+    a = torch.nn.functional.gelu(pre)
+    # the hidden row is rounded to bf16 before (|gelu'| < 1.2) and after the activation, and the result: 2^-9 each
+    tol = 2.0 ** -9 * (1.2 * pre.abs() + a.abs()) @ sd.double().abs().t() + 2.0 ** -8 * (a @ sd.double().t()).abs() + 1e-5
+    assert torch.all((out.double() - a @ sd.double().t()).abs() <= tol)
