@@ -330,8 +330,7 @@ class PackedSession:
             plan.append((self._slot[name], len(tokens)))
         b = self.state.begin(plan)
         dev = self.program.device
-        out = self.program.forward(torch.tensor(toks, dtype=torch.long).to(dev), b, self.state,
-                                   torch.tensor(want, dtype=torch.int32).to(dev))
+        out = self.program.forward(ops.upload(toks, torch.long, dev), b, self.state, ops.upload(want, torch.int32, dev))
         return None if out is None else out.float()
 
     def slots(self, names) -> list[int]:

@@ -17,6 +17,16 @@ from penroz.ops._ext import kernels, use_kernels
 from penroz.ops import gemm as gemm_ops
 
 
+def upload(values, dtype: torch.dtype, device: torch.device) -> Tensor:
+    """Host values as a tensor on ``device``. By way of pinned memory, whose copy is one more piece of the stream's work: a copy from
+    pageable memory waits for all that the stream has been given, and the GPU then idles until the next kernels arrive (64 sequences
+    of Golepel stepped token by token, 0.15 of 1.25 ms a step)."""
+    t = torch.tensor(values, dtype=dtype)
+    if device.type != "cuda" or t.numel() == 0:
+        return t.to(device)
+    return t.pin_memory().to(device, non_blocking=True)
+
+
 @dataclass
 class PackedBatch:
     """Rows of one step. Per row (int32 [N]): ``slot`` of its sequence, ``pos`` in it, ``first`` row of the
@@ -49,7 +59,7 @@ class PackedBatch:
             off = [0]
             for n in self.lens:
                 off.append(off[-1] + n)
-            self._kv = {"cu": torch.tensor(off, dtype=torch.int32).to(self.slot.device), "n": off[-1]}
+            self._kv = {"cu": upload(off, torch.int32, self.slot.device), "n": off[-1]}
         return self._kv["cu"], self._kv["n"]
 
     def query_blocks(self, size: int = 128) -> Tensor:
@@ -59,7 +69,7 @@ class PackedBatch:
             blk = [(l - n + min(q + size, n), s, q) for s, (n, l) in enumerate(zip(self.counts, self.lens))
                    for q in range(0, n, size)]
             blk.sort(key=lambda b: -b[0])
-            self._blocks = torch.tensor([b[1:] for b in blk], dtype=torch.int32).to(self.slot.device)
+            self._blocks = upload([b[1:] for b in blk], torch.int32, self.slot.device)
         return self._blocks
 
     def spans(self, size: int) -> tuple[Tensor, Tensor]:
@@ -72,7 +82,7 @@ class PackedBatch:
             off = [0]
             for n in self.counts:
                 off.append(off[-1] - (-n // size))
-            self._spans[size] = tuple(torch.tensor(t, dtype=torch.int32).to(self.slot.device) for t in (rows, off))
+            self._spans[size] = tuple(upload(t, torch.int32, self.slot.device) for t in (rows, off))
         return self._spans[size]
 
 
