@@ -400,6 +400,29 @@ def test_experts_in_large_tiles(kind, C, F):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", [1, P.UNGATED])
+@pytest.mark.parametrize("C,F", [(32, 64), (96, 160), (192, 96), (224, 256)])
+def test_experts_in_large_tiles_of_few_steps(kind, C, F):
+    """Reductions of half a step to four (a tile's last three steps bring the next tile's rows), several choices per token, workgroups
+    with several tiles of unequal heights, and an expert that few chose."""
+    dev, E, N, top = "cuda", 10, 50000, 3
+    g = torch.Generator().manual_seed(3)
+    ids = torch.stack([torch.randperm(E - 1, generator=g)[:top] for _ in range(500)]).repeat(N // 500, 1)
+    ids[7, 1] = E - 1
+    ids = ids.to(dev)
+    h = rand(N, C, dtype=torch.bfloat16).to(dev)
+    wg, u, d = (rand(E, *sh, seed=i, scale=2 * sh[1] ** -0.5, dtype=torch.bfloat16).to(dev)
+                for i, sh in enumerate([(F, C), (F, C), (C, F)]))
+    w = P.pack_experts(None if kind == P.UNGATED else wg, u, d)
+    y = P.experts(h, ids.int(), w, kind, 0.7).view(N, top, C)
+    for e in range(E):
+        tok, k = (ids == e).nonzero(as_tuple=True)
+        x = h[tok].float()
+        a = P.expert_activation(None if kind == P.UNGATED else x @ wg[e].float().t(), x @ u[e].float().t(), kind, 0.7)
+        near(y[tok, k], (a @ d[e].float().t()).cpu(), torch.bfloat16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", [1, P.UNGATED])
 @pytest.mark.parametrize("E,C,F", [(512, 1024, 64), (512, 992, 32), (40, 96, 160), (20, 512, 544), (20, 544, 512),
                                    (20, 1056, 1024), (70, 992, 512), (70, 992, 544)])
 def test_experts_of_few_pairs(kind, E, C, F):
