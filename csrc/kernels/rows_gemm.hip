@@ -28,6 +28,15 @@ typedef float rg_f32x4 __attribute__((ext_vector_type(4)));
 // not of 16-byte pieces
 enum { kRgPlain = 0, kRgAdd = 1, kRgGelu = 2, kRgNarrow = 4 };
 
+// glds16 of memory that nobody reads again soon
+__device__ __forceinline__ void glds16_once(const void* g, unsigned lds_addr) {
+  unsigned keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep)
+               : "v"(g), "s"(lds_addr)
+               : "memory");
+}
+
 template <int P, int LEFT>
 __device__ __forceinline__ void wait_stages(int left) {  // all but the newest `left` stages of P loads have landed
   if constexpr (LEFT > 0) {
@@ -41,7 +50,8 @@ __device__ __forceinline__ void wait_stages(int left) {  // all but the newest `
   }
 }
 
-template <int FM, int FN, int WM, int WN, int WK, int KS, int NBUF, typename OUT>
+// ONCE: no cache keeps the weights (a kernel of its own: a choice between two loads costs the small products up to 0.4 us)
+template <int FM, int FN, int WM, int WN, int WK, int KS, int NBUF, bool ONCE, typename OUT>
 __global__ void __launch_bounds__(64 * WM * WN * WK) rows_gemm_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
                                                                       const bf16* __restrict__ bias, OUT* __restrict__ out, int M,
                                                                       int N, int K, int ldx, int ldw, int ldo, int tiles_m,
@@ -77,7 +87,10 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) rows_gemm_kernel(const bf16
     const int k0 = st * COLS;
     if (k0 + COLS <= K) {
 #pragma unroll
-      for (int i = 0; i < PIECES; ++i) glds16(src[i] + (size_t)k0 * 2, lds + buf * STAGE + i * 1024);
+      for (int i = 0; i < PIECES; ++i) {
+        if (!ONCE || (wv * PIECES + i) % PER_SUB * 8 < TM) glds16(src[i] + (size_t)k0 * 2, lds + buf * STAGE + i * 1024);
+        else glds16_once(src[i] + (size_t)k0 * 2, lds + buf * STAGE + i * 1024);
+      }
     } else {
 #pragma unroll
       for (int i = 0; i < PIECES; ++i)
@@ -185,16 +198,25 @@ static void rg_launch(int tile, bool in_order, const torch::Tensor& x, const tor
                       const torch::Tensor& out, int end) {
   const int64_t M = x.size(0), N = w.size(0), K = x.size(1);
   auto stream = at::hip::getCurrentHIPStream();
-  auto launch = [&](auto kern, int threads, int lds, int TM, int TN, auto* o) {
+  // Weights of 16 MB and more that one workgroup each reads pass the caches, which keep the smaller ones of a decode step. us, from
+  // memory, kept / not: 16 x 8192 x 2048 9.1 / 8.1, 16 x 7232 x 2048 8.3 / 7.6, 16 x 12288 x 2048 14.0 / 12.8, 16 x 32768 x 1024
+  // 16.7 / 13.8; of 4 to 8 MB 2 % or nothing. ms: 64 tokens of GPT-2 124M, 64 rows 29.0 / 28.6, 12 rows 22.5 / 21.8; 32 of Zozenex large,
+  // 16 rows, 46.4 / 44.8 (with the tile below). Where all that the caches are left with fits them, a head of 64 MB is better kept:
+  // Zozenex small, 16 rows 33.9 / 34.1.
+  const bool large = N * K >= (int64_t)8 << 20;
+  auto launch = [&](auto kern, auto kern_once, int threads, int lds, int TM, int TN, auto* o) {
     const int64_t tiles_m = (M + TM - 1) / TM, tiles = tiles_m * ((N + TN - 1) / TN);
+    if (large && tiles_m == 1) kern = kern_once;
     hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(threads), lds, stream, reinterpret_cast<const bf16*>(x.data_ptr()),
                        reinterpret_cast<const bf16*>(w.data_ptr()), bias, o, (int)M, (int)N, (int)K, (int)x.stride(0),
                        (int)w.stride(0), (int)out.stride(0), (int)tiles_m, end);
   };
 #define PENROZ_RG(FM, FN, WM, WN, WK, KS, NB)                                                                    \
-  launch(rows_gemm_kernel<FM, FN, WM, WN, WK, KS, NB, OUT>, 64 * WM * WN * WK,                                   \
-         NB * WK * KS * 128 * 16 * (FM * WM + FN * WN), 16 * FM * WM, 16 * FN * WN, o)
+  launch(rows_gemm_kernel<FM, FN, WM, WN, WK, KS, NB, false, OUT>, rows_gemm_kernel<FM, FN, WM, WN, WK, KS, NB, true, OUT>, \
+         64 * WM * WN * WK, NB * WK * KS * 128 * 16 * (FM * WM + FN * WN), 16 * FM * WM, 16 * FN * WN, o)
+  // Tile 5 of up to 16 rows is 16×64, columns split, two workgroups to a CU and all of them at once: 64×128 brings 64 rows of x where
+  // 16 are there, on one CU each. us, both past the caches: 16 x 32768 x 2048 33.7 / 26.8; 1024 columns are the other's (13.8 / 14.5).
   auto typed = [&](auto* o) {
     using OUT = std::remove_pointer_t<decltype(o)>;
     if (tile == 6) PENROZ_RG(1, 1, 1, 1, 4, 1, 6);
@@ -204,6 +226,7 @@ static void rg_launch(int tile, bool in_order, const torch::Tensor& x, const tor
     else if (tile == 2) PENROZ_RG(2, 4, 1, 1, 4, 1, 3);
     else if (tile == 3) PENROZ_RG(2, 2, 2, 2, 1, 2, 4);
     else if (tile == 4) PENROZ_RG(2, 2, 2, 2, 1, 2, 2);
+    else if (!in_order && M <= 16 && K > 1024 && N <= 32768) PENROZ_RG(1, 4, 1, 1, 4, 1, 2);
     else PENROZ_RG(2, 4, 2, 2, 1, 1, 3);
   };
 #undef PENROZ_RG

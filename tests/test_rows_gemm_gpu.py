@@ -162,3 +162,21 @@ def test_gelu_is_the_erf_form(M, N):
     bound = 2.0 ** -8 * erf.abs() + 2.0 ** -22 * lin.abs()
     assert ((act - erf).abs() <= bound).all()
     assert ((tanh - erf).abs() > bound).float().mean() > 0.05  # the other form would not pass
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(9, 32768, 1032), (16, 30001, 1280), (13, 32768, 2048), (16, 17000, 1992), (16, 8192, 1032),
+                                   (64, 50304, 192), (64, 9001, 1024), (33, 9000, 1024)])
+def test_large_weights_of_few_rows(M, N, K):
+    """Outputs of up to 16 rows in tiles of 16 x 64, and weights past the caches in other tiles: ragged rows, columns and stages."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    w = torch.randn(N, K, generator=g, device="cuda").bfloat16()
+    bias = torch.randn(N, generator=g, device="cuda").bfloat16()
+    want = x.double() @ w.double().t()
+    full = gemm.rows_linear(x, w, fp32=True)
+    # fp32 sums of K products: in blocks of 32 in the MFMA, K / 32 of them
+    assert torch.linalg.norm(full.double() - want) <= 2.0 ** -24 * (K / 32 + 32) ** 0.5 * torch.linalg.norm(want)
+    got, ref = gemm.rows_linear(x, w, bias), want + bias.double()
+    # half a step of bf16 at each value, and the sums' own error where they cancel
+    assert ((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -18 * K ** 0.5).all()
