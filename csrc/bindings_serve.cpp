@@ -22,20 +22,20 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
                  c10::optional<torch::Tensor> gamma, c10::optional<torch::Tensor> beta, double eps, torch::Tensor w,
                  c10::optional<torch::Tensor> bias, torch::Tensor out, int64_t act, int64_t rows_per_wave,
                  c10::optional<torch::Tensor> emb_idx, c10::optional<torch::Tensor> emb_wte,
-                 c10::optional<torch::Tensor> emb_wpe, c10::optional<torch::Tensor> emb_pos);
+                 c10::optional<torch::Tensor> emb_wpe, c10::optional<torch::Tensor> emb_pos, bool past);
 void decode_gemv_pair(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64_t mode, int64_t kind, int64_t D,
                       int64_t nrot, c10::optional<torch::Tensor> cosv, c10::optional<torch::Tensor> sinv,
-                      int64_t pairs_per_wave);
+                      int64_t pairs_per_wave, bool past);
 void decode_norm_pair(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> a, c10::optional<torch::Tensor> w1, torch::Tensor w2,
                       int64_t step, double eps1, double eps2, c10::optional<torch::Tensor> h, torch::Tensor w, torch::Tensor out,
                       int64_t mode, int64_t kind, int64_t D, int64_t nrot, c10::optional<torch::Tensor> cosv,
                       c10::optional<torch::Tensor> sinv, c10::optional<torch::Tensor> tok, c10::optional<torch::Tensor> table,
-                      double scale);
-void decode_gemm_acc(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias, torch::Tensor resid);
+                      double scale, bool past);
+void decode_gemm_acc(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias, torch::Tensor resid, bool past);
 void decode_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64_t kind);
 // rows_gemm.hip
 c10::optional<torch::Tensor> rows_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
-                                       c10::optional<torch::Tensor> out, bool fp32, bool in_order, bool gelu);
+                                       c10::optional<torch::Tensor> out, bool fp32, bool in_order, bool gelu, bool past);
 int64_t rows_gemm_tile(int64_t M, int64_t N, int64_t K, bool in_order);
 // packed_rows.hip
 void row_norm_add(c10::optional<torch::Tensor> tok, c10::optional<torch::Tensor> table,
@@ -84,9 +84,9 @@ void router_topk(c10::optional<torch::Tensor> logits, c10::optional<torch::Tenso
 void experts_plain(torch::Tensor h, torch::Tensor ids, torch::Tensor wgu, torch::Tensor wd, int64_t kind, double limit,
                    torch::Tensor act, torch::Tensor y);
 void experts_rows(torch::Tensor h, torch::Tensor ids, torch::Tensor wgu, torch::Tensor wd, int64_t kind, double limit,
-                  torch::Tensor act, torch::Tensor y);
+                  torch::Tensor act, torch::Tensor y, bool past);
 bool experts_rows_shared(torch::Tensor h, torch::Tensor ids, torch::Tensor wgu, torch::Tensor wd, double limit, torch::Tensor act,
-                         torch::Tensor y, torch::Tensor up, torch::Tensor down, torch::Tensor sact, torch::Tensor sy);
+                         torch::Tensor y, torch::Tensor up, torch::Tensor down, torch::Tensor sact, torch::Tensor sy, bool past);
 void experts_grouped(torch::Tensor h, torch::Tensor ids, torch::Tensor wgu, torch::Tensor wd, int64_t kind, double limit,
                      torch::Tensor act, torch::Tensor y, torch::Tensor perm, torch::Tensor tiles);
 void gelu_rows(torch::Tensor u);
@@ -147,26 +147,26 @@ PYBIND11_MODULE(penroz_serve, m) {
         pybind11::arg("eps"), pybind11::arg("w"), pybind11::arg("bias"), pybind11::arg("out"), pybind11::arg("act") = 0,
         pybind11::arg("rows_per_wave") = 0, pybind11::arg("emb_idx") = pybind11::none(),
         pybind11::arg("emb_wte") = pybind11::none(), pybind11::arg("emb_wpe") = pybind11::none(),
-        pybind11::arg("emb_pos") = pybind11::none(),
+        pybind11::arg("emb_pos") = pybind11::none(), pybind11::arg("past") = false,
         "decode GEMV for 1..4 rows: act(x · Wᵀ + bias), or act(LN(resid_in + delta + dbias) · Wᵀ + bias), or "
         "act(LN(wte[idx] + wpe[pos]) · Wᵀ + bias) with the embedding rows written to resid_out");
   m.def("decode_gemv_pair", &decode_gemv_pair, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("out"),
         pybind11::arg("mode"), pybind11::arg("kind") = 0, pybind11::arg("D") = 0, pybind11::arg("nrot") = 0,
         pybind11::arg("cos") = pybind11::none(), pybind11::arg("sin") = pybind11::none(),
-        pybind11::arg("pairs_per_wave") = 0,
+        pybind11::arg("pairs_per_wave") = 0, pybind11::arg("past") = false,
         "paired-row decode GEMV for 1..4 rows: gated MLP (mode 1) or RoPE QKV (mode 2) epilogue");
   m.def("decode_norm_pair", &decode_norm_pair, pybind11::arg("x"), pybind11::arg("a"), pybind11::arg("w1"), pybind11::arg("w2"),
         pybind11::arg("step"), pybind11::arg("eps1"), pybind11::arg("eps2"), pybind11::arg("h"), pybind11::arg("w"),
         pybind11::arg("out"), pybind11::arg("mode"), pybind11::arg("kind") = 0, pybind11::arg("D") = 0, pybind11::arg("nrot") = 0,
         pybind11::arg("cos") = pybind11::none(), pybind11::arg("sin") = pybind11::none(), pybind11::arg("tok") = pybind11::none(),
-        pybind11::arg("table") = pybind11::none(), pybind11::arg("scale") = 1.0,
+        pybind11::arg("table") = pybind11::none(), pybind11::arg("scale") = 1.0, pybind11::arg("past") = false,
         "decode_gemv_pair behind the residual add and norms of a Gemma block (rms_residual), for 1..4 rows");
   m.def("rows_gemm", &rows_gemm, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("bias"), pybind11::arg("out"),
-        pybind11::arg("fp32") = false, pybind11::arg("in_order") = false, pybind11::arg("gelu") = false);
+        pybind11::arg("fp32") = false, pybind11::arg("in_order") = false, pybind11::arg("gelu") = false, pybind11::arg("past") = false);
   m.def("rows_gemm_tile", &rows_gemm_tile, pybind11::arg("M"), pybind11::arg("N"), pybind11::arg("K"),
         pybind11::arg("in_order") = false);
   m.def("decode_gemm_acc", &decode_gemm_acc, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("bias"),
-        pybind11::arg("resid"),
+        pybind11::arg("resid"), pybind11::arg("past") = false,
         "batched decode: resid += x·wᵀ + bias (fp32 residual, in place)");
   m.def("decode_gemm", &decode_gemm, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("out"),
         pybind11::arg("kind") = -1,
@@ -190,8 +190,13 @@ PYBIND11_MODULE(penroz_serve, m) {
   m.def("latent_decode", &latent_decode, "latent attention of single rows over the cache, split over key ranges (MFMA)");
   m.def("latent_flash_ok", &latent_flash_ok, "latent_flash takes these sizes");
   m.def("latent_flash", &latent_flash, "causal attention of packed prompts / portions over expanded keys (MFMA)");
-  m.def("experts_rows", &experts_rows, "gated experts of few (token, expert) pairs (MFMA)");
-  m.def("experts_rows_shared", &experts_rows_shared);
+  m.def("experts_rows", &experts_rows, pybind11::arg("h"), pybind11::arg("ids"), pybind11::arg("wgu"), pybind11::arg("wd"),
+        pybind11::arg("kind"), pybind11::arg("limit"), pybind11::arg("act"), pybind11::arg("y"), pybind11::arg("past") = false,
+        "gated experts of few (token, expert) pairs (MFMA)");
+  m.def("experts_rows_shared", &experts_rows_shared, pybind11::arg("h"), pybind11::arg("ids"), pybind11::arg("wgu"),
+        pybind11::arg("wd"), pybind11::arg("limit"), pybind11::arg("act"), pybind11::arg("y"), pybind11::arg("up"),
+        pybind11::arg("down"), pybind11::arg("sact"), pybind11::arg("sy"), pybind11::arg("past") = false,
+        "experts_rows of ungated experts with a shared expert of twice their width in the same launches; False: nothing done");
   m.def("experts_grouped", &experts_grouped, "gated experts of pairs grouped by expert (MFMA tiles)");
   m.def("gated_rows", &gated_rows, "act(g)·u of packed [g | u] rows");
   m.def("gelu_rows", &gelu_rows, "gelu (erf form) in place");

@@ -443,19 +443,20 @@ __device__ __forceinline__ float other_half(float v, int half) {  // lane ^ 32
   return __uint_as_float(half ? r[0] : r[1]);
 }
 
-// 16 bytes of weights. NT: by a load that no cache keeps, 6.4 to 7.2 TB/s from memory where others take 5.7 to 6.3 (200 to 640 MB).
-// The vocabulary's projection, gate | up and long rows (K > 4608) are read so: nothing holds those from one step to the next, and
-// what they leave in the 256 MB in front of the memory is what a step finds there of its other weights. Generation of 64 tokens, GPT-2
-// 124M, one row: 14.95 -> 14.45 ms, but 14.94 with its layers' weights (170 MB) read so too; of 32 tokens, Gemma-3 1B, 3 rows: 34.9 ->
-// 33.4, 33.7 with QKV and output projections too. (A choice at run time costs a kernel 0.3 us.)
-template <bool NT>
+// 16 bytes of weights. PAST: by a load that no cache keeps, 6.4 to 7.2 TB/s from memory where others take 5.7 to 6.3 (200 to 640 MB).
+// The caller says so for weights that the 256 MB in front of the memory cannot hold from one step to the next (past_caches,
+// ops/gemm.py); what they leave there is what a step finds of its other weights. Generation of 64 tokens, GPT-2 124M, one row, the head
+// so: 14.95 -> 14.45 ms, but 14.94 with its layers' weights (170 MB) read so too; of 32 tokens, Gemma-3 1B, 3 rows: 34.9 -> 33.4, 33.7
+// with QKV and output projections too. Weights that the caches do hold are slower so: 2 x 1024 x 1792 gated, 22 MB in all, 4 rows 5.6 ->
+// 7.0 us, 6912 x 6912 24.0 -> 26.8. (Kernels of their own: a choice at run time costs one 0.3 us.)
+template <bool PAST>
 __device__ __forceinline__ uint4 weight16(const bf16* p) {
-  if constexpr (NT) return __builtin_bit_cast(uint4, __builtin_nontemporal_load(reinterpret_cast<const dl_u32x4*>(p)));
+  if constexpr (PAST) return __builtin_bit_cast(uint4, __builtin_nontemporal_load(reinterpret_cast<const dl_u32x4*>(p)));
   else return *reinterpret_cast<const uint4*>(p);
 }
 
 // PRO: 0 — x is the bf16 operand; 1 — LN mode (GPT: fp32 residual + delta + dbias, LayerNorm)
-template <int M, int PRO, int RP, int CPL>
+template <int M, int PRO, int RP, int CPL, bool PAST>
 __global__ void __launch_bounds__(64) decode_gemv_kernel(
     const float* __restrict__ rin, const bf16* __restrict__ delta, const float* __restrict__ dbias,
     float* __restrict__ rout, const float* __restrict__ gamma, const float* __restrict__ beta, float eps,
@@ -479,7 +480,7 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
   int cc[CPL];  // chunks past the row are read from its last one and count as zero
 #pragma unroll
   for (int i = 0; i < CPL; ++i) cc[i] = min(l32 + 32 * i, nc - 1);
-  uint4 wv[RP][CPL], xb[M][CPL];  // (8 rows per wave: the vocabulary's)
+  uint4 wv[RP][CPL], xb[M][CPL];
   auto weights = [&]() {
 #pragma unroll
     for (int rp = 0; rp < RP; ++rp) {
@@ -487,7 +488,7 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
 #pragma unroll
       for (int i = 0; i < CPL; ++i) {
         const int c = l32 + 32 * i;
-        wv[rp][i] = c < nc ? weight16<RP == 4>(wr + 8 * c) : uint4{0u, 0u, 0u, 0u};
+        wv[rp][i] = c < nc ? weight16<PAST>(wr + 8 * c) : uint4{0u, 0u, 0u, 0u};
       }
     }
   };
@@ -686,7 +687,7 @@ __global__ void __launch_bounds__(64) decode_gemv_kernel(
 // weight row that there was before, so long rows (K > 4608) are shared out two to a pair of waves: half the reads of x. us before /
 // now at 1, 3 and 4 rows: 1152 x 6912 5.3 / 5.2, 8.6 / 6.2, 9.9 / 6.7 (rows alone in 4 waves 6.8 at 3 rows, 4 rows in 4 waves 6.9, 8
 // in 7 waves 6.3), 768 x 3072 2.8 / 2.7, 3.3 / 3.0, 3.5 / 3.2, 1152 x 1024 2.4 / 2.4, 2.8 / 2.6, 3.0 / 2.7.
-template <int M, int RP, int NW, int CPL, bool ADD>
+template <int M, int RP, int NW, int CPL, bool ADD, bool PAST>
 __global__ void __launch_bounds__(64 * NW) decode_gemv_rows_kernel(const bf16* __restrict__ x, int64_t x_rs,
                                                                    const bf16* __restrict__ w, const bf16* __restrict__ bias,
                                                                    void* __restrict__ out, int64_t o_rs, int N, int K, int act) {
@@ -712,7 +713,7 @@ __global__ void __launch_bounds__(64 * NW) decode_gemv_rows_kernel(const bf16* _
 #pragma unroll
   for (int r = 0; r < RP; ++r)
 #pragma unroll
-    for (int i = 0; i < CPL; ++i) wv[r][i] = weight16<RP == 2>(w + (size_t)min(n0 + r, N - 1) * K + 8 * cc[i]);
+    for (int i = 0; i < CPL; ++i) wv[r][i] = weight16<PAST>(w + (size_t)min(n0 + r, N - 1) * K + 8 * cc[i]);
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("" : "+v"(bias_v), "+v"(old));  // asked for with the others: left to itself, each is fetched where it is needed
 #pragma unroll
@@ -778,7 +779,7 @@ struct PairNorm {
 // NORM: the first M waves each make a row of x from nm, while the weights are on their way; workgroup 0 writes h. Gated, 8 waves and
 // 2 pairs a wave, so that each CU repeats the rows' work at most twice, in 128 registers, so that it holds two (one with 132: 12.1 us).
 // In steps of Gemma-3 1B, 3 rows: step and QKV 4.0 + 3.5 us as two kernels, 5.4 as one, step and gate|up 4.0 + 8.6, 10.9 as one.
-template <int M, int RP, int CPL, int NW, bool GATED, bool NORM>
+template <int M, int RP, int CPL, int NW, bool GATED, bool NORM, bool PAST>
 __global__ void __launch_bounds__(64 * NW, NORM && CPL <= 5 ? 4 : 1) decode_gemv_pair_kernel(const bf16* __restrict__ x, int64_t x_rs,
                                                                    const bf16* __restrict__ w, bf16* __restrict__ out, int64_t o_rs,
                                                                    int N, int K, int kind, int D, int nrot,
@@ -796,7 +797,7 @@ __global__ void __launch_bounds__(64 * NW, NORM && CPL <= 5 ? 4 : 1) decode_gemv
     for (int r = 0; r < RP; ++r) {
       const int p = min(p0 + r, npair - 1), row = GATED ? p + h * npair : p / hd * D + p % hd + h * hd;
 #pragma unroll
-      for (int i = 0; i < CPL; ++i) wv[r][i] = weight16<GATED>(w + (size_t)row * K + 8 * min(l32 + 32 * i, nc - 1));
+      for (int i = 0; i < CPL; ++i) wv[r][i] = weight16<PAST>(w + (size_t)row * K + 8 * min(l32 + 32 * i, nc - 1));
     }
   };
   const int p = p0 + l32 / M;  // this lane's output pair, row l32 % M of x
@@ -1073,15 +1074,19 @@ void decode_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64_t ki
                      (int64_t)out.stride(0), M, N, K, (int)(gated ? kind : 0));
 }
 
-// decode_gemv_rows_kernel by the length of a row; M <= 4, K <= 8192
+// decode_gemv_rows_kernel by the length of a row; M <= 4, K <= 8192. past: weight16 (of rows of more than 4608 columns; shorter ones are
+// kept, what a model has of them fits the caches)
 template <bool ADD>
 static void gemv_rows_launch(const bf16* x, int64_t x_rs, const bf16* w, const bf16* bias, void* out, int64_t o_rs, int M, int N,
-                             int K, int act) {
+                             int K, int act, bool past) {
   auto stream = at::hip::getCurrentHIPStream();
   auto go = [&](auto mt, auto rpt, auto nwt, auto cplt) {
     constexpr int MM = decltype(mt)::value, RP = decltype(rpt)::value, NW = decltype(nwt)::value, CPL = decltype(cplt)::value;
-    hipLaunchKernelGGL((decode_gemv_rows_kernel<MM, RP, NW, CPL, ADD>), dim3((N + RP - 1) / RP), dim3(64 * NW), 0, stream, x, x_rs, w,
-                       bias, out, o_rs, N, K, act);
+    auto kern = decode_gemv_rows_kernel<MM, RP, NW, CPL, ADD, false>;
+    if constexpr (RP == 2) {
+      if (past) kern = decode_gemv_rows_kernel<MM, RP, NW, CPL, ADD, true>;
+    }
+    hipLaunchKernelGGL(kern, dim3((N + RP - 1) / RP), dim3(64 * NW), 0, stream, x, x_rs, w, bias, out, o_rs, N, K, act);
   };
   auto by_len = [&](auto mt) {
     using C1 = std::integral_constant<int, 1>;
@@ -1104,19 +1109,19 @@ static void gemv_rows_launch(const bf16* x, int64_t x_rs, const bf16* w, const b
   }
 }
 
-void gemv_add(const bf16* x, int64_t x_rs, const bf16* w, const bf16* bias, float* resid, int M, int N, int K) {
-  gemv_rows_launch<true>(x, x_rs, w, bias, resid, N, M, N, K, 0);
+void gemv_add(const bf16* x, int64_t x_rs, const bf16* w, const bf16* bias, float* resid, int M, int N, int K, bool past) {
+  gemv_rows_launch<true>(x, x_rs, w, bias, resid, N, M, N, K, 0, past);
 }
 
 // out[M, N] = act(x · Wᵀ + bias) for M <= 4 decode rows (decode_gemv_kernel). LN mode (x
 // undefined): x = LayerNorm(resid_in + delta + dbias) with γ / β, resid_out receives the sum.
-// act 0 none, 1 GELU (erf), 2 GELU (tanh). rows_per_wave 2, 4 or 8 (0: by N).
+// act 0 none, 1 GELU (erf), 2 GELU (tanh). rows_per_wave 2, 4 or 8 (0: by N). past: weight16, of 16384 outputs on and of long rows.
 void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> rin, c10::optional<torch::Tensor> delta,
                  c10::optional<torch::Tensor> dbias, c10::optional<torch::Tensor> rout,
                  c10::optional<torch::Tensor> gamma, c10::optional<torch::Tensor> beta, double eps, torch::Tensor w,
                  c10::optional<torch::Tensor> bias, torch::Tensor out, int64_t act, int64_t rows_per_wave,
                  c10::optional<torch::Tensor> emb_idx, c10::optional<torch::Tensor> emb_wte,
-                 c10::optional<torch::Tensor> emb_wpe, c10::optional<torch::Tensor> emb_pos) {
+                 c10::optional<torch::Tensor> emb_wpe, c10::optional<torch::Tensor> emb_pos, bool past) {
   const bool ln = !(x.has_value() && x->defined());
   const bool emb = emb_wte.has_value() && emb_wte->defined();
   const int64_t* eip = nullptr;
@@ -1207,7 +1212,8 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
     return e ? std::atoi(e) : 0;
   }();
   // a LayerNorm product of whole tiles: one workgroup normalises for 16 columns (decode_ln_few_kernel). The vocabulary's many columns
-  // stay with the waves below (50304 x 768, one row: 15.9 us through the caches, 77 MB at 4.9 TB/s)
+  // stay with the waves below (50304 x 768, 77 MB, one row, in steps of GPT-2 124M: 14.3 us through the caches, which hold part of it, 16.2
+  // past them)
   if (ln && !dp && rows_per_wave <= 0 && rpw_env <= 0 && K % 32 == 0 && N % 16 == 0 && N < 16384 && out.stride(0) % 4 == 0 &&
       reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0 && reinterpret_cast<uintptr_t>(bp) % 8 == 0) {
     const LnEmb e{eip, ewp, epp, eps_p, eV, eP};
@@ -1217,7 +1223,7 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
   }
   if (!ln && rows_per_wave <= 0 && N < 16384)
     return gemv_rows_launch<false>(xp, x_rs, reinterpret_cast<const bf16*>(w.data_ptr()), bp, out.data_ptr(), out.stride(0), M, N, K,
-                                   (int)act);
+                                   (int)act, past);
   const int cpl = (K / 8 + 31) / 32;
   int rpw = (int)rows_per_wave;
   // by shape: the vocabulary projection wants fewer, longer-lived waves (8 rows); behind a LayerNorm 4 rows, since every
@@ -1236,7 +1242,11 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
   auto launch = [&](auto mt, auto lnt, auto rpt, auto cplt) {
     constexpr int MM = decltype(mt)::value, RR = decltype(rpt)::value, CC = decltype(cplt)::value;
     constexpr int LL = decltype(lnt)::value ? 1 : 0;
-    hipLaunchKernelGGL((decode_gemv_kernel<MM, LL, RR, CC>), grid, dim3(64), 0, stream, rp, dp, dbp, rop, gp, bt,
+    auto kern = decode_gemv_kernel<MM, LL, RR, CC, false>;
+    if constexpr (RR == 4) {
+      if (past) kern = decode_gemv_kernel<MM, LL, RR, CC, true>;
+    }
+    hipLaunchKernelGGL(kern, grid, dim3(64), 0, stream, rp, dp, dbp, rop, gp, bt,
                        (float)eps, xp, x_rs, wp, bp, op, o_rs, N, K, (int)act, eip, ewp, epp, eps_p, eV, eP);
   };
   auto by_cpl = [&](auto mt, auto lnt, auto rpt) {
@@ -1285,10 +1295,10 @@ void decode_gemv(c10::optional<torch::Tensor> x, c10::optional<torch::Tensor> ri
 // Paired-row decode GEMV for 1..4 rows (decode_gemv_pair_kernel):
 //   mode 1 (gated): out[M, I] = act_f(x·Wgᵀ, kind) ⊙ (x·Wuᵀ), w = [Wg; Wu] [2I, K];
 //   mode 2 (RoPE QKV): out[M, (H + 2Hkv)·D] = rope(x · Wᵀ) for the first nrot heads, cos / sin [D/2].
-// x is given, or nm makes it.
+// x is given, or nm makes it. past: weight16, of gated weights.
 static void gemv_pair_launch(const bf16* xp, int64_t x_rs, const PairNorm* nm, int M, const torch::Tensor& w, const torch::Tensor& out,
                              int64_t mode, int64_t kind, int64_t D, int64_t nrot, const c10::optional<torch::Tensor>& cosv,
-                             const c10::optional<torch::Tensor>& sinv, int64_t pairs_per_wave, const char* who) {
+                             const c10::optional<torch::Tensor>& sinv, int64_t pairs_per_wave, bool past, const char* who) {
   const int N = w.size(0), K = w.size(1);
   TORCH_CHECK(mode == 1 || mode == 2, who, ": mode 1 (gated) or 2 (RoPE)");
   TORCH_CHECK(w.is_cuda() && w.scalar_type() == torch::kBFloat16 && w.dim() == 2 && w.is_contiguous() &&
@@ -1327,7 +1337,11 @@ static void gemv_pair_launch(const bf16* xp, int64_t x_rs, const PairNorm* nm, i
     constexpr bool GATED = decltype(et)::value, NORM = decltype(nt)::value;
     constexpr int NW = NORM && GATED ? 8 : 4;
     const dim3 grid((N / 2 + NW * RR - 1) / (NW * RR));
-    hipLaunchKernelGGL((decode_gemv_pair_kernel<MM, RR, CC, NW, GATED, NORM>), grid, dim3(64 * NW), 0, stream, xp, x_rs, wp, op, o_rs,
+    auto kern = decode_gemv_pair_kernel<MM, RR, CC, NW, GATED, NORM, false>;
+    if constexpr (GATED && (NORM || RR == 1)) {
+      if (past) kern = decode_gemv_pair_kernel<MM, RR, CC, NW, GATED, NORM, true>;
+    }
+    hipLaunchKernelGGL(kern, grid, dim3(64 * NW), 0, stream, xp, x_rs, wp, op, o_rs,
                        N, K, (int)kind, mode == 1 ? 2 : (int)D, (int)nrot, cp, sp, nm ? *nm : PairNorm{});
   };
   auto by_cpl = [&](auto mt, auto rpt, auto et, auto nt) {
@@ -1361,12 +1375,12 @@ static void gemv_pair_launch(const bf16* xp, int64_t x_rs, const PairNorm* nm, i
 
 void decode_gemv_pair(torch::Tensor x, torch::Tensor w, torch::Tensor out, int64_t mode, int64_t kind, int64_t D,
                       int64_t nrot, c10::optional<torch::Tensor> cosv, c10::optional<torch::Tensor> sinv,
-                      int64_t pairs_per_wave) {
+                      int64_t pairs_per_wave, bool past) {
   TORCH_CHECK(w.dim() == 2 && x.scalar_type() == torch::kBFloat16 && x.dim() == 2 && x.size(1) == w.size(1) && x.stride(1) == 1 &&
                   x.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
               "decode_gemv_pair: bf16 x [M, K], rows 16-B aligned");
   gemv_pair_launch(reinterpret_cast<const bf16*>(x.data_ptr()), x.stride(0), nullptr, (int)x.size(0), w, out, mode, kind, D, nrot, cosv,
-                   sinv, pairs_per_wave, "decode_gemv_pair");
+                   sinv, pairs_per_wave, past, "decode_gemv_pair");
 }
 
 // decode_gemv_pair of x' = rms(v)·w2 with v of `step` (PairNorm's modes 0 to 3); h [M, K] receives v (optional in mode 3 without
@@ -1375,7 +1389,7 @@ void decode_norm_pair(c10::optional<torch::Tensor> x, c10::optional<torch::Tenso
                       int64_t step, double eps1, double eps2, c10::optional<torch::Tensor> h, torch::Tensor w, torch::Tensor out,
                       int64_t mode, int64_t kind, int64_t D, int64_t nrot, c10::optional<torch::Tensor> cosv,
                       c10::optional<torch::Tensor> sinv, c10::optional<torch::Tensor> tok, c10::optional<torch::Tensor> table,
-                      double scale) {
+                      double scale, bool past) {
   const char* who = "decode_norm_pair";
   TORCH_CHECK(w.dim() == 2 && w.size(1) > 0 && step >= 0 && step <= 3, who, ": W [N, K], step 0 to 3");
   const int64_t K = w.size(1);
@@ -1416,5 +1430,5 @@ void decode_norm_pair(c10::optional<torch::Tensor> x, c10::optional<torch::Tenso
     nm.table = rows(*table, nm.vocab);
     nm.scale = (float)scale;
   }
-  gemv_pair_launch(nullptr, 0, &nm, (int)M, w, out, mode, kind, D, nrot, cosv, sinv, 0, who);
+  gemv_pair_launch(nullptr, 0, &nm, (int)M, w, out, mode, kind, D, nrot, cosv, sinv, 0, past, who);
 }

@@ -195,18 +195,18 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) rows_gemm_kernel(const bf16
 using namespace penroz;
 
 static void rg_launch(int tile, bool in_order, const torch::Tensor& x, const torch::Tensor& w, const bf16* bias,
-                      const torch::Tensor& out, int end) {
+                      const torch::Tensor& out, int end, bool past) {
   const int64_t M = x.size(0), N = w.size(0), K = x.size(1);
   auto stream = at::hip::getCurrentHIPStream();
-  // Weights of 16 MB and more that one workgroup each reads pass the caches, which keep the smaller ones of a decode step. us, from
-  // memory, kept / not: 16 x 8192 x 2048 9.1 / 8.1, 16 x 7232 x 2048 8.3 / 7.6, 16 x 12288 x 2048 14.0 / 12.8, 16 x 32768 x 1024
-  // 16.7 / 13.8; of 4 to 8 MB 2 % or nothing. ms: 64 tokens of GPT-2 124M, 64 rows 29.0 / 28.6, 12 rows 22.5 / 21.8; 32 of Zozenex large,
-  // 16 rows, 46.4 / 44.8 (with the tile below). Where all that the caches are left with fits them, a head of 64 MB is better kept:
-  // Zozenex small, 16 rows 33.9 / 34.1.
-  const bool large = N * K >= (int64_t)8 << 20;
+  // past: nothing holds the weights from one call to the next (past_caches, ops/gemm.py). Of 16 MB and more, each read by one workgroup,
+  // they pass the caches then, which keep the smaller ones of a decode step. us, from memory, kept / not: 16 x 8192 x 2048 9.1 / 8.1, 16 x
+  // 7232 x 2048 8.3 / 7.6, 16 x 12288 x 2048 14.0 / 12.8, 16 x 32768 x 1024 16.7 / 13.8; of 4 to 8 MB 2 % or nothing. Zozenex large, 16 rows,
+  // 32 tokens 46.4 / 44.8 ms (with the tile below). Weights that the caches hold come from there sooner: 32 x 8192 x 2048 14.9 / 19.7, 32 x 4096 x
+  // 2048, 117 MB in all, 6.6 / 7.6, 9 x 32768 x 2048 26.6 / 29.6.
+  const bool once = past && N * K >= (int64_t)8 << 20;
   auto launch = [&](auto kern, auto kern_once, int threads, int lds, int TM, int TN, auto* o) {
     const int64_t tiles_m = (M + TM - 1) / TM, tiles = tiles_m * ((N + TN - 1) / TN);
-    if (large && tiles_m == 1) kern = kern_once;
+    if (once && tiles_m == 1) kern = kern_once;
     hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(threads), lds, stream, reinterpret_cast<const bf16*>(x.data_ptr()),
                        reinterpret_cast<const bf16*>(w.data_ptr()), bias, o, (int)M, (int)N, (int)K, (int)x.stride(0),
@@ -235,9 +235,9 @@ static void rg_launch(int tile, bool in_order, const torch::Tensor& x, const tor
 }
 
 // x · wᵀ (+ bias) into out, or (none given) into a new tensor, fp32 or of x's type; in_order: each sum in one chain over k; gelu: its
-// gelu (erf form). None where rows_gemm_plan leaves the product to the library or a row is not of 16-byte pieces.
+// gelu (erf form); past: rg_launch. None where rows_gemm_plan leaves the product to the library or a row is not of 16-byte pieces.
 c10::optional<torch::Tensor> rows_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
-                                       c10::optional<torch::Tensor> out_opt, bool fp32, bool in_order, bool gelu) {
+                                       c10::optional<torch::Tensor> out_opt, bool fp32, bool in_order, bool gelu, bool past) {
   const bool given = out_opt.has_value() && out_opt->defined(), has_bias = bias.has_value() && bias->defined();
   if (!(x.is_cuda() && w.is_cuda() && x.get_device() == w.get_device() && x.scalar_type() == torch::kBFloat16 &&
         w.scalar_type() == torch::kBFloat16 && x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1)))
@@ -261,17 +261,17 @@ c10::optional<torch::Tensor> rows_gemm(torch::Tensor x, torch::Tensor w, c10::op
   }
   torch::Tensor out = given ? *out_opt : torch::empty({M, N}, x.options().dtype(fp32 ? torch::kFloat32 : torch::kBFloat16));
   const bf16* bp = has_bias ? reinterpret_cast<const bf16*>(bias->data_ptr()) : nullptr;
-  rg_launch(tile, in_order, x, w, bp, out, gelu ? kRgGelu : kRgPlain);
+  rg_launch(tile, in_order, x, w, bp, out, gelu ? kRgGelu : kRgPlain, past);
   return out;
 }
 
 int64_t rows_gemm_tile(int64_t M, int64_t N, int64_t K, bool in_order) { return rows_gemm_plan(M, N, K, in_order); }
 
 // decode_linear.hip
-void gemv_add(const bf16* x, int64_t x_rs, const bf16* w, const bf16* bias, float* resid, int M, int N, int K);
+void gemv_add(const bf16* x, int64_t x_rs, const bf16* w, const bf16* bias, float* resid, int M, int N, int K, bool past);
 
 // resid[M, N] += x · wᵀ + bias (fp32 residual, in place); up to 4 rows by decode_gemv's kernel (768 x 768 3.3 us here, 2.1 to 2.4 there)
-void decode_gemm_acc(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias, torch::Tensor resid) {
+void decode_gemm_acc(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias, torch::Tensor resid, bool past) {
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == torch::kBFloat16 && x.dim() == 2 && x.stride(1) == 1 &&
                   x.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
               "decode_gemm_acc: bf16 x [M, K], rows 16-B aligned");
@@ -297,9 +297,9 @@ void decode_gemm_acc(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tens
   }
   if (M <= 4 && K <= 8192 && N < 16384)
     return gemv_add(reinterpret_cast<const bf16*>(x.data_ptr()), x.stride(0), reinterpret_cast<const bf16*>(w.data_ptr()), bp,
-                    resid.data_ptr<float>(), (int)M, (int)N, (int)K);
+                    resid.data_ptr<float>(), (int)M, (int)N, (int)K, past);
   if (x.stride(0) >= (int64_t)1 << 30) x = x.contiguous();  // the kernel takes strides of 32 bits
   const int tile = rows_gemm_plan(M, N, K, false);
   const bool narrow = reinterpret_cast<uintptr_t>(resid.data_ptr()) % 16 != 0;
-  rg_launch(tile ? tile : 3, false, x, w, bp, resid, narrow ? kRgAdd | kRgNarrow : kRgAdd);
+  rg_launch(tile ? tile : 3, false, x, w, bp, resid, narrow ? kRgAdd | kRgNarrow : kRgAdd, past);
 }

@@ -185,6 +185,8 @@ class GPTDecodeProgram:
         # launches an extra bias-broadcast copy per call)
         self.out_bias = [(b.proj.bias.float(), b.fc2.bias.float()) for b in spec.blocks]
         self.device = dev
+        self.past, _ = gemm_ops.past_caches([l.weight for b in spec.blocks for l in (b.qkv, b.proj, b.fc, b.fc2)]
+                                            + [spec.head.weight])
 
     @staticmethod
     def build(model):
@@ -198,7 +200,7 @@ class GPTDecodeProgram:
 
     def _linear(self, x: Tensor, lin, bias: bool = True) -> Tensor:
         b = lin.bias if bias else None
-        y = gemm_ops.rows_linear(x, lin.weight, b)
+        y = gemm_ops.rows_linear(x, lin.weight, b, past=lin.weight.nbytes >= self.past)
         if y is not None:
             return y
         if x.shape[0] <= SKINNY_MAX_ROWS and gemm_ops.skinny_ok(x, lin.weight):
@@ -345,11 +347,13 @@ class GPTDecodeProgram:
             K.decode_gemv(None, x, d, pb, x2, w2, b2, e2, blk.fc.weight, blk.fc.bias, h, act)
             x, x2 = x2, x
             delta = torch.empty(rows, C, dtype=torch.bfloat16, device=x.device)
-            K.decode_gemv(h, None, None, None, None, None, None, 0.0, blk.fc2.weight, None, delta, 0)
+            K.decode_gemv(h, None, None, None, None, None, None, 0.0, blk.fc2.weight, None, delta, 0,
+                          past=blk.fc2.weight.nbytes >= self.past)
             dbias = fb
         wf, bf, ef = self.lnf
         logits = torch.empty(rows, sp.head.weight.shape[0], dtype=torch.bfloat16, device=x.device)
-        K.decode_gemv(None, x, delta, dbias, x2, wf, bf, ef, sp.head.weight, None, logits, 0)
+        K.decode_gemv(None, x, delta, dbias, x2, wf, bf, ef, sp.head.weight, None, logits, 0,
+                      past=sp.head.weight.nbytes >= self.past)
         return logits
 
     def _forward_batched(self, x: Tensor, rows: int, cache, emb=None) -> Tensor:
@@ -377,15 +381,16 @@ class GPTDecodeProgram:
             K.decode_gemm_acc(o.view(rows, C), blk.proj.weight, blk.proj.bias, x)
             h = torch.empty(rows, blk.fc.out_features, dtype=torch.bfloat16, device=x.device)
             K.decode_ln_gemm(x, w2, b2, e2, blk.fc.weight, blk.fc.bias, h, act)
-            K.decode_gemm_acc(h, blk.fc2.weight, blk.fc2.bias, x)
+            K.decode_gemm_acc(h, blk.fc2.weight, blk.fc2.bias, x, past=blk.fc2.weight.nbytes >= self.past)
         wf, bf, ef = self.lnf
         if rows <= 4:  # one row: LN in front of the product, whose waves all repeat it; more rows: once
             logits = torch.empty(rows, sp.head.weight.shape[0], dtype=torch.bfloat16, device=x.device)
+            past = sp.head.weight.nbytes >= self.past
             if rows == 1:
-                K.decode_gemv(None, x, None, None, None, wf, bf, ef, sp.head.weight, None, logits, 0)
+                K.decode_gemv(None, x, None, None, None, wf, bf, ef, sp.head.weight, None, logits, 0, past=past)
             else:
                 y, _, _ = norm_ops.ln_fwd(x, wf, bf, ef)
-                K.decode_gemv(y, None, None, None, None, None, None, 0.0, sp.head.weight, None, logits, 0)
+                K.decode_gemv(y, None, None, None, None, None, None, 0.0, sp.head.weight, None, logits, 0, past=past)
             return logits
         y, _, _ = norm_ops.ln_fwd(x, wf, bf, ef)
         return self._linear(y, sp.head)
@@ -435,6 +440,7 @@ class GemmaDecodeProgram:
                 post_attn=b.post_attn_norm, post_mlp=b.post_mlp_norm,
                 gu=_packed_gate_up(mlp), down=mlp.down_proj.weight,
                 kind=act_ops._GATED[mlp.act_kind], inter=mlp.gate_proj.out_features))
+        self.past, _ = gemm_ops.past_caches([b[k] for b in self.blocks for k in ("qkv", "o", "gu", "down")] + [head.weight])
 
     @staticmethod
     def build(model):
@@ -494,9 +500,9 @@ class GemmaDecodeProgram:
         def lin(x: Tensor, w: Tensor) -> Tensor:
             if gemv and w.shape[1] % 8 == 0 and w.shape[1] <= GEMV_MAX_K:
                 out = torch.empty(rows, w.shape[0], device=x.device, dtype=torch.bfloat16)
-                K.decode_gemv(x.contiguous(), None, None, None, None, None, None, 0.0, w, None, out, 0)
+                K.decode_gemv(x.contiguous(), None, None, None, None, None, None, 0.0, w, None, out, 0, past=w.nbytes >= self.past)
                 return out
-            return _linear(x, w)
+            return _linear(x, w, w.nbytes >= self.past)
 
         if gemv and DECODE_EPILOGUES and all(b["attn"].rope_theta is not None and b["attn"].head_dim % 2 == 0
                                              for b in self.blocks) and self._norm_pair_ok():
@@ -518,14 +524,14 @@ class GemmaDecodeProgram:
                     qkv = gemm_ops.skinny_qkv_rope(y, b["qkv"], cos, sin, D, H + Hkv).view(rows, 1, -1)
                 elif getattr(cache, "rope_attend_ok", None) is not None and cache.rope_attend_ok(rows, H, Hkv, D):
                     # 17-64 rows: q and the new key rotated inside the decode attention kernel
-                    qkv = _linear(y, b["qkv"]).view(rows, 1, -1)
+                    qkv = _linear(y, b["qkv"], b["qkv"].nbytes >= self.past).view(rows, 1, -1)
                     q, k, v = qkv.split([H * D, Hkv * D, Hkv * D], dim=2)
                     att = cache.attend_rope(l, q.reshape(rows, 1, H, D), k.view(rows, 1, Hkv, D),
                                             v.view(rows, 1, Hkv, D), cos, sin)
                     qkv = None
                 else:
-                    qkv = rope_ops.apply_rope_qkv(_linear(y, b["qkv"]).view(rows, 1, -1), H, Hkv, D, inv, 0,
-                                                  table=(cos, sin))
+                    qkv = _linear(y, b["qkv"], b["qkv"].nbytes >= self.past).view(rows, 1, -1)
+                    qkv = rope_ops.apply_rope_qkv(qkv, H, Hkv, D, inv, 0, table=(cos, sin))
             else:
                 qkv = lin(y, b["qkv"]).view(rows, 1, -1)
             if qkv is not None:
@@ -537,9 +543,9 @@ class GemmaDecodeProgram:
                                   pa.eps if pa is not None else 0.0, pre.eps)
             if gemv and DECODE_EPILOGUES:
                 g = torch.empty(rows, b["inter"], device=y.device, dtype=torch.bfloat16)
-                K.decode_gemv_pair(y.contiguous(), b["gu"], g, 1, b["kind"])
+                K.decode_gemv_pair(y.contiguous(), b["gu"], g, 1, b["kind"], past=b["gu"].nbytes >= self.past)
             else:
-                g = _gated(y, b["gu"], b["kind"])
+                g = _gated(y, b["gu"], b["kind"], b["gu"].nbytes >= self.past)
             d = lin(g, b["down"])
             nxt = self.blocks[l + 1]["in_norm"] if l + 1 < len(self.blocks) else self.norm_f
             x, y = K.rms_residual(h, d, pm.weight if pm is not None else None, nxt.weight, b["mode"],
@@ -566,17 +572,20 @@ class GemmaDecodeProgram:
             q, k, v = qkv.view(rows, 1, -1).split([H * D, Hkv * D, Hkv * D], dim=2)
             att = cache.attend(l, q.reshape(rows, 1, H, D), k.view(rows, 1, Hkv, D), v.view(rows, 1, Hkv, D))
             o = new(b["o"].shape[0])
-            K.decode_gemv(att.reshape(rows, H * D).contiguous(), None, None, None, None, None, None, 0.0, b["o"], None, o, 0)
+            K.decode_gemv(att.reshape(rows, H * D).contiguous(), None, None, None, None, None, None, 0.0, b["o"], None, o, 0,
+                          past=b["o"].nbytes >= self.past)
             post, mode, h, g = b["post_attn"], b["mode"], new(C), new(b["inter"])
             K.decode_norm_pair(x, o, post.weight if post is not None else None, pre.weight, mode,
-                               post.eps if post is not None else 0.0, pre.eps, h, b["gu"], g, 1, b["kind"])
+                               post.eps if post is not None else 0.0, pre.eps, h, b["gu"], g, 1, b["kind"],
+                               past=b["gu"].nbytes >= self.past)
             d = new(C)
-            K.decode_gemv(g, None, None, None, None, None, None, 0.0, b["down"], None, d, 0)
+            K.decode_gemv(g, None, None, None, None, None, None, 0.0, b["down"], None, d, 0, past=b["down"].nbytes >= self.past)
             x, post = h, b["post_mlp"]
         y = K.rms_residual(x, d, post.weight if post is not None else None, self.norm_f.weight, mode,
                            post.eps if post is not None else 0.0, self.norm_f.eps)[1]
         logits = torch.empty(rows, self.head.weight.shape[0], device=x.device, dtype=torch.bfloat16)
-        K.decode_gemv(y, None, None, None, None, None, None, 0.0, self.head.weight, None, logits, 0)
+        K.decode_gemv(y, None, None, None, None, None, None, 0.0, self.head.weight, None, logits, 0,
+                      past=self.head.weight.nbytes >= self.past)
         return logits
 
 
@@ -601,7 +610,7 @@ def _decode_gemm_ok(x: Tensor, w: Tensor, gated: bool = False) -> bool:
             and _ext.available("penroz_serve"))
 
 
-def _gated(x: Tensor, gu: Tensor, kind: int) -> Tensor:
+def _gated(x: Tensor, gu: Tensor, kind: int, past: bool = False) -> Tensor:
     """act(x·Wgᵀ) ⊙ (x·Wuᵀ) from the packed gate|up weight: one fused launch with the activation
     in the GEMM epilogue (the skinny kernel up to SKINNY_MAX_ROWS rows, decode_gemm up to 64), else
     GEMM + packed activation."""
@@ -611,13 +620,13 @@ def _gated(x: Tensor, gu: Tensor, kind: int) -> Tensor:
         out = torch.empty(x.shape[0], gu.shape[0] // 2, device=x.device, dtype=torch.bfloat16)
         _ext.kernels().decode_gemm(x, gu, out, kind)
         return out
-    return _ext.kernels().gated_act_packed(_linear(x, gu), kind)
+    return _ext.kernels().gated_act_packed(_linear(x, gu, past), kind)
 
 
-def _linear(x: Tensor, w: Tensor) -> Tensor:
-    """x [M, K] · wᵀ without bias: the kernel of short steps, what its rule leaves by the decode-shaped MFMA kernels up to
-    32 rows, else by the library."""
-    y = gemm_ops.rows_linear(x, w)
+def _linear(x: Tensor, w: Tensor, past: bool = False) -> Tensor:
+    """x [M, K] · wᵀ without bias: the kernel of short steps (``past``: past the caches), what its rule leaves by the
+    decode-shaped MFMA kernels up to 32 rows, else by the library."""
+    y = gemm_ops.rows_linear(x, w, past=past)
     if y is not None:
         return y
     if x.shape[0] <= SKINNY_MAX_ROWS and gemm_ops.skinny_ok(x, w):

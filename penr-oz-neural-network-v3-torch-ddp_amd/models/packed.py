@@ -27,50 +27,66 @@ from torch import Tensor, nn
 
 from penroz.models import layers as L
 from penroz.models.kv_cache import SequenceState
+from penroz.ops import gemm as gemm_ops
 from penroz.ops import linear_attn as linear_ops
 from penroz.ops import packed as ops
 from penroz.ops import window as window_ops
 
 
 # --------------------------------------------------------------------------- sublayers
-class _LatentMixer:
+class _Sublayer:
+    """``weights``, ``experts``: what a decode step multiplies its rows with; ``past``, ``experts_past``: what of it is read past
+    the caches (``gemm.past_caches``, of the whole program's)."""
+    past, experts, experts_past = gemm_ops.KEEP, (), False
+
+    @property
+    def weights(self) -> list[Tensor]:
+        return [t for t in self.w.values() if t is not None and t.dim() > 1]
+
+
+class _LatentMixer(_Sublayer):
     def __init__(self, m: L.LatentAttention, cache_index: int):
         self.s, self.w = m.sizes, m.packed()
         self.nw = m.dkv_norm.float() if m.kv_from is None else None
         self.cache_index = cache_index
         self.rotation = (m.sizes.base, m.sizes.rot)
 
+    @property
+    def weights(self) -> list[Tensor]:
+        return [self.w[k] for k in ("z", "uka", "uv", "o")]
+
     def run(self, h: Tensor, b: ops.PackedBatch, st: SequenceState) -> ops.Delta:
-        z = ops.linear(h, self.w["z"])
+        z = ops.linear(h, self.w["z"], self.past)
         o = ops.latent_attention(self.s, self.w, z, st.latent[self.cache_index], self.nw, st.tables[self.rotation], b)
-        return ops.Delta(ops.linear(o, self.w["o"]))
+        return ops.Delta(ops.linear(o, self.w["o"], self.past))
 
 
-class _WindowMixer:
+class _WindowMixer(_Sublayer):
     def __init__(self, m: L.WindowAttention, index: int):
         self.s, self.w, self.index = m.sizes, m.packed(), index
         self.pb = m.pb.float().contiguous()
 
     def attend(self, z: Tensor, b: ops.PackedBatch, st: SequenceState) -> Tensor:
         o = window_ops.window_attention(self.s, z, st.window[self.index], st.pooled[self.index], self.pb, st.tables, b)
-        return ops.linear(o, self.w["o"])
+        return ops.linear(o, self.w["o"], self.past)
 
     def run(self, h, b, st) -> ops.Delta:
-        return ops.Delta(self.attend(ops.linear(h, self.w["z"]), b, st))
+        return ops.Delta(self.attend(ops.linear(h, self.w["z"], self.past), b, st))
 
 
-class _LinearMixer:
+class _LinearMixer(_Sublayer):
     def __init__(self, m, index: int):
         self.s, self.w, self.index = m.sizes, m.packed(), index
 
     def attend(self, z: Tensor, b: ops.PackedBatch, st: SequenceState) -> Tensor:
-        return ops.linear(linear_ops.linear_attention(self.s, self.w, z, st.linear[self.index], b), self.w["o"])
+        return ops.linear(linear_ops.linear_attention(self.s, self.w, z, st.linear[self.index], b), self.w["o"],
+                          self.past)
 
     def run(self, h, b, st) -> ops.Delta:
-        return ops.Delta(self.attend(ops.linear(h, self.w["z"]), b, st))
+        return ops.Delta(self.attend(ops.linear(h, self.w["z"], self.past), b, st))
 
 
-class _ParallelMixer:
+class _ParallelMixer(_Sublayer):
     """Two mixers on one stacked projection of the same input."""
 
     def __init__(self, m: L.ParallelMixers, left, right):
@@ -78,34 +94,47 @@ class _ParallelMixer:
         self.z = torch.cat([left.w["z"], right.w["z"]]).contiguous()
         self.lw, self.rw = m.left_out.float().contiguous(), m.right_out.float().contiguous()
 
+    @property
+    def weights(self) -> list[Tensor]:
+        return [self.z] + [t for m in (self.left, self.right) for t in m.weights if t is not m.w["z"]]
+
     def run(self, h, b, st) -> ops.Delta:
-        z, n = ops.linear(h, self.z), self.left.s.width
+        z, n = ops.linear(h, self.z, self.past), self.left.s.width
         return ops.Delta(self.left.attend(z[:, :n], b, st), self.right.attend(z[:, n:], b, st), self.lw, self.rw, 0.5,
                          self.eps)
 
 
-class _DenseFF:
+class _DenseFF(_Sublayer):
     def __init__(self, m: L.GatedMLP):
         F, C = m.gate_proj.weight.shape
         Fp = (F + 7) // 8 * 8  # zero rows up to the kernels' vector width
         self.gu = torch.cat([ops._pad(m.gate_proj.weight, 0, Fp), ops._pad(m.up_proj.weight, 0, Fp)]).contiguous()
         self.down = ops._pad(m.down_proj.weight, 1, Fp).contiguous()
 
+    @property
+    def weights(self) -> list[Tensor]:
+        return [self.gu, self.down]
+
     def run(self, h: Tensor, b, st) -> ops.Delta:
-        return ops.Delta(ops.linear(ops.gated_linear(h, self.gu, 0), self.down))
+        return ops.Delta(ops.linear(ops.gated_linear(h, self.gu, 0, past=self.past), self.down, self.past))
 
 
-class _Experts:
+class _Experts(_Sublayer):
     def __init__(self, m: L.MixtureOfExperts):
         self.w, self.kind, self.limit = m.packed(), m.kind, m.limit
         self.router, self.rule = m.routing()
         self.shared = None if m.shared is None else m.shared.packed()
+        self.experts = (self.w["gu"], self.w["down"])
+
+    @property
+    def weights(self) -> list[Tensor]:
+        return [self.router] + ([] if self.shared is None else list(self.shared.values()))
 
     def run(self, h: Tensor, b, st) -> ops.Delta:
         ids, wts = ops.route(h, self.router, **self.rule)
         if self.shared is None:
-            return ops.Delta(ops.experts(h, ids, self.w, self.kind, self.limit), pair_w=wts)
-        y, shared = ops.experts_beside_shared(h, ids, self.w, self.kind, self.limit, self.shared)
+            return ops.Delta(ops.experts(h, ids, self.w, self.kind, self.limit, self.experts_past), pair_w=wts)
+        y, shared = ops.experts_beside_shared(h, ids, self.w, self.kind, self.limit, self.shared, self.past, self.experts_past)
         return ops.Delta(y, pair_w=wts, shared=shared)
 
 
@@ -246,6 +275,12 @@ class PackedProgram:
             self.steps.append((e, self._sublayer(sub), post))
         # the output scale rides on the final norm's weight
         self.norm_f = (plan.norm.weight.float() * plan.head_scale, plan.norm.groups, plan.norm.eps)
+        subs = [sub for _, sub, _ in self.steps]
+        self.past, experts_past = gemm_ops.past_caches([w for s in subs for w in s.weights] + [self.head],
+                                                       [w for s in subs for w in s.experts])
+        for s in subs + [m for s in subs if isinstance(s, _ParallelMixer) for m in (s.left, s.right)]:
+            s.past = self.past
+            s.experts_past = experts_past
 
     def _sublayer(self, m: nn.Module):
         if isinstance(m, L.MixtureOfExperts):
@@ -299,7 +334,7 @@ class PackedProgram:
         if want is not None and want.numel() == 0:
             return None
         w, groups, eps = self.norm_f
-        return ops.logits(ops.row_norm(x, w, groups, eps, self.dtype, rows=want), self.head)
+        return ops.logits(ops.row_norm(x, w, groups, eps, self.dtype, rows=want), self.head, self.past)
 
 
 class PackedSession:

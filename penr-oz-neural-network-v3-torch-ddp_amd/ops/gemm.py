@@ -94,20 +94,44 @@ def wgrad_together(shapes: tuple, tokens: int, device: torch.device, shared: boo
     return _wgrad_tile(shapes, tokens, torch.cuda.get_device_properties(device).multi_processor_count, shared) != 0
 
 
+# ---- weights that a decode step reads past the caches ----------------------------------------
+# Of the 256 MB in front of the memory keys, values, states and activations have a part. A model of up to CACHE_BYTES is left to them;
+# of a larger one they are to hold the smaller weights, up to HELD_BYTES. ms with nothing past them / this rule / all of the larger ones:
+# 32 tokens of GPT-2 124M (247 MB), 1 and 64 rows 8.44 / 8.31 / 8.38 and 15.4 / 14.8 / 14.7, with 5 layers (148 MB), 1 row 4.12 / 4.12 /
+# 4.14; Gemma-3 1B, 3 rows 33.3 / 31.7 / 32.0; two layers of its width and a vocabulary of 32768 (150 MB), 1 row 3.08 / 3.08 / 3.14. Room for
+# 192 MB instead of 128 beside experts that pass: Zozenex small, 48 tokens, 16 rows 26.2 -> 26.7, 64 rows 32.2 -> 32.9.
+CACHE_BYTES, HELD_BYTES = 192 << 20, 128 << 20
+KEEP = 1 << 62  # a size that no weight has
+
+
+def past_caches(weights, experts=()) -> tuple[int, bool]:
+    """What of the weights that a decode step multiplies its rows with should pass the caches (loads that keep nothing): the size
+    in bytes from which on ``weights`` do, and whether ``experts`` (of which each step reads others) do."""
+    sizes = sorted(w.nbytes for w in weights)
+    if sum(sizes) + sum(w.nbytes for w in experts) <= CACHE_BYTES:
+        return KEEP, False
+    held = 0
+    for size in dict.fromkeys(sizes):
+        held += size * sizes.count(size)
+        if held > HELD_BYTES:
+            return size, True
+    return KEEP, True
+
+
 # ---- linear layers of short steps (csrc/kernels/rows_gemm.hip) ------------------------------
 ROWS_GEMM = os.environ.get("PENROZ_ROWS_GEMM", "1") != "0"  # "0": the library (A/B)
 
 
 def rows_linear(x: Tensor, w: Tensor, bias: Tensor | None = None, out: Tensor | None = None,
-                fp32: bool = False, in_order: bool = False, gelu: bool = False) -> Tensor | None:
+                fp32: bool = False, in_order: bool = False, gelu: bool = False, past: bool = False) -> Tensor | None:
     """x [M, K] · wᵀ (+ bias), bf16 (``fp32``: the sums themselves; ``in_order``: each sum in one chain over k; ``gelu``: the
-    erf gelu of the bf16 result), by the kernel of short steps; None for what its rule (``rows_gemm_plan`` in
-    ``csrc/kernels/host_plan.h``) leaves to the library."""
+    erf gelu of the bf16 result; ``past``: :func:`past_caches`), by the kernel of short steps; None for what its rule
+    (``rows_gemm_plan`` in ``csrc/kernels/host_plan.h``) leaves to the library."""
     if not (ROWS_GEMM and x.is_cuda and x.dtype == torch.bfloat16 and use_kernels(x)):
         return None
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, w, bias)):
         return None
-    return kernels().rows_gemm(x, w, bias, out, fp32, in_order, gelu)
+    return kernels().rows_gemm(x, w, bias, out, fp32, in_order, gelu, past)
 
 
 def linear(x: Tensor, w: Tensor, bias: Tensor | None = None, out: Tensor | None = None) -> Tensor:
@@ -181,9 +205,9 @@ def _apply(mod: torch.nn.Module, x: Tensor, device: int) -> Tensor:
     return mod(x)
 
 
-def linear_fp32(x: Tensor, w: Tensor) -> Tensor:
+def linear_fp32(x: Tensor, w: Tensor, past: bool = False) -> Tensor:
     """x [M, K] · wᵀ of bf16 operands in fp32."""
-    y = rows_linear(x, w, fp32=True)
+    y = rows_linear(x, w, fp32=True, past=past)
     return torch.mm(x, w.t(), out_dtype=torch.float32) if y is None else y
 
 

@@ -244,41 +244,42 @@ def _gemv_ok(x: Tensor, w: Tensor, max_k: int) -> bool:
             and w.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0 and x.is_contiguous())
 
 
-def linear(x: Tensor, w: Tensor) -> Tensor:
-    """x [M, K] · wᵀ in x's dtype (decode-shaped kernels at few rows, the library GEMM otherwise)."""
+def linear(x: Tensor, w: Tensor, past: int = gemm_ops.KEEP) -> Tensor:
+    """x [M, K] · wᵀ in x's dtype (decode-shaped kernels at few rows, the library GEMM otherwise). ``past``, here and below:
+    weights from this size on are read past the caches (``gemm.past_caches``)."""
     if x.is_cuda and x.dtype == torch.bfloat16:
         if _gemv_ok(x, w, 8192):
             out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
-            kernels().decode_gemv(x, None, None, None, None, None, None, 0.0, w, None, out, 0)
+            kernels().decode_gemv(x, None, None, None, None, None, None, 0.0, w, None, out, 0, past=w.nbytes >= past)
             return out
         from penroz.models.graph_decode import _linear
-        return _linear(x, w)
+        return _linear(x, w, w.nbytes >= past)
     return torch.mm(x, w.t())
 
 
-def logits(h: Tensor, table: Tensor) -> Tensor:
+def logits(h: Tensor, table: Tensor, past: int = gemm_ops.KEEP) -> Tensor:
     """fp32 (bf16 at decode-shaped row counts) logits of normed rows over the embedding table."""
     if h.is_cuda and h.dtype == torch.bfloat16:
         if h.shape[0] <= 4 and _gemv_ok(h, table, 8192):
-            return linear(h, table)
+            return linear(h, table, past)
         if h.shape[0] <= 16 and gemm_ops.skinny_ok(h, table):
-            y = gemm_ops.rows_linear(h, table)
+            y = gemm_ops.rows_linear(h, table, past=table.nbytes >= past)
             return gemm_ops.skinny_linear(h, table, None) if y is None else y
-        return gemm_ops.linear_fp32(h, table)
+        return gemm_ops.linear_fp32(h, table, past=table.nbytes >= past)
     return torch.mm(h, table.t()).float()
 
 
-def gated_linear(x: Tensor, gu: Tensor, kind: int, limit: float = 0.0) -> Tensor:
+def gated_linear(x: Tensor, gu: Tensor, kind: int, limit: float = 0.0, past: int = gemm_ops.KEEP) -> Tensor:
     """act(x·Wgᵀ, x·Wuᵀ) of the packed [gate; up] weight; kind 0 silu, 1 clamped (``expert_activation``)."""
     if x.is_cuda:
         from penroz.models.graph_decode import DECODE_EPILOGUES, SKINNY_MAX_ROWS
         if kind == 0 and DECODE_EPILOGUES and _gemv_ok(x, gu, 1792):
             out = torch.empty(x.shape[0], gu.shape[0] // 2, dtype=x.dtype, device=x.device)
-            kernels().decode_gemv_pair(x, gu, out, 1, 2)
+            kernels().decode_gemv_pair(x, gu, out, 1, 2, past=gu.nbytes >= past)
             return out
         if (kind == 0 and DECODE_EPILOGUES and x.shape[0] <= SKINNY_MAX_ROWS and gemm_ops.skinny_ok(x, gu)):
             return gemm_ops.skinny_gated(x, gu, 2)
-        z = linear(x, gu)
+        z = linear(x, gu, past)
         out = torch.empty(x.shape[0], gu.shape[0] // 2, dtype=x.dtype, device=x.device)
         kernels().gated_rows(z, kind, float(limit), out)
         return out
@@ -286,20 +287,20 @@ def gated_linear(x: Tensor, gu: Tensor, kind: int, limit: float = 0.0) -> Tensor
     return expert_activation(g.float(), u.float(), kind, limit).to(x.dtype)
 
 
-def gelu_mlp(x: Tensor, up: Tensor, down: Tensor) -> Tensor:
+def gelu_mlp(x: Tensor, up: Tensor, down: Tensor, past: int = gemm_ops.KEEP) -> Tensor:
     """gelu(x · upᵀ) · downᵀ (erf form, no biases)."""
     if x.is_cuda:
         if _gemv_ok(x, up, 8192):
             u = torch.empty(x.shape[0], up.shape[0], dtype=x.dtype, device=x.device)
-            kernels().decode_gemv(x, None, None, None, None, None, None, 0.0, up, None, u, 1)
+            kernels().decode_gemv(x, None, None, None, None, None, None, 0.0, up, None, u, 1, past=up.nbytes >= past)
         else:
-            u = gemm_ops.rows_linear(x, up, gelu=True)
+            u = gemm_ops.rows_linear(x, up, gelu=True, past=up.nbytes >= past)
             if u is None:
-                u = linear(x, up)
+                u = linear(x, up, past)
                 kernels().gelu_rows(u)
     else:
         u = torch.nn.functional.gelu(torch.mm(x, up.t()).float()).to(x.dtype)
-    return linear(u, down)
+    return linear(u, down, past)
 
 
 def expert_activation(g: Tensor | None, u: Tensor, kind: int, limit: float) -> Tensor:
@@ -502,7 +503,8 @@ def route(h: Tensor, wr: Tensor, top: int, renorm: bool = False, *, sigmoid: boo
     return ids.int(), (wts if g is None else torch.cat([wts, torch.sigmoid(g)], dim=1))
 
 
-def experts_beside_shared(h: Tensor, ids: Tensor, w: dict, kind: int, limit: float, shared: dict) -> tuple[Tensor, Tensor]:
+def experts_beside_shared(h: Tensor, ids: Tensor, w: dict, kind: int, limit: float, shared: dict, past: int = gemm_ops.KEEP,
+                          experts_past: bool = False) -> tuple[Tensor, Tensor]:
     """:func:`experts` and :func:`gelu_mlp` of a shared expert on the same rows, in the same launches where there are kernels for that
     (``experts_rows_shared`` in csrc/kernels/experts.hip)."""
     if (kind == UNGATED and h.shape[0] <= 16 and h.dtype == torch.bfloat16 and use_kernels(h) and h.shape[1] % 32 == 0
@@ -510,13 +512,15 @@ def experts_beside_shared(h: Tensor, ids: Tensor, w: dict, kind: int, limit: flo
         (P, C), F, S = (ids.numel(), h.shape[1]), w["down"].shape[2], shared["up"].shape[0]
         act, y, hidden, out = (torch.empty(n, m, dtype=h.dtype, device=h.device)
                                for n, m in ((P, F), (P, C), (h.shape[0], S), (h.shape[0], C)))
-        if kernels().experts_rows_shared(h, ids, w["gu"], w["down"], float(limit), act, y, shared["up"], shared["down"], hidden, out):
+        if kernels().experts_rows_shared(h, ids, w["gu"], w["down"], float(limit), act, y, shared["up"], shared["down"], hidden, out,
+                                         experts_past):
             return y, out
-    return experts(h, ids, w, kind, limit), gelu_mlp(h, **shared)
+    return experts(h, ids, w, kind, limit, experts_past), gelu_mlp(h, **shared, past=past)
 
 
-def experts(h: Tensor, ids: Tensor, w: dict, kind: int, limit: float) -> Tensor:
-    """Outputs of the chosen experts, one row per (token, choice): [N·top, C]."""
+def experts(h: Tensor, ids: Tensor, w: dict, kind: int, limit: float, past: bool = False) -> Tensor:
+    """Outputs of the chosen experts, one row per (token, choice): [N·top, C]. ``past``: few pairs read the weights past the caches
+    (``gemm.past_caches``)."""
     P, C, F = ids.numel(), h.shape[1], w["down"].shape[2]
     if use_kernels(h):
         act = torch.empty(P, F, dtype=h.dtype, device=h.device)
@@ -525,7 +529,7 @@ def experts(h: Tensor, ids: Tensor, w: dict, kind: int, limit: float) -> Tensor:
         if h.dtype != torch.bfloat16 or C % 32:
             K.experts_plain(*a)
         elif P <= EXPERT_ROWS_MAX_PAIRS:
-            K.experts_rows(*a)
+            K.experts_rows(*a, past)
         else:
             i32 = dict(dtype=torch.int32, device=h.device)
             top, E = ids.shape[1], w["gu"].shape[0]
