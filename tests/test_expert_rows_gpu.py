@@ -22,7 +22,8 @@ def _chosen(N, E, top, spread):
                                             (512, 64, 2, 64)])
 # widths: every kernel of 256 columns per step, and widths in between, off 64 columns, and above
 @pytest.mark.parametrize("kind,C,F", [(P.UNGATED, 256, 512), (1, 512, 256), (1, 768, 1024), (P.UNGATED, 1024, 768), (1, 1536, 32),
-                                      (P.UNGATED, 2048, 1536), (0, 2304, 96), (P.UNGATED, 32, 2048), (1, 160, 1280), (0, 2080, 64)])
+                                      (P.UNGATED, 2048, 1536), (0, 2304, 96), (P.UNGATED, 32, 2048), (1, 160, 1280), (0, 2080, 64),
+                                      (0, 1664, 448)])
 def test_expert_rows(N, E, top, spread, kind, C, F):
     torch.manual_seed(N + 31 * E + C)
     ids = _chosen(N, E, top, spread)
