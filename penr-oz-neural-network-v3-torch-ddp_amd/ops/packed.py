@@ -518,6 +518,17 @@ def experts_beside_shared(h: Tensor, ids: Tensor, w: dict, kind: int, limit: flo
     return experts(h, ids, w, kind, limit, experts_past), gelu_mlp(h, **shared, past=past)
 
 
+def few_pairs(P: int, w: dict) -> bool:
+    """Whether ``P`` (token, choice) pairs of bf16 experts are the few-pairs kernel's: it reads an expert's weights again for every 16 of
+    its pairs, where the tiles of ``experts_grouped`` read them once behind a sort (13 to 20 us). Both products, gated, us, few pairs /
+    tiles at 32 and 96 pairs per expert: 8 experts, C 2048, F 1024 54 / 38 and 129 / 53; 4 of them (48 MB) 36 / 34 and 81 / 50; 8, C 1024,
+    F 768 (36 MB) 29 / 26 and 63 / 36; 8, C 512, F 512 (12 MB) 15 / 17 and 29 / 22; 2, C 2048, F 1024 24 / 33 and 47 / 49, but 59 / 50 at 128."""
+    E, F, C = w["gu"].shape[0], w["down"].shape[2], w["down"].shape[1]
+    large = E >= 4 and w["gu"].nbytes + w["down"].nbytes >= 36 << 20
+    many = P >= max(96 * E, 256) or (large and P >= 32 * E)
+    return P <= EXPERT_ROWS_MAX_PAIRS and not (many and 2 * F * C < 1 << 31)  # (the tiles' byte offsets have 32 bits)
+
+
 def experts(h: Tensor, ids: Tensor, w: dict, kind: int, limit: float, past: bool = False) -> Tensor:
     """Outputs of the chosen experts, one row per (token, choice): [N·top, C]. ``past``: few pairs read the weights past the caches
     (``gemm.past_caches``)."""
@@ -528,7 +539,7 @@ def experts(h: Tensor, ids: Tensor, w: dict, kind: int, limit: float, past: bool
         K, a = kernels(), (h, ids, w["gu"], w["down"], kind, float(limit), act, y)
         if h.dtype != torch.bfloat16 or C % 32:
             K.experts_plain(*a)
-        elif P <= EXPERT_ROWS_MAX_PAIRS:
+        elif few_pairs(P, w):
             K.experts_rows(*a, past)
         else:
             i32 = dict(dtype=torch.int32, device=h.device)

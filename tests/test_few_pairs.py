@@ -1,0 +1,68 @@
+"""Which kernel a step's experts take (ops/packed.py: few_pairs), and both against float64 on either side of the line."""
+import pytest
+import torch
+
+from penroz.ops import packed as P
+
+DEV = "cuda"
+
+
+def _w(E, C, F, gated=True):
+    t = lambda *s: torch.empty(*s, dtype=torch.bfloat16, device="meta")
+    return {"gu": t(E, 2 * F if gated else F, C), "down": t(E, C, F)}
+
+
+@pytest.mark.parametrize("w,P_,few", [
+    (_w(64, 2048, 1024), 1024, True), (_w(64, 2048, 1024), 1025, False),  # the pair list
+    (_w(8, 2048, 1024), 255, True), (_w(8, 2048, 1024), 256, False),      # 32 pairs per expert of large ones
+    (_w(4, 2048, 1024), 128, False), (_w(4, 2048, 1024, gated=False), 128, True),  # 48 and 32 MB
+    (_w(4, 64, 64), 383, True), (_w(4, 64, 64), 384, False),              # 96 of any
+    (_w(2, 4096, 4096), 255, True), (_w(1, 64, 64), 256, False),          # of two or one, 256 in all
+    (_w(1, 32768, 32768), 1024, True),                                    # past the tiles' 32-bit offsets
+    (_w(8, 2048, 1024), 0, True),
+])
+def test_rule(w, P_, few):
+    assert P.few_pairs(P_, w) == few
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,E,C,F,N,top", [(1, 8, 2048, 800, 127, 2), (1, 8, 2048, 800, 128, 2), (P.UNGATED, 3, 96, 160, 95, 3),
+                                              (P.UNGATED, 3, 96, 160, 96, 3), (0, 1, 32, 32, 255, 1), (0, 1, 32, 32, 256, 1), (1, 5, 544, 64, 200, 5)])
+def test_either_side(kind, E, C, F, N, top):
+    g = torch.Generator().manual_seed(E + N)
+    ids = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(N)])
+    r = lambda *s, scale=1.0: (torch.randn(*s, generator=g) * scale).bfloat16().to(DEV)
+    h, wg, u, d = r(N, C), r(E, F, C, scale=C ** -0.5), r(E, F, C, scale=C ** -0.5), r(E, C, F, scale=F ** -0.5)
+    gated = kind != P.UNGATED
+    y = P.experts(h, ids.int().to(DEV), P.pack_experts(wg if gated else None, u, d), kind, 0.7).view(N, top, C).double()
+    for e in range(E):
+        t, k = (ids == e).nonzero(as_tuple=True)
+        x = h[t.to(DEV)].double()
+        a = P.expert_activation(x @ wg[e].double().t() if gated else None, x @ u[e].double().t(), kind, 0.7)
+        want = a @ d[e].double().t()
+        # the hidden row is rounded to bf16 (2^-9), and the result (2^-9); fp32 sums of C and F terms are far below
+        tol = 2.0 ** -8 * (a.abs() @ d[e].double().abs().t()) + 2.0 ** -8 * want.abs() + 1e-6
+        assert torch.all((y[t.to(DEV), k.to(DEV)] - want).abs() <= tol), e
+
+
+@pytest.mark.gpu
+def test_tiles_in_a_captured_step():
+    """What was a captured step of the few-pairs kernel is one of the sort and the tiles: every replay on new rows and choices."""
+    E, C, F, N, top = 8, 2048, 800, 128, 2
+    g = torch.Generator(device=DEV).manual_seed(5)
+    r = lambda *s, scale=1.0: (torch.randn(*s, generator=g, device=DEV) * scale).bfloat16()
+    w = {"gu": r(E, F, C, scale=C ** -0.5), "down": r(E, C, F, scale=F ** -0.5)}
+    assert not P.few_pairs(N * top, w)
+    choose = lambda: torch.rand(N, E, generator=g, device=DEV).topk(top, dim=1).indices.int()
+    h, ids = r(N, C), choose()
+    P.experts(h, ids, w, P.UNGATED, 0.0)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = P.experts(h, ids, w, P.UNGATED, 0.0)
+    for _ in range(4):
+        h.copy_(r(N, C))
+        ids.copy_(choose())
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, P.experts(h, ids, w, P.UNGATED, 0.0))

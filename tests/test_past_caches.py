@@ -111,6 +111,7 @@ def test_experts(N, E, top, kind, C, F):
     ids = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(i))[:top] for i in range(N)]).int().to(DEV)
     w = {"gu": _randn(E, F if kind == P.UNGATED else 2 * F, C, seed=8, scale=C ** -0.5), "down": _randn(E, C, F, seed=9, scale=F ** -0.5)}
     h = _randn(N, C, seed=10)
+    assert P.few_pairs(N * top, w)
     a, b = (P.experts(h, ids, w, kind, 0.7, past) for past in (False, True))
     assert torch.equal(a, b) and a.isfinite().all()
 
