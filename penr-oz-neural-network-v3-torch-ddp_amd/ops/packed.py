@@ -24,6 +24,8 @@ def upload(values, dtype: torch.dtype, device: torch.device) -> Tensor:
     t = torch.tensor(values, dtype=dtype)
     if device.type != "cuda" or t.numel() == 0:
         return t.to(device)
+    if torch.cuda.is_current_stream_capturing():  # each replay would copy what the pinned block holds by then
+        raise RuntimeError("a captured graph cannot bring values from the host: make them tensors before the capture")
     return t.pin_memory().to(device, non_blocking=True)
 
 

@@ -511,3 +511,28 @@ def test_key_ranges_fill_the_gpu_without_tiny_ranges():
         p = P.key_ranges(rows, heads, n)
         assert 1 <= p <= P.MAX_KEY_RANGES and (p == 1 or n / p >= 32)
         assert p == 1 or rows * math.ceil(heads / 32) * (p - 1) < P.DECODE_WORKGROUPS
+
+
+def test_upload_is_no_part_of_a_graph(monkeypatch):
+    """Refused before anything reaches the device or the host's allocator, where a capture would keep the pinned block's address."""
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    monkeypatch.setattr(torch.Tensor, "pin_memory", lambda t: pytest.fail("pinned under capture"))
+    with pytest.raises(RuntimeError, match="captured graph"):
+        P.upload([1, 2], torch.int32, torch.device("cuda"))
+    assert torch.equal(P.upload([1, 2], torch.int32, torch.device("cpu")), torch.tensor([1, 2], dtype=torch.int32))
+
+
+@pytest.mark.gpu
+def test_upload_refused_under_capture():
+    dev = torch.device("cuda")
+    x = P.upload([3, 4], torch.int64, dev)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        with pytest.raises(RuntimeError, match="captured graph"):
+            P.upload([1, 2], torch.int64, dev)
+        y = x + 1
+    for _ in range(3):
+        assert torch.equal(P.upload([5, 6], torch.int64, dev).cpu(), torch.tensor([5, 6]))
+        graph.replay()
+        assert torch.equal(y.cpu(), torch.tensor([4, 5]))
