@@ -85,8 +85,9 @@ void experts_plain(torch::Tensor h, torch::Tensor ids, torch::Tensor wgu, torch:
                    torch::Tensor act, torch::Tensor y);
 void experts_rows(torch::Tensor h, torch::Tensor ids, torch::Tensor wgu, torch::Tensor wd, int64_t kind, double limit,
                   torch::Tensor act, torch::Tensor y, bool past);
-bool experts_rows_shared(torch::Tensor h, torch::Tensor ids, torch::Tensor wgu, torch::Tensor wd, double limit, torch::Tensor act,
-                         torch::Tensor y, torch::Tensor up, torch::Tensor down, torch::Tensor sact, torch::Tensor sy, bool past);
+c10::optional<std::tuple<torch::Tensor, torch::Tensor>> experts_rows_shared(torch::Tensor h, torch::Tensor ids, torch::Tensor wgu,
+                                                                            torch::Tensor wd, double limit, torch::Tensor up,
+                                                                            torch::Tensor down, bool past);
 void experts_grouped(torch::Tensor h, torch::Tensor ids, torch::Tensor wgu, torch::Tensor wd, int64_t kind, double limit,
                      torch::Tensor act, torch::Tensor y, torch::Tensor perm, torch::Tensor tiles);
 void gelu_rows(torch::Tensor u);
@@ -194,9 +195,8 @@ PYBIND11_MODULE(penroz_serve, m) {
         pybind11::arg("kind"), pybind11::arg("limit"), pybind11::arg("act"), pybind11::arg("y"), pybind11::arg("past") = false,
         "gated experts of few (token, expert) pairs (MFMA)");
   m.def("experts_rows_shared", &experts_rows_shared, pybind11::arg("h"), pybind11::arg("ids"), pybind11::arg("wgu"),
-        pybind11::arg("wd"), pybind11::arg("limit"), pybind11::arg("act"), pybind11::arg("y"), pybind11::arg("up"),
-        pybind11::arg("down"), pybind11::arg("sact"), pybind11::arg("sy"), pybind11::arg("past") = false,
-        "experts_rows of ungated experts with a shared expert of twice their width in the same launches; False: nothing done");
+        pybind11::arg("wd"), pybind11::arg("limit"), pybind11::arg("up"), pybind11::arg("down"), pybind11::arg("past") = false,
+        "experts_rows of ungated experts and a shared expert of twice their width in the same launches, or None");
   m.def("experts_grouped", &experts_grouped, "gated experts of pairs grouped by expert (MFMA tiles)");
   m.def("gated_rows", &gated_rows, "act(g)·u of packed [g | u] rows");
   m.def("gelu_rows", &gelu_rows, "gelu (erf form) in place");

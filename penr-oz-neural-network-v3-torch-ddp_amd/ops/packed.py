@@ -509,14 +509,10 @@ def experts_beside_shared(h: Tensor, ids: Tensor, w: dict, kind: int, limit: flo
                           experts_past: bool = False) -> tuple[Tensor, Tensor]:
     """:func:`experts` and :func:`gelu_mlp` of a shared expert on the same rows, in the same launches where there are kernels for that
     (``experts_rows_shared`` in csrc/kernels/experts.hip)."""
-    if (kind == UNGATED and h.shape[0] <= 16 and h.dtype == torch.bfloat16 and use_kernels(h) and h.shape[1] % 32 == 0
-            and ids.numel() <= EXPERT_ROWS_MAX_PAIRS):
-        (P, C), F, S = (ids.numel(), h.shape[1]), w["down"].shape[2], shared["up"].shape[0]
-        act, y, hidden, out = (torch.empty(n, m, dtype=h.dtype, device=h.device)
-                               for n, m in ((P, F), (P, C), (h.shape[0], S), (h.shape[0], C)))
-        if kernels().experts_rows_shared(h, ids, w["gu"], w["down"], float(limit), act, y, shared["up"], shared["down"], hidden, out,
-                                         experts_past):
-            return y, out
+    if kind == UNGATED and h.shape[0] <= 16 and h.dtype == torch.bfloat16 and use_kernels(h):
+        both = kernels().experts_rows_shared(h, ids, w["gu"], w["down"], float(limit), shared["up"], shared["down"], experts_past)
+        if both is not None:
+            return both
     return experts(h, ids, w, kind, limit, experts_past), gelu_mlp(h, **shared, past=past)
 
 

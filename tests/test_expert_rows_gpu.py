@@ -56,10 +56,37 @@ def test_shared_expert_beside(N, E, top, C, F, S):
     u, d = ((torch.randn(E, *s) * s[1] ** -0.5).bfloat16().to(DEV) for s in ((F, C), (C, F)))
     su, sd = ((torch.randn(*s) * s[1] ** -0.5).bfloat16().to(DEV) for s in ((S, C), (C, S)))
     w = P.pack_experts(None, u, d)
+    both = P.kernels().experts_rows_shared(h, ids, w["gu"], w["down"], 0.0, su, sd)
+    assert (both is not None) == (N <= 16 and S == 2 * F and F <= 1024 and C % 256 == 0)
     y, out = P.experts_beside_shared(h, ids, w, P.UNGATED, 0.0, {"up": su, "down": sd})
+    if both is not None:
+        assert torch.equal(y, both[0]) and torch.equal(out, both[1])
     assert torch.equal(y, P.experts(h, ids, w, P.UNGATED, 0.0))
     pre = h.double() @ su.double().t()
     a = torch.nn.functional.gelu(pre)
     # the hidden row is rounded to bf16 before (|gelu'| < 1.2) and after the activation, and the result: 2^-9 each
     tol = 2.0 ** -9 * (1.2 * pre.abs() + a.abs()) @ sd.double().abs().t() + 2.0 ** -8 * (a @ sd.double().t()).abs() + 1e-5
     assert torch.all((out.double() - a @ sd.double().t()).abs() <= tol)
+
+
+@pytest.mark.parametrize("N,C,F,S", [(16, 512, 256, 768), (4, 512, 256, 256), (17, 512, 256, 512), (2, 288, 96, 192)])
+def test_refused_shared_expert_allocates_nothing(N, C, F, S):
+    """Where the shared expert keeps its own launches, a step allocates what those do."""
+    ids = _chosen(N, 8, 2, 8).int().to(DEV)
+    r = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=DEV)
+    h, w, shared = r(N, C), {"gu": r(8, F, C), "down": r(8, C, F)}, {"up": r(S, C), "down": r(C, S)}
+    count = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+
+    def both():
+        return P.experts_beside_shared(h, ids, w, P.UNGATED, 0.0, shared)
+
+    def alone():
+        return P.experts(h, ids, w, P.UNGATED, 0.0), P.gelu_mlp(h, **shared)
+
+    used = []
+    for f in (both, alone, both, alone):
+        n = count()
+        out = f()
+        used.append(count() - n)
+        del out
+    assert used[2] == used[3]
