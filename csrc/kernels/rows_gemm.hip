@@ -201,7 +201,7 @@ static void rg_launch(int tile, bool in_order, const torch::Tensor& x, const tor
   // past: nothing holds the weights from one call to the next (past_caches, ops/gemm.py). Of 16 MB and more, each read by one workgroup,
   // they pass the caches then, which keep the smaller ones of a decode step. us, from memory, kept / not: 16 x 8192 x 2048 9.1 / 8.1, 16 x
   // 7232 x 2048 8.3 / 7.6, 16 x 12288 x 2048 14.0 / 12.8, 16 x 32768 x 1024 16.7 / 13.8; of 4 to 8 MB 2 % or nothing. Zozenex large, 16 rows,
-  // 32 tokens 46.4 / 44.8 ms (with the tile below). Weights that the caches hold come from there sooner: 32 x 8192 x 2048 14.9 / 19.7, 32 x 4096 x
+  // 32 tokens 46.4 / 44.8 ms (with rows_gemm_low's tile). Weights that the caches hold come from there sooner: 32 x 8192 x 2048 14.9 / 19.7, 32 x 4096 x
   // 2048, 117 MB in all, 6.6 / 7.6, 9 x 32768 x 2048 26.6 / 29.6.
   const bool once = past && N * K >= (int64_t)8 << 20;
   auto launch = [&](auto kern, auto kern_once, int threads, int lds, int TM, int TN, auto* o) {
@@ -215,8 +215,6 @@ static void rg_launch(int tile, bool in_order, const torch::Tensor& x, const tor
 #define PENROZ_RG(FM, FN, WM, WN, WK, KS, NB)                                                                    \
   launch(rows_gemm_kernel<FM, FN, WM, WN, WK, KS, NB, false, OUT>, rows_gemm_kernel<FM, FN, WM, WN, WK, KS, NB, true, OUT>, \
          64 * WM * WN * WK, NB * WK * KS * 128 * 16 * (FM * WM + FN * WN), 16 * FM * WM, 16 * FN * WN, o)
-  // Tile 5 of up to 16 rows is 16×64, columns split, two workgroups to a CU and all of them at once: 64×128 brings 64 rows of x where
-  // 16 are there, on one CU each. us, both past the caches: 16 x 32768 x 2048 33.7 / 26.8; 1024 columns are the other's (13.8 / 14.5).
   auto typed = [&](auto* o) {
     using OUT = std::remove_pointer_t<decltype(o)>;
     if (tile == 6) PENROZ_RG(1, 1, 1, 1, 4, 1, 6);
@@ -226,7 +224,7 @@ static void rg_launch(int tile, bool in_order, const torch::Tensor& x, const tor
     else if (tile == 2) PENROZ_RG(2, 4, 1, 1, 4, 1, 3);
     else if (tile == 3) PENROZ_RG(2, 2, 2, 2, 1, 2, 4);
     else if (tile == 4) PENROZ_RG(2, 2, 2, 2, 1, 2, 2);
-    else if (!in_order && M <= 16 && K > 1024 && N <= 32768) PENROZ_RG(1, 4, 1, 1, 4, 1, 2);
+    else if (!in_order && rows_gemm_low(M, N, K)) PENROZ_RG(1, 4, 1, 1, 4, 1, 2);
     else PENROZ_RG(2, 4, 2, 2, 1, 1, 3);
   };
 #undef PENROZ_RG
