@@ -134,9 +134,9 @@ inline int plan_wgrad_group(const int* M, const int* N, int n, int K, int n_cu, 
 //     1152 8.0 / 9.6, but 400 x 2048 x 2048 11.9 / 11.0 and 1024 x 576 x 2048 11.9 / 10.5, at a fifth of its host time
 //   * 4 and 5 only for K <= 1024, where their shorter rings do not wait: 512 x 2304 x 768 7.7 (4) / 8.5, 1024 x 3072 x 768
 //     11.2 (5) / 11.4, 700 x 4096 x 1024 12.6 (5) / 11.8 (again a fifth of the host time), 2048 x 3072 x 768 18 (5) / 15.7
-//   * 5 of up to 64 rows also to K = 2048: 64 x 32768 x 2048 35; up to 16 rows by way of rows_gemm_low's tile, which skinny_gemm beats
-//     below 5 rows and, up to 8, below 1280 columns (rows_gemm_low)
-inline bool rows_gemm_low(int64_t M, int64_t N, int64_t K);
+//   * 5 of up to 64 rows also to K = 2048: 64 x 32768 x 2048 35. Up to 8 rows those stay with skinny_gemm, so that the results of such
+//     steps, a prompt of 8 sequences among them, keep their bits; rows_gemm_low's tile would be faster (5 x 32768 x 2048: skinny_gemm
+//     32.0, 64×128 36.5, 16×64 27.1)
 inline int rows_gemm_plan(int64_t M, int64_t N, int64_t K, bool in_order) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 8 != 0 || M > 1 << 20 || N > 1 << 20 || K > 1 << 20) return 0;
   auto tiles = [&](int64_t tm, int64_t tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
@@ -145,8 +145,7 @@ inline int rows_gemm_plan(int64_t M, int64_t N, int64_t K, bool in_order) {
   if (!in_order && tiles(32, 64) <= 256) return 2;
   if (tiles(64, 64) <= 256 && K <= 2048) return 3;
   if (tiles(64, 64) <= 512 && K <= 1024) return 4;
-  const bool low = !in_order && M > 4 && K >= 1280 && rows_gemm_low(M, N, K);
-  if ((tiles(64, 128) <= 384 && K <= 1024) || (M <= 64 && tiles(64, 128) <= 512 && K <= (M > 8 || low ? 2048 : 1024))) return 5;
+  if ((tiles(64, 128) <= 384 && K <= 1024) || (M <= 64 && tiles(64, 128) <= 512 && K <= (M > 8 ? 2048 : 1024))) return 5;
   return 0;
 }
 
@@ -159,9 +158,9 @@ inline bool rows_gemm_narrow(int64_t M, int64_t N) { return ((M + 31) / 32) * ((
 // Tile 5 of up to 16 rows, columns split, is 16×64, two workgroups to a CU and all of them at once: 64×128 brings 64 rows of x where 16
 // are there, on one CU each. us, weights past the caches, 64×128 / 16×64, 16 rows: 16400 x 1152 13.7 / 11.8, 2048 23.9 / 17.6; 24576 x
 // 1280 17.0 / 15.1, 2048 26.1 / 21.2; 32768 x 1152 15.9 / 15.8, 1536 20.4 / 19.1, 2048 33.1 / 26.8; but 32768 x 1024 14.6 / 14.7 and 50304 x
-// 768 17.0 / 17.9, more than one round. (Narrower outputs of 1024 columns and fewer would gain too: 16400 x 1024 12.6 / 10.1.) Of 5 and 8
-// rows, skinny_gemm / 16×64: 16400 x 1280 17.8, 19.1 / 12.4, 2048 18.8, 19.8 / 17.5; 32768 x 1280 28.8, 30.9 / 16.6, 2048 32.0, 34.6 / 27.2;
-// but 16400 x 1056 10.4, 11.0 / 12.4.
+// 768 17.0 / 17.9, more than one round. (Narrower outputs of 1024 columns and fewer would gain too: 16400 x 1024 12.6 / 10.1.) 5 and 8 rows,
+// skinny_gemm / 16×64: 16400 x 1280 17.8, 19.1 / 12.4, 2048 18.8, 19.8 / 17.5; 32768 x 1280 28.8, 30.9 / 16.6, 2048 32.0, 34.6 / 27.2; but
+// 16400 x 1056 10.4, 11.0 / 12.4.
 inline bool rows_gemm_low(int64_t M, int64_t N, int64_t K) { return M <= 16 && K > 1024 && N <= 32768; }
 
 // Slices of the deterministic column reduction (reduce.h): ~sqrt(G) balances its two steps.

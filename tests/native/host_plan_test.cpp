@@ -103,7 +103,7 @@ int main() {
           const int64_t tm[] = {1, 32, 32, 64, 64, 64, 16}, tn[] = {1, 32, 64, 64, 64, 128, 16};
           if (t) EXPECT(((m + tm[t] - 1) / tm[t]) * ((n + tn[t] - 1) / tn[t]) <= 512);
         }
-  // wide outputs of 5 to 16 rows: the low tile in one round of 512 workgroups, from 9 rows on beyond 1024 columns, below from 1280 on
+  // wide outputs of 9 to 16 rows of more than 1024 columns: the low tile in one round of 512 workgroups
   for (int64_t m : {4, 5, 8, 9, 16, 17, 64})
     for (int64_t n : {16384, 16385, 32768, 32769, 65536, 65537})
       for (int64_t k : {1024, 1032, 1272, 1280, 2048, 2056}) {
@@ -111,9 +111,9 @@ int main() {
         EXPECT(low == (m <= 16 && n <= 32768 && k > 1024));
         if (low) EXPECT((n + 63) / 64 <= 512);
         if (n == 16384 || k == 1024) continue;
-        const int want = k > 2048 || n > 65536 || m < 5 ? 0 : m > 8 ? 5 : n <= 32768 && k >= 1280 ? 5 : 0;
+        const int want = k > 2048 || n > 65536 || m < 9 ? 0 : 5;
         EXPECT(penroz::rows_gemm_plan(m, n, k, false) == want);
-        EXPECT(penroz::rows_gemm_plan(m, n, k, true) == (m > 8 ? want : 0));
+        EXPECT(penroz::rows_gemm_plan(m, n, k, true) == want);
       }
   std::printf("host_plan_test: %s (%d failures)\n", fails ? "FAILED" : "ok", fails);
   return fails ? 1 : 0;

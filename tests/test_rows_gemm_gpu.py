@@ -17,10 +17,9 @@ def test_rows_gemm_rule(M, N, K, tile):
 
 
 @pytest.mark.skipif(not _ext.available("penroz_serve"), reason="HIP extension not built")
-@pytest.mark.parametrize("M,N,K,tile", [(4, 32768, 2048, 0), (5, 32768, 2048, 5), (8, 32768, 2048, 5), (9, 32768, 2048, 5),
-                                        (8, 32768, 1272, 0), (9, 32768, 1272, 5), (8, 32776, 2048, 0), (5, 50304, 768, 5)])
+@pytest.mark.parametrize("M,N,K,tile", [(5, 32768, 2048, 0), (8, 32768, 2048, 0), (9, 32768, 2048, 5), (5, 50304, 768, 5)])
 def test_wide_outputs_of_few_rows(M, N, K, tile):
-    """Up to 8 rows of more than 1024 columns skinny_gemm is faster below 1280 columns, and beyond the low tile's one round."""
+    """Up to 8 rows of more than 1024 columns stay with skinny_gemm."""
     assert _ext.kernels().rows_gemm_tile(M, N, K) == tile
 
 
@@ -166,7 +165,7 @@ def test_gelu_is_the_erf_form(M, N):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(5, 30001, 1280), (8, 32768, 2040), (9, 32768, 1032), (16, 30001, 1280), (13, 32768, 2048), (16, 17000, 1992), (16, 8192, 1032),
+@pytest.mark.parametrize("M,N,K", [(9, 32768, 1032), (16, 30001, 1280), (13, 32768, 2048), (16, 17000, 1992), (16, 8192, 1032),
                                    (64, 50304, 192), (64, 9001, 1024), (33, 9000, 1024)])
 def test_large_weights_of_few_rows(M, N, K):
     """Outputs of up to 16 rows in tiles of 16 x 64, and large weights in other tiles: ragged rows, columns and stages."""
