@@ -46,6 +46,7 @@ def test_either_side(kind, E, C, F, N, top):
 
 
 @pytest.mark.gpu
+@torch.inference_mode()  # (as decoders capture; torch's generator state of a process is of the first capture's mode)
 def test_tiles_in_a_captured_step():
     """What was a captured step of the few-pairs kernel is one of the sort and the tiles: every replay on new rows and choices."""
     E, C, F, N, top = 8, 2048, 800, 128, 2

@@ -523,6 +523,7 @@ def test_upload_is_no_part_of_a_graph(monkeypatch):
 
 
 @pytest.mark.gpu
+@torch.inference_mode()  # (as decoders capture; torch's generator state of a process is of the first capture's mode)
 def test_upload_refused_under_capture():
     dev = torch.device("cuda")
     x = P.upload([3, 4], torch.int64, dev)
