@@ -537,18 +537,20 @@ def experts(h: Tensor, ids: Tensor, w: dict, kind: int, limit: float, past: bool
         K, a = kernels(), (h, ids, w["gu"], w["down"], kind, float(limit), act, y)
         if h.dtype != torch.bfloat16 or C % 32:
             K.experts_plain(*a)
-        elif few_pairs(P, w):
-            K.experts_rows(*a, past)
         else:
             i32 = dict(dtype=torch.int32, device=h.device)
-            top, E = ids.shape[1], w["gu"].shape[0]
-            # the kernel's 32-bit byte offsets bound the rows of one call
-            rows = max(1, (1 << 31) // max(C, top * F) - 1)
+            top, E, few = ids.shape[1], w["gu"].shape[0], few_pairs(P, w)
+            # the kernels' 32-bit byte offsets bound the rows of one call
+            rows = max(1, (1 << 31) // max(C, top * F, 1) - 1)
             for r in range(0, h.shape[0], rows):
                 n = min(rows, h.shape[0] - r)
-                p = slice(r * top, (r + n) * top)
-                K.experts_grouped(h[r:r + n], ids[r:r + n], *a[2:6], act[p], y[p], torch.empty(n * top, **i32),
-                                  torch.empty(1 + 3 * (n * top // 128 + E), **i32))
+                if n < h.shape[0]:
+                    p = slice(r * top, (r + n) * top)
+                    a = (h[r:r + n], ids[r:r + n], *a[2:6], act[p], y[p])
+                if few:
+                    K.experts_rows(*a, past)
+                else:
+                    K.experts_grouped(*a, torch.empty(n * top, **i32), torch.empty(1 + 3 * (n * top // 128 + E), **i32))
         return y
     y = torch.empty(P, C, dtype=h.dtype)
     flat, top = ids.reshape(-1).long(), ids.shape[1]

@@ -67,3 +67,44 @@ def test_tiles_in_a_captured_step():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, P.experts(h, ids, w, P.UNGATED, 0.0))
+
+
+class _Kernels:
+    """Takes the kernels' calls, and gives each output row its place's number."""
+
+    def __init__(self):
+        self.calls, self.rows = [], 0
+
+    def experts_rows(self, h, ids, gu, down, kind, limit, act, y, past):
+        self.calls.append((h.numel(), act.numel()))
+        assert ids.shape[0] == h.shape[0] and act.shape[0] == y.shape[0] == ids.numel() and past
+        self.rows += y.shape[0]
+
+
+@pytest.mark.parametrize("N,top,C,F,calls", [(16, 6, 2048, 1024, 1), (100, 2, 32, (1 << 24) - 32, 2), (64, 1, 32, 1 << 25, 2),
+                                             (127, 1, 1 << 24, 32, 1), (128, 1, 1 << 24, 32, 2), (3, 2, 32, (1 << 30) - 32, 3)])
+def test_few_pairs_within_32_bit_offsets(monkeypatch, N, top, C, F, calls):
+    """One call where the input rows lie within them, more of fewer tokens where not."""
+    K = _Kernels()
+    monkeypatch.setattr(P, "kernels", lambda: K)
+    monkeypatch.setattr(P, "use_kernels", lambda h: True)
+    t = lambda *s, dtype=torch.bfloat16: torch.empty(*s, dtype=dtype, device="meta")
+    w = {"gu": t(8, F, C), "down": t(8, C, F)}
+    assert P.few_pairs(N * top, w)
+    P.experts(t(N, C), t(N, top, dtype=torch.int32), w, P.UNGATED, 0.0, True)
+    assert K.rows == N * top and len(K.calls) == calls and max(max(c) for c in K.calls) < 1 << 31
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("C,F", [(32, (1 << 24) + (1 << 15)), ((1 << 24) + (1 << 15), 32)])
+def test_rows_past_32_bit_offsets(C, F):
+    """Input or hidden rows of 4 GiB and more: the last pairs, of another expert than the first, have the bits that they have alone."""
+    N = 128
+    ids = (torch.arange(N, device=DEV) >= N // 2).int().view(N, 1)
+    g = torch.Generator(device=DEV).manual_seed(C)
+    r = lambda *s, scale: torch.empty(*s, dtype=torch.bfloat16, device=DEV).normal_(0, scale, generator=g)
+    h, w = r(N, C, scale=1.0), {"gu": r(2, F, C, scale=C ** -0.5), "down": r(2, C, F, scale=F ** -0.5)}
+    assert P.few_pairs(N, w)
+    y = P.experts(h, ids, w, P.UNGATED, 0.0)
+    last = P.experts(h[-4:], ids[-4:], w, P.UNGATED, 0.0)
+    assert torch.equal(y[-4:], last) and last.float().std() > 0.1 and not torch.equal(y[:4], last)
