@@ -70,7 +70,7 @@ def test_tiles_in_a_captured_step():
 
 
 class _Kernels:
-    """Takes the kernels' calls, and gives each output row its place's number."""
+    """Notes the elements of each call's input and hidden rows, and counts its pairs."""
 
     def __init__(self):
         self.calls, self.rows = [], 0
